@@ -37,7 +37,8 @@ EXPORTS = ("arm_create", "arm_destroy", "arm_last_error", "arm_domain_violations
            "arm_rollout_backward", "arm_update_params", "arm_set_objective",
            "arm_rollout_param_grads", "arm_conservation3", "arm_upload_h", "arm_download_h",
            "arm_ghost_particles", "arm_ghost_count", "arm_download_ghosts",
-           "arm_set_deposition", "arm_set_deposition_binning", "arm_link_list_static")
+           "arm_set_deposition", "arm_set_deposition_binning", "arm_link_list_static",
+           "arm_download_axes", "arm_download_rates_axes")
 ARM_STATIC_MAX_PARTICLES = 1 << 20  # arm_link_list_static limits (include/armando.h)
 ARM_STATIC_MAX_CELLS = 1 << 20
 
@@ -98,6 +99,8 @@ def load_library(path=LIB_PATH):
         "arm_upload": (C.c_int, [vp, C.c_int, C.c_int, dpn, dpn, dpn, dpn]),
         "arm_download": (C.c_int, [vp, dpn, dpn, dpn, dpn, dpn]),
         "arm_download_rates": (C.c_int, [vp, dpn, dpn, dpn, dpn, dpn]),
+        "arm_download_axes": (C.c_int, [vp, C.POINTER(dpn), C.POINTER(dpn), dpn, dpn, dpn]),
+        "arm_download_rates_axes": (C.c_int, [vp, dpn, C.POINTER(dpn), dpn, C.POINTER(dpn), dpn]),
         "arm_link_list": (C.c_int, [vp, C.POINTER(C.c_int)]),
         "arm_get_pairs": (C.c_int, [vp, C.c_int, C.POINTER(C.c_int), _ip, _ip]),
         "arm_get_cells": (C.c_int, [vp, _ip, _ip, _ip]),
@@ -222,18 +225,21 @@ class Simulation:
         self._check(self.L.arm_time_integration(self.ctx, its0, nsteps))
 
     # ---- data ---------------------------------------------------------------
+    def _columns(self, count):
+        """`count` FP64 arrays of n entries, and their addresses."""
+        cols = [np.empty(self.n) for _ in range(count)]
+        return cols, [_ptr(a) for a in cols]
+
     def state(self):
-        n, d = self.n, self.dim
-        X = np.zeros((n, d))
-        V = np.zeros((n, d))
-        rho = np.zeros(n)
-        p = np.zeros(n)
-        u = np.zeros(n)
-        self._check(self.L.arm_download(self.ctx, _ptr(X), _ptr(V), _ptr(rho), _ptr(p), _ptr(u)))
-        out = dict(rho=rho, p=p, u=u)
+        d = self.dim
+        cols, p = self._columns(2 * d + 3)
+        axes = C.POINTER(C.c_double) * d
+        self._check(self.L.arm_download_axes(self.ctx, axes(*p[:d]), axes(*p[d:2 * d]),
+                                             *p[2 * d:]))
+        out = dict(rho=cols[2 * d], p=cols[2 * d + 1], u=cols[2 * d + 2])
         for a, k in enumerate(self._axes()):
-            out[k] = X[:, a].copy()
-            out["v" + k] = V[:, a].copy()
+            out[k] = cols[a]
+            out["v" + k] = cols[d + a]
         return out
 
     # ---- mirror ghosts (ghost.f) -------------------------------------------
@@ -260,18 +266,15 @@ class Simulation:
                     vy=V[:ng, 1].copy(), rho=rho[:ng], p=p[:ng], u=u[:ng], parent=par[:ng])
 
     def rates(self):
-        n, d = self.n, self.dim
-        dr = np.zeros(n)
-        A = np.zeros((n, d))
-        du = np.zeros(n)
-        W = np.zeros((n, d))
-        dv = np.zeros(n)
-        self._check(self.L.arm_download_rates(self.ctx, _ptr(dr), _ptr(A), _ptr(du), _ptr(W),
-                                              _ptr(dv)))
-        out = dict(drho=dr, du=du, divv=dv)
+        d = self.dim
+        cols, p = self._columns(2 * d + 3)
+        axes = C.POINTER(C.c_double) * d
+        self._check(self.L.arm_download_rates_axes(self.ctx, p[2 * d], axes(*p[:d]), p[2 * d + 1],
+                                                   axes(*p[d:2 * d]), p[2 * d + 2]))
+        out = dict(drho=cols[2 * d], du=cols[2 * d + 1], divv=cols[2 * d + 2])
         for a, k in enumerate(self._axes()):
-            out["a" + k] = A[:, a].copy()
-            out["av" + k] = W[:, a].copy()
+            out["a" + k] = cols[a]
+            out["av" + k] = cols[d + a]
         return out
 
     def pairs(self, cap=None):

@@ -26,6 +26,7 @@
 #include "sph3d.h"
 #include "sph3d_adjoint.h"
 #include "sph_ghost.h"
+#include "sph_output.h"
 
 using namespace arm;
 
@@ -1253,42 +1254,6 @@ template <typename T> int d2h(arm_ctx* c, std::vector<T>& dst, const T* src, int
   return ARM_OK;
 }
 
-template <typename R> int download_t(arm_ctx* c, double* x, double* v, double* rho, double* p,
-                                     double* u) {
-  using R2 = typename V2<R>::type;
-  const int n = c->n;
-  St<R>& A = stA<R>(c);
-  std::vector<int32_t> id;
-  std::vector<double2> xy;
-  std::vector<R2> vv;
-  std::vector<R> rr, pp;
-  std::vector<double> uu;
-  int rc;
-  if ((rc = d2h(c, id, A.id, n))) return rc;
-  if (x && (rc = d2h(c, xy, A.xy, n))) return rc;
-  if (v && (rc = d2h(c, vv, A.v, n))) return rc;
-  if (rho && (rc = d2h(c, rr, A.rho, n))) return rc;
-  if (p && (rc = d2h(c, pp, A.p, n))) return rc;
-  if (u && (rc = d2h(c, uu, A.u, n))) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int s = 0; s < n; ++s) {
-    const int i = id[s];
-    if (i >= c->nb) continue;  // ghosts: arm_download_ghosts
-    if (x) {
-      x[2 * i] = xy[s].x;
-      x[2 * i + 1] = xy[s].y;
-    }
-    if (v) {
-      v[2 * i] = (double)vv[s].x;
-      v[2 * i + 1] = (double)vv[s].y;
-    }
-    if (rho) rho[i] = Layout<R>::f32 ? c->prm.rho0 + (double)rr[s] : (double)rr[s];
-    if (p) p[i] = (double)pp[s];
-    if (u) u[i] = uu[s];
-  }
-  return ARM_OK;
-}
-
 template <typename R> int download_ghosts_t(arm_ctx* c, double* x, double* v, double* rho,
                                             double* p, double* u, int32_t* parent) {
   using R2 = typename V2<R>::type;
@@ -1327,37 +1292,96 @@ template <typename R> int download_ghosts_t(arm_ctx* c, double* x, double* v, do
   return ARM_OK;
 }
 
-template <typename R> int download_rates_t(arm_ctx* c, double* drho, double* dvdt, double* dudt,
-                                           double* av, double* divv) {
-  using R2 = typename V2<R>::type;
-  const int n = c->n;
-  St<R>& A = stA<R>(c);
-  std::vector<int32_t> id;
-  std::vector<R> dr, du, dv;
-  std::vector<R2> aa, ww;
-  int rc;
-  if ((rc = d2h(c, id, A.id, n))) return rc;
-  if (drho && (rc = d2h(c, dr, A.drho, n))) return rc;
-  if (dudt && (rc = d2h(c, du, A.du, n))) return rc;
-  if (divv && (rc = d2h(c, dv, A.divv, n))) return rc;
-  if (dvdt && (rc = d2h(c, aa, A.a, n))) return rc;
-  if (av && (rc = d2h(c, ww, A.av, n))) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int s = 0; s < n; ++s) {
-    const int i = id[s];
-    if (i >= c->nb) continue;  // ghosts carry no rates of their own
-    if (drho) drho[i] = (double)dr[s];
-    if (dudt) dudt[i] = (double)du[s];
-    if (divv) divv[i] = (double)dv[s];
-    if (dvdt) {
-      dvdt[2 * i] = (double)aa[s].x;
-      dvdt[2 * i + 1] = (double)aa[s].y;
-    }
-    if (av) {
-      av[2 * i] = (double)ww[s].x;
-      av[2 * i + 1] = (double)ww[s].y;
-    }
+// ---- state and rates in the original order -----------------------------------
+// A vector field on the host: component a of particle i at p[a][stride i].
+// Interleaved arrays (the x(dim, n) of the C ABI) have stride dim and
+// p[a] = base + a; arrays of one axis each have stride 1.
+struct Axes {
+  double* p[3] = {nullptr, nullptr, nullptr};
+  int stride = 1;
+  bool on() const { return p[0] != nullptr; }
+};
+
+Axes interleaved(double* x, int dim) {
+  Axes a;
+  a.stride = dim;
+  for (int k = 0; x && k < dim; ++k) a.p[k] = x + k;
+  return a;
+}
+
+// Copies the first nb entries of a field, unsorted by its kernel into the
+// device scratch d with the host's layout, to the host.
+int fetch_axes(arm_ctx* c, const Axes& h, const double* d, int dim) {
+  if (!h.on()) return ARM_OK;
+  const size_t nb = (size_t)c->nb;
+  if (h.stride == dim) {
+    HIPCHK(c, hipMemcpyAsync(h.p[0], d, sizeof(double) * nb * dim, hipMemcpyDeviceToHost, c->stream));
+  } else {
+    for (int a = 0; a < dim; ++a)
+      HIPCHK(c, hipMemcpyAsync(h.p[a], d + (size_t)a * nb, sizeof(double) * nb,
+                               hipMemcpyDeviceToHost, c->stream));
   }
+  return ARM_OK;
+}
+
+int fetch(arm_ctx* c, double* h, const double* d) {
+  if (h)
+    HIPCHK(c, hipMemcpyAsync(h, d, sizeof(double) * (size_t)c->nb, hipMemcpyDeviceToHost, c->stream));
+  return ARM_OK;
+}
+
+double* as_double(void* p) { return static_cast<double*>(p); }
+
+// Device scratch of the downloads: arrays of the inactive state buffer, whose
+// contents no later pass reads before it writes them (the next reorder fills
+// that buffer), so a download allocates nothing.  vec[2] hold dim doubles
+// per particle, sc[3] one.
+struct OutScratch {
+  double* vec[2];
+  double* sc[3];
+};
+template <typename R> OutScratch out_scratch(arm_ctx* c) {
+  St<R>& B = stB<R>(c);
+  if constexpr (sizeof(R) == 8)
+    return {{as_double(B.xy), as_double(B.v)}, {B.rho, B.p, B.u}};
+  else
+    return {{as_double(B.xy), as_double(B.tau)}, {as_double(B.v), as_double(B.a), B.u}};
+}
+
+// Unsorts on the device (one kernel writes the asked fields as FP64 in id
+// order) and copies the results straight into the caller's arrays: the 720k
+// dam break's five fields took 8.3 ms of host gathering before.
+template <typename ST>
+int state_out(arm_ctx* c, const ST& S, const OutScratch& o, const Axes& x, const Axes& v,
+              double* rho, double* p, double* u) {
+  const int dim = c->K.dim, apart = (x.on() ? x.stride : v.stride) == 1;
+  hipLaunchKernelGGL(k_state_out<ST>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream, S, c->K,
+                     apart, x.on() ? o.vec[0] : nullptr, v.on() ? o.vec[1] : nullptr,
+                     rho ? o.sc[0] : nullptr, p ? o.sc[1] : nullptr, u ? o.sc[2] : nullptr);
+  HIPCHK(c, hipGetLastError());
+  int rc;
+  if ((rc = fetch_axes(c, x, o.vec[0], dim)) || (rc = fetch_axes(c, v, o.vec[1], dim)) ||
+      (rc = fetch(c, rho, o.sc[0])) || (rc = fetch(c, p, o.sc[1])) || (rc = fetch(c, u, o.sc[2])))
+    return rc;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return ARM_OK;
+}
+
+template <typename ST>
+int rates_out(arm_ctx* c, const ST& S, const OutScratch& o, double* drho, const Axes& a,
+              double* dudt, const Axes& av, double* divv) {
+  const int dim = c->K.dim, apart = (a.on() ? a.stride : av.stride) == 1;
+  hipLaunchKernelGGL(k_rates_out<ST>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream, S, c->K,
+                     apart, drho ? o.sc[0] : nullptr, a.on() ? o.vec[0] : nullptr,
+                     dudt ? o.sc[1] : nullptr, av.on() ? o.vec[1] : nullptr,
+                     divv ? o.sc[2] : nullptr);
+  HIPCHK(c, hipGetLastError());
+  int rc;
+  if ((rc = fetch(c, drho, o.sc[0])) || (rc = fetch_axes(c, a, o.vec[0], dim)) ||
+      (rc = fetch(c, dudt, o.sc[1])) || (rc = fetch_axes(c, av, o.vec[1], dim)) ||
+      (rc = fetch(c, divv, o.sc[2])))
+    return rc;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   return ARM_OK;
 }
 
@@ -1696,77 +1720,30 @@ template <typename R> int upload3_t(arm_ctx* c, const double* x, const double* v
   return check_domain(c);
 }
 
-template <typename R> int download3_t(arm_ctx* c, double* x, double* v, double* rho, double* p,
-                                      double* u) {
-  using R4 = typename V4<R>::type;
-  const int n = c->n;
-  St3<R>& A = st3A<R>(c);
-  std::vector<int32_t> id;
-  std::vector<double4> xyz;
-  std::vector<R4> vv;
-  std::vector<R> rr, pp;
-  std::vector<double> uu;
-  int rc;
-  if ((rc = d2h(c, id, A.id, n))) return rc;
-  if (x && (rc = d2h(c, xyz, A.xyz, n))) return rc;
-  if (v && (rc = d2h(c, vv, A.v, n))) return rc;
-  if (rho && (rc = d2h(c, rr, A.rho, n))) return rc;
-  if (p && (rc = d2h(c, pp, A.p, n))) return rc;
-  if (u && (rc = d2h(c, uu, A.u, n))) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int s = 0; s < n; ++s) {
-    const int i = id[s];
-    if (x) {
-      x[3 * i] = xyz[s].x;
-      x[3 * i + 1] = xyz[s].y;
-      x[3 * i + 2] = xyz[s].z;
-    }
-    if (v) {
-      v[3 * i] = (double)vv[s].x;
-      v[3 * i + 1] = (double)vv[s].y;
-      v[3 * i + 2] = (double)vv[s].z;
-    }
-    if (rho) rho[i] = Layout<R>::f32 ? c->prm.rho0 + (double)rr[s] : (double)rr[s];
-    if (p) p[i] = (double)pp[s];
-    if (u) u[i] = uu[s];
-  }
-  return ARM_OK;
+template <typename R> OutScratch out_scratch3(arm_ctx* c) {
+  St3<R>& B = st3B<R>(c);
+  // the packed records of the force pass are written anew by every one
+  if constexpr (sizeof(R) == 8)
+    return {{as_double(B.xyz), as_double(B.v)}, {B.rho, B.p, B.u}};
+  else
+    return {{as_double(B.xyz), as_double(c->pack3_vq)}, {B.u_min, as_double(B.v), B.u}};
 }
 
-template <typename R> int download_rates3_t(arm_ctx* c, double* drho, double* dvdt, double* dudt,
-                                            double* av, double* divv) {
-  using R4 = typename V4<R>::type;
-  const int n = c->n;
-  St3<R>& A = st3A<R>(c);
-  std::vector<int32_t> id;
-  std::vector<R> dr, du, dv;
-  std::vector<R4> aa, ww;
-  int rc;
-  if ((rc = d2h(c, id, A.id, n))) return rc;
-  if (drho && (rc = d2h(c, dr, A.drho, n))) return rc;
-  if (dudt && (rc = d2h(c, du, A.du, n))) return rc;
-  if (divv && (rc = d2h(c, dv, A.divv, n))) return rc;
-  if (dvdt && (rc = d2h(c, aa, A.a, n))) return rc;
-  if (av && (rc = d2h(c, ww, A.av, n))) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (int s = 0; s < n; ++s) {
-    const int i = id[s];
-    if (i >= c->nb) continue;  // ghosts carry no rates of their own
-    if (drho) drho[i] = (double)dr[s];
-    if (dudt) dudt[i] = (double)du[s];
-    if (divv) divv[i] = (double)dv[s];
-    if (dvdt) {
-      dvdt[3 * i] = (double)aa[s].x;
-      dvdt[3 * i + 1] = (double)aa[s].y;
-      dvdt[3 * i + 2] = (double)aa[s].z;
-    }
-    if (av) {
-      av[3 * i] = (double)ww[s].x;
-      av[3 * i + 1] = (double)ww[s].y;
-      av[3 * i + 2] = (double)ww[s].z;
-    }
-  }
-  return ARM_OK;
+int download(arm_ctx* c, const Axes& x, const Axes& v, double* rho, double* p, double* u) {
+  if (is3d(c))
+    return is32(c) ? state_out(c, c->A3_32, out_scratch3<float>(c), x, v, rho, p, u)
+                   : state_out(c, c->A3_64, out_scratch3<double>(c), x, v, rho, p, u);
+  return is32(c) ? state_out(c, c->A32, out_scratch<float>(c), x, v, rho, p, u)
+                 : state_out(c, c->A64, out_scratch<double>(c), x, v, rho, p, u);
+}
+
+int download_rates(arm_ctx* c, double* drho, const Axes& a, double* dudt, const Axes& av,
+                   double* divv) {
+  if (is3d(c))
+    return is32(c) ? rates_out(c, c->A3_32, out_scratch3<float>(c), drho, a, dudt, av, divv)
+                   : rates_out(c, c->A3_64, out_scratch3<double>(c), drho, a, dudt, av, divv);
+  return is32(c) ? rates_out(c, c->A32, out_scratch<float>(c), drho, a, dudt, av, divv)
+                 : rates_out(c, c->A64, out_scratch<double>(c), drho, a, dudt, av, divv);
 }
 
 template <typename R> int conservation3_t(arm_ctx* c, double out[6]) {
@@ -2378,16 +2355,43 @@ int arm_upload(arm_ctx* c, int np, int nv, const double* x, const double* v, con
 int arm_download(arm_ctx* c, double* x, double* v, double* rho, double* p, double* u) {
   if (!c) return ARM_ERR_ARG;
   if (!c->loaded) return fail(c, ARM_ERR_STATE, "no state uploaded");
-  if (is3d(c)) return DISPATCH(c, download3_t)(c, x, v, rho, p, u);
-  return DISPATCH(c, download_t)(c, x, v, rho, p, u);
+  const int d = c->K.dim;
+  return download(c, interleaved(x, d), interleaved(v, d), rho, p, u);
 }
 
 int arm_download_rates(arm_ctx* c, double* drho, double* dvdt, double* dudt, double* av,
                        double* divv) {
   if (!c) return ARM_ERR_ARG;
   if (!c->loaded) return fail(c, ARM_ERR_STATE, "no state uploaded");
-  if (is3d(c)) return DISPATCH(c, download_rates3_t)(c, drho, dvdt, dudt, av, divv);
-  return DISPATCH(c, download_rates_t)(c, drho, dvdt, dudt, av, divv);
+  const int d = c->K.dim;
+  return download_rates(c, drho, interleaved(dvdt, d), dudt, interleaved(av, d), divv);
+}
+
+// one array per axis, for bindings that keep them so (all of a field's axes or none)
+int arm_download_axes(arm_ctx* c, double* const* x, double* const* v, double* rho, double* p,
+                      double* u) {
+  if (!c) return ARM_ERR_ARG;
+  if (!c->loaded) return fail(c, ARM_ERR_STATE, "no state uploaded");
+  Axes ax, av;
+  for (int k = 0; k < c->K.dim; ++k) {
+    ax.p[k] = x ? x[k] : nullptr;
+    av.p[k] = v ? v[k] : nullptr;
+    if ((x && !x[k]) || (v && !v[k])) return fail(c, ARM_ERR_ARG, "null axis %d", k);
+  }
+  return download(c, ax, av, rho, p, u);
+}
+
+int arm_download_rates_axes(arm_ctx* c, double* drho, double* const* dvdt, double* dudt,
+                            double* const* av, double* divv) {
+  if (!c) return ARM_ERR_ARG;
+  if (!c->loaded) return fail(c, ARM_ERR_STATE, "no state uploaded");
+  Axes aa, ax;
+  for (int k = 0; k < c->K.dim; ++k) {
+    aa.p[k] = dvdt ? dvdt[k] : nullptr;
+    ax.p[k] = av ? av[k] : nullptr;
+    if ((dvdt && !dvdt[k]) || (av && !av[k])) return fail(c, ARM_ERR_ARG, "null axis %d", k);
+  }
+  return download_rates(c, drho, aa, dudt, ax, divv);
 }
 
 int arm_upload_h(arm_ctx* c, const double* h) {

@@ -153,6 +153,13 @@ int arm_download(arm_ctx* ctx, double* x, double* v, double* rho, double* p, dou
 int arm_download_rates(arm_ctx* ctx, double* drho, double* dvdt, double* dudt, double* av,
                        double* divv);
 
+/* arm_download and arm_download_rates with the axes apart: x[k], v[k], dvdt[k]
+   and av[k] (k < dim) receive component k, n entries each. */
+int arm_download_axes(arm_ctx* ctx, double* const* x, double* const* v, double* rho, double* p,
+                      double* u);
+int arm_download_rates_axes(arm_ctx* ctx, double* drho, double* const* dvdt, double* dudt,
+                            double* const* av, double* divv);
+
 /* Per-particle smoothing lengths h(n) in the original order (sle != 0), the
    reference's h array [CERNsource/time_integration.f:62]: set after
    arm_upload, read back after steps. */
