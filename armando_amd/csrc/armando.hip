@@ -84,6 +84,7 @@ struct arm_ctx {
   St3<double> A3_64{}, B3_64{};
   St3<float> A3_32{}, B3_32{};
   uint32_t* nbm3 = nullptr;  // 3D neighbour masks (M3_TOTAL words per particle)
+  Mask3 mask3{};             // where the current step's masks lie: nbm3, or a tape's own
   void* pack3_vq = nullptr;  // 3D force pass: packed neighbour records (Pack3)
   void* d_cd = nullptr;      // ARM_CONTACT: contact displacement per slot (V2<R>)
   // sort workspace
@@ -1474,7 +1475,7 @@ template <typename R> int link_list3_t(arm_ctx* c) {
 // LDS for few lanes).  Records the neighbour masks for the force pass.
 template <typename R, bool SUM, bool EOS> void launch_density3(arm_ctx* c) {
   hipLaunchKernelGGL((k3_density<R, SUM, EOS>), dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream,
-                     st3A<R>(c), c->K, c->skey, c->cstart, Mask3{c->nbm3, c->cap});
+                     st3A<R>(c), c->K, c->skey, c->cstart, c->mask3);
   c->masks_valid = true;
 }
 
@@ -1501,7 +1502,7 @@ template <typename R> Pack3<R> pack3(arm_ctx* c) {
 }
 
 template <typename R, bool P, bool AV, bool AH, bool XS> void launch_force3(arm_ctx* c) {
-  const Mask3 m{c->masks_valid ? c->nbm3 : nullptr, c->cap};
+  const Mask3 m{c->masks_valid ? c->mask3.w : nullptr, c->mask3.stride};
   const Pack3<R> pk = pack3<R>(c);
   hipLaunchKernelGGL(k3_force_pack<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream,
                      st3A<R>(c), c->K, pk);
@@ -1591,16 +1592,19 @@ template <typename R> int fused_step3(arm_ctx* c, int its, const StepHooks& hk =
   }
   if (!xs && (rc = zero_av3<R>(c))) return rc;
   c->sorted = true;
+  const Tape3<R>* tape = static_cast<const Tape3<R>*>(hk.tape);
+  c->mask3 = tape ? Mask3{tape->nbm, n} : Mask3{c->nbm3, c->cap};
   if ((rc = density3_t<R>(c, c->prm.density_method, true))) return rc;
   if (hk.jpart)
     hipLaunchKernelGGL(k3_objective<R>, dim3(grid_of(n)), dim3(BLOCK), 0, c->stream, st3A<R>(c),
                        c->K, hk.kind, hk.objmask, hk.jpart);
   if ((rc = force3_t<R>(c, true, c->prm.flags, xs))) return rc;
-  if (hk.tape) {
+  if (tape) {
     const int nb = std::max(grid_of(n), grid_of(c->K.ncell + 1));
     hipLaunchKernelGGL(k3_tape<R>, dim3(nb), dim3(BLOCK), 0, c->stream, st3A<R>(c), c->K, c->skey,
-                       c->cstart, Mask3{c->masks_valid ? c->nbm3 : nullptr, c->cap},
-                       *static_cast<const Tape3<R>*>(hk.tape));
+                       c->cstart, *tape);
+    c->mask3 = Mask3{c->nbm3, c->cap};
+    c->masks_valid = false;
   }
   return corrector3_t<R>(c, its, true);
 }
@@ -1810,7 +1814,7 @@ template <typename R>
 void adj_force3(arm_ctx* c, const Tape3<R>& T, const AdjScratch3<R>& W, double* apart) {
   const int f = c->prm.flags;
   const int code = ((f & ARM_ART_VISC) ? 4 : 0) | ((f & ARM_ART_HEAT) ? 2 : 0) | ((f & ARM_AV_VEL) ? 1 : 0);
-  const dim3 g(grid_of(c->n)), b(BLOCK);
+  const dim3 g((c->n + 63) / 64), b(64);
   switch (code) {
     case 0: hipLaunchKernelGGL((k3_adj_force<R, false, false, false>), g, b, 0, c->stream, T, c->K, W, apart); break;
     case 1: hipLaunchKernelGGL((k3_adj_force<R, false, false, true>), g, b, 0, c->stream, T, c->K, W, apart); break;
@@ -1839,7 +1843,8 @@ int rollout_forward3(arm_ctx* c, int nsteps, int ckpt, const int32_t* obj_ids, i
   R->ckpt = ckpt;
   R->nck = (nsteps + ckpt - 1) / ckpt;
   R->kind = c->objkind;
-  if ((rc = sc.get(&R->obj, n)) || (rc = sc.get(&R->jpart, nb)) || (rc = sc.get(&R->apart, nb)))
+  const int nw = (n + 63) / 64;  // k3_adj_force's partials
+  if ((rc = sc.get(&R->obj, n)) || (rc = sc.get(&R->jpart, nb)) || (rc = sc.get(&R->apart, nw)))
     return rc;
   {
     std::vector<uint8_t> h(n, 0);
@@ -1866,11 +1871,11 @@ int rollout_forward3(arm_ctx* c, int nsteps, int ckpt, const int32_t* obj_ids, i
   for (double** q : lf)
     if ((rc = sc.get(q, n))) return rc;
   AdjScratch3<Rf>& W = Ar.W;
-  Rf** wf[] = {&W.lax, &W.lay, &W.laz, &W.ldrho, &W.ldu, &W.lavx, &W.lavy, &W.lavz,
-               &W.lp,  &W.lQ,  &W.lA,  &W.lpsi,  &W.lS,  &W.lrhoh, &W.lu, &W.lvx,
-               &W.lvy, &W.lvz, &W.lx,  &W.ly,    &W.lz,  &W.lus};
+  Rf** wf[] = {&W.ldrho, &W.lp,  &W.lQ,  &W.lA,  &W.lpsi, &W.lrhoh, &W.lu,
+               &W.lvx,   &W.lvy, &W.lvz, &W.lx,  &W.ly,   &W.lz,    &W.lus};
   for (Rf** q : wf)
     if ((rc = sc.get(q, n))) return rc;
+  if ((rc = sc.get(&W.rec, 2 * (size_t)n)) || (rc = sc.get(&W.frec, 3 * (size_t)n))) return rc;
   hipEvent_t e0, e1;
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
@@ -1910,7 +1915,7 @@ int rollout_forward3(arm_ctx* c, int nsteps, int ckpt, const int32_t* obj_ids, i
 template <typename Rf>
 int rollout_backward3(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0, double* ms) {
   AdjRun* R = c->adj;
-  const int n = c->n, nb = grid_of(n);
+  const int n = c->n, nb = grid_of(n), nw = (n + 63) / 64;
   const int nsteps = R->nsteps, ckpt = R->ckpt, nck = R->nck;
   AdjState3& L = R->L3;
   AdjArrays3<Rf>& Ar = R->arrays3<Rf>();
@@ -1919,7 +1924,7 @@ int rollout_backward3(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0
   double** lf[] = {&L.x,  &L.y,   &L.z,   &L.vx,  &L.vy,    &L.vz,  &L.rho,
                    &L.u,  &L.cax, &L.cay, &L.caz, &L.cdrho, &L.cdu};
   for (double** q : lf) HIPCHK(c, hipMemsetAsync(*q, 0, sizeof(double) * n, c->stream));
-  HIPCHK(c, hipMemsetAsync(R->apart, 0, sizeof(double) * nb, c->stream));
+  HIPCHK(c, hipMemsetAsync(R->apart, 0, sizeof(double) * nw, c->stream));
   hipEvent_t e0, e1;
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
@@ -1941,7 +1946,7 @@ int rollout_backward3(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0
                          L, W, R->obj, R->kind, seed);
       adj_force3<Rf>(c, T, W, R->apart);
       hipLaunchKernelGGL(k3_adj_eos<Rf>, dim3(nb), dim3(BLOCK), 0, c->stream, T, c->K, W);
-      hipLaunchKernelGGL(k3_adj_density<Rf>, dim3(nb), dim3(BLOCK), 0, c->stream, T, c->K, W);
+      hipLaunchKernelGGL(k3_adj_density<Rf>, dim3(nw), dim3(64), 0, c->stream, T, c->K, W);
       hipLaunchKernelGGL(k3_adj_predictor<Rf>, dim3(nb), dim3(BLOCK), 0, c->stream, T, c->K, its,
                          L, W);
       HIPCHK(c, hipGetLastError());
@@ -1957,8 +1962,8 @@ int rollout_backward3(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0
   }
   HIPCHK(c, hipEventRecord(e1, c->stream));
   if ((rc = copy_checkpoint3(c, st3A<Rf>(c), Ar.ck[nck], false))) return rc;
-  std::vector<double> ap(nb), gx(n), gy(n), gz(n);
-  HIPCHK(c, hipMemcpyAsync(ap.data(), R->apart, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
+  std::vector<double> ap(nw), gx(n), gy(n), gz(n);
+  HIPCHK(c, hipMemcpyAsync(ap.data(), R->apart, sizeof(double) * nw, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(gx.data(), L.vx, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(gy.data(), L.vy, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(gz.data(), L.vz, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
@@ -1968,7 +1973,7 @@ int rollout_backward3(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   double As = 0;
-  for (int k = 0; k < nb; ++k) As += ap[k];
+  for (int k = 0; k < nw; ++k) As += ap[k];
   c->grads[ARM_GRAD_ALPHA] = As;
   c->grads[ARM_GRAD_Q0] = 0.0;
   c->grads[ARM_GRAD_VISC] = 0.0;
@@ -2230,6 +2235,7 @@ int arm_create(const arm_params* prm, int capacity, arm_ctx** out) {
     if (!rc) rc = dalloc(c, &c->npieces, 1);
   }
   if (!rc && is3d(c)) rc = dalloc(c, &c->nbm3, (size_t)M3_TOTAL * capacity);
+  if (!rc && is3d(c)) c->mask3 = Mask3{c->nbm3, capacity};
   if (!rc && is3d(c)) {
     const size_t r4 = is32(c) ? sizeof(float4) : sizeof(double4);
     double4* q = nullptr;

@@ -17,7 +17,8 @@
 
 namespace arm {
 
-// one recorded 3D step: the sorted state after the force pass
+// one recorded 3D step: the sorted state after the force pass; the density
+// pass of a recorded step writes its masks here itself
 template <typename R> struct Tape3 {
   using R4 = typename V4<R>::type;
   int32_t* id;
@@ -59,18 +60,37 @@ struct AdjState3 {
   double *cax, *cay, *caz, *cdrho, *cdu;
 };
 
-// per-step scratch in sorted order
+// per-step scratch in sorted order.  What the reverse gathers read of a
+// neighbour lies in two records, written by k3_adj_corrector: for both passes
+//   rec   position (pf / xyz), (v, Q)
+//   frec  (la, A), (lav, psi), (u, ldu, -, -)
+// for the force pass, with Q = 1/rho, A = p/rho and la, lav, ldu the adjoints
+// of the rates; k3_adj_eos puts the density pass's lt = ldrho - lS in the
+// place of Q.  (One record of five vectors for both made the density pass
+// fetch two and a half times its lines: 798 us
+// instead of 538 at 2.2M particles in FP32.)
 template <typename R> struct AdjScratch3 {
-  R *lax, *lay, *laz, *ldrho, *ldu, *lavx, *lavy, *lavz, *lp;
-  R *lQ, *lA, *lpsi, *lS, *lrhoh, *lu, *lvx, *lvy, *lvz, *lx, *ly, *lz;
+  typename V4<R>::type *rec, *frec;  // 2 and 3 vectors per particle
+  R *ldrho, *lp;
+  R *lQ, *lA, *lpsi, *lrhoh, *lu, *lvx, *lvy, *lvz, *lx, *ly, *lz;
   R* lus;
 };
+
+__device__ __forceinline__ float4 tape_rec3(const Tape3<float>& T, int t) { return T.pf[t]; }
+__device__ __forceinline__ double4 tape_rec3(const Tape3<double>& T, int t) { return T.xyz[t]; }
+
+// 1/x: the FP32 form's from the hardware's reciprocal (1 ulp) and one Newton
+// step, which rounds it as well as a division in a third of the instructions.
+__device__ __forceinline__ double rcp_n(double x) { return 1.0 / x; }
+__device__ __forceinline__ float rcp_n(float x) {
+  const float y = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, y, 1.f), y, y);
+}
 
 template <typename R>
 __global__ __launch_bounds__(BLOCK) void k3_tape(St3<R> S, KParams K,
                                                  const uint32_t* __restrict__ skey,
-                                                 const int* __restrict__ cstart, Mask3 nbm,
-                                                 Tape3<R> T) {
+                                                 const int* __restrict__ cstart, Tape3<R> T) {
   const int t = blockIdx.x * BLOCK + threadIdx.x;
   const int stride = gridDim.x * BLOCK;
   for (int c = t; c <= K.ncell; c += stride) T.cstart[c] = cstart[c];
@@ -93,36 +113,53 @@ __global__ __launch_bounds__(BLOCK) void k3_tape(St3<R> S, KParams K,
   T.v_min[t] = S.v_min[t];
   T.flag[t] = S.flag[t];
   T.skey[t] = skey[t];
-  for (int q = 0; q < M3_TOTAL; ++q)
-    T.nbm[(size_t)q * K.n + t] = nbm.w ? nbm.get(q, t) : 0u;
 }
+
+// The lane columns of a wavefront's walk over its mask words.
+struct WalkLds3 {
+  uint32_t w[M3_OK][64];
+  int t0[9][64];
+};
 
 // Calls visit(l, uy, uz) for every neighbour l of particle k of the taped
 // step, in the forward's order: from the recorded masks when they are
-// complete, else by testing the candidates again.
+// complete, in one loop over the set bits of all 27 words (a wavefront runs
+// for its longest lane's neighbour count), else by testing the candidates
+// again.
 template <typename R, typename Visit>
 __device__ __forceinline__ void for_tape_neighbours3(const Tape3<R>& T, const KParams& K, int k,
-                                                     Visit&& visit) {
+                                                     WalkLds3& L, Visit&& visit) {
   const Rows9 rw = rows3_of(K, T.skey[k], T.cstart);
   const size_t st = (size_t)K.n;
+  const int lane = threadIdx.x & 63;
   if (T.nbm[M3_OK * st + k]) {
-    // per row, one loop over the bits of its three words (in word order)
-    for (int row = 0; row < 9; ++row) {
-      const R uy = row_u3<R>(K, 1 - row % 3), uz = row_u3<R>(K, 1 - row / 3);
-      uint32_t m0 = T.nbm[(size_t)(row * M3_WORDS + 0) * st + k];
-      uint32_t m1 = T.nbm[(size_t)(row * M3_WORDS + 1) * st + k];
-      uint32_t m2 = T.nbm[(size_t)(row * M3_WORDS + 2) * st + k];
-      const int t0 = rw.t0[row];
-      while (m0 | m1 | m2) {
-        const bool s0 = m0 != 0u, s1 = !s0 && m1 != 0u;
-        const uint32_t m = s0 ? m0 : (s1 ? m1 : m2);
-        const int l = t0 + (s0 ? 0 : (s1 ? 32 : 64)) + (int)__builtin_ctz(m);
-        const uint32_t rest = m & (m - 1u);
-        m0 = s0 ? rest : m0;
-        m1 = s1 ? rest : m1;
-        m2 = (s0 || s1) ? m2 : rest;
-        visit(l, uy, uz);
+    uint32_t nz = 0u;
+#pragma unroll
+    for (int q = 0; q < M3_OK; ++q) {
+      const uint32_t m = T.nbm[(size_t)q * st + k];
+      L.w[q][lane] = m;
+      nz |= (m != 0u ? 1u : 0u) << q;
+    }
+#pragma unroll
+    for (int q = 0; q < 9; ++q) L.t0[q][lane] = rw.t0[q];
+    uint32_t m = 0u;
+    int tb = 0;
+    R uy = (R)0, uz = (R)0;
+    while (true) {
+      if (m == 0u) {
+        if (nz == 0u) break;
+        const int w = __builtin_ctz(nz);
+        nz &= nz - 1u;
+        m = L.w[w][lane];
+        const int row = (w * 11) >> 5;   // w / 3 for w < 27
+        const int ky = (row * 11) >> 5;  // row / 3 for row < 9
+        uy = row_u3<R>(K, 1 - (row - 3 * ky));
+        uz = row_u3<R>(K, 1 - ky);
+        tb = L.t0[row][lane] + 32 * (w - 3 * row);
       }
+      const int l = tb + (int)__builtin_ctz(m);
+      m &= m - 1u;
+      visit(l, uy, uz);
     }
     return;
   }
@@ -211,120 +248,130 @@ __global__ __launch_bounds__(BLOCK) void k3_adj_corrector(Tape3<R> T, KParams K,
   L.bvz[id] = bvz;
   L.brho[id] = brho;
   L.bu[id] = bu;
-  W.lax[k] = (R)lax;
-  W.lay[k] = (R)lay;
-  W.laz[k] = (R)laz;
   W.ldrho[k] = is_rate(K, id) ? (R)ldrho : (R)0;
-  W.ldu[k] = (R)ldu;
-  W.lavx[k] = (R)lavx;
-  W.lavy[k] = (R)lavy;
-  W.lavz[k] = (R)lavz;
+  {
+    using R4 = typename V4<R>::type;
+    const R Q = (R)1 / dens(K, T.rho[k]);
+    const R4 v = T.v[k];
+    W.rec[2 * (size_t)k] = tape_rec3(T, k);
+    W.rec[2 * (size_t)k + 1] = R4{v.x, v.y, v.z, Q};
+    W.frec[3 * (size_t)k] = R4{(R)lax, (R)lay, (R)laz, T.p[k] * Q};
+    W.frec[3 * (size_t)k + 1] = R4{(R)lavx, (R)lavy, (R)lavz, T.psi[k]};
+    W.frec[3 * (size_t)k + 2] = R4{(R)T.u[k], (R)ldu, (R)0, (R)0};
+  }
   W.lp[k] = (objmask[id] && kind == 0) ? (R)(seed * 2.0 * dt * (double)T.p[k]) : (R)0;
   W.lus[k] = (objmask[id] && kind == 1) ? (R)(seed * 2.0 * dt * T.u[k]) : (R)0;
 }
 
-template <typename R>
-__device__ __forceinline__ void wendland3_q(const KParams& K, R r2, R& q, R& F, R& Wv) {
-  q = fsqrt(r2) * (R)K.invh;
-  const R t = q - (R)2;
-  F = (R)K.C1 * (t * t * t);
-  const R s = (R)1 - (R)0.5 * q;
-  Wv = (R)K.wnorm * (s * s) * (s * s) * ((R)1 + (R)2 * q);
-}
-
 // 2. force-pass adjoint, gathered: particle k (as i) against every
-//    neighbour l (as j); accumulates k's own input adjoints.
+//    neighbour l (as j); accumulates k's own input adjoints.  One wavefront
+//    per workgroup; a neighbour is two records (five vectors) instead of
+//    thirteen scattered loads, and the pair divides by reciprocals.
+//    Bound by VALU issue and the records' latency.  Measured: FP32, 2.2M
+//    particles 2130 -> 1233 us; FP64, 24,874 particles 206 -> 78 us.  Contiguous
+//    shares per XCD: 1384 -> 1233 us.
 template <typename R, bool AV, bool AH, bool XS>
-__global__ __launch_bounds__(BLOCK) void k3_adj_force(Tape3<R> T, KParams K, AdjScratch3<R> W,
-                                                      double* __restrict__ alpha_part) {
-  __shared__ double sh[BLOCK];
+__global__ __launch_bounds__(64) void k3_adj_force(Tape3<R> T, KParams K, AdjScratch3<R> W,
+                                                   double* __restrict__ alpha_part) {
+  __shared__ WalkLds3 L;
   double lal = 0.0;
-  const int k = blockIdx.x * BLOCK + threadIdx.x;
+  const int kb = xcd_block();
+  const int k = kb * 64 + threadIdx.x;
   if (k < K.n) {
-    const R m = (R)K.mass, h = (R)K.h;
-    const auto pk = tape_pos3(T, k);
-    const auto vk = T.v[k];
-    const R Qk = (R)1 / dens(K, T.rho[k]), Ak = T.p[k] * Qk;
-    const R lak[3] = {W.lax[k], W.lay[k], W.laz[k]};
-    const R lavk[3] = {W.lavx[k], W.lavy[k], W.lavz[k]};
-    const R lduk = W.ldu[k];
-    const R psik = T.psi[k], uk = (R)T.u[k];
-    const R c0 = (R)K.c0, al = (R)K.av_alpha, be = (R)K.av_beta;
+    using R4 = typename V4<R>::type;
+    const R m = (R)K.mass, h = (R)K.h, invh = (R)K.invh, C1 = (R)K.C1;
+    const auto pk = pos_of_rec(W.rec[2 * (size_t)k]);
+    const R4 vk = W.rec[2 * (size_t)k + 1];
+    const R4 ak = W.frec[3 * (size_t)k], xk = W.frec[3 * (size_t)k + 1],
+             uk = W.frec[3 * (size_t)k + 2];
+    const R Qk = vk.w, Ak = ak.w, psik = xk.w, lduk = uk.y;
+    const R alc0 = (R)(K.av_alpha * K.c0), be = (R)K.av_beta, c0 = (R)K.c0;
+    const R ave2 = (R)K.av_e2, ahe2 = (R)K.ah_e2;
+    const R em = (R)(K.xsph_eps * K.mass), wn = (R)K.wnorm;
+    const R iq2 = (R)(0.5 / (K.h * K.h)), c3 = (R)(3.0 * K.C1);
+    const bool pa0 = K.pa_sph == 0, se = K.same_e2 != 0;
     R lr_acc[3] = {0, 0, 0}, lv_acc[3] = {0, 0, 0};
     R lQ = 0, lA = 0, lpsi = 0, lu = 0;
-    for_tape_neighbours3<R>(T, K, k, [&](int l, R uy, R uz) {
-        R r[3];
-        const R r2 = delta3(pk, tape_pos3(T, l), K, uy, uz, r[0], r[1], r[2]);
-        R q, F, Wv;
-        wendland3_q(K, r2, q, F, Wv);
-        const auto vl = T.v[l];
-        const R dv[3] = {vk.x - vl.x, vk.y - vl.y, vk.z - vl.z};
-        const R vr = dv[0] * r[0] + dv[1] * r[1] + dv[2] * r[2];
-        const R Ql = (R)1 / dens(K, T.rho[l]), Al = T.p[l] * Ql;
-        const R sQ = Qk + Ql;
-        const R M = (R)2 * Qk * Ql / sQ;
-        R Kc = (K.pa_sph == 0) ? (Ak * Ql + Al * Qk) : (Ak * Qk + Al * Ql);
-        const bool av_on = AV && vr < (R)0;
-        const R einv = (R)1 / (r2 + (R)K.av_e2);
-        const R phi = h * vr * einv;
-        if (av_on) Kc += (be * phi - al * c0) * phi * M;
-        const R G = m * F * Kc;
-        const R Da[3] = {lak[0] - W.lax[l], lak[1] - W.lay[l], lak[2] - W.laz[l]};
-        const R sig = lduk + W.ldu[l];
-        const R lG = -(Da[0] * r[0] + Da[1] * r[1] + Da[2] * r[2]) + (R)0.5 * sig * vr;
-        R lr[3] = {-G * Da[0], -G * Da[1], -G * Da[2]};
-        R lvr = (R)0.5 * sig * G;
-        R ldv[3] = {0, 0, 0};
-        R lF = lG * m * Kc;
-        const R lK = lG * m * F;
-        R lM = 0, lr2 = 0, lW = 0;
-        if (K.pa_sph == 0) {
-          lA += lK * Ql;
-          lQ += lK * Al;
-        } else {
-          lA += lK * Qk;
-          lQ += lK * Ak;
-        }
-        if (av_on) {
-          const R dPi = ((R)2 * be * phi - al * c0) * M;
-          lM += lK * (be * phi - al * c0) * phi;
-          lal += (double)(lK * (-c0 * phi * M));
-          const R lphi = lK * dPi;
-          lvr += lphi * h * einv;
-          lr2 += lphi * (-phi * einv);
-        }
-        if (AH) {
-          const R eh = (R)1 / (r2 + (R)K.ah_e2);
-          const R du_ = uk - (R)T.u[l];
-          const R dl = lduk - W.ldu[l];
-          const R ps = psik + T.psi[l];
-          const R H = m * ps * F * r2 * M * eh;
-          const R lH = dl * du_;
-          lu += dl * H;
-          lpsi += lH * m * F * r2 * M * eh;
-          lF += lH * m * ps * r2 * M * eh;
-          lr2 += lH * m * ps * F * M * (R)K.ah_e2 * eh * eh;
-          lM += lH * m * ps * F * r2 * eh;
-        }
-        if (XS) {
-          const R Dv[3] = {lavk[0] - W.lavx[l], lavk[1] - W.lavy[l], lavk[2] - W.lavz[l]};
-          const R w = (R)K.xsph_eps * m * M * Wv;
-          const R lw = -(Dv[0] * dv[0] + Dv[1] * dv[1] + Dv[2] * dv[2]);
-          for (int c = 0; c < 3; ++c) ldv[c] += -w * Dv[c];
-          lM += lw * (R)K.xsph_eps * m * Wv;
-          lW += lw * (R)K.xsph_eps * m * M;
-        }
-        lQ += lM * (R)2 * Ql * Ql / (sQ * sQ);
+    for_tape_neighbours3<R>(T, K, k, L, [&](int l, R uy, R uz) {
+      const R4* o = W.rec + ((unsigned)l << 1);
+      const R4* f = W.frec + (((unsigned)l << 1) + (unsigned)l);
+      const auto pl = pos_of_rec(o[0]);
+      const R4 vl = o[1], al = f[0], xl = f[1], ul = f[2];
+      R r[3];
+      const R r2 = delta3(pk, pl, K, uy, uz, r[0], r[1], r[2]);
+      const R q = fsqrt(r2) * invh;
+      const R t = q - (R)2;
+      const R t2 = t * t;
+      const R F = C1 * (t2 * t);
+      const R dv[3] = {vk.x - vl.x, vk.y - vl.y, vk.z - vl.z};
+      const R vr = dv[0] * r[0] + dv[1] * r[1] + dv[2] * r[2];
+      const R Ql = vl.w, Al = al.w;
+      const R is = rcp_n(Qk + Ql);
+      const R g2 = (R)2 * Ql * is;  // dM/dQk = g2 Ql/(Qk + Ql)
+      const R M = Qk * g2;
+      R Kc = pa0 ? (Ak * Ql + Al * Qk) : (Ak * Qk + Al * Ql);
+      const R mF = m * F;
+      const R Da[3] = {ak.x - al.x, ak.y - al.y, ak.z - al.z};
+      const R sig = lduk + ul.y;
+      const R lG = -(Da[0] * r[0] + Da[1] * r[1] + Da[2] * r[2]) + (R)0.5 * sig * vr;
+      const R lK = lG * mF;
+      R lM = 0, lr2 = 0, lW = 0, lvr = 0;
+      R einv = 0;
+      if (AV) {
+        einv = rcp_n(r2 + ave2);
+        const bool on = vr < (R)0;
+        const R phi = on ? h * vr * einv : (R)0;  // 0: every term below is 0
+        const R pc = be * phi - alc0;
+        Kc += pc * phi * M;
+        lM += lK * pc * phi;
+        lal += (double)(lK * (-c0 * phi * M));
+        const R lphi = on ? lK * (be * phi + pc) * M : (R)0;
+        lvr += lphi * h * einv;
+        lr2 -= lphi * phi * einv;
+      }
+      const R G = mF * Kc;
+      lvr += (R)0.5 * sig * G;
+      R lF = lG * m * Kc;
+      if (pa0) {
+        lA += lK * Ql;
+        lQ += lK * Al;
+      } else {
+        lA += lK * Qk;
+        lQ += lK * Ak;
+      }
+      if (AH) {
+        const R eh = (AV && se) ? einv : rcp_n(r2 + ahe2);
+        const R dl = lduk - ul.y, ps = psik + xl.w;
+        const R re = r2 * eh;
+        const R mMe = m * M * re;        // H = mMe ps F
+        const R lH = dl * (uk.x - ul.x);
+        const R lHp = lH * ps;
+        lu += dl * ps * (mMe * F);
+        lpsi += lH * (mMe * F);
+        lF += lHp * mMe;
+        lr2 += lHp * (mF * M) * ahe2 * eh * eh;
+        lM += lHp * mF * re;
+      }
+      R ldv[3] = {lvr * r[0], lvr * r[1], lvr * r[2]};
+      if (XS) {
         const R s = (R)1 - (R)0.5 * q;
-        const R lq = lF * (R)3 * (R)K.C1 * (q - (R)2) * (q - (R)2) +
-                     lW * (R)K.wnorm * s * s * s * ((R)-5 * q);
-        lr2 += lq / ((R)2 * h * h * q);
-        for (int c = 0; c < 3; ++c) {
-          ldv[c] += lvr * r[c];
-          lr[c] += lvr * dv[c] + (R)2 * lr2 * r[c];
-          lr_acc[c] += lr[c];
-          lv_acc[c] += ldv[c];
-        }
+        const R s2 = s * s;
+        const R Wv = wn * (s2 * s2) * ((R)1 + (R)2 * q);
+        const R Dv[3] = {xk.x - xl.x, xk.y - xl.y, xk.z - xl.z};
+        const R lw = -em * (Dv[0] * dv[0] + Dv[1] * dv[1] + Dv[2] * dv[2]);
+        const R w = em * M * Wv;
+        for (int c = 0; c < 3; ++c) ldv[c] -= w * Dv[c];
+        lM += lw * Wv;
+        lW = lw * M * wn * (s2 * s) * ((R)-5 * q);
+      }
+      lQ += lM * g2 * Ql * is;
+      const R lq = lF * c3 * t2 + lW;
+      lr2 += lq * iq2 * rcp_n(q);
+      const R r22 = (R)2 * lr2;
+      for (int c = 0; c < 3; ++c) {
+        lr_acc[c] += lvr * dv[c] + r22 * r[c] - G * Da[c];
+        lv_acc[c] += ldv[c];
+      }
     });
     W.lx[k] = lr_acc[0];
     W.ly[k] = lr_acc[1];
@@ -338,13 +385,10 @@ __global__ __launch_bounds__(BLOCK) void k3_adj_force(Tape3<R> T, KParams K, Adj
     W.lu[k] = lu + W.lus[k];
   }
   // each pair is visited from both ends: half of its alpha derivative each
-  sh[threadIdx.x] = 0.5 * lal;
-  __syncthreads();
-  for (int s = BLOCK / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) alpha_part[blockIdx.x] += sh[0];
+  lal *= 0.5;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) lal += __shfl_down(lal, d, 64);
+  if (threadIdx.x == 0) alpha_part[kb] += lal;
 }
 
 // 3. EOS and art_heat coefficient adjoint (per particle)
@@ -359,7 +403,7 @@ __global__ __launch_bounds__(BLOCK) void k3_adj_eos(Tape3<R> T, KParams K, AdjSc
   const R dv = T.divv[k];
   const R dpsi = (dv < (R)0) ? (R)(-2.0 * K.g2h2) : (R)0;
   const R ldv = W.lpsi[k] * dpsi;
-  W.lS[k] = ldv / rho;
+  W.rec[2 * (size_t)k + 1].w = W.ldrho[k] - ldv / rho;  // lt = ldrho - lS
   lrhoe += -ldv * dv / rho;
   R lrhoh = 0;
   if (is_rate(K, T.id[k]) && !(T.flag[k] & 2u)) {
@@ -375,32 +419,36 @@ __global__ __launch_bounds__(BLOCK) void k3_adj_eos(Tape3<R> T, KParams K, AdjSc
 }
 
 // 4. density adjoint, gathered; adds to the position / velocity adjoints
+//    (FP32, 2.2M particles 726 -> 538 us; FP64, 24,874 particles 73 -> 45 us)
 template <typename R>
-__global__ __launch_bounds__(BLOCK) void k3_adj_density(Tape3<R> T, KParams K,
-                                                        AdjScratch3<R> W) {
-  const int k = blockIdx.x * BLOCK + threadIdx.x;
+__global__ __launch_bounds__(64) void k3_adj_density(Tape3<R> T, KParams K, AdjScratch3<R> W) {
+  __shared__ WalkLds3 L;
+  const int k = xcd_block() * 64 + threadIdx.x;
   if (k >= K.n) return;
-  const R m = (R)K.mass, h = (R)K.h;
-  const auto pk = tape_pos3(T, k);
-  const auto vk = T.v[k];
-  const R ltk = W.ldrho[k] - W.lS[k];
+  using R4 = typename V4<R>::type;
+  const R m = (R)K.mass, invh = (R)K.invh, C1 = (R)K.C1;
+  const R c3 = (R)(1.5 * K.C1 / (K.h * K.h)) * m;  // m 3 C1 / (2 h^2)
+  const auto pk = pos_of_rec(W.rec[2 * (size_t)k]);
+  const R4 vk = W.rec[2 * (size_t)k + 1];
   R lr[3] = {0, 0, 0}, lv[3] = {0, 0, 0};
-  for_tape_neighbours3<R>(T, K, k, [&](int l, R uy, R uz) {
-      R r[3];
-      const R r2 = delta3(pk, tape_pos3(T, l), K, uy, uz, r[0], r[1], r[2]);
-      const R lt = ltk + W.ldrho[l] - W.lS[l];
-      R q, F, Wv;
-      wendland3_q(K, r2, q, F, Wv);
-      const auto vl = T.v[l];
-      const R dv[3] = {vk.x - vl.x, vk.y - vl.y, vk.z - vl.z};
-      const R vr = dv[0] * r[0] + dv[1] * r[1] + dv[2] * r[2];
-      const R lvr = lt * m * F;
-      const R lF = lt * m * vr;
-      const R lr2 = lF * (R)3 * (R)K.C1 * (q - (R)2) * (q - (R)2) / ((R)2 * h * h * q);
-      for (int c = 0; c < 3; ++c) {
-        lr[c] += lvr * dv[c] + (R)2 * lr2 * r[c];
-        lv[c] += lvr * r[c];
-      }
+  for_tape_neighbours3<R>(T, K, k, L, [&](int l, R uy, R uz) {
+    const R4* o = W.rec + ((unsigned)l << 1);
+    const auto pl = pos_of_rec(o[0]);
+    const R4 vl = o[1];
+    R r[3];
+    const R r2 = delta3(pk, pl, K, uy, uz, r[0], r[1], r[2]);
+    const R lt = vk.w + vl.w;
+    const R q = fsqrt(r2) * invh;
+    const R t = q - (R)2;
+    const R t2 = t * t;
+    const R dv[3] = {vk.x - vl.x, vk.y - vl.y, vk.z - vl.z};
+    const R vr = dv[0] * r[0] + dv[1] * r[1] + dv[2] * r[2];
+    const R lvr = lt * m * (C1 * (t2 * t));
+    const R r22 = (R)2 * (lt * vr * c3 * t2) * rcp_n(q);
+    for (int c = 0; c < 3; ++c) {
+      lr[c] += lvr * dv[c] + r22 * r[c];
+      lv[c] += lvr * r[c];
+    }
   });
   W.lx[k] += lr[0];
   W.ly[k] += lr[1];
