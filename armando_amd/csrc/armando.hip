@@ -1470,11 +1470,10 @@ template <typename R> int link_list3_t(arm_ctx* c) {
   return check_domain(c);
 }
 
-// 3D density gather (direct: per-particle walks of the nine rows; an
-// LDS-tiled variant measured twice as slow, the 27-cell halo filling the
-// LDS for few lanes).  Records the neighbour masks for the force pass.
+// 3D density gather, one wavefront per workgroup (k3_density).  Records the
+// neighbour masks for the force pass.
 template <typename R, bool SUM, bool EOS> void launch_density3(arm_ctx* c) {
-  hipLaunchKernelGGL((k3_density<R, SUM, EOS>), dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream,
+  hipLaunchKernelGGL((k3_density<R, SUM, EOS>), dim3((c->n + 63) / 64), dim3(64), 0, c->stream,
                      st3A<R>(c), c->K, c->skey, c->cstart, c->mask3);
   c->masks_valid = true;
 }
@@ -2044,6 +2043,14 @@ void set_kparams(KParams& K, const arm_params& P) {
     const double E = u * (2.0 * nmax * P.cell + 4.0 * P.cell + 16.0 * P.h);
     const double b = 2.0 * P.h + 2.0 * E;
     K.pre2f = std::nextafter((float)(b * b * (1.0 + 1e-5)), INFINITY);
+    // pretest3: coordinates relative to the sweep's first cell are at most
+    // L = P3_SPAN + 3 cells along x and 2 along y and z, so |x|^2 is at most
+    // X = (L^2 + 8) cell^2.  Each coordinate is rounded once or twice (u L
+    // cell), which moves r^2 < cell^2 by at most 8 sqrt(3) u L cell^2; the two
+    // norms (three roundings each), the bound's subtraction and the four
+    // products' sum add at most 3 u X each norm and 5 u 4 X: below 64 u X
+    const double X = ((P3_SPAN + 3.0) * (P3_SPAN + 3.0) + 8.0) * P.cell * P.cell;
+    K.pre3f = std::nextafter((float)(K.cut2 * (1.0 + 1e-5) + 64.0 * u * X), INFINITY);
   }
   K.eos = P.eos;
   K.lin_c2 = P.c0 * P.c0;

@@ -273,18 +273,32 @@ __device__ __forceinline__ Rows9 rows3_of(const KParams& K, uint32_t key,
 // ------------------------------------------------------------------------
 // pair arithmetic (the 2D forms with a z component)
 // ------------------------------------------------------------------------
+// ok = false: no neighbour, the sums keep every word.
 template <typename R, bool SUM>
 __device__ __forceinline__ void dens3_pair(const KParams& K, R dx, R dy, R dz, R r2, R dvx,
-                                           R dvy, R dvz, Acc<R>& sum, Acc<R>& rs) {
+                                           R dvy, R dvz, Acc<R>& sum, Acc<R>& rs, bool ok = true) {
+  if constexpr (sizeof(R) == 4) {
+    // m dW.dv = m C1 (q - 2)^3 (dx dvx + dy dvy + dz dvz), m C1 one constant
+    const float q = fsqrt(r2) * K.kf.invh;
+    const float tq = q - 2.f;
+    const float vr = __builtin_fmaf(dvz, dz, __builtin_fmaf(dvy, dy, dvx * dx));
+    sum.add_if(K.kf.mC1 * ((tq * tq) * tq * vr), ok);
+    if (SUM) {
+      const float s = __builtin_fmaf(-0.5f, q, 1.f);
+      const float s2 = s * s;
+      rs.add_if(K.kf.mw * ((s2 * s2) * __builtin_fmaf(2.f, q, 1.f)), ok);
+    }
+    return;
+  }
   const R q = fsqrt(r2) * (R)K.invh;
   const R tq = q - (R)2;
   const R F = (R)K.C1 * (tq * tq * tq);
   const R vcc = fmr(dvz, F * dz, fmr(dvy, F * dy, dvx * (F * dx)));
-  sum.add((R)K.mass * vcc);
+  sum.add_if((R)K.mass * vcc, ok);
   if (SUM) {
     const R s = fmr((R)-0.5, q, (R)1);
     const R s2 = s * s;
-    rs.add((R)K.mass * ((R)K.wnorm * (s2 * s2) * fmr((R)2, q, (R)1)));
+    rs.add_if((R)K.mass * ((R)K.wnorm * (s2 * s2) * fmr((R)2, q, (R)1)), ok);
   }
 }
 
@@ -309,194 +323,322 @@ struct Mask3 {
   }
 };
 
+// ---- neighbour pre-test on the matrix cores ---------------------------------
+// A particle has about 490 candidates in its nine rows, of which 68 are
+// neighbours, so the candidate test dominates a density pass that makes it
+// per lane (92 VALU instructions and eight 16-byte loads per lane for eight
+// candidates).  Squared distances are a contraction:
+//   r^2 = |x_j|^2 - 2 x_j . x_i + |x_i|^2,
+// so a wavefront computes them with v_mfma_f32_16x16x4_f32, 16 candidates by
+// 16 of its particles at a time: A row j = (-2x, -2y, -2z, |x|^2)_j,
+// B column i = (x, y, z, 1)_i, C = |x_i|^2 - bound, and the sign of each
+// result is the test (one v_alignbit per 64 of them collects it).  Positions
+// are FP32 and relative to the wavefront's first cell, and the bound
+// (KParams::pre3f) covers their rounding and the cancellation, so every pair
+// with r < 2h passes; the survivors (about one in a thousand too many) take
+// the exact test in the pair walk.
+//
+// The wavefront's 64 consecutive particles form four tiles of 16; two tiles
+// share a row's staged candidates (in LDS, one record each) but each tests its
+// own union of candidates: the lanes 16 q .. 16 q + 15 of D hold rows 4q .. 4q+3,
+// and row 4q + r of step s is candidate q 4 steps + 4 s + r, so that a lane
+// collects 4 steps consecutive candidates of one particle in one word.  Two
+// permlane32 and two permlane16 swaps then bring a particle's four words to
+// its own lane, which cuts its window [t0, t1) out of them.
+//
+// Bound: VALU issue (7,500 instructions a wavefront, 70 % of the launch; the
+// MFMAs are busy a tenth of it).  Measured, density pass: FP32, 2,236,171-
+// particle dam break 807 -> 612 us against the per-lane pre-test; FP64 (which
+// tested every candidate in FP64), 83,630-particle tank 245 -> 78 us.  A
+// wavefront's 64 particles staging a row at once, with the next row's loads
+// ahead, took more registers and came out no faster (616 and 95 us).
+constexpr int P3_CAP = 160;   // staged records of two tiles in one row (16 bytes each)
+constexpr int P3_TILE = 128;  // candidates of a tile in one row, at most 4 x 32
+constexpr int P3_SPAN = 12;   // cells between the first and last particle of a sweep
+
+using f32x4 = __attribute__((ext_vector_type(4))) float;
+
+// A particle's position relative to the corner of cell (cx0, cy, cz), for a
+// candidate in row k the row's own offset included.
+struct Local3 {
+  float x, y, z;
+};
+__device__ __forceinline__ Local3 local3(const KParams& K, float4 q, int cx0, int, int, int k) {
+  return {__builtin_fmaf(q.w - (float)cx0, K.cellf, q.x), q.y - row_u3<float>(K, 1 - k % 3),
+          q.z - row_u3<float>(K, 1 - k / 3)};
+}
+__device__ __forceinline__ Local3 local3(const KParams& K, double4 q, int cx0, int cy, int cz,
+                                         int) {
+  return {(float)(q.x - (K.ox + (double)cx0 * K.cell)),
+          (float)(q.y - (K.oy + (double)cy * K.cell)),
+          (float)(q.z - (K.oz + (double)cz * K.cell))};
+}
+__device__ __forceinline__ float4 pos_rec3(const St3<float>& S, int i) { return S.pf[i]; }
+__device__ __forceinline__ double4 pos_rec3(const St3<double>& S, int i) { return S.xyz[i]; }
+
+// The 96-bit window [d, d + len) of the four words p of ch bits each
+// (ch a multiple of 4, at most 32; len <= 96).
+__device__ __forceinline__ void window3(const uint32_t* p, int ch, int d, int len, uint32_t* m) {
+  const uint64_t a = (uint64_t)p[0] | ((uint64_t)p[1] << ch);
+  const uint64_t b = (uint64_t)p[2] | ((uint64_t)p[3] << ch);  // from bit 2 ch on
+  uint64_t lo = a | ((b << ch) << ch);
+  uint64_t hi = ch ? b >> (64 - 2 * ch) : 0ull;
+  if (d >= 64) {
+    lo = hi;
+    hi = 0ull;
+    d -= 64;
+  }
+  lo = (lo >> d) | ((hi << 1) << (63 - d));
+  hi = hi >> d;
+  lo &= len >= 64 ? ~0ull : (1ull << len) - 1ull;
+  const int l2 = len - 64;
+  m[0] = (uint32_t)lo;
+  m[1] = (uint32_t)(lo >> 32);
+  m[2] = l2 <= 0 ? 0u : (uint32_t)hi & (l2 >= 32 ? ~0u : (1u << l2) - 1u);
+}
+
+// Mask words lw[3k + q][lane] of the nine rows of every lane with on set (rows
+// of at most 96 candidates), the particle's own bit cleared.  Called by the
+// whole wavefront.  cx, row = cy + cz ny: the lane's cell; rec: LDS for the
+// records staged of a row, P3_CAP and P3_TILE + 16 more that may be read.
+template <typename R>
+__device__ __forceinline__ void pretest3(const St3<R>& S, const KParams& K, int i, bool on, int cx,
+                                         int row, const Rows9& rw, float4* __restrict__ rec,
+                                         uint32_t (*__restrict__ lw)[64]) {
+  const int* t0 = rw.t0;
+  const int* t1 = rw.t1;
+  const int lane = threadIdx.x & 63;
+  const auto own = pos_rec3(S, i);
+  const int ar = (lane & 15) >> 2, ac = lane & 3, ak = lane >> 4;
+  uint64_t todo = __ballot(on);
+  int span = P3_SPAN;
+  while (todo) {
+    // the sweep: lanes of one cell row within span cells of the first (a gap
+    // of empty cells ends it; its rows hold the candidates of what lies between)
+    const int a = __builtin_ctzll(todo);
+    const int row0 = __builtin_amdgcn_readlane(row, a), cx0 = __builtin_amdgcn_readlane(cx, a);
+    const bool in = ((todo >> lane) & 1ull) && row == row0 && cx - cx0 <= span;
+    const uint64_t im = __ballot(in);
+    const int cz = row0 / K.ny, cy = row0 - cz * K.ny;
+    int first[4], last[4];
+#pragma unroll
+    for (int T = 0; T < 4; ++T) {
+      const uint32_t mt = (uint32_t)(im >> (16 * T)) & 0xffffu;
+      first[T] = mt ? 16 * T + __builtin_ctz(mt) : a;
+      last[T] = mt ? 16 * T + 31 - __builtin_clz(mt) : -1;
+    }
+    const Local3 me = local3(K, own, cx0, cy, cz, 4);
+    const float c = __builtin_fmaf(me.x, me.x, __builtin_fmaf(me.y, me.y, me.z * me.z)) - K.pre3f;
+    float B[4];
+    f32x4 C[4];
+#pragma unroll
+    for (int T = 0; T < 4; ++T) {
+      const int src = 16 * T + (lane & 15);
+      const float bx = __shfl(me.x, src, 64), by = __shfl(me.y, src, 64),
+                  bz = __shfl(me.z, src, 64), cc = __shfl(c, src, 64);
+      B[T] = ak == 0 ? bx : (ak == 1 ? by : (ak == 2 ? bz : 1.f));
+      C[T] = f32x4{cc, cc, cc, cc};
+    }
+    bool fits = true;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      uint32_t p[4] = {0u, 0u, 0u, 0u};
+      int u0 = 0, ch = 0;  // of the lane's tile: first candidate, candidates per word
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (last[2 * h] < 0 && last[2 * h + 1] < 0) continue;
+        int at[2], most = 0, U0 = 0x7fffffff, U1 = 0;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int T = 2 * h + e;
+          at[e] = 0;
+          if (last[T] < 0) continue;
+          at[e] = __builtin_amdgcn_readlane(t0[k], first[T]);
+          const int end = __builtin_amdgcn_readlane(t1[k], last[T]);
+          most = max(most, end - at[e]);
+          U0 = min(U0, at[e]);
+          U1 = max(U1, end);
+        }
+        fits = fits && U1 - U0 <= P3_CAP && most <= P3_TILE;
+        if (!fits) break;
+        const int steps = (most + 15) >> 4;
+        const int UL = U1 - U0;
+        for (int q = lane; q < UL; q += 64) {
+          const Local3 r = local3(K, pos_rec3(S, U0 + q), cx0, cy, cz, k);
+          rec[q] = make_float4(-2.f * r.x, -2.f * r.y, -2.f * r.z,
+                               __builtin_fmaf(r.x, r.x, __builtin_fmaf(r.y, r.y, r.z * r.z)));
+        }
+        __syncthreads();
+        const float* ap[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          ap[e] = reinterpret_cast<const float*>(rec) +
+                  4 * (max(at[e] - U0, 0) + 4 * (ar * steps + steps - 1) + ac) + ak;
+        for (int s = 0; s < steps; ++s) {
+          f32x4 d[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            d[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(*ap[e], B[2 * h + e], C[2 * h + e], 0, 0, 0);
+            ap[e] -= 16;
+          }
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int r = 3; r >= 0; --r)
+              p[2 * h + e] =
+                  __builtin_amdgcn_alignbit(p[2 * h + e], __float_as_uint(d[e][r]), 31);
+        }
+        __syncthreads();
+        if ((lane >> 5) == h) {
+          u0 = (lane >> 4) & 1 ? at[1] : at[0];
+          ch = 4 * steps;
+        }
+      }
+      if (!fits) break;
+      // word T of lane group q -> word q of lane group T
+      auto s2 = __builtin_amdgcn_permlane32_swap(p[0], p[2], false, false);
+      p[0] = s2[0], p[2] = s2[1];
+      s2 = __builtin_amdgcn_permlane32_swap(p[1], p[3], false, false);
+      p[1] = s2[0], p[3] = s2[1];
+      s2 = __builtin_amdgcn_permlane16_swap(p[0], p[1], false, false);
+      p[0] = s2[0], p[1] = s2[1];
+      s2 = __builtin_amdgcn_permlane16_swap(p[2], p[3], false, false);
+      p[2] = s2[0], p[3] = s2[1];
+      if (in) {
+        uint32_t m[3];
+        window3(p, ch, t0[k] - u0, t1[k] - t0[k], m);
+        if (k == 4) {
+          const int sb = i - t0[4];
+          const uint32_t bit = 1u << (sb & 31);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) m[q] &= (sb >> 5) == q ? ~bit : ~0u;
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) lw[3 * k + q][lane] = m[q];
+      }
+    }
+    if (fits) {
+      todo &= ~im;
+      span = P3_SPAN;
+    } else {
+      // a shorter sweep; one cell's own window (at most 96) always fits
+      span = span > 2 ? 2 : 0;
+    }
+  }
+}
+
+// Density gather of a wavefront's 64 consecutive particles: the pre-test of
+// all nine rows (pretest3) into 27 mask words per lane, then one loop over a
+// lane's set bits in (row, word, bit) order, two at a time so that their
+// loads are in flight together, each through the exact test and the pair
+// sums (a wavefront runs for its longest lane's survivor count).  The words
+// are kept in the lane's own LDS column, which the staged records use
+// before.  A lane with a row of more than 96 candidates tests and sums its
+// candidates one by one instead, in the same order.
 template <typename R, bool SUM, bool EOS>
-__device__ __forceinline__ void density3_direct(St3<R>& S, const KParams& K, int i,
-                                                const uint32_t* __restrict__ skey,
-                                                const int* __restrict__ cstart, Mask3 nbm) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3))) void k3_density(St3<R> S, KParams K,
+                                                 const uint32_t* __restrict__ skey,
+                                                 const int* __restrict__ cstart, Mask3 nbm) {
+  if (halted(K)) return;
+  // contiguous shares per XCD (633 -> 616 us at 2.2M particles in FP32, 86 ->
+  // 78 us in FP64 at 84k): the neighbour rows stay in one L2
+  // staged records, then (in their place) the lanes' row starts; the reads
+  // past the records end in the words
+  struct Lds {
+    union {
+      float4 rec[P3_CAP];
+      int lt[9][64];
+    };
+    uint32_t lw[M3_OK][64];
+  };
+  __shared__ Lds L;
+  static_assert(sizeof(Lds) >= sizeof(float4) * (P3_CAP + P3_TILE + 16), "reads past the records");
+  const int lane = threadIdx.x;
+  const int i0 = xcd_block() * 64 + lane;
+  const bool valid = i0 < K.n;
+  const int i = valid ? i0 : K.n - 1;
+  const uint32_t key = skey[i];
+  const int row = (int)(key / (uint32_t)K.nx), cx = (int)key - row * K.nx;
+  const Rows9 rw = rows3_of(K, key, cstart);
+  bool ok = true;
+#pragma unroll
+  for (int k = 0; k < 9; ++k) ok = ok && rw.t1[k] - rw.t0[k] <= 32 * M3_WORDS;
+  pretest3(S, K, i, valid && ok, cx, row, rw, L.rec, L.lw);
+  uint32_t(*lw)[64] = L.lw;
+  int(*lt)[64] = L.lt;
+  uint32_t nz = 0u;  // the lane's non-empty words
+  if (valid && ok) {
+#pragma unroll
+    for (int q = 0; q < M3_OK; ++q) nz |= (lw[q][lane] != 0u ? 1u : 0u) << q;
+  }
+#pragma unroll
+  for (int k = 0; k < 9; ++k) lt[k][lane] = rw.t0[k];
+  if (!valid) return;
   const auto pi = load_pos3(S, i);
   const auto vi = S.v[i];
-  const Rows9 rw = rows3_of(K, skey[i], cstart);
   const R cut2 = cutoff2<R>(K);
   DensOwn<R> o;
   dens_begin<R, SUM>(K, o);
-  bool ok = true;
-  // FP32 form: the neighbour pre-test of every row's candidates (at most 96
-  // per row), eight at a time with no branch, into three mask words per row
-  // kept in the lane's own LDS column; then one loop over the set bits of
-  // all 27 words in (row, word, bit) order, each survivor through the exact
-  // test and the pair sums (a wavefront runs for its longest lane's survivor
-  // count, not for the sum of the nine per-row maxima).  A lane with a row of
-  // more than 96 candidates tests and sums its candidates one by one
-  // instead.  Either way the pairs are summed in ascending position, row by
-  // row, as the single test-and-sum walk of the FP64 form (below) does.
-  if constexpr (sizeof(R) == 4) {
-    constexpr int NB = 8;
-    __shared__ uint32_t lw[M3_OK][BLOCK];
-    __shared__ int lt[9][BLOCK];
-    const int lane = threadIdx.x;
-    // pre-test positions: x = cx cell + off rounded once (K.pre2f bounds
-    // the exact test's cut-off through that rounding)
-    const float cellf = K.cellf;
-    const float xi = __builtin_fmaf(pi.cxf, cellf, pi.ox);
-    const float pre2 = K.pre2f;
-    uint32_t nz = 0u;  // the lane's non-empty words
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      const int t0 = rw.t0[k], t1 = rw.t1[k];
-      if (t1 - t0 > 32 * M3_WORDS) ok = false;
-      const int tA = t1 < t0 + 32 * M3_WORDS ? t1 : t0 + 32 * M3_WORDS;
-      const float yi = pi.oy + row_u3<float>(K, 1 - k % 3), zi = pi.oz + row_u3<float>(K, 1 - k / 3);
-      uint32_t m0 = 0, m1 = 0, m2 = 0;
-      for (int c0 = t0; c0 < tA; c0 += NB) {
-        // a batch starts a multiple of NB past t0, so its bits lie in one
-        // mask word: test into a byte, then place the byte once.  The
-        // position records are padded by NB - 1 past the last particle.
-        uint32_t bb = 0u;
-        const float4* pb = S.pf + c0;
-#pragma unroll
-        for (int q = 0; q < NB; ++q) {
-          const float4 pj = pb[q];
-          const float dx = xi - __builtin_fmaf(pj.w, cellf, pj.x);
-          const float dy = yi - pj.y;
-          const float dz = zi - pj.z;
-          const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-          bb |= (r2 < pre2 ? 1u : 0u) << q;
-        }
-        const int len = tA - c0;
-        if (len < NB) bb &= (1u << len) - 1u;
-        const int b0 = c0 - t0;
-        const uint32_t mb = bb << (b0 & 31);
-        m0 |= b0 < 32 ? mb : 0u;
-        m1 |= (b0 >= 32 && b0 < 64) ? mb : 0u;
-        m2 |= b0 >= 64 ? mb : 0u;
+  if (ok) {
+    uint32_t m = 0u;
+    int tb = 0, wc = 0;
+    R uy = (R)0, uz = (R)0;
+    // the next word: its first candidate and its row's y and z terms
+    auto enter = [&]() {
+      wc = __builtin_ctz(nz);
+      nz &= nz - 1u;
+      m = lw[wc][lane];
+      const int k = (wc * 11) >> 5;  // wc / 3 for wc < 27
+      const int ky = (k * 11) >> 5;  // k / 3 for k < 9
+      uy = row_u3<R>(K, 1 - (k - 3 * ky));
+      uz = row_u3<R>(K, 1 - ky);
+      tb = lt[k][lane] + 32 * (wc - 3 * k);
+    };
+    while (true) {
+      if (m == 0u) {
+        if (nz == 0u) break;
+        enter();
       }
-      {
-        // the lane's own position passed the test at r = 0: clear it
-        const int sb = i - t0;
-        if (sb >= 0 && sb < tA - t0) {
-          const uint32_t keep = ~(1u << (sb & 31));
-          m0 &= sb < 32 ? keep : ~0u;
-          m1 &= (sb >= 32 && sb < 64) ? keep : ~0u;
-          m2 &= sb >= 64 ? keep : ~0u;
-        }
-      }
-      lw[3 * k + 0][lane] = m0;
-      lw[3 * k + 1][lane] = m1;
-      lw[3 * k + 2][lane] = m2;
-      nz |= (m0 != 0u ? 1u : 0u) << (3 * k);
-      nz |= (m1 != 0u ? 2u : 0u) << (3 * k);
-      nz |= (m2 != 0u ? 4u : 0u) << (3 * k);
-      lt[k][lane] = t0;
+      const int b0 = __builtin_ctz(m), w0 = wc, t0 = tb + b0;
+      const R uy0 = uy, uz0 = uz;
+      m &= m - 1u;
+      if (m == 0u && nz != 0u) enter();
+      const bool two = m != 0u;
+      const int b1 = two ? __builtin_ctz(m) : b0, t1 = two ? tb + b1 : t0;
+      m &= m - 1u;  // 0 stays 0
+      const auto p0 = load_pos3(S, t0), p1 = load_pos3(S, t1);
+      const auto v0 = S.v[t0], v1 = S.v[t1];
+      R ax, ay, az, bx, by, bz;
+      const R ra = delta3(pi, p0, K, uy0, uz0, ax, ay, az);
+      const R rb = delta3(pi, p1, K, uy, uz, bx, by, bz);
+      const bool in0 = ra < cut2, in1 = two && rb < cut2;
+      dens3_pair<R, SUM>(K, ax, ay, az, ra, vi.x - v0.x, vi.y - v0.y, vi.z - v0.z, o.sum, o.rs,
+                         in0);
+      dens3_pair<R, SUM>(K, bx, by, bz, rb, vi.x - v1.x, vi.y - v1.y, vi.z - v1.z, o.sum, o.rs,
+                         in1);
+      // passed the pre-test only: out of the recorded masks
+      if (!in0) lw[w0][lane] &= ~(1u << b0);
+      if (two && !in1) lw[wc][lane] &= ~(1u << b1);
     }
-    if (ok) {
-      // the word's first candidate and its row's y and z terms are found
-      // when the walk enters the word; a survivor that fails the exact test
-      // leaves the lane's copy of the word
-      uint32_t m = 0u;
-      int tb = 0, wc = 0;
-      float uy = 0.f, uz = 0.f;
-      while (true) {
-        if (m == 0u) {
-          if (nz == 0u) break;
-          const int w = __builtin_ctz(nz);
-          nz &= nz - 1u;
-          m = lw[w][lane];
-          wc = w;
-          const int k = (w * 11) >> 5;  // w / 3 for w < 27
-          const int q = w - 3 * k;
-          const int ky = (k * 11) >> 5;  // k / 3 for k < 9
-          uy = row_u3<float>(K, 1 - (k - 3 * ky));
-          uz = row_u3<float>(K, 1 - ky);
-          tb = lt[k][lane] + 32 * q;
-        }
-        const int b = __builtin_ctz(m);
-        m &= m - 1u;
-        const int t = tb + b;
-        const auto pj = load_pos3(S, t);
-        const auto vj = S.v[t];
-        float dx, dy, dz;
-        const float r2 = delta3(pi, pj, K, uy, uz, dx, dy, dz);
-        // both loads in flight together: keep the velocity load out of
-        // the branch below
-        asm volatile("" ::"v"(vj.x), "v"(vj.y), "v"(vj.z));
-        if (!(r2 < cut2)) {
-          lw[wc][lane] &= ~(1u << b);  // passed the pre-test only
-          continue;
-        }
-        dens3_pair<R, SUM>(K, dx, dy, dz, r2, vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, o.sum,
-                           o.rs);
-      }
-      if (nbm.w)
-        for (int q = 0; q < M3_OK; ++q) nbm.put(q, i, lw[q][lane]);
-    } else {
-      // a row of more than 96 candidates: test and sum one by one, in the
-      // same order; masks of the first 96 candidates of each row
-#pragma unroll
-      for (int k = 0; k < 9; ++k) {
-        const int t0 = rw.t0[k], t1 = rw.t1[k];
-        const float uy = row_u3<float>(K, 1 - k % 3), uz = row_u3<float>(K, 1 - k / 3);
-        uint32_t m0 = 0, m1 = 0, m2 = 0;
-        for (int t = t0; t < t1; ++t) {
-          if (t == i) continue;
-          const auto pj = load_pos3(S, t);
-          float dx, dy, dz;
-          const float r2 = delta3(pi, pj, K, uy, uz, dx, dy, dz);
-          if (!(r2 < cut2)) continue;
-          const int b = t - t0;
-          const uint32_t bit = 1u << (b & 31);
-          m0 |= b < 32 ? bit : 0u;
-          m1 |= (b >= 32 && b < 64) ? bit : 0u;
-          m2 |= (b >= 64 && b < 96) ? bit : 0u;
-          const auto vj = S.v[t];
-          dens3_pair<R, SUM>(K, dx, dy, dz, r2, vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, o.sum,
-                             o.rs);
-        }
-        if (nbm.w) {
-          nbm.put(k * M3_WORDS + 0, i, m0);
-          nbm.put(k * M3_WORDS + 1, i, m1);
-          nbm.put(k * M3_WORDS + 2, i, m2);
-        }
-      }
-    }
+    if (nbm.w)
+      for (int q = 0; q < M3_OK; ++q) nbm.put(q, i, lw[q][lane]);
   } else {
     for (int k = 0; k < 9; ++k) {
       const int t0 = rw.t0[k], t1 = rw.t1[k];
       const R uy = row_u3<R>(K, 1 - k % 3), uz = row_u3<R>(K, 1 - k / 3);
-      if (t1 - t0 > 32 * M3_WORDS) ok = false;
-      uint32_t m0 = 0, m1 = 0, m2 = 0;
       for (int t = t0; t < t1; ++t) {
         if (t == i) continue;
         const auto pj = load_pos3(S, t);
         R dx, dy, dz;
         const R r2 = delta3(pi, pj, K, uy, uz, dx, dy, dz);
         if (!(r2 < cut2)) continue;
-        const int b = t - t0;
-        const uint32_t bit = 1u << (b & 31);
-        m0 |= b < 32 ? bit : 0u;
-        m1 |= (b >= 32 && b < 64) ? bit : 0u;
-        m2 |= (b >= 64 && b < 96) ? bit : 0u;
         const auto vj = S.v[t];
         dens3_pair<R, SUM>(K, dx, dy, dz, r2, vi.x - vj.x, vi.y - vj.y, vi.z - vj.z, o.sum, o.rs);
-      }
-      if (nbm.w) {
-        nbm.put(k * M3_WORDS + 0, i, m0);
-        nbm.put(k * M3_WORDS + 1, i, m1);
-        nbm.put(k * M3_WORDS + 2, i, m2);
       }
     }
   }
   if (nbm.w) nbm.put(M3_OK, i, ok ? 1u : 0u);
   dens_end<R, SUM, EOS>(S, K, i, o);
-}
-
-template <typename R, bool SUM, bool EOS>
-__global__ __launch_bounds__(BLOCK) void k3_density(St3<R> S, KParams K,
-                                                    const uint32_t* __restrict__ skey,
-                                                    const int* __restrict__ cstart, Mask3 nbm) {
-  if (halted(K)) return;
-  const int i = blockIdx.x * BLOCK + threadIdx.x;
-  if (i >= K.n) return;
-  density3_direct<R, SUM, EOS>(S, K, i, skey, cstart, nbm);
 }
 
 template <typename R>
@@ -625,8 +767,6 @@ template <typename R> struct Pack3 {
   R4* rec;  // 3 per particle
 };
 
-__device__ __forceinline__ float4 pos_rec3(const St3<float>& S, int i) { return S.pf[i]; }
-__device__ __forceinline__ double4 pos_rec3(const St3<double>& S, int i) { return S.xyz[i]; }
 __device__ __forceinline__ Pos3F pos_of_rec(float4 q) { return {q.w, q.x, q.y, q.z}; }
 __device__ __forceinline__ Pos3D pos_of_rec(double4 q) { return {q.x, q.y, q.z}; }
 

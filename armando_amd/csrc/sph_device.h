@@ -37,6 +37,7 @@ struct KParams {
   // FP32 neighbour pre-test: a bound on (2h)^2 for r^2 computed from
   // x = cx cell + off rounded once per particle (the exact test follows)
   float pre2f;
+  float pre3f;  // the same for the 3D pre-test on the matrix cores (pretest3)
   // FP32 roundings of the constants the FP32 pair bodies use, so that they
   // stay in scalar registers (a conversion in the kernel lands in a vector
   // register); each is (float) of the double field it is named after, apart
