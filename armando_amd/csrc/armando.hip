@@ -1470,11 +1470,16 @@ template <typename R> int link_list3_t(arm_ctx* c) {
   return check_domain(c);
 }
 
+template <typename R> Pack3<R> pack3(arm_ctx* c) {
+  using R4 = typename V4<R>::type;
+  return Pack3<R>{static_cast<R4*>(c->pack3_vq)};
+}
+
 // 3D density gather, one wavefront per workgroup (k3_density).  Records the
 // neighbour masks for the force pass.
 template <typename R, bool SUM, bool EOS> void launch_density3(arm_ctx* c) {
   hipLaunchKernelGGL((k3_density<R, SUM, EOS>), dim3((c->n + 63) / 64), dim3(64), 0, c->stream,
-                     st3A<R>(c), c->K, c->skey, c->cstart, c->mask3);
+                     st3A<R>(c), c->K, c->skey, c->cstart, c->mask3, pack3<R>(c));
   c->masks_valid = true;
 }
 
@@ -1495,21 +1500,25 @@ template <typename R> int eos3_t(arm_ctx* c) {
   return ARM_OK;
 }
 
-template <typename R> Pack3<R> pack3(arm_ctx* c) {
-  using R4 = typename V4<R>::type;
-  return Pack3<R>{static_cast<R4*>(c->pack3_vq)};
-}
-
-template <typename R, bool P, bool AV, bool AH, bool XS> void launch_force3(arm_ctx* c) {
+// packed: the records are those of the current state (density3_t with eos)
+template <typename R, bool P, bool AV, bool AH, bool XS>
+void launch_force3(arm_ctx* c, bool packed) {
   const Mask3 m{c->masks_valid ? c->mask3.w : nullptr, c->mask3.stride};
   const Pack3<R> pk = pack3<R>(c);
-  hipLaunchKernelGGL(k3_force_pack<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream,
-                     st3A<R>(c), c->K, pk);
-  hipLaunchKernelGGL((k3_force<R, P, AV, AH, XS>), dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream,
-                     st3A<R>(c), pk, c->K, c->skey, c->cstart, m);
+  if (!packed)
+    hipLaunchKernelGGL(k3_force_pack<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream,
+                       st3A<R>(c), c->K, pk);
+  const dim3 g((c->n + 63) / 64), b(64);
+  if (AV && AH && c->K.same_e2)
+    hipLaunchKernelGGL((k3_force<R, P, AV, AH, XS, AV && AH>), g, b, 0, c->stream, st3A<R>(c), pk,
+                       c->K, c->skey, c->cstart, m);
+  else
+    hipLaunchKernelGGL((k3_force<R, P, AV, AH, XS, false>), g, b, 0, c->stream, st3A<R>(c), pk,
+                       c->K, c->skey, c->cstart, m);
 }
 
-template <typename R> int force3_t(arm_ctx* c, bool press, int flags, bool xs) {
+template <typename R>
+int force3_t(arm_ctx* c, bool press, int flags, bool xs, bool packed = false) {
   const bool av = (flags & ARM_ART_VISC) != 0, ah = (flags & ARM_ART_HEAT) != 0;
   if (press && (flags & ARM_VISC))
     return fail(c, ARM_ERR_UNSUPPORTED, "physical viscosity is implemented in 2D only");
@@ -1517,15 +1526,15 @@ template <typename R> int force3_t(arm_ctx* c, bool press, int flags, bool xs) {
   PassTimer tm(c, ARM_PASS_FORCE);
   const int code = (press ? 8 : 0) | (av ? 4 : 0) | (ah ? 2 : 0) | (xs ? 1 : 0);
   switch (code) {
-    case 8: launch_force3<R, true, false, false, false>(c); break;
-    case 9: launch_force3<R, true, false, false, true>(c); break;
-    case 10: launch_force3<R, true, false, true, false>(c); break;
-    case 11: launch_force3<R, true, false, true, true>(c); break;
-    case 12: launch_force3<R, true, true, false, false>(c); break;
-    case 13: launch_force3<R, true, true, false, true>(c); break;
-    case 14: launch_force3<R, true, true, true, false>(c); break;
-    case 15: launch_force3<R, true, true, true, true>(c); break;
-    case 1: launch_force3<R, false, false, false, true>(c); break;
+    case 8: launch_force3<R, true, false, false, false>(c, packed); break;
+    case 9: launch_force3<R, true, false, false, true>(c, packed); break;
+    case 10: launch_force3<R, true, false, true, false>(c, packed); break;
+    case 11: launch_force3<R, true, false, true, true>(c, packed); break;
+    case 12: launch_force3<R, true, true, false, false>(c, packed); break;
+    case 13: launch_force3<R, true, true, false, true>(c, packed); break;
+    case 14: launch_force3<R, true, true, true, false>(c, packed); break;
+    case 15: launch_force3<R, true, true, true, true>(c, packed); break;
+    case 1: launch_force3<R, false, false, false, true>(c, packed); break;
     default: return fail(c, ARM_ERR_ARG, "force pass with nothing to compute");
   }
   if (press && (c->K.flags & KF_DEPOSITION))
@@ -1543,7 +1552,7 @@ template <typename R> int single_step3_t(arm_ctx* c) {
   int rc;
   if ((rc = density3_t<R>(c, c->prm.density_method, true))) return rc;
   const bool xs = (c->prm.flags & ARM_AV_VEL) != 0;
-  if ((rc = force3_t<R>(c, true, c->prm.flags, xs))) return rc;
+  if ((rc = force3_t<R>(c, true, c->prm.flags, xs, true))) return rc;
   if (!xs && (rc = zero_av3<R>(c))) return rc;
   c->have_rates = true;
   return ARM_OK;
@@ -1597,7 +1606,7 @@ template <typename R> int fused_step3(arm_ctx* c, int its, const StepHooks& hk =
   if (hk.jpart)
     hipLaunchKernelGGL(k3_objective<R>, dim3(grid_of(n)), dim3(BLOCK), 0, c->stream, st3A<R>(c),
                        c->K, hk.kind, hk.objmask, hk.jpart);
-  if ((rc = force3_t<R>(c, true, c->prm.flags, xs))) return rc;
+  if ((rc = force3_t<R>(c, true, c->prm.flags, xs, true))) return rc;
   if (tape) {
     const int nb = std::max(grid_of(n), grid_of(c->K.ncell + 1));
     hipLaunchKernelGGL(k3_tape<R>, dim3(nb), dim3(BLOCK), 0, c->stream, st3A<R>(c), c->K, c->skey,
@@ -2505,7 +2514,7 @@ int arm_internal_force(arm_ctx* c, int flags) {
   if (!c) return ARM_ERR_ARG;
   int rc = need_sorted(c);
   if (rc) return rc;
-  rc = is3d(c) ? DISPATCH(c, force3_t)(c, true, flags, false)
+  rc = is3d(c) ? DISPATCH(c, force3_t)(c, true, flags, false, false)
                : DISPATCH(c, force_t)(c, true, flags, false);
   if (!rc) HIPCHK(c, hipStreamSynchronize(c->stream));
   return rc;
@@ -2515,7 +2524,7 @@ int arm_av_vel(arm_ctx* c) {
   if (!c) return ARM_ERR_ARG;
   int rc = need_sorted(c);
   if (rc) return rc;
-  rc = is3d(c) ? DISPATCH(c, force3_t)(c, false, 0, true)
+  rc = is3d(c) ? DISPATCH(c, force3_t)(c, false, 0, true, false)
                : DISPATCH(c, force_t)(c, false, 0, true);
   if (!rc) HIPCHK(c, hipStreamSynchronize(c->stream));
   return rc;

@@ -323,6 +323,36 @@ struct Mask3 {
   }
 };
 
+// Neighbour data of the force pass packed per particle into one record of
+// three vectors, so that a neighbour's loads fall in one or two cache lines:
+// the position record of the state (FP32: pf; FP64: xyz), (v, Q = 1/rho) and
+// (A = p/rho, psi, u, 0), with q_and_a's arithmetic.  Written at the end of a
+// density pass with the EOS in it, whose particles hold most of it already,
+// or by k3_force_pack.
+template <typename R> struct Pack3 {
+  using R4 = typename V4<R>::type;
+  R4* rec;  // 3 per particle
+};
+
+__device__ __forceinline__ float4 pos_rec3(const St3<float>& S, int i) { return S.pf[i]; }
+__device__ __forceinline__ double4 pos_rec3(const St3<double>& S, int i) { return S.xyz[i]; }
+template <typename R> __device__ __forceinline__ R u3_of(const St3<R>& S, int t) {
+  if constexpr (sizeof(R) == 4) return S.uf[t]; else return (R)S.u[t];
+}
+
+template <typename R>
+__device__ __forceinline__ void force3_record(const St3<R>& S, const KParams& K, const Pack3<R>& P,
+                                              int i) {
+  using R4 = typename V4<R>::type;
+  R Q, A;
+  q_and_a(K, S.rho[i], S.p[i], Q, A);
+  const R4 v = S.v[i];
+  R4* r = P.rec + 3 * (size_t)i;
+  r[0] = pos_rec3(S, i);
+  r[1] = R4{v.x, v.y, v.z, Q};
+  r[2] = R4{A, S.psi[i], u3_of(S, i), (R)0};
+}
+
 // ---- neighbour pre-test on the matrix cores ---------------------------------
 // A particle has about 490 candidates in its nine rows, of which 68 are
 // neighbours, so the candidate test dominates a density pass that makes it
@@ -373,8 +403,6 @@ __device__ __forceinline__ Local3 local3(const KParams& K, double4 q, int cx0, i
           (float)(q.y - (K.oy + (double)cy * K.cell)),
           (float)(q.z - (K.oz + (double)cz * K.cell))};
 }
-__device__ __forceinline__ float4 pos_rec3(const St3<float>& S, int i) { return S.pf[i]; }
-__device__ __forceinline__ double4 pos_rec3(const St3<double>& S, int i) { return S.xyz[i]; }
 
 // The 96-bit window [d, d + len) of the four words p of ch bits each
 // (ch a multiple of 4, at most 32; len <= 96).
@@ -538,7 +566,8 @@ __device__ __forceinline__ void pretest3(const St3<R>& S, const KParams& K, int 
 template <typename R, bool SUM, bool EOS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3))) void k3_density(St3<R> S, KParams K,
                                                  const uint32_t* __restrict__ skey,
-                                                 const int* __restrict__ cstart, Mask3 nbm) {
+                                                 const int* __restrict__ cstart, Mask3 nbm,
+                                                 Pack3<R> P) {
   if (halted(K)) return;
   // contiguous shares per XCD (633 -> 616 us at 2.2M particles in FP32, 86 ->
   // 78 us in FP64 at 84k): the neighbour rows stay in one L2
@@ -639,6 +668,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) ==
   }
   if (nbm.w) nbm.put(M3_OK, i, ok ? 1u : 0u);
   dens_end<R, SUM, EOS>(S, K, i, o);
+  if (EOS) force3_record(S, K, P, i);
 }
 
 template <typename R>
@@ -654,6 +684,9 @@ template <typename R> struct ForceOwn3 {
   using R4 = typename V4<R>::type;
   R4 v;
   R Q, A, psi, u;
+  // FP32 pair body: the particle's factors as in ForceOwn, and the pressure
+  // term f_cm (..) = (a1 Q_j + a0) + A_j (b1 Q_j + b0) for either pa_sph
+  R a0, a1, b0, b1, avb, ava, c4, c4psi, xw, xw2;
   R fx = 0, fy = 0, fz = 0, xsx = 0, xsy = 0, xsz = 0;
   Acc<R> du;
 };
@@ -664,19 +697,79 @@ __device__ __forceinline__ void force3_begin(const St3<R>& S, const KParams& K, 
   o.v = S.v[i];
   q_and_a(K, S.rho[i], S.p[i], o.Q, o.A);
   o.psi = S.psi[i];
-  if constexpr (sizeof(R) == 4) o.u = S.uf[i]; else o.u = (R)S.u[i];
+  if constexpr (sizeof(R) == 4) {
+    o.u = S.uf[i];
+    const float cm = K.kf.cm, q4 = 4.f * o.Q, c4 = cm * q4, cA = cm * o.A;
+    const bool pa0 = K.pa_sph == 0;
+    o.a0 = pa0 ? 0.f : cA * o.Q;
+    o.a1 = pa0 ? cA : 0.f;
+    o.b0 = pa0 ? cm * o.Q : 0.f;
+    o.b1 = pa0 ? 0.f : cm;
+    o.avb = c4 * K.kf.avbh2;
+    o.ava = c4 * K.kf.avah;
+    o.c4 = c4;
+    o.c4psi = c4 * o.psi;
+    o.xw = K.kf.xs * q4;
+    o.xw2 = 2.f * o.xw;
+  } else {
+    o.u = (R)S.u[i];
+  }
 }
 
-template <typename R, bool PRESS, bool AV, bool AH, bool XS>
-__device__ __forceinline__ void force3_pair(const KParams& K, ForceOwn3<R>& o, R dx, R dy, R dz,
-                                            R r2, R vjx, R vjy, R vjz, R Qj, R Aj, R psij,
-                                            R uj) {
+// The terms of one pair apart from their accumulation: the particle gains
+// -G r, the energy rate d and -wf dv.
+template <typename R> struct Terms3 {
+  R G, dx, dy, dz, d, wf, dvx, dvy, dvz;
+};
+
+// SE: artificial viscosity and heat share (h eta)^2.  The FP32 form has the
+// operations of force_terms_f32 (sph_kernels.h), the energy rate doubled; the
+// FP64 form the plain products and sums.
+template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool SE>
+__device__ __forceinline__ Terms3<R> force3_terms(const KParams& K, const ForceOwn3<R>& o, R dx,
+                                                  R dy, R dz, R r2, R vjx, R vjy, R vjz, R Qj,
+                                                  R Aj, R psij, R uj) {
+  Terms3<R> t;
+  t.dx = dx;
+  t.dy = dy;
+  t.dz = dz;
+  t.dvx = o.v.x - vjx;
+  t.dvy = o.v.y - vjy;
+  t.dvz = o.v.z - vjz;
+  t.G = (R)0;
+  t.d = (R)0;
+  t.wf = (R)0;
+  const R vr = fmr(t.dvz, dz, fmr(t.dvy, dy, t.dvx * dx));
+  if constexpr (sizeof(R) == 4) {
+    const float rr = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+    const float q = fsqrt(rr) * K.kf.invh;
+    const float s = __builtin_fmaf(-0.5f, q, 1.f);
+    const float s3 = s * s * s;
+    const float M = s3 * (Qj * frcp(o.Q + Qj));
+    float G = 0.f, inv_ea = 0.f;
+    if (PRESS) G = s3 * __builtin_fmaf(Aj, __builtin_fmaf(o.b1, Qj, o.b0), __builtin_fmaf(o.a1, Qj, o.a0));
+    if (AV) {
+      inv_ea = frcp(rr + K.kf.ave2);
+      const float e = __builtin_fminf(vr, 0.f) * inv_ea;
+      G = __builtin_fmaf(e * __builtin_fmaf(o.avb, e, o.ava), M, G);
+    }
+    float d = 0.f;
+    if (PRESS || AV) {
+      t.G = G;
+      d = G * vr;
+    }
+    if (AH) {
+      const float inv_eh = (AV && SE) ? inv_ea : frcp(rr + K.kf.ahe2);
+      d = __builtin_fmaf(__builtin_fmaf(o.c4, psij, o.c4psi) * M * (rr * inv_eh), o.u - uj, d);
+    }
+    t.d = d;
+    if (XS) t.wf = __builtin_fmaf(o.xw2, q, o.xw) * s * M;
+    return t;
+  }
   const R m = (R)K.mass;
   const R q = fsqrt(r2) * (R)K.invh;
   const R tq = q - (R)2;
   const R F = (R)K.C1 * (tq * tq * tq);
-  const R dvx = o.v.x - vjx, dvy = o.v.y - vjy, dvz = o.v.z - vjz;
-  const R vr = fmr(dvz, dz, fmr(dvy, dy, dvx * dx));
   const R inv_mrho = (R)2 * o.Q * Qj * frcp(o.Q + Qj);
   R coef = 0;
   if (PRESS) coef = (K.pa_sph == 0) ? fmr(o.A, Qj, Aj * o.Q) : fmr(o.A, o.Q, Aj * Qj);
@@ -690,28 +783,35 @@ __device__ __forceinline__ void force3_pair(const KParams& K, ForceOwn3<R>& o, R
     }
   }
   if (PRESS || AV) {
-    const R G = m * F * coef;
-    o.fx = fmr(-G, dx, o.fx);
-    o.fy = fmr(-G, dy, o.fy);
-    o.fz = fmr(-G, dz, o.fz);
-    R dut = (R)0.5 * G * vr;
-    if (AH) {
-      const R inv_eh = (AV && K.same_e2) ? inv_ea : frcp(r2 + (R)K.ah_e2);
-      dut = fmr(m * (o.psi + psij) * F * r2 * inv_mrho * inv_eh, o.u - uj, dut);
-    }
-    o.du.add(dut);
-  } else if (AH) {
-    const R inv_eh = frcp(r2 + (R)K.ah_e2);
-    o.du.add(m * (o.psi + psij) * F * r2 * inv_mrho * inv_eh * (o.u - uj));
+    t.G = m * F * coef;
+    t.d = (R)0.5 * t.G * vr;
+  }
+  if (AH) {
+    const R inv_eh = (AV && SE) ? inv_ea : frcp(r2 + (R)K.ah_e2);
+    t.d = fmr(m * (o.psi + psij) * F * r2 * inv_mrho * inv_eh, o.u - uj, t.d);
   }
   if (XS) {
     const R s = fmr((R)-0.5, q, (R)1);
     const R s2 = s * s;
     const R w = (R)K.wnorm * (s2 * s2) * fmr((R)2, q, (R)1);
-    const R wf = (R)K.eps_m * inv_mrho * w;
-    o.xsx = fmr(-wf, dvx, o.xsx);
-    o.xsy = fmr(-wf, dvy, o.xsy);
-    o.xsz = fmr(-wf, dvz, o.xsz);
+    t.wf = (R)K.eps_m * inv_mrho * w;
+  }
+  return t;
+}
+
+// Adds the terms of one pair when ok (else nothing), without a branch.
+template <typename R, bool PRESS, bool AV, bool AH, bool XS>
+__device__ __forceinline__ void force3_acc(ForceOwn3<R>& o, const Terms3<R>& t, bool ok) {
+  if (PRESS || AV) {
+    o.fx = ok ? fmr(-t.G, t.dx, o.fx) : o.fx;
+    o.fy = ok ? fmr(-t.G, t.dy, o.fy) : o.fy;
+    o.fz = ok ? fmr(-t.G, t.dz, o.fz) : o.fz;
+  }
+  if (PRESS || AV || AH) o.du.add_if(t.d, ok);
+  if (XS) {
+    o.xsx = ok ? fmr(-t.wf, t.dvx, o.xsx) : o.xsx;
+    o.xsy = ok ? fmr(-t.wf, t.dvy, o.xsy) : o.xsy;
+    o.xsz = ok ? fmr(-t.wf, t.dvz, o.xsz) : o.xsz;
   }
 }
 
@@ -741,7 +841,7 @@ __device__ __forceinline__ void force3_end(St3<R>& S, const KParams& K, int i,
     acc.z = o.fz + (grav ? (R)K.gz : (R)0);
     acc.w = (R)0;
     S.a[i] = acc;
-    S.du[i] = o.du.get();
+    S.du[i] = sizeof(R) == 4 ? (R)0.5 * o.du.get() : o.du.get();  // FP32: doubled sums
   }
   if (XS) {
     R4 w;
@@ -753,78 +853,59 @@ __device__ __forceinline__ void force3_end(St3<R>& S, const KParams& K, int i,
   }
 }
 
-template <typename R> __device__ __forceinline__ R u3_of(const St3<R>& S, int t) {
-  if constexpr (sizeof(R) == 4) return S.uf[t]; else return (R)S.u[t];
-}
-
-// Neighbour data of the force pass packed per particle into one record of
-// three vectors, so that a neighbour's loads fall in one or two cache lines:
-// the position record of the state (FP32: pf; FP64: xyz), (v, Q = 1/rho) and
-// (A = p/rho, psi, u, 0), written by k3_force_pack right before the gather
-// with q_and_a's arithmetic.
-template <typename R> struct Pack3 {
-  using R4 = typename V4<R>::type;
-  R4* rec;  // 3 per particle
-};
-
 __device__ __forceinline__ Pos3F pos_of_rec(float4 q) { return {q.w, q.x, q.y, q.z}; }
 __device__ __forceinline__ Pos3D pos_of_rec(double4 q) { return {q.x, q.y, q.z}; }
 
+// The records on their own (after the routines that do not write them).
 template <typename R>
 __global__ __launch_bounds__(BLOCK) void k3_force_pack(St3<R> S, KParams K, Pack3<R> P) {
   if (halted(K)) return;
-  using R4 = typename V4<R>::type;
   const int i = blockIdx.x * BLOCK + threadIdx.x;
   if (i >= K.n) return;
-  R Q, A;
-  q_and_a(K, S.rho[i], S.p[i], Q, A);
-  const R4 v = S.v[i];
-  R4 vq, ap;
-  vq.x = v.x;
-  vq.y = v.y;
-  vq.z = v.z;
-  vq.w = Q;
-  ap.x = A;
-  ap.y = S.psi[i];
-  ap.z = u3_of(S, i);
-  ap.w = (R)0;
-  P.rec[3 * (size_t)i] = pos_rec3(S, i);
-  P.rec[3 * (size_t)i + 1] = vq;
-  P.rec[3 * (size_t)i + 2] = ap;
+  force3_record(S, K, P, i);
 }
 
-// One neighbour t of particle i in the direct path.
-template <typename R, bool PRESS, bool AV, bool AH, bool XS, typename P3>
-__device__ __forceinline__ void force3_visit(const St3<R>& S, const Pack3<R>& P, const KParams& K,
-                                             const P3& pi, R uy, R uz, ForceOwn3<R>& o, int t) {
-  const auto* rp = P.rec + (((unsigned)t << 1) + (unsigned)t);  // 3 t, no 64-bit multiply
-  const auto pj = pos_of_rec(rp[0]);
-  const auto vq = rp[1];
-  const auto ap = rp[2];
-  R dx, dy, dz;
-  const R r2 = delta3(pi, pj, K, uy, uz, dx, dy, dz);
-  force3_pair<R, PRESS, AV, AH, XS>(K, o, dx, dy, dz, r2, vq.x, vq.y, vq.z, vq.w, ap.x, ap.y,
-                                    ap.z);
-}
-
-template <typename R, bool PRESS, bool AV, bool AH, bool XS>
-__device__ __forceinline__ void force3_direct(St3<R>& S, const Pack3<R>& P, const KParams& K,
-                                              int i, const uint32_t* __restrict__ skey,
-                                              const int* __restrict__ cstart, Mask3 nbm) {
+// The force gather of a wavefront's 64 consecutive particles: one loop over
+// every set bit of a lane's 27 mask words in (row, word, bit) order (a
+// wavefront runs for its longest lane's neighbour count).  The FP32 form takes
+// two neighbours at a time, whose six record loads are in flight together,
+// each added in walk order; in FP64 the second one's registers cost a
+// wavefront per SIMD (2.2M particles: 1507 us against 1398).  Each lane keeps its words and row starts in its own LDS column and
+// a bitmap of its non-empty words.  A particle without complete masks tests
+// its candidates one by one, in the same order with the same pair body.
+// Contiguous shares per XCD: the packed records of the neighbour rows stay in
+// one L2 (3.6x less traffic beyond L2, 915 -> 880 us in FP32 at 2.2M).
+// Bound at 2.2M particles in FP32: the vector cache's tag accesses, one a cycle
+// (a record load of 64 lanes touches 46 lines; three loads a neighbour keep it
+// 92 % busy), so fewer instructions (2.71e8 -> 2.39e8) and two neighbours at
+// once leave it at 790 us.  Below that size latency: 83,630 particles FP32
+// 51.6 -> 39.8 us; FP64 at 2.2M 1638 -> 1398 us.  The records written by the
+// density pass take 41 us there instead of a launch of 53 (FP64 106 of 121).
+template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool SE>
+__global__ __launch_bounds__(64) void k3_force(
+    St3<R> S, Pack3<R> P, KParams K, const uint32_t* __restrict__ skey,
+    const int* __restrict__ cstart, Mask3 nbm) {
+  if (halted(K)) return;
+  __shared__ uint32_t lw[M3_OK][64];
+  __shared__ int lt[9][64];
+  const int lane = threadIdx.x;
+  const int i = xcd_block() * 64 + lane;
+  if (i >= K.n) return;
   const auto pi = load_pos3(S, i);
   ForceOwn3<R> o;
   force3_begin(S, K, i, o);
   const Rows9 rw = rows3_of(K, skey[i], cstart);
+  auto terms = [&](int t, R uy, R uz) {
+    const auto* rp = P.rec + (((unsigned)t << 1) + (unsigned)t);  // 3 t, no 64-bit multiply
+    const auto pj = pos_of_rec(rp[0]);
+    const auto vq = rp[1];
+    const auto ap = rp[2];
+    R dx, dy, dz;
+    const R r2 = delta3(pi, pj, K, uy, uz, dx, dy, dz);
+    return force3_terms<R, PRESS, AV, AH, XS, SE>(K, o, dx, dy, dz, r2, vq.x, vq.y, vq.z, vq.w,
+                                                  ap.x, ap.y, ap.z);
+  };
   if (nbm.w && nbm.get(M3_OK, i)) {
-    // One loop over every set bit of the 27 words in (row, word, bit) order,
-    // the order of the per-word walk: a wavefront runs for its longest
-    // lane's neighbour count instead of the sum of the 27 per-word maxima.
-    // Each lane keeps its words and row starts in its own LDS column (they
-    // are indexed by the lane's position in the walk) and a bitmap of its
-    // non-empty words.
-    __shared__ uint32_t lw[M3_OK][BLOCK];
-    __shared__ int lt[9][BLOCK];
-    const int lane = threadIdx.x;
     uint32_t nz = 0u;
 #pragma unroll
     for (int q = 0; q < M3_OK; ++q) {
@@ -834,28 +915,39 @@ __device__ __forceinline__ void force3_direct(St3<R>& S, const Pack3<R>& P, cons
     }
 #pragma unroll
     for (int k = 0; k < 9; ++k) lt[k][lane] = rw.t0[k];
-    if (nz) {
-      // the word's first candidate and its row's y and z terms are found
-      // when the walk enters the word, and kept until it leaves it
-      uint32_t m = 0u;
-      int tb = 0;
-      R uy = (R)0, uz = (R)0;
-      while (true) {
-        if (m == 0u) {
-          if (nz == 0u) break;
-          const int w = __builtin_ctz(nz);
-          nz &= nz - 1u;
-          m = lw[w][lane];
-          const int k = (w * 11) >> 5;  // w / 3 for w < 27
-          const int q = w - 3 * k;
-          const int ky = (k * 11) >> 5;  // k / 3 for k < 9
-          uy = row_u3<R>(K, 1 - (k - 3 * ky));
-          uz = row_u3<R>(K, 1 - ky);
-          tb = lt[k][lane] + 32 * q;
-        }
-        const int b = __builtin_ctz(m);
-        m &= m - 1u;
-        force3_visit<R, PRESS, AV, AH, XS>(S, P, K, pi, uy, uz, o, tb + b);
+    uint32_t m = 0u;
+    int tb = 0;
+    R uy = (R)0, uz = (R)0;
+    // the next word: its first candidate and its row's y and z terms
+    auto enter = [&]() {
+      const int w = __builtin_ctz(nz);
+      nz &= nz - 1u;
+      m = lw[w][lane];
+      const int k = (w * 11) >> 5;   // w / 3 for w < 27
+      const int ky = (k * 11) >> 5;  // k / 3 for k < 9
+      uy = row_u3<R>(K, 1 - (k - 3 * ky));
+      uz = row_u3<R>(K, 1 - ky);
+      tb = lt[k][lane] + 32 * (w - 3 * k);
+    };
+    while (true) {
+      if (m == 0u) {
+        if (nz == 0u) break;
+        enter();
+      }
+      const int ta = tb + (int)__builtin_ctz(m);
+      const R ya = uy, za = uz;
+      m &= m - 1u;
+      if constexpr (sizeof(R) == 4) {
+        if (m == 0u && nz != 0u) enter();
+        const bool two = m != 0u;
+        const int tc = two ? tb + (int)__builtin_ctz(m) : ta;
+        m &= m - 1u;  // 0 stays 0
+        const Terms3<R> A = terms(ta, ya, za);
+        const Terms3<R> B = terms(tc, uy, uz);
+        force3_acc<R, PRESS, AV, AH, XS>(o, A, true);
+        force3_acc<R, PRESS, AV, AH, XS>(o, B, two);
+      } else {
+        force3_acc<R, PRESS, AV, AH, XS>(o, terms(ta, ya, za), true);
       }
     }
   } else {
@@ -868,25 +960,11 @@ __device__ __forceinline__ void force3_direct(St3<R>& S, const Pack3<R>& P, cons
         R dx, dy, dz;
         const R r2 = delta3(pi, pj, K, uy, uz, dx, dy, dz);
         if (!(r2 < cut2)) continue;
-        force3_visit<R, PRESS, AV, AH, XS>(S, P, K, pi, uy, uz, o, t);
+        force3_acc<R, PRESS, AV, AH, XS>(o, terms(t, uy, uz), true);
       }
     }
   }
   force3_end<R, PRESS, XS>(S, K, i, o);
-}
-
-template <typename R, bool PRESS, bool AV, bool AH, bool XS>
-__global__ __launch_bounds__(BLOCK) void k3_force(St3<R> S, Pack3<R> P, KParams K,
-                                                  const uint32_t* __restrict__ skey,
-                                                  const int* __restrict__ cstart, Mask3 nbm) {
-  if (halted(K)) return;
-  // contiguous shares per XCD: the packed records of the neighbour rows
-  // stay in one L2 (3.6x less traffic beyond L2, 915 -> 880 us in FP32);
-  // the density pass, bound by instruction issue, keeps the plain order,
-  // where the XCDs' shares of work are even
-  const int i = xcd_block() * BLOCK + threadIdx.x;
-  if (i >= K.n) return;
-  force3_direct<R, PRESS, AV, AH, XS>(S, P, K, i, skey, cstart, nbm);
 }
 
 // ------------------------------------------------------------------------
