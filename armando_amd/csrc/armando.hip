@@ -66,7 +66,8 @@ struct arm_ctx {
   bool masks_valid = false;  // nbm holds the neighbour masks of the current order
   uint4* nbm = nullptr;
   // 2D tiled gathers: the row pieces of the current order (RowPieces)
-  int2* pieces = nullptr;
+  int4* pieces = nullptr;
+  int2* cuts = nullptr;
   int* npieces = nullptr;
   bool pieces_valid = false;
   // deposition heat source (arm_set_deposition): the map on the device, the
@@ -267,7 +268,7 @@ Ent ent_of(arm_ctx* c) {
 }
 
 RowPieces row_pieces_of(const arm_ctx* c) {
-  return c->pieces ? RowPieces{c->pieces, c->npieces, c->K.nx, c->K.ny} : RowPieces{};
+  return c->pieces ? RowPieces{c->pieces, c->cuts, c->npieces, c->K.nx, c->K.ny} : RowPieces{};
 }
 
 int run_sort(arm_ctx* c, const int32_t* id_of, const uint32_t** sval_out, bool* ranges_done,
@@ -434,23 +435,24 @@ template <typename R> int link_list_t(arm_ctx* c) {
 
 // Where the tiled gathers' workgroups find their segments, and how many
 // workgroups they take: row pieces (CW = 0; the piece table is rebuilt after
-// each sort, and the grid is the bound n / PIECE + ny on the piece count) or
+// each sort, and the grid is ny for the cut parts and the bound n / PIECE + ny
+// on the piece count) or
 // runs of CW cells of every row.
 template <int CW> SegArg seg_arg(arm_ctx* c) {
   if constexpr (CW > 0) {
-    return SegArg{(c->K.nx + CW - 1) / CW, nullptr, nullptr};
+    return SegArg{(c->K.nx + CW - 1) / CW, nullptr, nullptr, nullptr};
   } else {
     if (!c->pieces_valid) {
       const RowPieces rp = row_pieces_of(c);
       hipLaunchKernelGGL(k_row_pieces, dim3(row_blocks(rp)), dim3(BLOCK), 0, c->stream,
-                         c->cstart, rp, Halt{c->K.halt, c->K.its});
+                         c->cstart, c->skey, rp, Halt{c->K.halt, c->K.its});
       c->pieces_valid = true;
     }
-    return SegArg{0, c->pieces, c->npieces};
+    return SegArg{0, c->pieces, c->cuts, c->npieces};
   }
 }
 template <int CW> int seg_grid(const arm_ctx* c, const SegArg& sa) {
-  return CW > 0 ? c->K.ny * sa.nseg : (c->n + PIECE - 1) / PIECE + c->K.ny;
+  return CW > 0 ? c->K.ny * sa.nseg : (c->n + PIECE - 1) / PIECE + 2 * c->K.ny;
 }
 
 template <typename R, bool SUM, bool EOS> void launch_density(arm_ctx* c) {
@@ -2248,6 +2250,7 @@ int arm_create(const arm_params* prm, int capacity, arm_ctx** out) {
   if (!rc) rc = dalloc(c, &c->nbm, capacity);
   if (!rc && !is3d(c)) {
     rc = dalloc(c, &c->pieces, (size_t)capacity / PIECE + c->K.ny + 2);
+    if (!rc) rc = dalloc(c, &c->cuts, (size_t)c->K.ny);
     if (!rc) rc = dalloc(c, &c->npieces, 1);
   }
   if (!rc && is3d(c)) rc = dalloc(c, &c->nbm3, (size_t)M3_TOTAL * capacity);

@@ -295,39 +295,83 @@ __global__ __launch_bounds__(CS_THREADS) void k_cs_scatter(const uint32_t* __res
 // Pieces of the cell rows, for the gathers that give each workgroup a run of
 // consecutive sorted positions of one row: the sorted range of row y,
 // [cstart[y nx], cstart[(y+1) nx]), cut into runs of PIECE positions from its
-// start (the last one shorter); pieces[s] = (first position, row), in row
+// start (the last one shorter); pieces[s] = (first position, row, end), in row
 // order, and *npieces their count, at most n / PIECE + ny.
+//
+// Above a tank's free surface a row holds wall particles on either side only,
+// and the row below everything between them, so that a piece over the gap
+// needs more records than a gather's tile holds and its workgroup runs on the
+// direct path, as long as a whole launch of the others (FP32 force of the
+// 111,119-particle dam break: 28.6 us, 12.8 without; density 20.5 and 14.5).  A piece of more than
+// GAP_SPAN cells whose three rows hold more than GAP_RECORDS particles is
+// therefore cut at the middle of its cells, at most one of each row: the
+// part after the cut is cuts[y] = (first position, end), (0, 0) if there is none.
 constexpr int PIECE = 128;
+constexpr int GAP_SPAN = 40;      // a full piece of 2h cells spans about 20
+constexpr int GAP_RECORDS = 592;  // the smallest tile of the gathers on pieces
 struct RowPieces {
-  int2* pieces = nullptr;
+  int4* pieces = nullptr;
+  int2* cuts = nullptr;
   int* npieces = nullptr;
   int nx = 0, ny = 0;
 };
 
-// Workgroup wg of a grid of ceil(ny / THREADS) lists the pieces of rows
-// wg THREADS .. wg THREADS + THREADS-1, one lane per row.  It counts the
-// pieces of the rows before its own itself (as k_cs_tile_scan adds up the
-// tile sums before its own), so the table needs neither atomics nor a
-// cleared counter; the workgroup of the last row writes *npieces.
+// Workgroup wg of a grid of ceil(ny / ROWS_PER_WG) lists the pieces of rows
+// wg ROWS_PER_WG .., one wavefront per row and one lane per piece (a lane that
+// walked a row's pieces itself waited for the keys of each in turn: 32 us for
+// a 17 us reorder).  It counts the pieces of the rows before its own itself
+// (as k_cs_tile_scan adds up the tile sums before its own), so the table needs
+// neither atomics nor a cleared counter; the workgroup of the last row writes
+// *npieces.  keys: the cell of every sorted position.
+constexpr int ROWS_PER_WG = 4;
 template <int THREADS>
 __device__ __forceinline__ void row_pieces_block(const int* __restrict__ cstart,
+                                                 const uint32_t* __restrict__ keys,
                                                  const RowPieces& rp, int wg) {
+  static_assert(THREADS == 64 * ROWS_PER_WG, "one wavefront per row");
   __shared__ int wsum[THREADS / 64];
   const int nx = rp.nx;
-  const int y0 = wg * THREADS;
+  const int y0 = wg * ROWS_PER_WG;
+  auto count = [&](int y) { return (cstart[(y + 1) * nx] - cstart[y * nx] + PIECE - 1) / PIECE; };
   int before = 0;
-  for (int y = threadIdx.x; y < y0; y += THREADS)
-    before += (cstart[(y + 1) * nx] - cstart[y * nx] + PIECE - 1) / PIECE;
+  for (int y = threadIdx.x; y < y0; y += THREADS) before += count(y);
   int base;
   block_exclusive_scan<THREADS>(before, wsum, &base);
-  __syncthreads();  // wsum is reused
-  const int y = y0 + (int)threadIdx.x;
-  const int a = y < rp.ny ? cstart[y * nx] : 0;
-  const int b = y < rp.ny ? cstart[(y + 1) * nx] : 0;
-  int total;
-  int s = base + block_exclusive_scan<THREADS>((b - a + PIECE - 1) / PIECE, wsum, &total);
-  for (int p = a; p < b; p += PIECE) rp.pieces[s++] = make_int2(p, y);
-  if (threadIdx.x == 0 && y0 + THREADS >= rp.ny) *rp.npieces = base + total;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int y = y0 + w;
+  if (y >= rp.ny) return;
+  for (int r = y0; r < y; ++r) base += count(r);
+  const int a = cstart[y * nx], b = cstart[(y + 1) * nx];
+  const int np = (b - a + PIECE - 1) / PIECE;
+  if (lane == 0 && y == rp.ny - 1) *rp.npieces = base + np;
+  // a row of at least four particles a cell has no gap worth looking for
+  const bool sparse = b > a && 4 * ((int)(keys[b - 1] - keys[a]) + 1) > b - a;
+  bool found = false;
+  for (int j0 = 0; j0 < np; j0 += 64) {
+    const int p = a + (j0 + lane) * PIECE;
+    int e = min(p + PIECE, b), m = 0;
+    if (sparse && !found && p < b) {
+      const int x0 = (int)keys[p] - y * nx, x1 = (int)keys[e - 1] - y * nx;
+      if (x1 - x0 > GAP_SPAN) {
+        const int lo = x0 > 0 ? x0 - 1 : 0, hi = (x1 + 1 < nx ? x1 + 1 : nx - 1) + 1;
+        int rec = cstart[y * nx + hi] - cstart[y * nx + lo];
+        if (y > 0) rec += cstart[(y - 1) * nx + hi] - cstart[(y - 1) * nx + lo];
+        if (y + 1 < rp.ny) rec += cstart[(y + 1) * nx + hi] - cstart[(y + 1) * nx + lo];
+        m = cstart[y * nx + (x0 + x1 + 1) / 2];
+        if (!(rec > GAP_RECORDS && m > p && m < e)) m = 0;
+      }
+    }
+    const uint64_t cutters = __ballot(m != 0);
+    if (cutters && !found) {
+      found = true;
+      if (lane == __builtin_ctzll(cutters)) {
+        rp.cuts[y] = make_int2(m, e);
+        e = m;
+      }
+    }
+    if (p < b) rp.pieces[base + j0 + lane] = make_int4(p, y, e, 0);
+  }
+  if (!found && lane == 0) rp.cuts[y] = make_int2(0, 0);
 }
 
 // skip: a cell whose order does not matter (the extra cell of stale ghosts,

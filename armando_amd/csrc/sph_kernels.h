@@ -187,17 +187,18 @@ __device__ __forceinline__ void ghost_slot(const St<R>& A, St<R>& Bs, const KPar
 
 // A reorder kernel launched with row pieces (rp.pieces set; cell_start
 // written by the sort) has row_blocks(rp) extra workgroups in front, one
-// lane per cell row, which list the rows' pieces (they run beside the first
-// particles' workgroups).  Returns true in those; *t is the sorted position
+// wavefront per cell row, which list the rows' pieces (they run beside the
+// first particles' workgroups).  Returns true in those; *t is the sorted position
 // of the lane in the others.
 __host__ __device__ inline int row_blocks(const RowPieces& rp) {
-  return rp.pieces ? (rp.ny + BLOCK - 1) / BLOCK : 0;
+  return rp.pieces ? (rp.ny + ROWS_PER_WG - 1) / ROWS_PER_WG : 0;
 }
 __device__ __forceinline__ bool reorder_row_pieces(const int* __restrict__ cstart,
+                                                   const uint32_t* __restrict__ keys,
                                                    const RowPieces& rp, int* t) {
   const int rb = row_blocks(rp);
   if ((int)blockIdx.x < rb) {
-    row_pieces_block<BLOCK>(cstart, rp, blockIdx.x);
+    row_pieces_block<BLOCK>(cstart, keys, rp, blockIdx.x);
     return true;
   }
   *t = ((int)blockIdx.x - rb) * BLOCK + threadIdx.x;
@@ -213,7 +214,7 @@ __global__ __launch_bounds__(BLOCK) void k_reorder_all(St<R> A, St<R> Bs, KParam
                                                        int* __restrict__ cstart, int fill,
                                                        Ghosts G, RowPieces rp) {
   int t;
-  if (reorder_row_pieces(cstart, rp, &t)) return;
+  if (reorder_row_pieces(cstart, skey, rp, &t)) return;
   const bool valid = t < K.n;
   if (fill) fill_cell_start(skey, t, valid, K.n, K.ncell, cstart);
   if (!valid) return;
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(BLOCK) void k_reorder_pred(St<R> A, St<R> Bs, KPara
                                                         int fill, Ghosts G, RowPieces rp) {
   if (halted(K)) return;
   int t;
-  if (reorder_row_pieces(cstart, rp, &t)) return;
+  if (reorder_row_pieces(cstart, skey, rp, &t)) return;
   using R2 = typename V2<R>::type;
   const bool valid = t < K.n;
   if (fill) fill_cell_start(skey, t, valid, K.n, K.ncell, cstart);

@@ -239,10 +239,12 @@ struct Segment {
 //  CW > 0: a fixed run of CW cells of a row (segment row * nseg + run).
 //  CW = 0: a piece of at most PIECE consecutive sorted positions of one row
 //          (RowPieces); every wavefront of a piece but the row's last is
-//          full.
+//          full.  The first ny workgroups take the parts cut from the rows'
+//          pieces (most rows have none).
 struct SegArg {
   int nseg;
-  const int2* pieces;
+  const int4* pieces;
+  const int2* cuts;
   const int* npieces;
 };
 
@@ -294,15 +296,22 @@ __device__ __forceinline__ Segment segment_of(const KParams& K, const int* __res
   } else {
     // pieces in even XCD-contiguous shares: neighbouring pieces, which stage
     // the same rows, share an L2 (the grid is a bound on the piece count)
-    const int sb = xcd_share(*sa.npieces);
-    if (sb < 0) {
-      g.O0 = g.O1 = 0;
-      return g;
+    g.cy = g.O0 = g.O1 = 0;
+    if ((int)blockIdx.x < K.ny) {
+      const int2 cut = sa.cuts[blockIdx.x];
+      g.cy = blockIdx.x;
+      g.O0 = cut.x;
+      g.O1 = cut.y;
+    } else {
+      const int sb = xcd_share(*sa.npieces, (int)blockIdx.x - K.ny);
+      if (sb >= 0) {
+        const int4 pc = sa.pieces[sb];
+        g.cy = pc.y;
+        g.O0 = pc.x;
+        g.O1 = pc.z;
+      }
     }
-    const int2 pc = sa.pieces[sb];
-    g.cy = pc.y;
-    g.O0 = pc.x;
-    g.O1 = min(pc.x + PIECE, cstart[(pc.y + 1) * nx]);
+    if (g.O0 >= g.O1) return g;
     cx0 = (int)skey[g.O0] - g.cy * nx;
     cx1 = (int)skey[g.O1 - 1] - g.cy * nx + 1;
   }
@@ -331,9 +340,10 @@ __device__ __forceinline__ Segment segment_of(const KParams& K, const int* __res
 
 // The row pieces on their own (after a sort that does not build them).
 __global__ __launch_bounds__(BLOCK) void k_row_pieces(const int* __restrict__ cstart,
+                                                      const uint32_t* __restrict__ skey,
                                                       RowPieces rp, Halt hl) {
   if (hl.on()) return;
-  row_pieces_block<BLOCK>(cstart, rp, blockIdx.x);
+  row_pieces_block<BLOCK>(cstart, skey, rp, blockIdx.x);
 }
 
 // A particle of the first or last cell column of a grid periodic in x: its
