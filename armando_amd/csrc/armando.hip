@@ -66,9 +66,8 @@ struct arm_ctx {
   bool masks_valid = false;  // nbm holds the neighbour masks of the current order
   uint4* nbm = nullptr;
   // 2D tiled gathers: the row pieces of the current order (RowPieces)
-  int4* pieces = nullptr;
-  int2* cuts = nullptr;
-  int* npieces = nullptr;
+  PieceRec* pieces = nullptr;
+  int piece_slots = 0;  // of the table last built
   bool pieces_valid = false;
   // deposition heat source (arm_set_deposition): the map on the device, the
   // deposition time and the number of the step the next force pass belongs
@@ -267,8 +266,10 @@ Ent ent_of(arm_ctx* c) {
   return Ent{p, p + c->cap};
 }
 
-RowPieces row_pieces_of(const arm_ctx* c) {
-  return c->pieces ? RowPieces{c->pieces, c->cuts, c->npieces, c->K.nx, c->K.ny} : RowPieces{};
+RowPieces row_pieces_of(arm_ctx* c) {
+  if (!c->pieces) return {};
+  c->piece_slots = (c->n + PIECE - 1) / PIECE + c->K.ny;
+  return {c->pieces, c->K.nx, c->K.ny, c->piece_slots};
 }
 
 int run_sort(arm_ctx* c, const int32_t* id_of, const uint32_t** sval_out, bool* ranges_done,
@@ -424,7 +425,7 @@ template <typename R> int link_list_t(arm_ctx* c) {
     hipLaunchKernelGGL(k_reorder_all<R>, dim3(grid_of(c->n) + row_blocks(rp)),
                        dim3(BLOCK), 0, c->stream, A, B, c->K, c->skey, sval, c->cstart,
                        ranges ? 0 : 1, c->G, rp);
-    c->pieces_valid = rp.pieces != nullptr;
+    c->pieces_valid = rp.tab != nullptr;
   }
   HIPCHK(c, hipGetLastError());
   std::swap(A, B);
@@ -435,12 +436,11 @@ template <typename R> int link_list_t(arm_ctx* c) {
 
 // Where the tiled gathers' workgroups find their segments, and how many
 // workgroups they take: row pieces (CW = 0; the piece table is rebuilt after
-// each sort, and the grid is ny for the cut parts and the bound n / PIECE + ny
-// on the piece count) or
+// each sort, and the grid is ny for the cut parts and piece_slots) or
 // runs of CW cells of every row.
 template <int CW> SegArg seg_arg(arm_ctx* c) {
   if constexpr (CW > 0) {
-    return SegArg{(c->K.nx + CW - 1) / CW, nullptr, nullptr, nullptr};
+    return SegArg{(c->K.nx + CW - 1) / CW, nullptr, c->masks_valid};
   } else {
     if (!c->pieces_valid) {
       const RowPieces rp = row_pieces_of(c);
@@ -448,11 +448,11 @@ template <int CW> SegArg seg_arg(arm_ctx* c) {
                          c->cstart, c->skey, rp, Halt{c->K.halt, c->K.its});
       c->pieces_valid = true;
     }
-    return SegArg{0, c->pieces, c->cuts, c->npieces};
+    return SegArg{0, c->pieces, c->masks_valid};
   }
 }
 template <int CW> int seg_grid(const arm_ctx* c, const SegArg& sa) {
-  return CW > 0 ? c->K.ny * sa.nseg : (c->n + PIECE - 1) / PIECE + 2 * c->K.ny;
+  return CW > 0 ? c->K.ny * sa.nseg : c->K.ny + c->piece_slots;
 }
 
 template <typename R, bool SUM, bool EOS> void launch_density(arm_ctx* c) {
@@ -507,12 +507,12 @@ template <typename R> int eos_t(arm_ctx* c) {
 
 // The FP32 tiled force gather of the dam-break flag set (pressure, artificial
 // viscosity and heat, XSPH) with pa_sph and same_e2 fixed at compile time.
-template <int PC> void launch_force_hot(arm_ctx* c, const uint4* nbm) {
+template <int PC> void launch_force_hot(arm_ctx* c) {
   using T = HotForceCfg;
   const SegArg sa = seg_arg<T::CW>(c);
   hipLaunchKernelGGL((k_force_hot<T::BLK, T::CAP, PC>), dim3(seg_grid<T::CW>(c, sa)),
                      dim3(T::BLK), 0, c->stream, stA<float>(c), c->K, c->skey, c->cstart, sa,
-                     nbm);
+                     c->nbm);
 }
 
 template <typename R, bool P, bool AV, bool AH, bool XS, bool VI = false>
@@ -520,14 +520,13 @@ void launch_force(arm_ctx* c) {
   St<R>& A = stA<R>(c);
   using T = ForceCfg<R, VI>;
   if (c->tiled && !c->K.sle) {
-    const uint4* nbm = c->masks_valid ? c->nbm : nullptr;
     if (sizeof(R) == 4 && P && AV && AH && XS && !VI && !c->K.periodic &&
         !(c->K.flags & ARM_CONDUCTION)) {
       switch ((c->K.pa_sph == 0 ? 1 : 0) | (c->K.same_e2 ? 2 : 0)) {
-        case 0: launch_force_hot<0>(c, nbm); break;
-        case 1: launch_force_hot<1>(c, nbm); break;
-        case 2: launch_force_hot<2>(c, nbm); break;
-        default: launch_force_hot<3>(c, nbm); break;
+        case 0: launch_force_hot<0>(c); break;
+        case 1: launch_force_hot<1>(c); break;
+        case 2: launch_force_hot<2>(c); break;
+        default: launch_force_hot<3>(c); break;
       }
     } else {
       const SegArg sa = seg_arg<T::CW>(c);
@@ -535,11 +534,11 @@ void launch_force(arm_ctx* c) {
       if (c->K.periodic)
         hipLaunchKernelGGL((k_force_tiled<R, P, AV, AH, XS, VI, true, T::BLK, T::CW, T::CAP>),
                            dim3(grid), dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart,
-                           sa, nbm);
+                           sa, c->nbm);
       else
         hipLaunchKernelGGL((k_force_tiled<R, P, AV, AH, XS, VI, false, T::BLK, T::CW, T::CAP>),
                            dim3(grid), dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart,
-                           sa, nbm);
+                           sa, c->nbm);
     }
   } else {
     hipLaunchKernelGGL((k_force<R, P, AV, AH, XS, VI>), dim3(grid_of(c->n)), dim3(BLOCK), 0,
@@ -552,15 +551,14 @@ template <typename R> void launch_tensor(arm_ctx* c) {
   St<R>& A = stA<R>(c);
   using T = TileCfg<R>;
   if (c->tiled && !c->K.sle) {
-    const uint4* nbm = c->masks_valid ? c->nbm : nullptr;
     const SegArg sa = seg_arg<T::CW>(c);
     const int grid = seg_grid<T::CW>(c, sa);
     if (c->K.periodic)
       hipLaunchKernelGGL((k_tensor_tiled<R, true, T::BLK, T::CW, T::CAP>), dim3(grid),
-                         dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart, sa, nbm);
+                         dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart, sa, c->nbm);
     else
       hipLaunchKernelGGL((k_tensor_tiled<R, false, T::BLK, T::CW, T::CAP>), dim3(grid),
-                         dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart, sa, nbm);
+                         dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart, sa, c->nbm);
   } else {
     hipLaunchKernelGGL(k_tensor<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream, A, c->K,
                        c->skey, c->cstart);
@@ -773,7 +771,7 @@ template <typename R> int fused_step(arm_ctx* c, int its, const StepHooks& hk) {
     hipLaunchKernelGGL(k_reorder_pred<R>, dim3(grid_of(n) + row_blocks(rp)),
                        dim3(BLOCK), 0, c->stream, A, B, c->K, c->skey, sval, c->cstart,
                        its != 1 ? 1 : 0, ranges ? 0 : 1, c->G, rp);
-    c->pieces_valid = rp.pieces != nullptr;
+    c->pieces_valid = rp.tab != nullptr;
     std::swap(A, B);
     c->masks_valid = false;
   }
@@ -2044,16 +2042,15 @@ void set_kparams(KParams& K, const arm_params& P) {
   K.cellf = (float)P.cell;
   K.cut2f = (float)K.cut2;
   {
-    // x_a = fl(cx cell + off) is within u |x_a| <= u nx cell of the exact
-    // value (u = 2^-24); a difference of two, rounded, and the y and z terms
-    // (oy_i + uy) - oy_j rounded in another order, are within
-    // E = u (2 nx cell + 4 cell + 16 h) of the exact path's per axis, so
-    // r < 2h implies r_a < 2h + 2E
     const double u = 1.0 / 16777216.0;
-    const double nmax = (double)std::max(P.nx, std::max(P.ny, P.dim == 3 ? P.nz : 1));
-    const double E = u * (2.0 * nmax * P.cell + 4.0 * P.cell + 16.0 * P.h);
-    const double b = 2.0 * P.h + 2.0 * E;
-    K.pre2f = std::nextafter((float)(b * b * (1.0 + 1e-5)), INFINITY);
+    // fixed-point positions: each is rounded by at most 1/2 unit (and the FP32
+    // product by u FIX), so a difference by less than 1.01 per axis and r by less
+    // than 1.43; the FP32 test's own rounding of r (a few u cell) is far below
+    // the rest of the margin
+    K.fix = FIX / P.cell;
+    K.fixf = (float)K.fix;
+    const double b = 2.0 * P.h * K.fix * (1.0 + 1e-6) + 1.6;
+    K.fix2 = (int)std::ceil(b * b);
     // pretest3: coordinates relative to the sweep's first cell are at most
     // L = P3_SPAN + 3 cells along x and 2 along y and z, so |x|^2 is at most
     // X = (L^2 + 8) cell^2.  Each coordinate is rounded once or twice (u L
@@ -2249,9 +2246,7 @@ int arm_create(const arm_params* prm, int capacity, arm_ctx** out) {
   if (!rc) rc = dalloc(c, &c->d_cnt, capacity);
   if (!rc) rc = dalloc(c, &c->nbm, capacity);
   if (!rc && !is3d(c)) {
-    rc = dalloc(c, &c->pieces, (size_t)capacity / PIECE + c->K.ny + 2);
-    if (!rc) rc = dalloc(c, &c->cuts, (size_t)c->K.ny);
-    if (!rc) rc = dalloc(c, &c->npieces, 1);
+    rc = dalloc(c, &c->pieces, (size_t)capacity / PIECE + 2 * (size_t)c->K.ny + 2);
   }
   if (!rc && is3d(c)) rc = dalloc(c, &c->nbm3, (size_t)M3_TOTAL * capacity);
   if (!rc && is3d(c)) c->mask3 = Mask3{c->nbm3, capacity};

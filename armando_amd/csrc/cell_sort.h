@@ -295,83 +295,129 @@ __global__ __launch_bounds__(CS_THREADS) void k_cs_scatter(const uint32_t* __res
 // Pieces of the cell rows, for the gathers that give each workgroup a run of
 // consecutive sorted positions of one row: the sorted range of row y,
 // [cstart[y nx], cstart[(y+1) nx]), cut into runs of PIECE positions from its
-// start (the last one shorter); pieces[s] = (first position, row, end), in row
-// order, and *npieces their count, at most n / PIECE + ny.
+// start (the last one shorter).  tab[b] is all that workgroup b of a gather
+// needs to begin: its particles [O0, O1) of row cy and the three ranges of
+// sorted positions that hold their candidates, so that one load stands
+// between the launch and the filling of the tile (a chain of five before, a
+// microsecond each for every workgroup).
 //
-// Above a tank's free surface a row holds wall particles on either side only,
-// and the row below everything between them, so that a piece over the gap
-// needs more records than a gather's tile holds and its workgroup runs on the
-// direct path, as long as a whole launch of the others (FP32 force of the
-// 111,119-particle dam break: 28.6 us, 12.8 without; density 20.5 and 14.5).  A piece of more than
-// GAP_SPAN cells whose three rows hold more than GAP_RECORDS particles is
-// therefore cut at the middle of its cells, at most one of each row: the
-// part after the cut is cuts[y] = (first position, end), (0, 0) if there is none.
+// tab[0 .. ny) hold the parts cut off the rows' pieces: above a tank's free
+// surface a row holds wall particles on either side only, and the row below
+// everything between them, so that a piece over the gap needs more records
+// than a gather's tile holds and its workgroup runs on the direct path, as
+// long as a whole launch of the others (FP32 force of the 111,119-particle
+// dam break: 28.6 us, 12.8 without; density 20.5 and 14.5).  A piece of more
+// than GAP_SPAN cells whose three rows hold more than GAP_RECORDS particles is
+// therefore cut at the middle of its cells, at most one of each row.
+//
+// tab[ny .. ny + slots) hold the pieces: the first count of them, dealt so
+// that the workgroups of one XCD take one contiguous share (neighbouring
+// pieces, which stage the same rows, then share an L2); the others are empty.
+// slots = n / PIECE + ny bounds the count.
 constexpr int PIECE = 128;
 constexpr int GAP_SPAN = 40;      // a full piece of 2h cells spans about 20
 constexpr int GAP_RECORDS = 592;  // the smallest tile of the gathers on pieces
+struct alignas(16) PieceRec {
+  int O0, O1, cy, total;  // total = rl[0] + rl[1] + rl[2]
+  int rs[3], rl[3];       // sorted start and length of rows cy-1, cy, cy+1
+  int pad[2];
+};
 struct RowPieces {
-  int4* pieces = nullptr;
-  int2* cuts = nullptr;
-  int* npieces = nullptr;
-  int nx = 0, ny = 0;
+  PieceRec* tab = nullptr;
+  int nx = 0, ny = 0, slots = 0;
 };
 
-// Workgroup wg of a grid of ceil(ny / ROWS_PER_WG) lists the pieces of rows
+// The workgroup of a run of workgroups that xcd_share gives logical block L
+// of count.
+__device__ __forceinline__ int share_slot(int count, int L) {
+  constexpr int X = 8;
+  const int q = count / X, r = count - q * X;
+  if (L < r * (q + 1)) return (L % (q + 1)) * X + L / (q + 1);
+  const int m = L - r * (q + 1);
+  return (m % q) * X + r + m / q;
+}
+
+// Workgroup wg of a grid of row_blocks() lists the pieces of rows
 // wg ROWS_PER_WG .., one wavefront per row and one lane per piece (a lane that
 // walked a row's pieces itself waited for the keys of each in turn: 32 us for
-// a 17 us reorder).  It counts the pieces of the rows before its own itself
-// (as k_cs_tile_scan adds up the tile sums before its own), so the table needs
-// neither atomics nor a cleared counter; the workgroup of the last row writes
-// *npieces.  keys: the cell of every sorted position.
+// a 17 us reorder).  It counts the pieces of all rows itself, so the table
+// needs neither atomics nor a cleared counter.  keys: the cell of every sorted
+// position.
 constexpr int ROWS_PER_WG = 4;
 template <int THREADS>
 __device__ __forceinline__ void row_pieces_block(const int* __restrict__ cstart,
                                                  const uint32_t* __restrict__ keys,
-                                                 const RowPieces& rp, int wg) {
+                                                 const RowPieces& rp, int wg, int nwg) {
   static_assert(THREADS == 64 * ROWS_PER_WG, "one wavefront per row");
   __shared__ int wsum[THREADS / 64];
-  const int nx = rp.nx;
+  const int nx = rp.nx, ny = rp.ny;
   const int y0 = wg * ROWS_PER_WG;
   auto count = [&](int y) { return (cstart[(y + 1) * nx] - cstart[y * nx] + PIECE - 1) / PIECE; };
-  int before = 0;
-  for (int y = threadIdx.x; y < y0; y += THREADS) before += count(y);
-  int base;
+  int before = 0, all = 0;
+  for (int y = threadIdx.x; y < ny; y += THREADS) {
+    const int c = count(y);
+    all += c;
+    before += y < y0 ? c : 0;
+  }
+  int base, total;
   block_exclusive_scan<THREADS>(before, wsum, &base);
+  __syncthreads();  // wsum is reused
+  block_exclusive_scan<THREADS>(all, wsum, &total);
+  PieceRec* slots = rp.tab + ny;
+  for (int s = total + wg * THREADS + (int)threadIdx.x; s < rp.slots; s += nwg * THREADS)
+    slots[s] = PieceRec{};
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int y = y0 + w;
-  if (y >= rp.ny) return;
+  if (y >= ny) return;
   for (int r = y0; r < y; ++r) base += count(r);
   const int a = cstart[y * nx], b = cstart[(y + 1) * nx];
   const int np = (b - a + PIECE - 1) / PIECE;
-  if (lane == 0 && y == rp.ny - 1) *rp.npieces = base + np;
-  // a row of at least four particles a cell has no gap worth looking for
-  const bool sparse = b > a && 4 * ((int)(keys[b - 1] - keys[a]) + 1) > b - a;
+  // the rows' ranges of the particles [p, e) in cells x0 .. x1
+  auto make = [&](int p, int e, int x0, int x1) {
+    PieceRec r{};
+    const int lo = x0 > 0 ? x0 - 1 : 0, hi = (x1 + 1 < nx ? x1 + 1 : nx - 1) + 1;
+    r.O0 = p;
+    r.O1 = e;
+    r.cy = y;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int ry = y - 1 + k;
+      if (ry >= 0 && ry < ny) {
+        r.rs[k] = cstart[ry * nx + lo];
+        r.rl[k] = cstart[ry * nx + hi] - r.rs[k];
+      }
+      r.total += r.rl[k];
+    }
+    return r;
+  };
   bool found = false;
   for (int j0 = 0; j0 < np; j0 += 64) {
     const int p = a + (j0 + lane) * PIECE;
-    int e = min(p + PIECE, b), m = 0;
-    if (sparse && !found && p < b) {
+    int m = 0;
+    PieceRec rec{}, cut{};
+    if (p < b) {
+      const int e = min(p + PIECE, b);
       const int x0 = (int)keys[p] - y * nx, x1 = (int)keys[e - 1] - y * nx;
-      if (x1 - x0 > GAP_SPAN) {
-        const int lo = x0 > 0 ? x0 - 1 : 0, hi = (x1 + 1 < nx ? x1 + 1 : nx - 1) + 1;
-        int rec = cstart[y * nx + hi] - cstart[y * nx + lo];
-        if (y > 0) rec += cstart[(y - 1) * nx + hi] - cstart[(y - 1) * nx + lo];
-        if (y + 1 < rp.ny) rec += cstart[(y + 1) * nx + hi] - cstart[(y + 1) * nx + lo];
+      rec = make(p, e, x0, x1);
+      if (!found && x1 - x0 > GAP_SPAN && rec.total > GAP_RECORDS) {
         m = cstart[y * nx + (x0 + x1 + 1) / 2];
-        if (!(rec > GAP_RECORDS && m > p && m < e)) m = 0;
+        if (m > p && m < e)
+          cut = make(m, e, (int)keys[m] - y * nx, x1);
+        else
+          m = 0;
       }
     }
     const uint64_t cutters = __ballot(m != 0);
     if (cutters && !found) {
       found = true;
       if (lane == __builtin_ctzll(cutters)) {
-        rp.cuts[y] = make_int2(m, e);
-        e = m;
+        rp.tab[y] = cut;
+        rec = make(p, m, (int)keys[p] - y * nx, (int)keys[m - 1] - y * nx);
       }
     }
-    if (p < b) rp.pieces[base + j0 + lane] = make_int4(p, y, e, 0);
+    if (p < b) slots[share_slot(total, base + j0 + lane)] = rec;
   }
-  if (!found && lane == 0) rp.cuts[y] = make_int2(0, 0);
+  if (!found && lane == 0) rp.tab[y] = PieceRec{};
 }
 
 // skip: a cell whose order does not matter (the extra cell of stale ghosts,

@@ -34,10 +34,13 @@ struct KParams {
   // (beta phi - alpha c0)/2 = f_avb phi + f_ava; XSPH wnorm eps m / 2; 2 cond
   double f_cm, f_ava, f_avb, f_xs, f_cond2;
   float cellf, cut2f;
-  // FP32 neighbour pre-test: a bound on (2h)^2 for r^2 computed from
-  // x = cx cell + off rounded once per particle (the exact test follows)
-  float pre2f;
-  float pre3f;  // the same for the 3D pre-test on the matrix cores (pretest3)
+  // neighbour pre-test of the 2D density pass on fixed-point positions
+  // (PreTile): FIX / cell, and a bound on (2h)^2 in squared units
+  double fix;
+  float fixf;
+  int fix2;
+  // a bound on (2h)^2 for the 3D pre-test on the matrix cores (pretest3)
+  float pre3f;
   // FP32 roundings of the constants the FP32 pair bodies use, so that they
   // stay in scalar registers (a conversion in the kernel lands in a vector
   // register); each is (float) of the double field it is named after, apart
@@ -105,16 +108,6 @@ __device__ __forceinline__ int xcd_block() {
   const int nb = (int)gridDim.x, b = (int)blockIdx.x;
   const int q = nb / NXCD, r = nb - q * NXCD, x = b - (b / NXCD) * NXCD;
   return x * q + (x < r ? x : r) + b / NXCD;
-}
-
-// The same for the first `count` logical blocks of a run of at least count
-// workgroups, b the workgroup's number in it: XCD x (or, when the run does not
-// begin at workgroup 0, the one as far from it) covers one contiguous share of
-// 0 .. count-1, the shares as even as the count allows; -1 for the
-// workgroups past them.
-__device__ __forceinline__ int xcd_share(int count, int b) {
-  const int q = count / NXCD, r = count - q * NXCD, x = b - (b / NXCD) * NXCD, j = b / NXCD;
-  return j < q + (x < r ? 1 : 0) ? x * q + (x < r ? x : r) + j : -1;
 }
 
 // Set in KParams::flags by the host for the steps whose time its dt lies

@@ -185,20 +185,20 @@ __device__ __forceinline__ void ghost_slot(const St<R>& A, St<R>& Bs, const KPar
   G.gpid[t] = A.id[ps];
 }
 
-// A reorder kernel launched with row pieces (rp.pieces set; cell_start
+// A reorder kernel launched with row pieces (rp.tab set; cell_start
 // written by the sort) has row_blocks(rp) extra workgroups in front, one
 // wavefront per cell row, which list the rows' pieces (they run beside the
 // first particles' workgroups).  Returns true in those; *t is the sorted position
 // of the lane in the others.
 __host__ __device__ inline int row_blocks(const RowPieces& rp) {
-  return rp.pieces ? (rp.ny + ROWS_PER_WG - 1) / ROWS_PER_WG : 0;
+  return rp.tab ? (rp.ny + ROWS_PER_WG - 1) / ROWS_PER_WG : 0;
 }
 __device__ __forceinline__ bool reorder_row_pieces(const int* __restrict__ cstart,
                                                    const uint32_t* __restrict__ keys,
                                                    const RowPieces& rp, int* t) {
   const int rb = row_blocks(rp);
   if ((int)blockIdx.x < rb) {
-    row_pieces_block<BLOCK>(cstart, keys, rp, blockIdx.x);
+    row_pieces_block<BLOCK>(cstart, keys, rp, blockIdx.x, rb);
     return true;
   }
   *t = ((int)blockIdx.x - rb) * BLOCK + threadIdx.x;
@@ -474,13 +474,15 @@ __device__ __forceinline__ void eos_point(SS& S, const KParams& K, int i, bool r
 // negative of the continuity sum; the EOS divides it by rho.  With EOS the
 // equation of state follows at once (single_step.f:119-186 comes right after
 // the density call).
+// id, rho_s: the particle's, loaded by the caller (before its walk).
 template <typename R, bool SUM, bool EOS = false, typename SS = St<R>>
-__device__ __forceinline__ void dens_end(SS& S, const KParams& K, int i, const DensOwn<R>& o) {
-  const bool rate = is_rate(K, S.id[i]);
+__device__ __forceinline__ void dens_end(SS& S, const KParams& K, int i, const DensOwn<R>& o,
+                                         int id, R rho_s) {
+  const bool rate = is_rate(K, id);
   R rho = (R)0;
   if (!SUM) {
     S.drho[i] = rate ? o.sum.get() : (R)0;
-    if (EOS) rho = S.rho[i];
+    if (EOS) rho = rho_s;
   } else {
     S.drho[i] = (R)0;
     if (rate) {
@@ -490,13 +492,17 @@ __device__ __forceinline__ void dens_end(SS& S, const KParams& K, int i, const D
         rho = o.rs.get();
       S.rho[i] = rho;
     } else if (EOS) {
-      rho = S.rho[i];
+      rho = rho_s;
     }
   }
   if (EOS)
     eos_point(S, K, i, rate, rho, -o.sum.get());
   else
     S.divv[i] = -o.sum.get();
+}
+template <typename R, bool SUM, bool EOS = false, typename SS = St<R>>
+__device__ __forceinline__ void dens_end(SS& S, const KParams& K, int i, const DensOwn<R>& o) {
+  dens_end<R, SUM, EOS>(S, K, i, o, S.id[i], EOS ? S.rho[i] : (R)0);
 }
 
 // force pass: int_force pressure part (internal_force.f:178-259, 309-430),
@@ -765,10 +771,10 @@ __device__ __forceinline__ void force_pair(const KParams& K, ForceOwn<R>& o, R d
 }
 
 template <typename R, bool PRESS, bool XS, bool VI = false>
-__device__ __forceinline__ void force_end(St<R>& S, const KParams& K, int i, const ForceOwn<R>& o) {
+__device__ __forceinline__ void force_end(St<R>& S, const KParams& K, int i, const ForceOwn<R>& o,
+                                          int id) {
   using R2 = typename V2<R>::type;
   if (PRESS) {
-    const int id = S.id[i];
     const bool grav = (K.flags & 16) && id < K.np;
     R gx, gy;
     if constexpr (sizeof(R) == 4) {
@@ -799,6 +805,11 @@ __device__ __forceinline__ void force_end(St<R>& S, const KParams& K, int i, con
     w.y = o.xsy;
     S.av[i] = w;
   }
+}
+
+template <typename R, bool PRESS, bool XS, bool VI = false>
+__device__ __forceinline__ void force_end(St<R>& S, const KParams& K, int i, const ForceOwn<R>& o) {
+  force_end<R, PRESS, XS, VI>(S, K, i, o, PRESS ? S.id[i] : 0);
 }
 
 // The deposition heat source after the force pass, in the steps where it

@@ -73,11 +73,16 @@ template <int CAP> struct DensTile<float, CAP> {
   // the neighbour test reads one 16-byte record per candidate
   float4 a[CAP + TPAD];  // offx, offy, cell column as float, vx
   float vy[CAP + TPAD];
-  __device__ __forceinline__ void put(int l, const St<float>& S, const KParams&, int t) {
-    const float2 o = S.off[t];
-    const float2 v = S.v[t];
-    a[l] = make_float4(o.x, o.y, (float)(S.cxy[t] & 0xffffu), v.x);
-    vy[l] = v.y;
+  struct Raw {
+    float2 o, v;
+    uint32_t c;
+  };
+  static __device__ __forceinline__ Raw load(const St<float>& S, int t) {
+    return {S.off[t], S.v[t], S.cxy[t]};
+  }
+  __device__ __forceinline__ void put(int l, const KParams&, const Raw& r) {
+    a[l] = make_float4(r.o.x, r.o.y, (float)(r.c & 0xffffu), r.v.x);
+    vy[l] = r.v.y;
   }
   __device__ __forceinline__ LaneF lane(int l) const {
     const float4 q = a[l];
@@ -94,9 +99,15 @@ template <int CAP> struct DensTile<float, CAP> {
 };
 template <int CAP> struct DensTile<double, CAP> {
   double2 x[CAP + TPAD], v[CAP + TPAD];
-  __device__ __forceinline__ void put(int l, const St<double>& S, const KParams&, int t) {
-    x[l] = S.xy[t];
-    v[l] = S.v[t];
+  struct Raw {
+    double2 x, v;
+  };
+  static __device__ __forceinline__ Raw load(const St<double>& S, int t) {
+    return {S.xy[t], S.v[t]};
+  }
+  __device__ __forceinline__ void put(int l, const KParams&, const Raw& r) {
+    x[l] = r.x;
+    v[l] = r.v;
   }
   __device__ __forceinline__ PosD lane(int l) const {
     const double2 q = x[l];
@@ -111,15 +122,49 @@ template <int CAP> struct DensTile<double, CAP> {
   __device__ __forceinline__ double2 vel(int l) const { return v[l]; }
 };
 
+// Positions of the neighbour pre-test: x and y as 16-bit fixed-point numbers of
+// FIX units per cell, modulo 2^16 (a particle and its candidates are less than
+// three cells apart, so their difference is exact through the wrap), in one
+// 4-byte record: a candidate's test is a packed subtraction, a dot product
+// against the bound and a shift of the sign into the mask, three instructions
+// in either form, instead of the eight (FP32) or seven in FP64 (at half the
+// rate) of a test on the staged floating-point positions.
+constexpr int FIX = 4096;
+using s16x2 = __attribute__((ext_vector_type(2))) short;
+
+template <int CAP> struct PreTile {
+  uint32_t p[CAP + TPAD];
+  __device__ __forceinline__ void put(int l, const KParams& K,
+                                      const typename DensTile<float, CAP>::Raw& r) {
+    const uint32_t c = r.c;
+    const uint32_t x = (c & 0xffffu) * FIX + (uint32_t)(int)__builtin_fmaf(r.o.x, K.fixf, 0.5f);
+    const uint32_t y = (c >> 16) * FIX + (uint32_t)(int)__builtin_fmaf(r.o.y, K.fixf, 0.5f);
+    p[l] = (x & 0xffffu) | (y << 16);
+  }
+  __device__ __forceinline__ void put(int l, const KParams& K,
+                                      const typename DensTile<double, CAP>::Raw& r) {
+    auto fix = [&](double d) {
+      const double u = d * K.fix;
+      return (uint32_t)(int)(u - 65536.0 * floor(u * (1.0 / 65536.0)) + 0.5);
+    };
+    p[l] = (fix(r.x.x - K.ox) & 0xffffu) | (fix(r.x.y - K.oy) << 16);
+  }
+};
+
 // Neighbour W = c T of the physical viscosity, staged only when VI.
 template <typename R, int CAP, bool VI> struct TauTile {
-  __device__ __forceinline__ void put(int, const St<R>&, int, R) {}
+  struct Raw {};
+  static __device__ __forceinline__ Raw load(const St<R>&, int) { return {}; }
+  __device__ __forceinline__ void put(int, const Raw&, R) {}
   __device__ __forceinline__ Tau3<R> get(int) const { return Tau3<R>{}; }
 };
 template <int CAP> struct TauTile<float, CAP, true> {
   float4 w[CAP];
-  __device__ __forceinline__ void put(int l, const St<float>& S, int t, float c) {
-    const float4 q = reinterpret_cast<const float4*>(S.tau)[t];
+  using Raw = float4;
+  static __device__ __forceinline__ Raw load(const St<float>& S, int t) {
+    return reinterpret_cast<const float4*>(S.tau)[t];
+  }
+  __device__ __forceinline__ void put(int l, const Raw& q, float c) {
     w[l] = make_float4(c * q.x, c * q.y, c * q.z, q.w);
   }
   __device__ __forceinline__ Tau3<float> get(int l) const {
@@ -130,10 +175,16 @@ template <int CAP> struct TauTile<float, CAP, true> {
 template <int CAP> struct TauTile<double, CAP, true> {
   double2 w01[CAP];
   double w2[CAP];
-  __device__ __forceinline__ void put(int l, const St<double>& S, int t, double c) {
+  struct Raw {
+    double xx, yy, xy;
+  };
+  static __device__ __forceinline__ Raw load(const St<double>& S, int t) {
     const double* q = S.tau + 4 * (size_t)t;
-    w01[l] = make_double2(c * q[0], c * q[1]);
-    w2[l] = c * q[2];
+    return {q[0], q[1], q[2]};
+  }
+  __device__ __forceinline__ void put(int l, const Raw& q, double c) {
+    w01[l] = make_double2(c * q.xx, c * q.yy);
+    w2[l] = c * q.xy;
   }
   __device__ __forceinline__ Tau3<double> get(int l) const {
     const double2 q = w01[l];
@@ -141,21 +192,51 @@ template <int CAP> struct TauTile<double, CAP, true> {
   }
 };
 
+// The particle's own viscous terms: W from its record, tds from the state.
+template <typename R>
+__device__ __forceinline__ void own_tau(const St<R>& S, ForceOwn<R>& o, int i, const Tau3<R>& w) {
+  o.wxx = w.xx;
+  o.wyy = w.yy;
+  o.wxy = w.xy;
+  o.tds = S.tau[4 * (size_t)i + 3];
+}
+
 template <typename R, int CAP, bool VI = false> struct ForceTile;
 template <int CAP, bool VI> struct ForceTile<float, CAP, VI> {
   float4 a[CAP + TPAD];  // offx, offy, vx, vy
   float4 b[CAP + TPAD];  // Q = 1/rho, A = p/rho, psi, u
   float cx[CAP + TPAD];  // cell column as float
   TauTile<float, CAP + TPAD, VI> tw;
-  __device__ __forceinline__ void put(int l, const St<float>& S, const KParams& K, int t, int) {
-    const float2 o = S.off[t];
-    const float2 v = S.v[t];
-    a[l] = make_float4(o.x, o.y, v.x, v.y);
+  struct Raw {
+    float2 o, v;
+    float rho, p, psi, u;
+    uint32_t c;
+    typename TauTile<float, CAP + TPAD, VI>::Raw w;
+  };
+  static __device__ __forceinline__ Raw load(const St<float>& S, int t) {
+    return {S.off[t], S.v[t],  S.rho[t], S.p[t],
+            S.psi[t], S.uf[t], S.cxy[t], TauTile<float, CAP + TPAD, VI>::load(S, t)};
+  }
+  __device__ __forceinline__ void put(int l, const KParams& K, const Raw& r) {
+    a[l] = make_float4(r.o.x, r.o.y, r.v.x, r.v.y);
     float Q, A;
-    q_and_a(K, S.rho[t], S.p[t], Q, A);
-    b[l] = make_float4(Q, A, S.psi[t], S.uf[t]);
-    cx[l] = (float)(S.cxy[t] & 0xffffu);
-    tw.put(l, S, t, visc_c(K, Q));
+    q_and_a(K, r.rho, r.p, Q, A);
+    b[l] = make_float4(Q, A, r.psi, r.u);
+    cx[l] = (float)(r.c & 0xffffu);
+    tw.put(l, r.w, visc_c(K, Q));
+  }
+  // force_begin from the particle's own record
+  __device__ __forceinline__ void own(const St<float>& S, const KParams& K, ForceOwn<float>& o,
+                                      int i, int l) const {
+    const float4 q = a[l];
+    const float4 w = b[l];
+    o.v = make_float2(q.z, q.w);
+    o.Q = w.x;
+    o.A = w.y;
+    o.psi = w.z;
+    o.u = w.w;
+    own_factors_f32(K, o);
+    if (VI) own_tau(S, o, i, tw.get(l));
   }
   __device__ __forceinline__ LaneF lane(int l) const {
     const float4 q = a[l];
@@ -178,14 +259,32 @@ template <int CAP, bool VI> struct ForceTile<float, CAP, VI> {
 template <int CAP, bool VI> struct ForceTile<double, CAP, VI> {
   double2 x[CAP + TPAD], v[CAP + TPAD], rp[CAP + TPAD], pu[CAP + TPAD];  // rp = (Q, A), pu = (psi, u)
   TauTile<double, CAP + TPAD, VI> tw;
-  __device__ __forceinline__ void put(int l, const St<double>& S, const KParams& K, int t, int) {
-    x[l] = S.xy[t];
-    v[l] = S.v[t];
+  struct Raw {
+    double2 x, v;
+    double rho, p, psi, u;
+    typename TauTile<double, CAP + TPAD, VI>::Raw w;
+  };
+  static __device__ __forceinline__ Raw load(const St<double>& S, int t) {
+    return {S.xy[t],  S.v[t], S.rho[t], S.p[t],
+            S.psi[t], S.u[t], TauTile<double, CAP + TPAD, VI>::load(S, t)};
+  }
+  __device__ __forceinline__ void put(int l, const KParams& K, const Raw& r) {
+    x[l] = r.x;
+    v[l] = r.v;
     double Q, A;
-    q_and_a(K, S.rho[t], S.p[t], Q, A);
+    q_and_a(K, r.rho, r.p, Q, A);
     rp[l] = make_double2(Q, A);
-    pu[l] = make_double2(S.psi[t], S.u[t]);
-    tw.put(l, S, t, visc_c(K, Q));
+    pu[l] = make_double2(r.psi, r.u);
+    tw.put(l, r.w, visc_c(K, Q));
+  }
+  __device__ __forceinline__ void own(const St<double>& S, const KParams&, ForceOwn<double>& o,
+                                      int i, int l) const {
+    o.v = v[l];
+    o.Q = rp[l].x;
+    o.A = rp[l].y;
+    o.psi = pu[l].x;
+    o.u = pu[l].y;
+    if (VI) own_tau(S, o, i, tw.get(l));
   }
   __device__ __forceinline__ PosD lane(int l) const {
     const double2 q = x[l];
@@ -212,9 +311,16 @@ template <int CAP, bool VI> struct ForceTile<double, CAP, VI> {
 template <typename R, int CAP> struct TensTile {
   DensTile<R, CAP> d;
   R q[CAP + TPAD];
-  __device__ __forceinline__ void put(int l, const St<R>& S, const KParams& K, int t) {
-    d.put(l, S, K, t);
-    q[l] = (R)1 / dens(K, S.rho[t]);
+  struct Raw {
+    typename DensTile<R, CAP>::Raw d;
+    R rho;
+  };
+  static __device__ __forceinline__ Raw load(const St<R>& S, int t) {
+    return {DensTile<R, CAP>::load(S, t), S.rho[t]};
+  }
+  __device__ __forceinline__ void put(int l, const KParams& K, const Raw& r) {
+    d.put(l, K, r.d);
+    q[l] = (R)1 / dens(K, r.rho);
   }
   __device__ __forceinline__ auto lane(int l) const { return d.lane(l); }
   template <typename LP>
@@ -239,13 +345,11 @@ struct Segment {
 //  CW > 0: a fixed run of CW cells of a row (segment row * nseg + run).
 //  CW = 0: a piece of at most PIECE consecutive sorted positions of one row
 //          (RowPieces); every wavefront of a piece but the row's last is
-//          full.  The first ny workgroups take the parts cut from the rows'
-//          pieces (most rows have none).
+//          full.
 struct SegArg {
   int nseg;
-  const int4* pieces;
-  const int2* cuts;
-  const int* npieces;
+  const PieceRec* tab;
+  int masks;  // the density pass has recorded the neighbour masks
 };
 
 // Width of the LDS copy of the cell starts (none for pieces, whose cells are
@@ -276,66 +380,163 @@ __device__ __forceinline__ CellBounds<CW> bounds_of(const KParams& K, const Segm
     return CellBounds<0>{cstart, (g.cy - 1) * K.nx, K.nx};
 }
 
+// A lane particle's cell column and its candidates [ta_k, tb_k) of row k
+// (sorted positions; empty for a row outside the grid).  On pieces a lane
+// looks them up before the tile is filled, so that the two loads they take
+// one after the other run beside the staging.
+struct LaneRows {
+  int cx;
+  int ta[3], tb[3];
+};
+template <typename BD>
+__device__ __forceinline__ LaneRows lane_rows(const KParams& K, const Segment& g, const BD& B,
+                                              uint32_t key) {
+  LaneRows r;
+  r.cx = (int)key - g.cy * K.nx;
+  const int ca = r.cx > 0 ? r.cx - 1 : 0;
+  const int cb = (r.cx + 1 < K.nx ? r.cx + 1 : K.nx - 1) + 1;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int kk = g.rl[k] ? k : 1;
+    const int a = B.at(kk, ca), b = B.at(kk, cb);
+    r.ta[k] = g.rl[k] ? a : 0;
+    r.tb[k] = g.rl[k] ? b : 0;
+  }
+  return r;
+}
+
 // The segment of this workgroup; O0 >= O1 when it has no particles.  With
 // CW > 0 the workgroup also copies the cell starts of its rows into cs.
 template <int CW>
 __device__ __forceinline__ Segment segment_of(const KParams& K, const int* __restrict__ cstart,
-                                              const uint32_t* __restrict__ skey,
                                               const SegArg& sa, int (*cs)[csw<CW>()]) {
   Segment g;
-  const int nx = K.nx;
-  int cx0, cx1;  // the particles' cells: cx0 .. cx1-1
   if constexpr (CW > 0) {
     // plain order: most cell runs of a tank are empty, and contiguous
     // shares per XCD would leave the XCDs of the empty rows idle
+    const int nx = K.nx;
     g.cy = blockIdx.x / sa.nseg;
-    cx0 = (blockIdx.x - g.cy * sa.nseg) * CW;
-    cx1 = min(cx0 + CW, nx);
+    const int cx0 = (blockIdx.x - g.cy * sa.nseg) * CW;
+    const int cx1 = min(cx0 + CW, nx);
     g.O0 = cstart[g.cy * nx + cx0];
     g.O1 = cstart[g.cy * nx + cx1];
-  } else {
-    // pieces in even XCD-contiguous shares: neighbouring pieces, which stage
-    // the same rows, share an L2 (the grid is a bound on the piece count)
-    g.cy = g.O0 = g.O1 = 0;
-    if ((int)blockIdx.x < K.ny) {
-      const int2 cut = sa.cuts[blockIdx.x];
-      g.cy = blockIdx.x;
-      g.O0 = cut.x;
-      g.O1 = cut.y;
-    } else {
-      const int sb = xcd_share(*sa.npieces, (int)blockIdx.x - K.ny);
-      if (sb >= 0) {
-        const int4 pc = sa.pieces[sb];
-        g.cy = pc.y;
-        g.O0 = pc.x;
-        g.O1 = pc.z;
-      }
-    }
-    if (g.O0 >= g.O1) return g;
-    cx0 = (int)skey[g.O0] - g.cy * nx;
-    cx1 = (int)skey[g.O1 - 1] - g.cy * nx + 1;
-  }
-  g.slo = cx0 > 0 ? cx0 - 1 : 0;
-  const int shi = cx1 < nx ? cx1 : nx - 1;
-  g.total = 0;
+    g.slo = cx0 > 0 ? cx0 - 1 : 0;
+    const int shi = cx1 < nx ? cx1 : nx - 1;
+    g.total = 0;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const int ry = g.cy - 1 + k;
-    if (ry < 0 || ry >= K.ny || g.O0 >= g.O1) {
-      g.rs[k] = 0;
-      g.rl[k] = 0;
-    } else {
-      g.rs[k] = cstart[ry * nx + g.slo];
-      g.rl[k] = cstart[ry * nx + shi + 1] - g.rs[k];
-      if constexpr (CW > 0) {
+    for (int k = 0; k < 3; ++k) {
+      const int ry = g.cy - 1 + k;
+      if (ry < 0 || ry >= K.ny || g.O0 >= g.O1) {
+        g.rs[k] = 0;
+        g.rl[k] = 0;
+      } else {
+        g.rs[k] = cstart[ry * nx + g.slo];
+        g.rl[k] = cstart[ry * nx + shi + 1] - g.rs[k];
         const int ncs = shi + 2 - g.slo;
         for (int j = threadIdx.x; j < ncs; j += blockDim.x) cs[k][j] = cstart[ry * nx + g.slo + j];
       }
+      g.lo[k] = g.total;
+      g.total += g.rl[k];
     }
-    g.lo[k] = g.total;
-    g.total += g.rl[k];
+  } else {
+    const PieceRec r = sa.tab[blockIdx.x];
+    g.cy = r.cy;
+    g.slo = 0;
+    g.O0 = r.O0;
+    g.O1 = r.O1;
+    g.total = r.total;
+    int l = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      g.rs[k] = r.rs[k];
+      g.rl[k] = r.rl[k];
+      g.lo[k] = l;
+      l += r.rl[k];
+    }
   }
   return g;
+}
+
+// Tile entries q0 + u BLK + lane, u < UN, of the three rows, read (load(t): the
+// record of sorted position t) before any is written (put(l, record)), so that
+// filling a tile waits for memory once or twice.  Past the last entry the last
+// one is read and written again: no branch for the compiler to move the loads
+// into.
+template <int BLK, int UN, typename Raw> struct Stage {
+  Raw r[UN];
+  template <typename Load>
+  __device__ __forceinline__ void load(const Segment& g, int q0, Load&& ld) {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int q = at(g, q0, u);
+      int t = q + g.rs[0];
+      t += q >= g.lo[1] ? g.rs[1] - g.lo[1] - g.rs[0] : 0;
+      t += q >= g.lo[2] ? g.rs[2] - g.lo[2] - (g.rs[1] - g.lo[1]) : 0;
+      r[u] = ld(t);
+    }
+  }
+  template <typename Put>
+  __device__ __forceinline__ void put(const Segment& g, int q0, Put&& pt) const {
+#pragma unroll
+    for (int u = 0; u < UN; ++u) pt(at(g, q0, u), r[u]);
+  }
+  static __device__ __forceinline__ int at(const Segment& g, int q0, int u) {
+    return min(q0 + u * BLK + (int)threadIdx.x, g.total - 1);
+  }
+};
+
+// The batches after the first.
+template <int BLK, int UN, typename Raw, typename Load, typename Put>
+__device__ __forceinline__ void stage_rest(const Segment& g, Load&& ld, Put&& pt) {
+  for (int q0 = UN * BLK; q0 < g.total; q0 += UN * BLK) {
+    Stage<BLK, UN, Raw> st;
+    st.load(g, q0, ld);
+    st.put(g, q0, pt);
+  }
+}
+
+// Fills the tile (if tiled), then calls lane(i, key, rows) for the workgroup's
+// particles, one lane each; early(i) loads what else lane() needs.  On pieces
+// (CW = 0) every lane has at most one particle, and its key, its rows and
+// early() are read beside the tile's records: after the piece's record that
+// takes two dependent loads, where a chain of staging, key and cell bounds
+// takes six, most of a workgroup's life on the small tiles of 2D.
+template <int CW, int BLK, int UN, typename Raw, typename BD, typename Early, typename Load,
+          typename Put, typename Lane>
+__device__ __forceinline__ void for_segment(const KParams& K, const Segment& g, const BD& B,
+                                            const uint32_t* __restrict__ skey, bool tiled,
+                                            Early&& early, Load&& ld, Put&& pt, Lane&& lane) {
+  if constexpr (CW == 0) {
+    static_assert(BLK >= PIECE, "a lane for every particle of a piece");
+    const int i = g.O0 + (int)threadIdx.x;
+    const int ic = min(i, g.O1 - 1);
+    const uint32_t key = skey[ic];
+    Stage<BLK, UN, Raw> st;
+    st.load(g, 0, ld);
+    early(ic);
+    const LaneRows r = lane_rows(K, g, B, key);
+    if (tiled) {
+      st.put(g, 0, pt);
+      stage_rest<BLK, UN, Raw>(g, ld, pt);
+    }
+    __syncthreads();
+    if (i < g.O1) lane(i, key, r);
+  } else {
+    if (tiled) {
+      Stage<BLK, UN, Raw> st;
+      st.load(g, 0, ld);
+      st.put(g, 0, pt);
+      stage_rest<BLK, UN, Raw>(g, ld, pt);
+    }
+    __syncthreads();
+    for (int i0 = g.O0; i0 < g.O1; i0 += BLK) {
+      const int i = i0 + threadIdx.x;
+      if (i >= g.O1) continue;
+      const uint32_t key = skey[i];
+      early(i);
+      lane(i, key, lane_rows(K, g, B, key));
+    }
+  }
 }
 
 // The row pieces on their own (after a sort that does not build them).
@@ -343,7 +544,7 @@ __global__ __launch_bounds__(BLOCK) void k_row_pieces(const int* __restrict__ cs
                                                       const uint32_t* __restrict__ skey,
                                                       RowPieces rp, Halt hl) {
   if (hl.on()) return;
-  row_pieces_block<BLOCK>(cstart, skey, rp, blockIdx.x);
+  row_pieces_block<BLOCK>(cstart, skey, rp, blockIdx.x, gridDim.x);
 }
 
 // A particle of the first or last cell column of a grid periodic in x: its
@@ -382,31 +583,20 @@ __device__ __forceinline__ uint32_t row_mask(const KParams& K, const Tile& T, co
 
 // Calls visit(l, uy) for every neighbour of lane particle i, rows bottom to
 // top, ascending sorted position within a row (uy: the cell-row term of the
-// row).  With rm != nullptr it also returns the neighbour masks of the three
-// rows (bit b = candidate ta_k + b) and whether they are complete (every
-// row at most 32 candidates).
-template <typename R, typename BD, typename Tile, typename LP, typename Visit>
-__device__ __forceinline__ void for_neighbours(const KParams& K, const Segment& g, const BD& B,
-                                               const Tile& T, const LP& pi, int i, uint32_t key,
-                                               Visit&& visit, uint32_t* rm = nullptr,
-                                               bool* ok = nullptr) {
-  const int nx = K.nx;
-  const int cx = (int)key - g.cy * nx;
-  const int ca = cx > 0 ? cx - 1 : 0;
-  const int cb = (cx + 1 < nx ? cx + 1 : nx - 1) + 1;
+// row).
+template <typename R, typename Tile, typename LP, typename Visit>
+__device__ __forceinline__ void for_neighbours(const KParams& K, const Segment& g,
+                                               const LaneRows& lr, const Tile& T, const LP& pi,
+                                               int i, Visit&& visit) {
   const int self = g.lo[1] + (i - g.rs[1]);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     if (g.rl[k] == 0) continue;
     const R uy = (R)row_uy(K, k);
-    const int ta = B.at(k, ca);
-    const int tb = B.at(k, cb);
     const int base = g.lo[k] - g.rs[k];
-    if (rm && tb - ta > 32) *ok = false;
-    for (int c0 = ta; c0 < tb; c0 += 32) {
-      const int len = min(32, tb - c0);
+    for (int c0 = lr.ta[k]; c0 < lr.tb[k]; c0 += 32) {
+      const int len = min(32, lr.tb[k] - c0);
       uint32_t m = row_mask<R>(K, T, pi, uy, base + c0, len, self);
-      if (rm && c0 == ta) rm[k] = m;
       while (m) {
         const int b = __builtin_ctz(m);
         m &= m - 1;
@@ -465,64 +655,21 @@ __device__ __forceinline__ void walk_rows(uint32_t m0, uint32_t m1, uint32_t m2,
   }
 }
 
-// for_neighbours with the masks of all three rows built first and one walk
-// over them (walk_rows): the same visits in the same order, but a wavefront
-// runs for its longest lane's neighbour count rather than for the sum over
-// the rows of the per-row maxima.  A particle with a row of more than 32
-// candidates takes for_neighbours.  The masks go to rm.
-template <typename R, typename BD, typename Tile, typename LP, typename Visit>
-__device__ __forceinline__ void for_neighbours_rows(const KParams& K, const Segment& g,
-                                                    const BD& B, const Tile& T, const LP& pi,
-                                                    int i, uint32_t key, Visit&& visit,
-                                                    uint32_t* rm, bool* ok) {
-  const int nx = K.nx;
-  const int cx = (int)key - g.cy * nx;
-  const int ca = cx > 0 ? cx - 1 : 0;
-  const int cb = (cx + 1 < nx ? cx + 1 : nx - 1) + 1;
-  const int self = g.lo[1] + (i - g.rs[1]);
-  uint32_t m[3];
-  int l[3];
-  bool small = true;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    m[k] = 0u;
-    l[k] = 0;
-    if (g.rl[k] == 0) continue;
-    const int ta = B.at(k, ca);
-    const int tb = B.at(k, cb);
-    l[k] = g.lo[k] - g.rs[k] + ta;
-    small = small && tb - ta <= 32;
-    m[k] = row_mask<R>(K, T, pi, (R)row_uy(K, k), l[k], min(32, tb - ta), self);
-  }
-  if (!small) {
-    for_neighbours<R>(K, g, B, T, pi, i, key, visit, rm, ok);
-    return;
-  }
-  walk_rows(m[0], m[1], m[2], l[0], l[1], l[2], (R)row_uy(K, 0), (R)row_uy(K, 1),
-            (R)row_uy(K, 2), visit);
-  rm[0] = m[0];
-  rm[1] = m[1];
-  rm[2] = m[2];
-}
-
-// FP32 density pass: the neighbour pre-test of candidates l0 .. l0+len-1
-// (len <= 32) of one row against K.pre2f, with x = cx cell + off rounded
-// once per record (xi, yi: the lane's x, and its y plus the row term); the
-// survivors take the exact test in dens_walk_f32.
+// The pre-test of candidates l0 .. l0+len-1 (len <= 32) of one row against
+// K.fix2, a bound on (2h)^2 in units of the fixed-point positions (own: the
+// lane's) that covers their rounding; the survivors (about one in two thousand
+// too many) take the exact test in the walk.
 template <int CAP>
-__device__ __forceinline__ uint32_t row_mask_pre(const KParams& K, const DensTile<float, CAP>& T,
-                                                 float xi, float yi, int l0, int len, int self) {
-  const float pre2 = K.pre2f, cellf = K.cellf;
+__device__ __forceinline__ uint32_t row_mask_pre(const KParams& K, const PreTile<CAP>& P, s16x2 own,
+                                                 int l0, int len, int self) {
+  const int bound = -K.fix2;
   uint32_t m = 0;
   for (int k0 = 0; k0 < len; k0 += 8) {
     uint32_t bb = 0u;  // the batch's bits, placed once
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const float4 a = T.a[l0 + k0 + q];
-      const float dx = xi - __builtin_fmaf(a.z, cellf, a.x);
-      const float dy = yi - a.y;
-      const float r2 = __builtin_fmaf(dx, dx, dy * dy);
-      bb |= (r2 < pre2 ? 1u : 0u) << q;
+    for (int q = 7; q >= 0; --q) {
+      const s16x2 d = own - __builtin_bit_cast(s16x2, P.p[l0 + k0 + q]);
+      bb = __builtin_amdgcn_alignbit(bb, (uint32_t)__builtin_amdgcn_sdot2(d, d, bound, false), 31);
     }
     m |= bb << k0;
   }
@@ -532,72 +679,62 @@ __device__ __forceinline__ uint32_t row_mask_pre(const KParams& K, const DensTil
   return m;
 }
 
-// for_neighbours of the FP32 density pass, row by row: the pre-test, then over
-// its survivors the exact test (r^2 < (2h)^2 with the direct path's
-// arithmetic) and the pair sums, without a branch: a survivor that fails the
-// exact test adds nothing (dens_pair with ok = false) and leaves the recorded
-// mask.  Same visiting order and sums as for_neighbours; the exact masks in rm.
-// Taken by dens_walk_f32 for a particle with a row of more than 32 candidates.
-template <bool SUM, int CAP, typename BD>
-__device__ __forceinline__ void dens_walk_rows_f32(const KParams& K, const Segment& g, const BD& B,
-                                              const DensTile<float, CAP>& T, const LaneF& pi,
-                                              float2 vi, int i, uint32_t key, DensOwn<float>& o,
-                                              uint32_t* rm, bool* ok) {
-  const int nx = K.nx;
-  const int cx = (int)key - g.cy * nx;
-  const int ca = cx > 0 ? cx - 1 : 0;
-  const int cb = (cx + 1 < nx ? cx + 1 : nx - 1) + 1;
+// for_neighbours of the density pass, row by row: the pre-test, then over its
+// survivors the exact test (r^2 < (2h)^2 with the direct path's arithmetic)
+// and the pair sums, without a branch: a survivor that fails the exact test
+// adds nothing (dens_pair with ok = false) and leaves the recorded mask.
+// Same visiting order and sums as for_neighbours; the exact masks in rm.
+// Taken by dens_walk for a particle with a row of more than 32 candidates.
+template <typename R, bool SUM, int CAP, typename LP, typename V>
+__device__ __forceinline__ void dens_walk_rows(const KParams& K, const Segment& g, const LaneRows& lr,
+                                               const DensTile<R, CAP>& T, const PreTile<CAP>& P,
+                                               const LP& pi, const V& vi, int i, DensOwn<R>& o,
+                                               uint32_t* rm, bool* ok) {
   const int self = g.lo[1] + (i - g.rs[1]);
-  const float cut2 = K.cut2f;
-  const float xi = __builtin_fmaf(pi.cxf, K.cellf, pi.ox);
+  const R cut2 = cutoff2<R>(K);
+  const s16x2 own = __builtin_bit_cast(s16x2, P.p[self]);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     if (g.rl[k] == 0) continue;
-    const float uy = row_uy(K, k);
-    const float yi = pi.oy + uy;
-    const int ta = B.at(k, ca);
-    const int tb = B.at(k, cb);
+    const R uy = (R)row_uy(K, k);
+    const int ta = lr.ta[k], tb = lr.tb[k];
     const int base = g.lo[k] - g.rs[k];
     if (tb - ta > 32) *ok = false;
     for (int c0 = ta; c0 < tb; c0 += 32) {
       const int len = min(32, tb - c0);
-      uint32_t m = row_mask_pre(K, T, xi, yi, base + c0, len, self);
+      uint32_t m = row_mask_pre(K, P, own, base + c0, len, self);
       uint32_t w = m;
       while (w) {
         const int b = __builtin_ctz(w);
         w &= w - 1;
         const int l = base + c0 + b;
-        float dx, dy;
+        R dx, dy;
         T.delta(K, pi, l, uy, dx, dy);
-        const float r2 = dx * dx + dy * dy;
+        const R r2 = dx * dx + dy * dy;
         const bool in = r2 < cut2;
         m = in ? m : (m & ~(1u << b));
-        const float2 vj = T.vel(l);
-        dens_pair<float, SUM>(K, dx, dy, r2, vi.x - vj.x, vi.y - vj.y, o.sum, o.rs, in);
+        const auto vj = T.vel(l);
+        dens_pair<R, SUM>(K, dx, dy, r2, vi.x - vj.x, vi.y - vj.y, o.sum, o.rs, in);
       }
       if (c0 == ta) rm[k] = m;
     }
   }
 }
 
-// The FP32 density walk: the pre-test of all three rows first, then one loop
-// over the survivors of the three masks in row order (so that a wavefront
-// runs for its longest lane's survivor count, not for the sum over the rows
-// of the per-row maxima), each through the exact test and the pair sums
-// without a branch.  Failed survivors are collected per row (fc, flushed at
-// each row change) and taken out of the recorded masks.  Same visiting order
-// and sums as for_neighbours; the exact masks in rm.
-template <bool SUM, int CAP, typename BD>
-__device__ __forceinline__ void dens_walk_f32(const KParams& K, const Segment& g, const BD& B,
-                                              const DensTile<float, CAP>& T, const LaneF& pi,
-                                              float2 vi, int i, uint32_t key, DensOwn<float>& o,
-                                              uint32_t* rm, bool* ok) {
-  const int nx = K.nx;
-  const int cx = (int)key - g.cy * nx;
-  const int ca = cx > 0 ? cx - 1 : 0;
-  const int cb = (cx + 1 < nx ? cx + 1 : nx - 1) + 1;
+// The density walk: the pre-test of all three rows first, then one loop over
+// the survivors of the three masks in row order (so that a wavefront runs for
+// its longest lane's survivor count, not for the sum over the rows of the
+// per-row maxima), each through the exact test and the pair sums without a
+// branch.  Failed survivors are collected per row (fc, flushed at each row
+// change) and taken out of the recorded masks.  Same visiting order and sums
+// as for_neighbours; the exact masks in rm.
+template <typename R, bool SUM, int CAP, typename LP, typename V>
+__device__ __forceinline__ void dens_walk(const KParams& K, const Segment& g, const LaneRows& lr,
+                                          const DensTile<R, CAP>& T, const PreTile<CAP>& P,
+                                          const LP& pi, const V& vi, int i, DensOwn<R>& o,
+                                          uint32_t* rm, bool* ok) {
   const int self = g.lo[1] + (i - g.rs[1]);
-  const float xi = __builtin_fmaf(pi.cxf, K.cellf, pi.ox);
+  const s16x2 own = __builtin_bit_cast(s16x2, P.p[self]);
   uint32_t pm[3];
   int pb[3];
   bool small = true;
@@ -606,22 +743,21 @@ __device__ __forceinline__ void dens_walk_f32(const KParams& K, const Segment& g
     pm[k] = 0u;
     pb[k] = 0;
     if (g.rl[k] == 0) continue;
-    const int ta = B.at(k, ca);
-    const int tb = B.at(k, cb);
+    const int ta = lr.ta[k], tb = lr.tb[k];
     pb[k] = g.lo[k] - g.rs[k] + ta;
     small = small && tb - ta <= 32;
-    pm[k] = row_mask_pre(K, T, xi, pi.oy + row_uy(K, k), pb[k], min(32, tb - ta), self);
+    pm[k] = row_mask_pre(K, P, own, pb[k], min(32, tb - ta), self);
   }
   if (!small) {
-    dens_walk_rows_f32<SUM>(K, g, B, T, pi, vi, i, key, o, rm, ok);
+    dens_walk_rows<R, SUM>(K, g, lr, T, P, pi, vi, i, o, rm, ok);
     return;
   }
-  const float cut2 = K.cut2f;
+  const R cut2 = cutoff2<R>(K);
   uint32_t f0 = 0u, f1 = 0u, f2 = 0u, fc = 0u;  // failed survivors: rows 0..2, current row
   int kc = 0;
   uint32_t m = pm[0];
   int base = pb[0];
-  float uy = row_uy(K, 0);
+  R uy = (R)row_uy(K, 0);
   while (true) {
     if (m == 0u) {
       f0 |= kc == 0 ? fc : 0u;
@@ -634,18 +770,18 @@ __device__ __forceinline__ void dens_walk_f32(const KParams& K, const Segment& g
       kc = t1 ? 1 : 2;
       m = t1 ? pm[1] : pm[2];
       base = t1 ? pb[1] : pb[2];
-      uy = t1 ? row_uy(K, 1) : row_uy(K, 2);
+      uy = t1 ? (R)row_uy(K, 1) : (R)row_uy(K, 2);
     }
     const int b = (int)__builtin_ctz(m);
     m &= m - 1u;
     const int l = base + b;
-    float dx, dy;
+    R dx, dy;
     T.delta(K, pi, l, uy, dx, dy);
-    const float r2 = dx * dx + dy * dy;
+    const R r2 = dx * dx + dy * dy;
     const bool in = r2 < cut2;
     fc |= in ? 0u : (1u << b);
-    const float2 vj = T.vel(l);
-    dens_pair<float, SUM>(K, dx, dy, r2, vi.x - vj.x, vi.y - vj.y, o.sum, o.rs, in);
+    const auto vj = T.vel(l);
+    dens_pair<R, SUM>(K, dx, dy, r2, vi.x - vj.x, vi.y - vj.y, o.sum, o.rs, in);
   }
   rm[0] = pm[0] & ~f0;
   rm[1] = pm[1] & ~f1;
@@ -654,28 +790,21 @@ __device__ __forceinline__ void dens_walk_f32(const KParams& K, const Segment& g
 
 // The same walk driven by masks recorded by the density pass.
 // (Rows outside the grid have empty masks: their entries are not looked up.)
-template <typename R, typename BD, typename Visit>
-__device__ __forceinline__ void for_masked(const KParams& K, const Segment& g, const BD& B,
-                                           uint32_t key, uint4 nm, Visit&& visit) {
-  const int nx = K.nx;
-  const int cx = (int)key - g.cy * nx;
-  const int ca = cx > 0 ? cx - 1 : 0;
-  walk_masks<R>(K, nm.x, nm.y, nm.z, g.rl[0] ? g.lo[0] - g.rs[0] + B.at(0, ca) : 0,
-                g.lo[1] - g.rs[1] + B.at(1, ca), g.rl[2] ? g.lo[2] - g.rs[2] + B.at(2, ca) : 0,
-                visit);
+template <typename R, typename Visit>
+__device__ __forceinline__ void for_masked(const KParams& K, const Segment& g, const LaneRows& lr,
+                                           uint4 nm, Visit&& visit) {
+  walk_masks<R>(K, nm.x, nm.y, nm.z, g.lo[0] - g.rs[0] + lr.ta[0], g.lo[1] - g.rs[1] + lr.ta[1],
+                g.lo[2] - g.rs[2] + lr.ta[2], visit);
 }
 
 // The same with walk_rows (a bit scan per neighbour, the row change only
 // where a lane needs it).
-template <typename R, typename BD, typename Visit>
-__device__ __forceinline__ void for_masked_rows(const KParams& K, const Segment& g, const BD& B,
-                                                uint32_t key, uint4 nm, Visit&& visit) {
-  const int nx = K.nx;
-  const int cx = (int)key - g.cy * nx;
-  const int ca = cx > 0 ? cx - 1 : 0;
-  walk_rows(nm.x, nm.y, nm.z, g.rl[0] ? g.lo[0] - g.rs[0] + B.at(0, ca) : 0,
-            g.lo[1] - g.rs[1] + B.at(1, ca), g.rl[2] ? g.lo[2] - g.rs[2] + B.at(2, ca) : 0,
-            (R)row_uy(K, 0), (R)row_uy(K, 1), (R)row_uy(K, 2), visit);
+template <typename R, typename Visit>
+__device__ __forceinline__ void for_masked_rows(const KParams& K, const Segment& g,
+                                                const LaneRows& lr, uint4 nm, Visit&& visit) {
+  walk_rows(nm.x, nm.y, nm.z, g.lo[0] - g.rs[0] + lr.ta[0], g.lo[1] - g.rs[1] + lr.ta[1],
+            g.lo[2] - g.rs[2] + lr.ta[2], (R)row_uy(K, 0), (R)row_uy(K, 1), (R)row_uy(K, 2),
+            visit);
 }
 
 template <typename R, bool SUM, bool EOS, bool PER, int BLK, int CW, int CAP>
@@ -683,50 +812,43 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
                                                        const uint32_t* __restrict__ skey,
                                                        const int* __restrict__ cstart, SegArg sa,
                                                        uint4* __restrict__ nbm) {
-  if (halted(K)) return;
   __shared__ DensTile<R, CAP> T;
+  __shared__ PreTile<CAP> P;
   __shared__ int cs[3][csw<CW>()];
-  const Segment g = segment_of<CW>(K, cstart, skey, sa, cs);
-  if (g.O0 >= g.O1) return;
+  const Segment g = segment_of<CW>(K, cstart, sa, cs);
+  if (halted(K) || g.O0 >= g.O1) return;
   const auto B = bounds_of<CW>(K, g, cstart, cs);
   const bool tiled = g.total <= CAP;
-  if (tiled) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      for (int q = threadIdx.x; q < g.rl[k]; q += BLK) T.put(g.lo[k] + q, S, K, g.rs[k] + q);
-  }
-  __syncthreads();
-  for (int i0 = g.O0; i0 < g.O1; i0 += BLK) {
-    const int i = i0 + threadIdx.x;
-    if (i >= g.O1) continue;
-    if (!tiled || seam<PER>(K, g, skey[i])) {
-      density_direct<R, SUM, EOS, PER>(S, K, i, skey, cstart, nbm);
-      continue;
-    }
-    const int self = g.lo[1] + (i - g.rs[1]);
-    const auto pi = T.lane(self);
-    const auto vi = T.vel(self);
-    DensOwn<R> o;
-    dens_begin<R, SUM>(K, o);
-    uint32_t rm[3] = {0u, 0u, 0u};
-    bool ok = true;
-    if constexpr (sizeof(R) == 4) {
-      dens_walk_f32<SUM>(K, g, B, T, pi, vi, i, skey[i], o, rm, &ok);
-    } else {
-      for_neighbours_rows<R>(
-          K, g, B, T, pi, i, skey[i],
-          [&](int l, R uy) {
-            R dx, dy;
-            T.delta(K, pi, l, uy, dx, dy);
-            const R r2 = dx * dx + dy * dy;
-            const auto vj = T.vel(l);
-            dens_pair<R, SUM>(K, dx, dy, r2, vi.x - vj.x, vi.y - vj.y, o.sum, o.rs);
-          },
-          rm, &ok);
-    }
-    nbm[i] = make_uint4(rm[0], rm[1], rm[2], ok ? 1u : 0u);
-    dens_end<R, SUM, EOS>(S, K, i, o);
-  }
+  using Raw = typename DensTile<R, CAP>::Raw;
+  int id = 0;
+  R rho = (R)0;
+  for_segment<CW, BLK, 4, Raw>(
+      K, g, B, skey, tiled,
+      [&](int i) {
+        id = S.id[i];
+        if (EOS) rho = S.rho[i];
+      },
+      [&](int t) { return T.load(S, t); },
+      [&](int l, const Raw& r) {
+        T.put(l, K, r);
+        P.put(l, K, r);
+      },
+      [&](int i, uint32_t key, const LaneRows& lr) {
+        if (!tiled || seam<PER>(K, g, key)) {
+          density_direct<R, SUM, EOS, PER>(S, K, i, skey, cstart, nbm);
+          return;
+        }
+        const int self = g.lo[1] + (i - g.rs[1]);
+        const auto pi = T.lane(self);
+        const auto vi = T.vel(self);
+        DensOwn<R> o;
+        dens_begin<R, SUM>(K, o);
+        uint32_t rm[3] = {0u, 0u, 0u};
+        bool ok = true;
+        dens_walk<R, SUM>(K, g, lr, T, P, pi, vi, i, o, rm, &ok);
+        nbm[i] = make_uint4(rm[0], rm[1], rm[2], ok ? 1u : 0u);
+        dens_end<R, SUM, EOS>(S, K, i, o, id, rho);
+      });
 }
 
 template <typename R, bool PER, int BLK, int CW, int CAP>
@@ -734,47 +856,45 @@ __global__ __launch_bounds__(BLK) void k_tensor_tiled(St<R> S, KParams K,
                                                       const uint32_t* __restrict__ skey,
                                                       const int* __restrict__ cstart, SegArg sa,
                                                       const uint4* __restrict__ nbm) {
-  if (halted(K)) return;
   __shared__ TensTile<R, CAP> T;
   __shared__ int cs[3][csw<CW>()];
-  const Segment g = segment_of<CW>(K, cstart, skey, sa, cs);
-  if (g.O0 >= g.O1) return;
+  const Segment g = segment_of<CW>(K, cstart, sa, cs);
+  if (halted(K) || g.O0 >= g.O1) return;
   const auto B = bounds_of<CW>(K, g, cstart, cs);
   const bool tiled = g.total <= CAP;
-  if (tiled) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      for (int q = threadIdx.x; q < g.rl[k]; q += BLK) T.put(g.lo[k] + q, S, K, g.rs[k] + q);
-  }
-  __syncthreads();
-  for (int i0 = g.O0; i0 < g.O1; i0 += BLK) {
-    const int i = i0 + threadIdx.x;
-    if (i >= g.O1) continue;
-    if (!tiled || seam<PER>(K, g, skey[i])) {
-      tensor_direct<R, PER>(S, K, i, skey, cstart);
-      continue;
-    }
-    const int self = g.lo[1] + (i - g.rs[1]);
-    const auto pi = T.lane(self);
-    const auto vi = T.d.vel(self);
-    TensOwn<R> o;
-    auto visit = [&](int l, R uy) {
-      R dx, dy;
-      T.delta(K, pi, l, uy, dx, dy);
-      const R r2 = dx * dx + dy * dy;
-      const auto vj = T.d.vel(l);
-      tens_pair(K, o, dx, dy, r2, vj.x - vi.x, vj.y - vi.y, T.q[l]);
-    };
-    const uint32_t key = skey[i];
-    const uint4 nm = nbm ? nbm[i] : make_uint4(0u, 0u, 0u, 0u);
-    if (nm.w && sizeof(R) == 4)
-      for_masked_rows<R>(K, g, B, key, nm, visit);
-    else if (nm.w)
-      for_masked<R>(K, g, B, key, nm, visit);
-    else
-      for_neighbours<R>(K, g, B, T, pi, i, key, visit);
-    tens_end(S, K, i, T.q[self], o);
-  }
+  using Raw = typename TensTile<R, CAP>::Raw;
+  uint4 nm;
+  for_segment<CW, BLK, 4, Raw>(
+      K, g, B, skey, tiled,
+      [&](int i) {
+        nm = nbm[i];
+        if (!sa.masks) nm.w = 0u;
+      },
+      [&](int t) { return T.load(S, t); }, [&](int l, const Raw& r) { T.put(l, K, r); },
+      [&](int i, uint32_t key, const LaneRows& lr) {
+        if (!tiled || seam<PER>(K, g, key)) {
+          tensor_direct<R, PER>(S, K, i, skey, cstart);
+          return;
+        }
+        const int self = g.lo[1] + (i - g.rs[1]);
+        const auto pi = T.lane(self);
+        const auto vi = T.d.vel(self);
+        TensOwn<R> o;
+        auto visit = [&](int l, R uy) {
+          R dx, dy;
+          T.delta(K, pi, l, uy, dx, dy);
+          const R r2 = dx * dx + dy * dy;
+          const auto vj = T.d.vel(l);
+          tens_pair(K, o, dx, dy, r2, vj.x - vi.x, vj.y - vi.y, T.q[l]);
+        };
+        if (nm.w && sizeof(R) == 4)
+          for_masked_rows<R>(K, g, lr, nm, visit);
+        else if (nm.w)
+          for_masked<R>(K, g, lr, nm, visit);
+        else
+          for_neighbours<R>(K, g, lr, T, pi, i, visit);
+        tens_end(S, K, i, T.q[self], o);
+      });
 }
 
 // PC: pa_sph and same_e2 fixed at compile time for the FP32 pair body
@@ -785,56 +905,46 @@ __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
                                                      const uint32_t* __restrict__ skey,
                                                      const int* __restrict__ cstart, SegArg sa,
                                                      const uint4* __restrict__ nbm) {
-  if (halted(K)) return;
   __shared__ ForceTile<R, CAP, VI> T;
   __shared__ int cs[3][csw<CW>()];
-  const Segment g = segment_of<CW>(K, cstart, skey, sa, cs);
-  if (g.O0 >= g.O1) return;
+  const Segment g = segment_of<CW>(K, cstart, sa, cs);
+  if (halted(K) || g.O0 >= g.O1) return;
   const auto B = bounds_of<CW>(K, g, cstart, cs);
   const bool tiled = g.total <= CAP;
-  if (tiled) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      for (int q = threadIdx.x; q < g.rl[k]; q += BLK)
-        T.put(g.lo[k] + q, S, K, g.rs[k] + q, k);
-  }
-  __syncthreads();
-  for (int i0 = g.O0; i0 < g.O1; i0 += BLK) {
-    const int i = i0 + threadIdx.x;
-    if (i >= g.O1) continue;
-    if (!tiled || seam<PER>(K, g, skey[i])) {
-      force_direct<R, PRESS, AV, AH, XS, VI, PER>(S, K, i, skey, cstart);
-      continue;
-    }
-    const int self = g.lo[1] + (i - g.rs[1]);
-    const auto pi = T.lane(self);
-    ForceOwn<R> o;
-    force_begin<R, VI>(S, K, i, o);
-    auto visit = [&](int l, R uy) {
-      R dx, dy;
-      T.delta(K, pi, l, uy, dx, dy);
-      const R r2 = dx * dx + dy * dy;
-      T.template pair<PRESS, AV, AH, XS, PC>(K, o, l, dx, dy, r2);
-    };
-    const uint32_t key = skey[i];
-    const uint4 nm = nbm ? nbm[i] : make_uint4(0u, 0u, 0u, 0u);
-    if (nm.w && sizeof(R) == 4) {
-      // FP32: the row-refill walk, the row term from the walk
-      const int cx = (int)key - g.cy * K.nx;
-      const int ca = cx > 0 ? cx - 1 : 0;
-      const int l0 = g.rl[0] ? g.lo[0] - g.rs[0] + B.at(0, ca) : 0;
-      const int l1 = g.lo[1] - g.rs[1] + B.at(1, ca);
-      const int l2 = g.rl[2] ? g.lo[2] - g.rs[2] + B.at(2, ca) : 0;
-      const R u0 = (R)row_uy(K, 0), u1 = (R)row_uy(K, 1), u2 = (R)row_uy(K, 2);
-      walk_rows(nm.x, nm.y, nm.z, l0, l1, l2, u0, u1, u2, visit);
-    } else if (nm.w) {
-      // FP64: walk_masks (walk_rows measured 0.6 % slower here)
-      for_masked<R>(K, g, B, key, nm, visit);
-    } else {
-      for_neighbours<R>(K, g, B, T, pi, i, key, visit);
-    }
-    force_end<R, PRESS, XS, VI>(S, K, i, o);
-  }
+  using Raw = typename ForceTile<R, CAP, VI>::Raw;
+  uint4 nm;
+  int id = 0;
+  for_segment<CW, BLK, VI ? 3 : 4, Raw>(
+      K, g, B, skey, tiled,
+      [&](int i) {
+        nm = nbm[i];
+        if (!sa.masks) nm.w = 0u;
+        if (PRESS) id = S.id[i];
+      },
+      [&](int t) { return T.load(S, t); }, [&](int l, const Raw& r) { T.put(l, K, r); },
+      [&](int i, uint32_t key, const LaneRows& lr) {
+        if (!tiled || seam<PER>(K, g, key)) {
+          force_direct<R, PRESS, AV, AH, XS, VI, PER>(S, K, i, skey, cstart);
+          return;
+        }
+        const int self = g.lo[1] + (i - g.rs[1]);
+        const auto pi = T.lane(self);
+        ForceOwn<R> o;
+        T.own(S, K, o, i, self);
+        auto visit = [&](int l, R uy) {
+          R dx, dy;
+          T.delta(K, pi, l, uy, dx, dy);
+          const R r2 = dx * dx + dy * dy;
+          T.template pair<PRESS, AV, AH, XS, PC>(K, o, l, dx, dy, r2);
+        };
+        if (nm.w && sizeof(R) == 4)
+          for_masked_rows<R>(K, g, lr, nm, visit);  // the row-refill walk
+        else if (nm.w)
+          for_masked<R>(K, g, lr, nm, visit);  // FP64 (walk_rows measured 0.6 % slower here)
+        else
+          for_neighbours<R>(K, g, lr, T, pi, i, visit);
+        force_end<R, PRESS, XS, VI>(S, K, i, o, id);
+      });
 }
 
 // ---- the hot FP32 force gather ---------------------------------------------
@@ -850,13 +960,18 @@ __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
 template <int CAP> struct HotForceTile {
   float4 a[CAP];  // offx, offy, vx, vy
   float4 b[CAP];  // Q = 1/rho, A = p/rho, psi, u
-  __device__ __forceinline__ void put(int l, const St<float>& S, const KParams& K, int t) {
-    const float2 o = S.off[t];
-    const float2 v = S.v[t];
-    a[l] = make_float4(o.x, o.y, v.x, v.y);
+  struct Raw {
+    float2 o, v;
+    float rho, p, psi, u;
+  };
+  static __device__ __forceinline__ Raw load(const St<float>& S, int t) {
+    return {S.off[t], S.v[t], S.rho[t], S.p[t], S.psi[t], S.uf[t]};
+  }
+  __device__ __forceinline__ void put(int l, const KParams& K, const Raw& r) {
+    a[l] = make_float4(r.o.x, r.o.y, r.v.x, r.v.y);
     float Q, A;
-    q_and_a(K, S.rho[t], S.p[t], Q, A);
-    b[l] = make_float4(Q, A, S.psi[t], S.uf[t]);
+    q_and_a(K, r.rho, r.p, Q, A);
+    b[l] = make_float4(Q, A, r.psi, r.u);
   }
 };
 
@@ -911,73 +1026,81 @@ template <int BLK, int CAP, int PC>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) void k_force_hot(
     St<float> S, KParams K, const uint32_t* __restrict__ skey, const int* __restrict__ cstart,
     SegArg sa, const uint4* __restrict__ nbm) {
-  if (halted(K)) return;
   __shared__ HotForceTile<CAP> T;
   __shared__ int cs[3][csw<0>()];
-  const Segment g = segment_of<0>(K, cstart, skey, sa, cs);
-  if (g.O0 >= g.O1) return;
+  const Segment g = segment_of<0>(K, cstart, sa, cs);
+  if (halted(K) || g.O0 >= g.O1) return;
   const auto B = bounds_of<0>(K, g, cstart, cs);
   const bool tiled = g.total <= CAP;
-  if (tiled) {
+  const int i = g.O0 + (int)threadIdx.x;
+  const int ic = min(i, g.O1 - 1);
+  const uint32_t key = skey[ic];
+  using Raw = typename HotForceTile<CAP>::Raw;
+  Stage<BLK, 4, Raw> st;  // as for_segment
+  auto ld = [&](int t) { return T.load(S, t); };
+  auto pt = [&](int l, const Raw& r) { T.put(l, K, r); };
+  st.load(g, 0, ld);
+  const int cx = (int)key - g.cy * K.nx;
+  const uint4 nm = nbm[ic];
+  const int id = S.id[ic];
+  HotRow rw[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-      for (int q = threadIdx.x; q < g.rl[k]; q += BLK) T.put(g.lo[k] + q, S, K, g.rs[k] + q);
+  for (int k = 0; k < 3; ++k) {
+    const int d = g.lo[k] - g.rs[k];
+    const int kk = g.rl[k] ? k : 1;  // a row outside the grid has an empty mask
+    rw[k].base = d + B.at(kk, cx > 0 ? cx - 1 : 0);
+    rw[k].e1 = d + B.at(kk, cx);
+    rw[k].e2 = d + B.at(kk, cx + 1);
+    rw[k].uy = row_uy(K, k);
+  }
+  if (tiled) {
+    st.put(g, 0, pt);
+    stage_rest<BLK, 4, Raw>(g, ld, pt);
   }
   __syncthreads();
-  for (int i0 = g.O0; i0 < g.O1; i0 += BLK) {
-    const int i = i0 + threadIdx.x;
-    if (i >= g.O1) continue;
-    const uint4 nm = nbm ? nbm[i] : make_uint4(0u, 0u, 0u, 0u);
-    if (!tiled || !nm.w) {
-      force_direct<float, true, true, true, true, false, false>(S, K, i, skey, cstart);
-      continue;
-    }
-    const int self = g.lo[1] + (i - g.rs[1]);
-    const float4 qs = T.a[self];
-    ForceOwn<float> o;
-    force_begin<float, false>(S, K, i, o);
-    const int cx = (int)skey[i] - g.cy * K.nx;
-    const int ca = cx > 0 ? cx - 1 : 0;
-    HotRow rw[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int d = g.lo[k] - g.rs[k];
-      const bool on = k == 1 || g.rl[k] != 0;  // rows outside the grid have empty masks
-      rw[k].base = on ? d + B.at(k, ca) : 0;
-      rw[k].e1 = on ? d + B.at(k, cx) : 0;
-      rw[k].e2 = on ? d + B.at(k, cx + 1) : 0;
-      rw[k].uy = row_uy(K, k);
-    }
-    const float cellf = K.cellf;
-    auto terms = [&](int l, const HotRow& r) {
-      const float4 q = T.a[l];
-      const float4 w = T.b[l];
-      const float ux = l < r.e1 ? cellf : (l < r.e2 ? 0.f : -cellf);
-      const float tx = qs.x - q.x;
-      const float dx = tx + ux;
-      const float ty = qs.y - q.y;
-      const float dy = ty + r.uy;
-      return force_terms_f32<true, true, true, true, PC>(K, o, dx, dy, q.z, q.w, w.x, w.y, w.z,
-                                                         w.w);
-    };
-    // two neighbours per step; each added in walk order
-    walk_rows2_hot(nm.x, nm.y, nm.z, rw[0], rw[1], rw[2],
-                   [&](int la, const HotRow& ra, int lb, const HotRow& rb, bool hb) {
-                     const TermsF ta = terms(la, ra);
-                     const TermsF tb = terms(lb, rb);
-                     force_acc_f32<true, true, true, true>(o, ta, true);
-                     // without a second neighbour G and wf are zeroed (adding
-                     // -0 dx to a sum that is never -0 leaves its bits), the
-                     // energy rate is skipped
-                     const float gb = hb ? tb.G : 0.f, wb = hb ? tb.wf : 0.f;
-                     o.fx = __builtin_fmaf(-gb, tb.dx, o.fx);
-                     o.fy = __builtin_fmaf(-gb, tb.dy, o.fy);
-                     o.du.add_if(tb.d, hb);
-                     o.xsx = __builtin_fmaf(-wb, tb.dvx, o.xsx);
-                     o.xsy = __builtin_fmaf(-wb, tb.dvy, o.xsy);
-                   });
-    force_end<float, true, true, false>(S, K, i, o);
+  if (i >= g.O1) return;
+  if (!tiled || !nm.w || !sa.masks) {
+    force_direct<float, true, true, true, true, false, false>(S, K, i, skey, cstart);
+    return;
   }
+  const int self = g.lo[1] + (i - g.rs[1]);
+  const float4 qs = T.a[self];
+  const float4 ws = T.b[self];
+  ForceOwn<float> o;
+  o.v = make_float2(qs.z, qs.w);
+  o.Q = ws.x;
+  o.A = ws.y;
+  o.psi = ws.z;
+  o.u = ws.w;
+  own_factors_f32(K, o);
+  const float cellf = K.cellf;
+  auto terms = [&](int l, const HotRow& r) {
+    const float4 q = T.a[l];
+    const float4 w = T.b[l];
+    const float ux = l < r.e1 ? cellf : (l < r.e2 ? 0.f : -cellf);
+    const float tx = qs.x - q.x;
+    const float dx = tx + ux;
+    const float ty = qs.y - q.y;
+    const float dy = ty + r.uy;
+    return force_terms_f32<true, true, true, true, PC>(K, o, dx, dy, q.z, q.w, w.x, w.y, w.z, w.w);
+  };
+  // two neighbours per step; each added in walk order
+  walk_rows2_hot(nm.x, nm.y, nm.z, rw[0], rw[1], rw[2],
+                 [&](int la, const HotRow& ra, int lb, const HotRow& rb, bool hb) {
+                   const TermsF ta = terms(la, ra);
+                   const TermsF tb = terms(lb, rb);
+                   force_acc_f32<true, true, true, true>(o, ta, true);
+                   // without a second neighbour G and wf are zeroed (adding
+                   // -0 dx to a sum that is never -0 leaves its bits), the
+                   // energy rate is skipped
+                   const float gb = hb ? tb.G : 0.f, wb = hb ? tb.wf : 0.f;
+                   o.fx = __builtin_fmaf(-gb, tb.dx, o.fx);
+                   o.fy = __builtin_fmaf(-gb, tb.dy, o.fy);
+                   o.du.add_if(tb.d, hb);
+                   o.xsx = __builtin_fmaf(-wb, tb.dvx, o.xsx);
+                   o.xsy = __builtin_fmaf(-wb, tb.dvy, o.xsy);
+                 });
+  force_end<float, true, true, false>(S, K, i, o, id);
 }
 
 // Launch shapes: cells per segment (0: row pieces of PIECE particles), lanes,
@@ -985,7 +1108,7 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) void k
 // gathers with the physical viscosity (ForceCfg), which run on cell runs.
 template <typename R> struct TileCfg;
 template <> struct TileCfg<float> {
-  static constexpr int BLK = PIECE, CW = 0, CAP = 640;
+  static constexpr int BLK = PIECE, CW = 0, CAP = 592;
 };
 // The hot FP32 force gather (k_force_hot): row pieces; the tile (592 records
 // of 32 bytes, 18.9 KB) lets eight workgroups share a CU (a piece's three
