@@ -237,10 +237,6 @@ struct PassTimer {
 };
 
 // ---- sort -------------------------------------------------------------------
-// Sorts (key_by_id, slot_by_id) into (skey, sval); returns the value array.
-// Sorts (key_by_id, slot_by_id) into (cell, id) order: skey and *sval_out
-// hold the sorted keys and source slots.  The counting sort also writes
-// cell_start (*ranges_done = true); the radix sort leaves it to the reorder.
 // Where the hashing kernels put the keys for the next sort.
 KeyOut key_out(arm_ctx* c) {
   if (c->counting) return KeyOut{nullptr, nullptr, c->key_by_id, c->cnt};
@@ -258,7 +254,6 @@ void zero_counts(arm_ctx* c) {
                        dim3(CS_THREADS), 0, c->stream, c->cnt, sort_cells(c));
 }
 
-// Sorts the first n slots (c->n when n < 0).
 // The entry arrays of the counting sort: ids then slots, capacity each, in
 // the context's 8-byte-per-particle buffer.
 Ent ent_of(arm_ctx* c) {
@@ -272,7 +267,11 @@ RowPieces row_pieces_of(arm_ctx* c) {
   return {c->pieces, c->K.nx, c->K.ny, c->piece_slots};
 }
 
-int run_sort(arm_ctx* c, const int32_t* id_of, const uint32_t** sval_out, bool* ranges_done,
+// Sorts the first n_sort slots (c->n when n_sort < 0) by (cell, id): skey holds
+// the sorted keys, *order the source slots (the counting sort leaves the ranks
+// within the cells to the reorder).  The counting sort also writes cell_start
+// (*ranges_done = true); the radix sort leaves it to the reorder.
+int run_sort(arm_ctx* c, const int32_t* id_of, Order* order, bool* ranges_done,
              int n_sort = -1) {
   const int n = n_sort < 0 ? c->n : n_sort;
   if (c->counting) {
@@ -290,11 +289,9 @@ int run_sort(arm_ctx* c, const int32_t* id_of, const uint32_t** sval_out, bool* 
                        ncell, n, c->cstart, c->tstat, c->scan_epoch, hl);
     hipLaunchKernelGGL(k_cs_scatter, dim3(nb), dim3(CS_THREADS), 0, c->stream, c->key_by_id,
                        id_of, n, c->cstart, c->cnt, ent_of(c), c->sk[1], hl);
-    hipLaunchKernelGGL(k_cs_rank, dim3(nb), dim3(CS_THREADS), 0, c->stream, ent_of(c), c->sk[1],
-                       n, c->cstart, c->sk[0], c->sv[0], c->ghosts ? c->K.ncell : -1, hl);
     HIPCHK(c, hipGetLastError());
-    c->skey = c->sk[0];
-    *sval_out = c->sv[0];
+    c->skey = c->sk[1];
+    *order = Order{ent_of(c).id, ent_of(c).slot};
     *ranges_done = true;
     c->pieces_valid = false;
     return ARM_OK;
@@ -320,7 +317,7 @@ int run_sort(arm_ctx* c, const int32_t* id_of, const uint32_t** sval_out, bool* 
   }
   HIPCHK(c, hipGetLastError());
   c->skey = const_cast<uint32_t*>(kin);
-  *sval_out = vin;
+  *order = Order{nullptr, vin};
   return ARM_OK;
 }
 
@@ -407,11 +404,11 @@ template <typename R> int link_list_t(arm_ctx* c) {
     hipLaunchKernelGGL(k_keys<R>, dim3(grid_of(n)), dim3(BLOCK), 0, c->stream, A, c->K,
                        key_out(c), c->d_err, gfirst);
   }
-  const uint32_t* sval = nullptr;
+  Order order{};
   bool ranges = false;
   {
     PassTimer tm(c, ARM_PASS_SORT);
-    int rc = run_sort(c, A.id, &sval, &ranges);
+    int rc = run_sort(c, A.id, &order, &ranges);
     if (rc) return rc;
   }
   c->ng = c->ghost_pending ? c->ng_new : 0;
@@ -423,7 +420,7 @@ template <typename R> int link_list_t(arm_ctx* c) {
     // with the sort's cell ranges the kernel also adds the row pieces
     const RowPieces rp = ranges ? row_pieces_of(c) : RowPieces{};
     hipLaunchKernelGGL(k_reorder_all<R>, dim3(grid_of(c->n) + row_blocks(rp)),
-                       dim3(BLOCK), 0, c->stream, A, B, c->K, c->skey, sval, c->cstart,
+                       dim3(BLOCK), 0, c->stream, A, B, c->K, c->skey, order, c->cstart,
                        ranges ? 0 : 1, c->G, rp);
     c->pieces_valid = rp.tab != nullptr;
   }
@@ -743,7 +740,7 @@ template <typename R> int fused_step(arm_ctx* c, int its, const StepHooks& hk) {
   int rc;
   c->its_next = its;
   c->K.its = its;
-  const uint32_t* sval = nullptr;
+  Order order{};
   bool ranges = false;
   // with ghosts: the new set goes after the live slots; the old set carries
   // the extra key (corrector) and drops out of the sort
@@ -754,7 +751,7 @@ template <typename R> int fused_step(arm_ctx* c, int its, const StepHooks& hk) {
   }
   {
     PassTimer tm(c, ARM_PASS_SORT);
-    if ((rc = run_sort(c, stA<R>(c).id, &sval, &ranges, n_sort))) return rc;
+    if ((rc = run_sort(c, stA<R>(c).id, &order, &ranges, n_sort))) return rc;
   }
   if (c->ghosts) {
     c->ng = c->ng_new;
@@ -769,7 +766,7 @@ template <typename R> int fused_step(arm_ctx* c, int its, const StepHooks& hk) {
     // with the sort's cell ranges the kernel also adds the row pieces
     const RowPieces rp = ranges ? row_pieces_of(c) : RowPieces{};
     hipLaunchKernelGGL(k_reorder_pred<R>, dim3(grid_of(n) + row_blocks(rp)),
-                       dim3(BLOCK), 0, c->stream, A, B, c->K, c->skey, sval, c->cstart,
+                       dim3(BLOCK), 0, c->stream, A, B, c->K, c->skey, order, c->cstart,
                        its != 1 ? 1 : 0, ranges ? 0 : 1, c->G, rp);
     c->pieces_valid = rp.tab != nullptr;
     std::swap(A, B);
@@ -1451,17 +1448,17 @@ template <typename R> int link_list3_t(arm_ctx* c) {
     hipLaunchKernelGGL(k3_keys<R>, dim3(grid_of(n)), dim3(BLOCK), 0, c->stream, A, c->K,
                        key_out(c), c->d_err);
   }
-  const uint32_t* sval = nullptr;
+  Order order{};
   bool ranges = false;
   {
     PassTimer tm(c, ARM_PASS_SORT);
-    int rc = run_sort(c, A.id, &sval, &ranges);
+    int rc = run_sort(c, A.id, &order, &ranges);
     if (rc) return rc;
   }
   {
     PassTimer tm(c, ARM_PASS_REORDER);
     hipLaunchKernelGGL(k3_reorder_all<R>, dim3(grid_of(n)), dim3(BLOCK), 0, c->stream, A, B,
-                       c->K, c->skey, sval, c->cstart, ranges ? 0 : 1);
+                       c->K, c->skey, order, c->cstart, ranges ? 0 : 1);
   }
   HIPCHK(c, hipGetLastError());
   std::swap(A, B);
@@ -1583,18 +1580,18 @@ template <typename R> int fused_step3(arm_ctx* c, int its, const StepHooks& hk =
   int rc;
   c->its_next = its;
   c->K.its = its;
-  const uint32_t* sval = nullptr;
+  Order order{};
   bool ranges = false;
   {
     PassTimer tm(c, ARM_PASS_SORT);
-    if ((rc = run_sort(c, st3A<R>(c).id, &sval, &ranges))) return rc;
+    if ((rc = run_sort(c, st3A<R>(c).id, &order, &ranges))) return rc;
   }
   {
     St3<R>& A = st3A<R>(c);
     St3<R>& B = st3B<R>(c);
     PassTimer tm(c, ARM_PASS_REORDER);
     hipLaunchKernelGGL(k3_reorder_pred<R>, dim3(grid_of(n)), dim3(BLOCK), 0, c->stream, A, B,
-                       c->K, c->skey, sval, c->cstart, its != 1 ? 1 : 0, ranges ? 0 : 1);
+                       c->K, c->skey, order, c->cstart, its != 1 ? 1 : 0, ranges ? 0 : 1);
     std::swap(A, B);
     c->masks_valid = false;
   }
@@ -2182,13 +2179,6 @@ int arm_create(const arm_params* prm, int capacity, arm_ctx** out) {
     if (!rc) rc = is32(c) ? alloc_state(c, c->B32, capacity) : alloc_state(c, c->B64, capacity);
   }
   if (!rc) rc = dalloc(c, &c->key_by_id, capacity);
-  if (!rc) rc = dalloc(c, &c->slot_by_id, capacity);
-  for (int k = 0; k < 2 && !rc; ++k) {
-    rc = dalloc(c, &c->sk[k], capacity);
-    if (!rc) rc = dalloc(c, &c->sv[k], capacity);
-  }
-  if (!rc) rc = dalloc(c, &c->hist, (size_t)(1 << c->sort_bits) * c->ntiles);
-  if (!rc) rc = dalloc(c, &c->tot, (size_t)(1 << c->sort_bits));
   c->ghosts = (P.flags & ARM_GHOSTS) != 0;
   // the counting sort runs over ncell cells, plus one with ghosts; its tile
   // sums also serve the ghost numbering (a scan over the real ids)
@@ -2211,6 +2201,16 @@ int arm_create(const arm_params* prm, int capacity, arm_ctx** out) {
       hipError_t ez = hipMemset(c->cnt, 0, sizeof(int) * ((size_t)ncell + 1));
       if (ez != hipSuccess) rc = fail(c, ARM_ERR_HIP, "hipMemset: %s", hipGetErrorString(ez));
     }
+    if (!rc) rc = dalloc(c, &c->sk[1], capacity);
+  }
+  if (!rc && !c->counting) {  // the radix sort
+    rc = dalloc(c, &c->slot_by_id, capacity);
+    for (int k = 0; k < 2 && !rc; ++k) {
+      rc = dalloc(c, &c->sk[k], capacity);
+      if (!rc) rc = dalloc(c, &c->sv[k], capacity);
+    }
+    if (!rc) rc = dalloc(c, &c->hist, (size_t)(1 << c->sort_bits) * c->ntiles);
+    if (!rc) rc = dalloc(c, &c->tot, (size_t)(1 << c->sort_bits));
   }
   if (!rc) rc = dalloc(c, &c->cstart, (size_t)ncell + 2);
   if (!rc && c->ghosts) {
@@ -2942,7 +2942,7 @@ extern "C" int arm_link_list_static(const arm_params* prm, int n, const double* 
     hipLaunchKernelGGL(k_cs_rank, dim3(nb), dim3(CS_THREADS), 0, s, ent, entc, n,
                        reinterpret_cast<const int*>(cell_start),
                        reinterpret_cast<uint32_t*>(key_sorted),
-                       reinterpret_cast<uint32_t*>(id_sorted), -1, Halt{});
+                       reinterpret_cast<uint32_t*>(id_sorted));
   }
   return hipGetLastError() == hipSuccess ? ARM_OK : ARM_ERR_HIP;
 }

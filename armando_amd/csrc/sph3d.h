@@ -156,14 +156,16 @@ __global__ __launch_bounds__(BLOCK) void k3_keys(St3<R> S, KParams K, KeyOut ko,
 template <typename R>
 __global__ __launch_bounds__(BLOCK) void k3_reorder_all(St3<R> A, St3<R> Bs, KParams K,
                                                         const uint32_t* __restrict__ skey,
-                                                        const uint32_t* __restrict__ sval,
+                                                        Order ord,
                                                         int* __restrict__ cstart, int fill) {
-  const int t = blockIdx.x * BLOCK + threadIdx.x;
-  const bool valid = t < K.n;
-  if (fill) fill_cell_start(skey, t, valid, K.n, K.ncell, cstart);
+  const int p = blockIdx.x * BLOCK + threadIdx.x;
+  const bool valid = p < K.n;
+  if (fill) fill_cell_start(skey, p, valid, K.n, K.ncell, cstart);
   if (!valid) return;
-  const int s = (int)sval[t];
-  Bs.id[t] = A.id[s];
+  const int s = (int)ord.slot[p];
+  const int id = A.id[s];
+  const int t = ord.place(skey, cstart, p, id);
+  Bs.id[t] = id;
   Bs.xyz[t] = A.xyz[s];
   if constexpr (sizeof(R) == 4) {
     Bs.pf[t] = A.pf[s];
@@ -189,41 +191,49 @@ __global__ __launch_bounds__(BLOCK) void k3_reorder_all(St3<R> A, St3<R> Bs, KPa
 template <typename R>
 __global__ __launch_bounds__(BLOCK) void k3_reorder_pred(St3<R> A, St3<R> Bs, KParams K,
                                                          const uint32_t* __restrict__ skey,
-                                                         const uint32_t* __restrict__ sval,
+                                                         Order ord,
                                                          int* __restrict__ cstart, int predict,
                                                          int fill) {
   if (halted(K)) return;
   using R4 = typename V4<R>::type;
-  const int t = blockIdx.x * BLOCK + threadIdx.x;
-  const bool valid = t < K.n;
-  if (fill) fill_cell_start(skey, t, valid, K.n, K.ncell, cstart);
+  const int p = blockIdx.x * BLOCK + threadIdx.x;
+  const bool valid = p < K.n;
+  if (fill) fill_cell_start(skey, p, valid, K.n, K.ncell, cstart);
   if (!valid) return;
-  const int s = (int)sval[t];
-  const int id = A.id[s];
-  Bs.id[t] = id;
+  const int s = (int)ord.slot[p];
+  const int id = ord.ids ? (int)ord.ids[p] : A.id[s];
+  // the fields before the rank: their loads overlap its own
   const double4 q = A.xyz[s];
-  Bs.xyz[t] = q;
-  if constexpr (sizeof(R) == 4) Bs.pf[t] = split3(K, q);
   R4 v = A.v[s];
   R rho = A.rho[s];
   double u = A.u[s];
+  R4 a{};
+  R du = (R)0, drho = (R)0;
+  if (predict) {
+    a = A.a[s];
+    du = A.du[s];
+    drho = A.drho[s];
+  }
+  const int t = ord.place(skey, cstart, p, id);
+  Bs.id[t] = id;
+  Bs.xyz[t] = q;
+  if constexpr (sizeof(R) == 4) Bs.pf[t] = split3(K, q);
   uint8_t fl = 0;
   if (predict) {
     const double hdt = K.dt / 2.0;
     if (is_rate(K, id)) {
       Bs.u_min[t] = u;
-      u = u + hdt * (double)A.du[s];
+      u = u + hdt * (double)du;
       if (u < 0.0) {
         u = 0.0;
         fl = 1u;
       }
       if (K.density_method == 0) {
         Bs.rho_min[t] = rho;
-        rho = rho + (R)hdt * A.drho[s];
+        rho = rho + (R)hdt * drho;
       }
     }
     if (id < K.np) {
-      const R4 a = A.a[s];
       Bs.v_min[t] = v;
       v.x = v.x + (R)hdt * a.x;
       v.y = v.y + (R)hdt * a.y;

@@ -188,7 +188,7 @@ __device__ __forceinline__ void ghost_slot(const St<R>& A, St<R>& Bs, const KPar
 // A reorder kernel launched with row pieces (rp.tab set; cell_start
 // written by the sort) has row_blocks(rp) extra workgroups in front, one
 // wavefront per cell row, which list the rows' pieces (they run beside the
-// first particles' workgroups).  Returns true in those; *t is the sorted position
+// first particles' workgroups).  Returns true in those; *t is the position
 // of the lane in the others.
 __host__ __device__ inline int row_blocks(const RowPieces& rp) {
   return rp.tab ? (rp.ny + ROWS_PER_WG - 1) / ROWS_PER_WG : 0;
@@ -210,17 +210,18 @@ __device__ __forceinline__ bool reorder_row_pieces(const int* __restrict__ cstar
 template <typename R>
 __global__ __launch_bounds__(BLOCK) void k_reorder_all(St<R> A, St<R> Bs, KParams K,
                                                        const uint32_t* __restrict__ skey,
-                                                       const uint32_t* __restrict__ sval,
+                                                       Order ord,
                                                        int* __restrict__ cstart, int fill,
                                                        Ghosts G, RowPieces rp) {
-  int t;
-  if (reorder_row_pieces(cstart, skey, rp, &t)) return;
-  const bool valid = t < K.n;
-  if (fill) fill_cell_start(skey, t, valid, K.n, K.ncell, cstart);
+  int p;
+  if (reorder_row_pieces(cstart, skey, rp, &p)) return;
+  const bool valid = p < K.n;
+  if (fill) fill_cell_start(skey, p, valid, K.n, K.ncell, cstart);
   if (!valid) return;
-  const int s = (int)sval[t];
+  const int s = (int)ord.slot[p];
+  const int id = A.id[s];
+  const int t = ord.place(skey, cstart, p, id);
   if (G.xprev) {
-    const int id = A.id[s];
     if (id >= K.nb) {
       ghost_slot(A, Bs, K, G, s, t, id, 0);
       return;
@@ -228,7 +229,7 @@ __global__ __launch_bounds__(BLOCK) void k_reorder_all(St<R> A, St<R> Bs, KParam
     G.xprev[t] = A.xy[s];
     if (id < K.np) G.sid[id] = t;
   }
-  Bs.id[t] = A.id[s];
+  Bs.id[t] = id;
   Bs.xy[t] = A.xy[s];
   if constexpr (sizeof(R) == 4) {
     Bs.cxy[t] = A.cxy[s];
@@ -257,28 +258,40 @@ __global__ __launch_bounds__(BLOCK) void k_reorder_all(St<R> A, St<R> Bs, KParam
 template <typename R>
 __global__ __launch_bounds__(BLOCK) void k_reorder_pred(St<R> A, St<R> Bs, KParams K,
                                                         const uint32_t* __restrict__ skey,
-                                                        const uint32_t* __restrict__ sval,
+                                                        Order ord,
                                                         int* __restrict__ cstart, int predict,
                                                         int fill, Ghosts G, RowPieces rp) {
   if (halted(K)) return;
-  int t;
-  if (reorder_row_pieces(cstart, skey, rp, &t)) return;
+  int p;
+  if (reorder_row_pieces(cstart, skey, rp, &p)) return;
   using R2 = typename V2<R>::type;
-  const bool valid = t < K.n;
-  if (fill) fill_cell_start(skey, t, valid, K.n, K.ncell, cstart);
+  const bool valid = p < K.n;
+  if (fill) fill_cell_start(skey, p, valid, K.n, K.ncell, cstart);
   if (!valid) return;
-  const int s = (int)sval[t];
-  const int id = A.id[s];
+  const int s = (int)ord.slot[p];
+  const int id = ord.ids ? (int)ord.ids[p] : A.id[s];
+  // the fields before the rank: their loads overlap its own
+  const double2 q = A.xy[s];
+  R2 v = A.v[s];
+  R rho = A.rho[s];
+  double u = A.u[s];
+  R2 a{};
+  R du = (R)0, drho = (R)0;
+  if (predict) {
+    a = A.a[s];
+    du = A.du[s];
+    drho = A.drho[s];
+  }
+  const int t = ord.place(skey, cstart, p, id);
   if (G.xprev) {
     if (id >= K.nb) {
       ghost_slot(A, Bs, K, G, s, t, id, predict);
       return;
     }
-    G.xprev[t] = A.xy[s];
+    G.xprev[t] = q;
     if (id < K.np) G.sid[id] = t;
   }
   Bs.id[t] = id;
-  const double2 q = A.xy[s];
   Bs.xy[t] = q;
   if (K.sle) Bs.hs[t] = A.hs[s];
   if constexpr (sizeof(R) == 4) {
@@ -291,27 +304,23 @@ __global__ __launch_bounds__(BLOCK) void k_reorder_pred(St<R> A, St<R> Bs, KPara
     Bs.cxy[t] = (uint32_t)ix | ((uint32_t)iy << 16);
     Bs.off[t] = make_float2((float)(q.x - bx), (float)(q.y - by));
   }
-  R2 v = A.v[s];
-  R rho = A.rho[s];
-  double u = A.u[s];
   uint8_t fl = 0;
   if (predict) {
     const double hdt = K.dt / 2.0;
     const bool rate = is_rate(K, id);
     if (rate) {
       Bs.u_min[t] = u;
-      u = u + hdt * (double)A.du[s];
+      u = u + hdt * (double)du;
       if (u < 0.0) {
         u = 0.0;
         fl = 1u;
       }
       if (K.density_method == 0) {
         Bs.rho_min[t] = rho;
-        rho = rho + (R)hdt * A.drho[s];
+        rho = rho + (R)hdt * drho;
       }
     }
     if (id < K.np) {
-      const R2 a = A.a[s];
       Bs.v_min[t] = v;
       v.x = v.x + (R)hdt * a.x;
       v.y = v.y + (R)hdt * a.y;
