@@ -329,7 +329,23 @@ template <> St<double>& stB<double>(arm_ctx* c) { return c->B64; }
 template <> St<float>& stB<float>(arm_ctx* c) { return c->B32; }
 
 // Swaps the active state buffer with the other one.
-void swap_state(arm_ctx* c) {
+template <typename R> void swap_moved(St<R>& A, St<R>& B) {
+  std::swap(A.xy, B.xy);
+  std::swap(A.v, B.v);
+  std::swap(A.rho, B.rho);
+  std::swap(A.u, B.u);
+}
+
+// Undoes the swaps of one step of a run: the reorder's of the two states and,
+// in 2D, the corrector's of the moved fields.
+void unstep_state(arm_ctx* c) {
+  if (c->prm.dim != 3) {
+    if (c->prm.precision == ARM_FP32)
+      swap_moved(c->A32, c->B32);
+    else
+      swap_moved(c->A64, c->B64);
+  }
+
   if (c->prm.dim == 3) {
     if (c->prm.precision == ARM_FP32)
       std::swap(c->A3_32, c->B3_32);
@@ -354,7 +370,7 @@ int check_domain(arm_ctx* c, int its_end = -1) {
   HIPCHK(c, hipMemcpyAsync(bad, c->d_err, 4 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   const int stop = bad[3];
-  if (stop && its_end >= 0 && (its_end - stop) % 2 != 0) swap_state(c);
+  if (stop && its_end >= 0 && (its_end - stop) % 2 != 0) unstep_state(c);
   if (bad[0] || bad[1] || stop) {
     c->domain_bad = bad[0] + bad[1];
     HIPCHK(c, hipMemsetAsync(c->d_err, 0, 2 * sizeof(int), c->stream));
@@ -504,26 +520,30 @@ template <typename R> int eos_t(arm_ctx* c) {
 
 // The FP32 tiled force gather of the dam-break flag set (pressure, artificial
 // viscosity and heat, XSPH) with pa_sph and same_e2 fixed at compile time.
-template <int PC> void launch_force_hot(arm_ctx* c) {
+template <int PC> void launch_force_hot(arm_ctx* c, const Moved<float>& mv) {
   using T = HotForceCfg;
   const SegArg sa = seg_arg<T::CW>(c);
   hipLaunchKernelGGL((k_force_hot<T::BLK, T::CAP, PC>), dim3(seg_grid<T::CW>(c, sa)),
                      dim3(T::BLK), 0, c->stream, stA<float>(c), c->K, c->skey, c->cstart, sa,
-                     c->nbm);
+                     c->nbm, mv);
 }
 
+// mv: the tiled gathers also move the particles (mv.its != 0); returns whether
+// they did.
 template <typename R, bool P, bool AV, bool AH, bool XS, bool VI = false>
-void launch_force(arm_ctx* c) {
+bool launch_force(arm_ctx* c, const Moved<R>& mv) {
   St<R>& A = stA<R>(c);
   using T = ForceCfg<R, VI>;
   if (c->tiled && !c->K.sle) {
-    if (sizeof(R) == 4 && P && AV && AH && XS && !VI && !c->K.periodic &&
-        !(c->K.flags & ARM_CONDUCTION)) {
-      switch ((c->K.pa_sph == 0 ? 1 : 0) | (c->K.same_e2 ? 2 : 0)) {
-        case 0: launch_force_hot<0>(c); break;
-        case 1: launch_force_hot<1>(c); break;
-        case 2: launch_force_hot<2>(c); break;
-        default: launch_force_hot<3>(c); break;
+    bool hot = false;
+    if constexpr (sizeof(R) == 4 && P && AV && AH && XS && !VI)
+      hot = !c->K.periodic && !(c->K.flags & ARM_CONDUCTION);
+    if (hot) {
+      if constexpr (sizeof(R) == 4) switch ((c->K.pa_sph == 0 ? 1 : 0) | (c->K.same_e2 ? 2 : 0)) {
+        case 0: launch_force_hot<0>(c, mv); break;
+        case 1: launch_force_hot<1>(c, mv); break;
+        case 2: launch_force_hot<2>(c, mv); break;
+        default: launch_force_hot<3>(c, mv); break;
       }
     } else {
       const SegArg sa = seg_arg<T::CW>(c);
@@ -531,16 +551,17 @@ void launch_force(arm_ctx* c) {
       if (c->K.periodic)
         hipLaunchKernelGGL((k_force_tiled<R, P, AV, AH, XS, VI, true, T::BLK, T::CW, T::CAP>),
                            dim3(grid), dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart,
-                           sa, c->nbm);
+                           sa, c->nbm, mv);
       else
         hipLaunchKernelGGL((k_force_tiled<R, P, AV, AH, XS, VI, false, T::BLK, T::CW, T::CAP>),
                            dim3(grid), dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart,
-                           sa, c->nbm);
+                           sa, c->nbm, mv);
     }
-  } else {
-    hipLaunchKernelGGL((k_force<R, P, AV, AH, XS, VI>), dim3(grid_of(c->n)), dim3(BLOCK), 0,
-                       c->stream, A, c->K, c->skey, c->cstart, c->d_err);
+    return mv.its != 0;
   }
+  hipLaunchKernelGGL((k_force<R, P, AV, AH, XS, VI>), dim3(grid_of(c->n)), dim3(BLOCK), 0,
+                     c->stream, A, c->K, c->skey, c->cstart, c->d_err);
+  return false;
 }
 
 // Shear tensor of the physical viscosity, after the EOS (tau of every particle).
@@ -572,7 +593,11 @@ void dep_window(arm_ctx* c) {
 }
 
 // dispatch over the compile-time flag combination
-template <typename R> int force_t(arm_ctx* c, bool press, int flags, bool xs) {
+// mv (in a run of steps): the corrector, which goes with the force pass where
+// nothing acts on the rates after it; *moved: it did.
+template <typename R>
+int force_and_move_t(arm_ctx* c, bool press, int flags, bool xs, const Moved<R>* mv,
+                     bool* moved) {
   const bool av = (flags & ARM_ART_VISC) != 0, ah = (flags & ARM_ART_HEAT) != 0;
   dep_window(c);
   const bool vi = press && (flags & ARM_VISC) != 0;
@@ -580,25 +605,28 @@ template <typename R> int force_t(arm_ctx* c, bool press, int flags, bool xs) {
     return fail(c, ARM_ERR_ARG, "ARM_CONTACT: the context was created without it");
   PassTimer tm(c, ARM_PASS_FORCE);
   if (vi) launch_tensor<R>(c);
+  const bool more = press && ((c->K.flags & KF_DEPOSITION) || (flags & ARM_CONTACT));
+  const Moved<R> m = mv && !more ? *mv : Moved<R>{};
+  bool did = false;
   const int code = (vi ? 16 : 0) | (press ? 8 : 0) | (av ? 4 : 0) | (ah ? 2 : 0) | (xs ? 1 : 0);
   switch (code) {
-    case 8: launch_force<R, true, false, false, false>(c); break;
-    case 9: launch_force<R, true, false, false, true>(c); break;
-    case 10: launch_force<R, true, false, true, false>(c); break;
-    case 11: launch_force<R, true, false, true, true>(c); break;
-    case 12: launch_force<R, true, true, false, false>(c); break;
-    case 13: launch_force<R, true, true, false, true>(c); break;
-    case 14: launch_force<R, true, true, true, false>(c); break;
-    case 15: launch_force<R, true, true, true, true>(c); break;
-    case 24: launch_force<R, true, false, false, false, true>(c); break;
-    case 25: launch_force<R, true, false, false, true, true>(c); break;
-    case 26: launch_force<R, true, false, true, false, true>(c); break;
-    case 27: launch_force<R, true, false, true, true, true>(c); break;
-    case 28: launch_force<R, true, true, false, false, true>(c); break;
-    case 29: launch_force<R, true, true, false, true, true>(c); break;
-    case 30: launch_force<R, true, true, true, false, true>(c); break;
-    case 31: launch_force<R, true, true, true, true, true>(c); break;
-    case 1: launch_force<R, false, false, false, true>(c); break;
+    case 8: did = launch_force<R, true, false, false, false>(c, m); break;
+    case 9: did = launch_force<R, true, false, false, true>(c, m); break;
+    case 10: did = launch_force<R, true, false, true, false>(c, m); break;
+    case 11: did = launch_force<R, true, false, true, true>(c, m); break;
+    case 12: did = launch_force<R, true, true, false, false>(c, m); break;
+    case 13: did = launch_force<R, true, true, false, true>(c, m); break;
+    case 14: did = launch_force<R, true, true, true, false>(c, m); break;
+    case 15: did = launch_force<R, true, true, true, true>(c, m); break;
+    case 24: did = launch_force<R, true, false, false, false, true>(c, m); break;
+    case 25: did = launch_force<R, true, false, false, true, true>(c, m); break;
+    case 26: did = launch_force<R, true, false, true, false, true>(c, m); break;
+    case 27: did = launch_force<R, true, false, true, true, true>(c, m); break;
+    case 28: did = launch_force<R, true, true, false, false, true>(c, m); break;
+    case 29: did = launch_force<R, true, true, false, true, true>(c, m); break;
+    case 30: did = launch_force<R, true, true, true, false, true>(c, m); break;
+    case 31: did = launch_force<R, true, true, true, true, true>(c, m); break;
+    case 1: did = launch_force<R, false, false, false, true>(c, m); break;
     default: return fail(c, ARM_ERR_ARG, "force pass with nothing to compute");
   }
   if (press && (c->K.flags & KF_DEPOSITION))
@@ -614,8 +642,14 @@ template <typename R> int force_t(arm_ctx* c, bool press, int flags, bool xs) {
     hipLaunchKernelGGL(k_contact_apply<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream,
                        stA<R>(c), c->K, c->skey, c->cstart, static_cast<const V*>(cd));
   }
+  *moved = did;
   HIPCHK(c, hipGetLastError());
   return ARM_OK;
+}
+
+template <typename R> int force_t(arm_ctx* c, bool press, int flags, bool xs) {
+  bool moved;
+  return force_and_move_t<R>(c, press, flags, xs, nullptr, &moved);
 }
 
 // Clears a device array inside the step with a fill kernel (not a memset
@@ -659,14 +693,21 @@ template <typename R> int predictor_t(arm_ctx* c) {
   return ARM_OK;
 }
 
-template <typename R> int corrector_t(arm_ctx* c, int its, bool keys) {
+// The corrector per routine, in place.
+template <typename R> int corrector_t(arm_ctx* c, int its) {
   St<R>& A = stA<R>(c);
   c->its_next = its + 1;
   PassTimer tm(c, ARM_PASS_INTEGRATE);
-  hipLaunchKernelGGL(k_corrector<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream, A, c->K,
-                     its, keys ? 1 : 0, keys ? key_out(c) : KeyOut{}, c->d_err);
+  const Moved<R> m{A.xy, A.v, A.rho, A.u, A.uf, KeyOut{}, c->d_err, its};
+  hipLaunchKernelGGL(k_corrector<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream, A, c->K, m);
   HIPCHK(c, hipGetLastError());
   return ARM_OK;
+}
+
+// The corrector of a run's step, with the keys of the next one.
+template <typename R> Moved<R> moved_of(arm_ctx* c, int its) {
+  St<R>& B = stB<R>(c);
+  return {B.xy, B.v, B.rho, B.u, nullptr, key_out(c), c->d_err, its};
 }
 
 // time_integration.f:131-235, fused: per step
@@ -778,7 +819,11 @@ template <typename R> int fused_step(arm_ctx* c, int its, const StepHooks& hk) {
   if (hk.jpart)
     hipLaunchKernelGGL(k_objective<R>, dim3(grid_of(n)), dim3(BLOCK), 0, c->stream, stA<R>(c),
                        c->K, hk.kind, hk.objmask, hk.jpart);
-  if ((rc = force_t<R>(c, true, c->prm.flags, xs))) return rc;
+  // the force pass moves its particles, unless the step is to be recorded first
+  const Moved<R> mv = moved_of<R>(c, its);
+  bool moved = false;
+  if ((rc = force_and_move_t<R>(c, true, c->prm.flags, xs, hk.tape ? nullptr : &mv, &moved)))
+    return rc;
   take_new_h<R>(c);
   if (hk.tape) {
     const int nb = std::max(grid_of(n), grid_of(c->K.ncell + 1));
@@ -786,7 +831,14 @@ template <typename R> int fused_step(arm_ctx* c, int its, const StepHooks& hk) {
                        c->cstart, c->masks_valid ? c->nbm : nullptr,
                        *static_cast<const Tape<R>*>(hk.tape));
   }
-  if ((rc = corrector_t<R>(c, its, true))) return rc;
+  c->its_next = its + 1;
+  if (!moved) {
+    PassTimer tm(c, ARM_PASS_INTEGRATE);
+    hipLaunchKernelGGL(k_corrector<R>, dim3(grid_of(n)), dim3(BLOCK), 0, c->stream, stA<R>(c),
+                       c->K, mv);
+    HIPCHK(c, hipGetLastError());
+  }
+  swap_moved(stA<R>(c), stB<R>(c));
   return ARM_OK;
 }
 
@@ -2549,8 +2601,7 @@ int arm_corrector(arm_ctx* c, int its) {
   if (!c) return ARM_ERR_ARG;
   if (!c->loaded) return fail(c, ARM_ERR_STATE, "no state uploaded");
   if (!c->have_rates) return fail(c, ARM_ERR_STATE, "no rates: run arm_single_step first");
-  int rc = is3d(c) ? DISPATCH(c, corrector3_t)(c, its, false)
-                    : DISPATCH(c, corrector_t)(c, its, false);
+  int rc = is3d(c) ? DISPATCH(c, corrector3_t)(c, its, false) : DISPATCH(c, corrector_t)(c, its);
   if (!rc) HIPCHK(c, hipStreamSynchronize(c->stream));
   // positions moved: the cell order and masks must be rebuilt before the next gather
   c->masks_valid = false;

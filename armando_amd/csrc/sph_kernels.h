@@ -234,11 +234,12 @@ __global__ __launch_bounds__(BLOCK) void k_reorder_all(St<R> A, St<R> Bs, KParam
   if constexpr (sizeof(R) == 4) {
     Bs.cxy[t] = A.cxy[s];
     Bs.off[t] = A.off[s];
-    Bs.uf[t] = A.uf[s];
   }
   Bs.v[t] = A.v[s];
   Bs.rho[t] = A.rho[s];
-  Bs.u[t] = A.u[s];
+  const double u = A.u[s];
+  Bs.u[t] = u;
+  if constexpr (sizeof(R) == 4) Bs.uf[t] = (float)u;  // the steps leave A.uf behind
   Bs.p[t] = A.p[s];
   Bs.psi[t] = A.psi[s];
   Bs.drho[t] = A.drho[s];
@@ -779,10 +780,17 @@ __device__ __forceinline__ void force_pair(const KParams& K, ForceOwn<R>& o, R d
   }
 }
 
+// What the corrector takes from the force pass.
+template <typename R> struct Rates {
+  typename V2<R>::type a{}, av{};
+  R du = (R)0;
+};
+
 template <typename R, bool PRESS, bool XS, bool VI = false>
-__device__ __forceinline__ void force_end(St<R>& S, const KParams& K, int i, const ForceOwn<R>& o,
-                                          int id) {
+__device__ __forceinline__ Rates<R> force_end(St<R>& S, const KParams& K, int i,
+                                              const ForceOwn<R>& o, int id) {
   using R2 = typename V2<R>::type;
+  Rates<R> out;
   if (PRESS) {
     const bool grav = (K.flags & 16) && id < K.np;
     R gx, gy;
@@ -798,6 +806,7 @@ __device__ __forceinline__ void force_end(St<R>& S, const KParams& K, int i, con
     acc.x = o.fx + ex;
     acc.y = o.fy + ey;
     S.a[i] = acc;
+    out.a = acc;
     // du = tds/dt + the pair sums (internal_force.f:433-435) [+ heat source];
     // the FP32 pair body accumulates the sums doubled
     const R sums = sizeof(R) == 4 ? (R)0.5 * o.du.get() : o.du.get();
@@ -807,18 +816,22 @@ __device__ __forceinline__ void force_end(St<R>& S, const KParams& K, int i, con
       du = du + (R)(K.hs_q0 * heat_shape(K, q.x, q.y)) * o.Q;
     }
     S.du[i] = du;
+    out.du = du;
   }
   if (XS) {
     R2 w;
     w.x = o.xsx;
     w.y = o.xsy;
     S.av[i] = w;
+    out.av = w;
   }
+  return out;
 }
 
 template <typename R, bool PRESS, bool XS, bool VI = false>
-__device__ __forceinline__ void force_end(St<R>& S, const KParams& K, int i, const ForceOwn<R>& o) {
-  force_end<R, PRESS, XS, VI>(S, K, i, o, PRESS ? S.id[i] : 0);
+__device__ __forceinline__ Rates<R> force_end(St<R>& S, const KParams& K, int i,
+                                              const ForceOwn<R>& o) {
+  return force_end<R, PRESS, XS, VI>(S, K, i, o, PRESS ? S.id[i] : 0);
 }
 
 // The deposition heat source after the force pass, in the steps where it
@@ -961,7 +974,7 @@ __device__ __forceinline__ void density_direct(St<R>& S, const KParams& K, int i
 }
 
 template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool VI = false, bool WRAP = true>
-__device__ __forceinline__ void force_direct(St<R>& S, const KParams& K, int i,
+__device__ __forceinline__ Rates<R> force_direct(St<R>& S, const KParams& K, int i,
                                              const uint32_t* __restrict__ skey,
                                              const int* __restrict__ cstart) {
   const auto pi = load_pos(S, i);
@@ -982,7 +995,7 @@ __device__ __forceinline__ void force_direct(St<R>& S, const KParams& K, int i,
                                          u_of(S, t),
                                          VI ? tau_of(S, t, visc_c(K, Qj)) : Tau3<R>{});
   });
-  force_end<R, PRESS, XS, VI>(S, K, i, o);
+  return force_end<R, PRESS, XS, VI>(S, K, i, o);
 }
 
 // ---- per-particle smoothing length (K.sle != 0): the direct gathers with
@@ -1250,70 +1263,121 @@ __global__ __launch_bounds__(BLOCK) void k_predictor(St<R> S, KParams K) {
   }
 }
 
-// Corrector; with keys it also hashes the updated position for the next
-// step's sort (the reorder then rebuilds the FP32 cell + offset).
+// ---- corrector ----------------------------------------------------------
+// Where the corrector puts the moved particles.  In a run of steps these are
+// the arrays of the inactive state (its xy, v, rho, u; the host then swaps the
+// four between the two states): the force gathers that move their own
+// particles still read their neighbours' old values in the active ones.  The
+// routine corrector writes in place.  its: the step, 0 for none; uf: null
+// where the next reorder writes it.
+template <typename R> struct Moved {
+  double2* xy;
+  typename V2<R>::type* v;
+  R* rho;
+  double* u;
+  float* uf;
+  KeyOut ko;
+  int* err;
+  int its;
+};
+
+// A particle's values before the corrector: those that the predictor kept,
+// or its own where that has not acted.
+template <typename R> struct MoveIn {
+  double2 q{};
+  typename V2<R>::type v{};
+  double u = 0.0;
+  R rho = (R)0, drho = (R)0;
+};
+
 template <typename R>
-__global__ __launch_bounds__(BLOCK) void k_corrector(St<R> S, KParams K, int its, int keys,
-                                                     KeyOut ko, int* __restrict__ err) {
-  if (halted(K)) return;
-  const int i = blockIdx.x * BLOCK + threadIdx.x;
-  const bool valid = i < K.n;
+__device__ __forceinline__ MoveIn<R> move_load(const St<R>& S, const KParams& K, int its, int i,
+                                               int id) {
+  const bool kept = its != 1 && is_rate(K, id);
+  MoveIn<R> m;
+  m.q = S.xy[i];
+  m.v = (its != 1 && id < K.np ? S.v_min : S.v)[i];
+  m.u = (kept ? S.u_min : S.u)[i];
+  m.rho = (kept && K.density_method == 0 ? S.rho_min : S.rho)[i];
+  m.drho = S.drho[i];
+  return m;
+}
+
+// The corrector of particle i; with keys in M.ko it also hashes the new
+// position for the next step's sort, for which all 64 lanes of the wavefront
+// must call it (on: the lane has a particle).  The reorder then rebuilds the
+// FP32 cell + offset.
+template <typename R>
+__device__ __forceinline__ void move_particle(const KParams& K, const Moved<R>& M, bool on, int i,
+                                              int id, MoveIn<R> m, const Rates<R>& r) {
   uint32_t key = 0;
-  int id = 0;
-  if (valid) {
-    id = S.id[i];
+  const bool keys = M.ko.key_by_slot || M.ko.key_by_id;
+  if (on) {
     const double dt = K.dt, hdt = K.dt / 2.0;
-    double2 q = S.xy[i];
+    const bool first = M.its == 1;
     if (is_rate(K, id)) {
-      double u;
-      if (its != 1) {
-        u = S.u_min[i] + dt * (double)S.du[i];
-        if (K.density_method == 0) S.rho[i] = S.rho_min[i] + (R)dt * S.drho[i];
-      } else {
-        u = S.u[i] + hdt * (double)S.du[i];
-        if (K.density_method == 0) S.rho[i] = S.rho[i] + (R)hdt * S.drho[i];
-      }
-      if (u < 0.0) u = 0.0;
-      S.u[i] = u;
-      if constexpr (sizeof(R) == 4) S.uf[i] = (float)u;
+      m.u = m.u + (first ? hdt : dt) * (double)r.du;
+      if (m.u < 0.0) m.u = 0.0;
+      if (K.density_method == 0) m.rho = m.rho + (R)(first ? hdt : dt) * m.drho;
       if (id < K.np) {
-        auto v = S.v[i];
-        const auto a = S.a[i];
-        if (its != 1) {
-          const auto vm = S.v_min[i];
-          const auto av = S.av[i];
-          v.x = vm.x + (R)dt * a.x + av.x;
-          v.y = vm.y + (R)dt * a.y + av.y;
+        if (!first) {
+          m.v.x = m.v.x + (R)dt * r.a.x + r.av.x;
+          m.v.y = m.v.y + (R)dt * r.a.y + r.av.y;
         } else {
-          v.x = v.x + (R)hdt * a.x;
-          v.y = v.y + (R)hdt * a.y;
+          m.v.x = m.v.x + (R)hdt * r.a.x;
+          m.v.y = m.v.y + (R)hdt * r.a.y;
         }
-        S.v[i] = v;
-        q.x = q.x + dt * (double)v.x;
-        q.y = q.y + dt * (double)v.y;
+        m.q.x = m.q.x + dt * (double)m.v.x;
+        m.q.y = m.q.y + dt * (double)m.v.y;
         if (K.periodic) {  // re-enter on the other side of the period
           const double L = (double)K.nx * K.cell;
-          if (q.x >= K.ox + L)
-            q.x = q.x - L;
-          else if (q.x < K.ox)
-            q.x = q.x + L;
+          if (m.q.x >= K.ox + L)
+            m.q.x = m.q.x - L;
+          else if (m.q.x < K.ox)
+            m.q.x = m.q.x + L;
         }
-        S.xy[i] = q;
       }
+    }
+    M.xy[i] = m.q;
+    M.v[i] = m.v;
+    M.rho[i] = m.rho;
+    M.u[i] = m.u;
+    if constexpr (sizeof(R) == 4) {
+      if (M.uf) M.uf[i] = (float)m.u;
     }
     if (keys && id >= K.nb) {
       key = (uint32_t)K.ncell;  // this step's ghost: out of the next sort
     } else if (keys) {
       int ix, iy;
       bool ok;
-      key = (uint32_t)cell_of(K, q.x, q.y, ix, iy, ok);
+      key = (uint32_t)cell_of(K, m.q.x, m.q.y, ix, iy, ok);
       if (!ok) {
-        atomicAdd(err, 1);
+        atomicAdd(M.err, 1);
         raise_halt(K);
       }
     }
   }
-  if (keys) emit_key(ko, valid, i, id, key);
+  if (keys) emit_key(M.ko, on, i, id, key);
+}
+
+// The corrector as a pass of its own: per routine, and in the steps whose
+// force pass is not the last to act on the rates.
+template <typename R>
+__global__ __launch_bounds__(BLOCK) void k_corrector(St<R> S, KParams K, Moved<R> M) {
+  if (halted(K)) return;
+  const int i = blockIdx.x * BLOCK + threadIdx.x;
+  const bool on = i < K.n;
+  int id = 0;
+  MoveIn<R> m;
+  Rates<R> r;
+  if (on) {
+    id = S.id[i];
+    m = move_load(S, K, M.its, i, id);
+    r.a = S.a[i];
+    r.av = S.av[i];
+    r.du = S.du[i];
+  }
+  move_particle(K, M, on, i, id, m, r);
 }
 
 // ------------------------------------------------------------------------

@@ -496,31 +496,35 @@ __device__ __forceinline__ void stage_rest(const Segment& g, Load&& ld, Put&& pt
 }
 
 // Fills the tile (if tiled), then calls lane(i, key, rows) for the workgroup's
-// particles, one lane each; early(i) loads what else lane() needs.  On pieces
+// particles, one lane each, and done(i, on) in all lanes (on: it has one);
+// early(i) loads what else lane() needs, late(i) what depends on that.  On pieces
 // (CW = 0) every lane has at most one particle, and its key, its rows and
 // early() are read beside the tile's records: after the piece's record that
 // takes two dependent loads, where a chain of staging, key and cell bounds
 // takes six, most of a workgroup's life on the small tiles of 2D.
-template <int CW, int BLK, int UN, typename Raw, typename BD, typename Early, typename Load,
-          typename Put, typename Lane>
+template <int CW, int BLK, int UN, typename Raw, typename BD, typename Early, typename Late,
+          typename Load, typename Put, typename Lane, typename Done>
 __device__ __forceinline__ void for_segment(const KParams& K, const Segment& g, const BD& B,
                                             const uint32_t* __restrict__ skey, bool tiled,
-                                            Early&& early, Load&& ld, Put&& pt, Lane&& lane) {
+                                            Early&& early, Late&& late, Load&& ld, Put&& pt,
+                                            Lane&& lane, Done&& done) {
   if constexpr (CW == 0) {
     static_assert(BLK >= PIECE, "a lane for every particle of a piece");
     const int i = g.O0 + (int)threadIdx.x;
     const int ic = min(i, g.O1 - 1);
     const uint32_t key = skey[ic];
+    early(ic);
     Stage<BLK, UN, Raw> st;
     st.load(g, 0, ld);
-    early(ic);
     const LaneRows r = lane_rows(K, g, B, key);
+    late(ic);
     if (tiled) {
       st.put(g, 0, pt);
       stage_rest<BLK, UN, Raw>(g, ld, pt);
     }
     __syncthreads();
     if (i < g.O1) lane(i, key, r);
+    done(i, i < g.O1);
   } else {
     if (tiled) {
       Stage<BLK, UN, Raw> st;
@@ -531,10 +535,13 @@ __device__ __forceinline__ void for_segment(const KParams& K, const Segment& g, 
     __syncthreads();
     for (int i0 = g.O0; i0 < g.O1; i0 += BLK) {
       const int i = i0 + threadIdx.x;
-      if (i >= g.O1) continue;
-      const uint32_t key = skey[i];
-      early(i);
-      lane(i, key, lane_rows(K, g, B, key));
+      if (i < g.O1) {
+        const uint32_t key = skey[i];
+        early(i);
+        late(i);
+        lane(i, key, lane_rows(K, g, B, key));
+      }
+      done(i, i < g.O1);
     }
   }
 }
@@ -828,6 +835,7 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
         id = S.id[i];
         if (EOS) rho = S.rho[i];
       },
+      [](int) {},
       [&](int t) { return T.load(S, t); },
       [&](int l, const Raw& r) {
         T.put(l, K, r);
@@ -848,7 +856,8 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
         dens_walk<R, SUM>(K, g, lr, T, P, pi, vi, i, o, rm, &ok);
         nbm[i] = make_uint4(rm[0], rm[1], rm[2], ok ? 1u : 0u);
         dens_end<R, SUM, EOS>(S, K, i, o, id, rho);
-      });
+      },
+      [](int, bool) {});
 }
 
 template <typename R, bool PER, int BLK, int CW, int CAP>
@@ -870,6 +879,7 @@ __global__ __launch_bounds__(BLK) void k_tensor_tiled(St<R> S, KParams K,
         nm = nbm[i];
         if (!sa.masks) nm.w = 0u;
       },
+      [](int) {},
       [&](int t) { return T.load(S, t); }, [&](int l, const Raw& r) { T.put(l, K, r); },
       [&](int i, uint32_t key, const LaneRows& lr) {
         if (!tiled || seam<PER>(K, g, key)) {
@@ -894,9 +904,14 @@ __global__ __launch_bounds__(BLK) void k_tensor_tiled(St<R> S, KParams K,
         else
           for_neighbours<R>(K, g, lr, T, pi, i, visit);
         tens_end(S, K, i, T.q[self], o);
-      });
+      },
+      [](int, bool) {});
 }
 
+// With M.its the workgroup also moves its particles (move_particle): the rates
+// are in registers and the corrector's own values were read beside the tile, so
+// the pass that read them back (14.8 us of a 115 us step of 720,000 FP32
+// particles, 4.4 of 41 us with 1,972 in FP64) costs a store.
 // PC: pa_sph and same_e2 fixed at compile time for the FP32 pair body
 // (force_pair_f32), -1 to read them from K (k_force_hot fixes them).
 template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool VI, bool PER, int BLK, int CW,
@@ -904,7 +919,7 @@ template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool VI, bool PER, 
 __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
                                                      const uint32_t* __restrict__ skey,
                                                      const int* __restrict__ cstart, SegArg sa,
-                                                     const uint4* __restrict__ nbm) {
+                                                     const uint4* __restrict__ nbm, Moved<R> M) {
   __shared__ ForceTile<R, CAP, VI> T;
   __shared__ int cs[3][csw<CW>()];
   const Segment g = segment_of<CW>(K, cstart, sa, cs);
@@ -914,6 +929,8 @@ __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
   using Raw = typename ForceTile<R, CAP, VI>::Raw;
   uint4 nm;
   int id = 0;
+  MoveIn<R> m;
+  Rates<R> rates;
   for_segment<CW, BLK, VI ? 3 : 4, Raw>(
       K, g, B, skey, tiled,
       [&](int i) {
@@ -921,10 +938,13 @@ __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
         if (!sa.masks) nm.w = 0u;
         if (PRESS) id = S.id[i];
       },
+      [&](int i) {
+        if (PRESS && M.its) m = move_load(S, K, M.its, i, id);
+      },
       [&](int t) { return T.load(S, t); }, [&](int l, const Raw& r) { T.put(l, K, r); },
       [&](int i, uint32_t key, const LaneRows& lr) {
         if (!tiled || seam<PER>(K, g, key)) {
-          force_direct<R, PRESS, AV, AH, XS, VI, PER>(S, K, i, skey, cstart);
+          rates = force_direct<R, PRESS, AV, AH, XS, VI, PER>(S, K, i, skey, cstart);
           return;
         }
         const int self = g.lo[1] + (i - g.rs[1]);
@@ -943,7 +963,10 @@ __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
           for_masked<R>(K, g, lr, nm, visit);  // FP64 (walk_rows measured 0.6 % slower here)
         else
           for_neighbours<R>(K, g, lr, T, pi, i, visit);
-        force_end<R, PRESS, XS, VI>(S, K, i, o, id);
+        rates = force_end<R, PRESS, XS, VI>(S, K, i, o, id);
+      },
+      [&](int i, bool on) {
+        if (PRESS && M.its) move_particle(K, M, on, i, id, m, rates);
       });
 }
 
@@ -1025,7 +1048,7 @@ __device__ __forceinline__ void walk_rows2_hot(uint32_t m0, uint32_t m1, uint32_
 template <int BLK, int CAP, int PC>
 __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) void k_force_hot(
     St<float> S, KParams K, const uint32_t* __restrict__ skey, const int* __restrict__ cstart,
-    SegArg sa, const uint4* __restrict__ nbm) {
+    SegArg sa, const uint4* __restrict__ nbm, Moved<float> M) {
   __shared__ HotForceTile<CAP> T;
   __shared__ int cs[3][csw<0>()];
   const Segment g = segment_of<0>(K, cstart, sa, cs);
@@ -1035,6 +1058,7 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) void k
   const int i = g.O0 + (int)threadIdx.x;
   const int ic = min(i, g.O1 - 1);
   const uint32_t key = skey[ic];
+  const int id = S.id[ic];
   using Raw = typename HotForceTile<CAP>::Raw;
   Stage<BLK, 4, Raw> st;  // as for_segment
   auto ld = [&](int t) { return T.load(S, t); };
@@ -1042,7 +1066,6 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) void k
   st.load(g, 0, ld);
   const int cx = (int)key - g.cy * K.nx;
   const uint4 nm = nbm[ic];
-  const int id = S.id[ic];
   HotRow rw[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -1053,54 +1076,59 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) void k
     rw[k].e2 = d + B.at(kk, cx + 1);
     rw[k].uy = row_uy(K, k);
   }
+  MoveIn<float> m;
+  if (M.its) m = move_load(S, K, M.its, ic, id);
   if (tiled) {
     st.put(g, 0, pt);
     stage_rest<BLK, 4, Raw>(g, ld, pt);
   }
   __syncthreads();
-  if (i >= g.O1) return;
-  if (!tiled || !nm.w || !sa.masks) {
-    force_direct<float, true, true, true, true, false, false>(S, K, i, skey, cstart);
-    return;
+  Rates<float> rates;
+  const bool on = i < g.O1;
+  if (on && (!tiled || !nm.w || !sa.masks)) {
+    rates = force_direct<float, true, true, true, true, false, false>(S, K, i, skey, cstart);
+  } else if (on) {
+    const int self = g.lo[1] + (i - g.rs[1]);
+    const float4 qs = T.a[self];
+    const float4 ws = T.b[self];
+    ForceOwn<float> o;
+    o.v = make_float2(qs.z, qs.w);
+    o.Q = ws.x;
+    o.A = ws.y;
+    o.psi = ws.z;
+    o.u = ws.w;
+    own_factors_f32(K, o);
+    const float cellf = K.cellf;
+    auto terms = [&](int l, const HotRow& r) {
+      const float4 q = T.a[l];
+      const float4 w = T.b[l];
+      const float ux = l < r.e1 ? cellf : (l < r.e2 ? 0.f : -cellf);
+      const float tx = qs.x - q.x;
+      const float dx = tx + ux;
+      const float ty = qs.y - q.y;
+      const float dy = ty + r.uy;
+      return force_terms_f32<true, true, true, true, PC>(K, o, dx, dy, q.z, q.w, w.x, w.y, w.z,
+                                                         w.w);
+    };
+    // two neighbours per step; each added in walk order
+    walk_rows2_hot(nm.x, nm.y, nm.z, rw[0], rw[1], rw[2],
+                   [&](int la, const HotRow& ra, int lb, const HotRow& rb, bool hb) {
+                     const TermsF ta = terms(la, ra);
+                     const TermsF tb = terms(lb, rb);
+                     force_acc_f32<true, true, true, true>(o, ta, true);
+                     // without a second neighbour G and wf are zeroed (adding
+                     // -0 dx to a sum that is never -0 leaves its bits), the
+                     // energy rate is skipped
+                     const float gb = hb ? tb.G : 0.f, wb = hb ? tb.wf : 0.f;
+                     o.fx = __builtin_fmaf(-gb, tb.dx, o.fx);
+                     o.fy = __builtin_fmaf(-gb, tb.dy, o.fy);
+                     o.du.add_if(tb.d, hb);
+                     o.xsx = __builtin_fmaf(-wb, tb.dvx, o.xsx);
+                     o.xsy = __builtin_fmaf(-wb, tb.dvy, o.xsy);
+                   });
+    rates = force_end<float, true, true, false>(S, K, i, o, id);
   }
-  const int self = g.lo[1] + (i - g.rs[1]);
-  const float4 qs = T.a[self];
-  const float4 ws = T.b[self];
-  ForceOwn<float> o;
-  o.v = make_float2(qs.z, qs.w);
-  o.Q = ws.x;
-  o.A = ws.y;
-  o.psi = ws.z;
-  o.u = ws.w;
-  own_factors_f32(K, o);
-  const float cellf = K.cellf;
-  auto terms = [&](int l, const HotRow& r) {
-    const float4 q = T.a[l];
-    const float4 w = T.b[l];
-    const float ux = l < r.e1 ? cellf : (l < r.e2 ? 0.f : -cellf);
-    const float tx = qs.x - q.x;
-    const float dx = tx + ux;
-    const float ty = qs.y - q.y;
-    const float dy = ty + r.uy;
-    return force_terms_f32<true, true, true, true, PC>(K, o, dx, dy, q.z, q.w, w.x, w.y, w.z, w.w);
-  };
-  // two neighbours per step; each added in walk order
-  walk_rows2_hot(nm.x, nm.y, nm.z, rw[0], rw[1], rw[2],
-                 [&](int la, const HotRow& ra, int lb, const HotRow& rb, bool hb) {
-                   const TermsF ta = terms(la, ra);
-                   const TermsF tb = terms(lb, rb);
-                   force_acc_f32<true, true, true, true>(o, ta, true);
-                   // without a second neighbour G and wf are zeroed (adding
-                   // -0 dx to a sum that is never -0 leaves its bits), the
-                   // energy rate is skipped
-                   const float gb = hb ? tb.G : 0.f, wb = hb ? tb.wf : 0.f;
-                   o.fx = __builtin_fmaf(-gb, tb.dx, o.fx);
-                   o.fy = __builtin_fmaf(-gb, tb.dy, o.fy);
-                   o.du.add_if(tb.d, hb);
-                   o.xsx = __builtin_fmaf(-wb, tb.dvx, o.xsx);
-                   o.xsy = __builtin_fmaf(-wb, tb.dvy, o.xsy);
-                 });
-  force_end<float, true, true, false>(S, K, i, o, id);
+  if (M.its) move_particle(K, M, on, i, id, m, rates);
 }
 
 // Launch shapes: cells per segment (0: row pieces of PIECE particles), lanes,
