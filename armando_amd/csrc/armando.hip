@@ -447,40 +447,31 @@ template <typename R> int link_list_t(arm_ctx* c) {
   return check_domain(c);
 }
 
-// Where the tiled gathers' workgroups find their segments, and how many
-// workgroups they take: row pieces (CW = 0; the piece table is rebuilt after
-// each sort, and the grid is ny for the cut parts and piece_slots) or
-// runs of CW cells of every row.
-template <int CW> SegArg seg_arg(arm_ctx* c) {
-  if constexpr (CW > 0) {
-    return SegArg{(c->K.nx + CW - 1) / CW, nullptr, c->masks_valid};
-  } else {
-    if (!c->pieces_valid) {
-      const RowPieces rp = row_pieces_of(c);
-      hipLaunchKernelGGL(k_row_pieces, dim3(row_blocks(rp)), dim3(BLOCK), 0, c->stream,
-                         c->cstart, c->skey, rp, Halt{c->K.halt, c->K.its});
-      c->pieces_valid = true;
-    }
-    return SegArg{0, c->pieces, c->masks_valid};
+// The row pieces of the tiled gathers (rebuilt after each sort) and how many
+// workgroups they take: ny for the cut parts and piece_slots.
+SegArg seg_arg(arm_ctx* c) {
+  if (!c->pieces_valid) {
+    const RowPieces rp = row_pieces_of(c);
+    hipLaunchKernelGGL(k_row_pieces, dim3(row_blocks(rp)), dim3(BLOCK), 0, c->stream,
+                       c->cstart, c->skey, rp, Halt{c->K.halt, c->K.its});
+    c->pieces_valid = true;
   }
+  return SegArg{c->pieces, c->masks_valid};
 }
-template <int CW> int seg_grid(const arm_ctx* c, const SegArg& sa) {
-  return CW > 0 ? c->K.ny * sa.nseg : c->K.ny + c->piece_slots;
-}
+int seg_grid(const arm_ctx* c) { return c->K.ny + c->piece_slots; }
 
 template <typename R, bool SUM, bool EOS> void launch_density(arm_ctx* c) {
   St<R>& A = stA<R>(c);
-  using T = TileCfg<R>;
   if (c->tiled && !c->K.sle) {
-    const SegArg sa = seg_arg<T::CW>(c);
-    const int grid = seg_grid<T::CW>(c, sa);
+    const SegArg sa = seg_arg(c);
+    const int grid = seg_grid(c);
     if (c->K.periodic)
-      hipLaunchKernelGGL((k_density_tiled<R, SUM, EOS, true, T::BLK, T::CW, T::CAP>),
-                         dim3(grid), dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart, sa,
+      hipLaunchKernelGGL((k_density_tiled<R, SUM, EOS, true>),
+                         dim3(grid), dim3(PIECE), 0, c->stream, A, c->K, c->skey, c->cstart, sa,
                          c->nbm);
     else
-      hipLaunchKernelGGL((k_density_tiled<R, SUM, EOS, false, T::BLK, T::CW, T::CAP>),
-                         dim3(grid), dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart, sa,
+      hipLaunchKernelGGL((k_density_tiled<R, SUM, EOS, false>),
+                         dim3(grid), dim3(PIECE), 0, c->stream, A, c->K, c->skey, c->cstart, sa,
                          c->nbm);
   } else {
     hipLaunchKernelGGL((k_density<R, SUM, EOS>), dim3(grid_of(c->n)), dim3(BLOCK), 0,
@@ -521,10 +512,9 @@ template <typename R> int eos_t(arm_ctx* c) {
 // The FP32 tiled force gather of the dam-break flag set (pressure, artificial
 // viscosity and heat, XSPH) with pa_sph and same_e2 fixed at compile time.
 template <int PC> void launch_force_hot(arm_ctx* c, const Moved<float>& mv) {
-  using T = HotForceCfg;
-  const SegArg sa = seg_arg<T::CW>(c);
-  hipLaunchKernelGGL((k_force_hot<T::BLK, T::CAP, PC>), dim3(seg_grid<T::CW>(c, sa)),
-                     dim3(T::BLK), 0, c->stream, stA<float>(c), c->K, c->skey, c->cstart, sa,
+  const SegArg sa = seg_arg(c);
+  hipLaunchKernelGGL((k_force_hot<PC>), dim3(seg_grid(c)),
+                     dim3(PIECE), 0, c->stream, stA<float>(c), c->K, c->skey, c->cstart, sa,
                      c->nbm, mv);
 }
 
@@ -533,7 +523,6 @@ template <int PC> void launch_force_hot(arm_ctx* c, const Moved<float>& mv) {
 template <typename R, bool P, bool AV, bool AH, bool XS, bool VI = false>
 bool launch_force(arm_ctx* c, const Moved<R>& mv) {
   St<R>& A = stA<R>(c);
-  using T = ForceCfg<R, VI>;
   if (c->tiled && !c->K.sle) {
     bool hot = false;
     if constexpr (sizeof(R) == 4 && P && AV && AH && XS && !VI)
@@ -546,15 +535,15 @@ bool launch_force(arm_ctx* c, const Moved<R>& mv) {
         default: launch_force_hot<3>(c, mv); break;
       }
     } else {
-      const SegArg sa = seg_arg<T::CW>(c);
-      const int grid = seg_grid<T::CW>(c, sa);
+      const SegArg sa = seg_arg(c);
+      const int grid = seg_grid(c);
       if (c->K.periodic)
-        hipLaunchKernelGGL((k_force_tiled<R, P, AV, AH, XS, VI, true, T::BLK, T::CW, T::CAP>),
-                           dim3(grid), dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart,
+        hipLaunchKernelGGL((k_force_tiled<R, P, AV, AH, XS, VI, true>),
+                           dim3(grid), dim3(PIECE), 0, c->stream, A, c->K, c->skey, c->cstart,
                            sa, c->nbm, mv);
       else
-        hipLaunchKernelGGL((k_force_tiled<R, P, AV, AH, XS, VI, false, T::BLK, T::CW, T::CAP>),
-                           dim3(grid), dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart,
+        hipLaunchKernelGGL((k_force_tiled<R, P, AV, AH, XS, VI, false>),
+                           dim3(grid), dim3(PIECE), 0, c->stream, A, c->K, c->skey, c->cstart,
                            sa, c->nbm, mv);
     }
     return mv.its != 0;
@@ -567,16 +556,15 @@ bool launch_force(arm_ctx* c, const Moved<R>& mv) {
 // Shear tensor of the physical viscosity, after the EOS (tau of every particle).
 template <typename R> void launch_tensor(arm_ctx* c) {
   St<R>& A = stA<R>(c);
-  using T = TileCfg<R>;
   if (c->tiled && !c->K.sle) {
-    const SegArg sa = seg_arg<T::CW>(c);
-    const int grid = seg_grid<T::CW>(c, sa);
+    const SegArg sa = seg_arg(c);
+    const int grid = seg_grid(c);
     if (c->K.periodic)
-      hipLaunchKernelGGL((k_tensor_tiled<R, true, T::BLK, T::CW, T::CAP>), dim3(grid),
-                         dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart, sa, c->nbm);
+      hipLaunchKernelGGL((k_tensor_tiled<R, true>), dim3(grid),
+                         dim3(PIECE), 0, c->stream, A, c->K, c->skey, c->cstart, sa, c->nbm);
     else
-      hipLaunchKernelGGL((k_tensor_tiled<R, false, T::BLK, T::CW, T::CAP>), dim3(grid),
-                         dim3(T::BLK), 0, c->stream, A, c->K, c->skey, c->cstart, sa, c->nbm);
+      hipLaunchKernelGGL((k_tensor_tiled<R, false>), dim3(grid),
+                         dim3(PIECE), 0, c->stream, A, c->K, c->skey, c->cstart, sa, c->nbm);
   } else {
     hipLaunchKernelGGL(k_tensor<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream, A, c->K,
                        c->skey, c->cstart);

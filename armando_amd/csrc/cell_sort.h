@@ -317,11 +317,11 @@ __global__ __launch_bounds__(CS_THREADS) void k_cs_scatter(const uint32_t* __res
 // slots = n / PIECE + ny bounds the count.
 constexpr int PIECE = 128;
 constexpr int GAP_SPAN = 40;      // a full piece of 2h cells spans about 20
-constexpr int GAP_RECORDS = 592;  // the smallest tile of the gathers on pieces
+constexpr int GAP_RECORDS = 592;  // the records of a gather's tile
 struct alignas(16) PieceRec {
   int O0, O1, cy, total;  // total = rl[0] + rl[1] + rl[2]
   int rs[3], rl[3];       // sorted start and length of rows cy-1, cy, cy+1
-  int pad[2];
+  int x0, x1;             // cells of its first and last particle
 };
 struct RowPieces {
   PieceRec* tab = nullptr;
@@ -380,6 +380,8 @@ __device__ __forceinline__ void row_pieces_block(const int* __restrict__ cstart,
     r.O0 = p;
     r.O1 = e;
     r.cy = y;
+    r.x0 = x0;
+    r.x1 = x1;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const int ry = y - 1 + k;

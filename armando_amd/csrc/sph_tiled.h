@@ -1,8 +1,7 @@
 // sph_tiled.h -- LDS-tiled gathers of the density and force passes.
 //
 // A workgroup owns a segment of one cell row: a piece of up to 128
-// consecutive sorted particles of the row (or, for the viscous force
-// gathers, a run of CW cells).  Its particles are one contiguous sorted
+// consecutive sorted particles of the row.  Its particles are one contiguous sorted
 // range, and the candidates of all of them lie in three contiguous sorted
 // ranges (the cell row below, the row itself and the row above, over the
 // segment's cells and one either side).  The workgroup copies those three
@@ -35,6 +34,13 @@ namespace arm {
 //   dy = (off_i.y - off_j.y) + (1 - k) cell
 // are the same operations, with the same roundings, as delta() on PosF.
 constexpr int TPAD = 8;
+// Records of a tile: a piece's three rows hold about 3 x 140 on the dam-break
+// lattice, 584 at most.  The FP32 force gather's 18.9 KB let eight workgroups
+// share a CU; with the physical viscosity's 52 bytes (FP32) or 88 (FP64) a
+// record, runs of 32 or 16 cells with smaller tiles were the faster form until
+// the loads of the prologue overlapped (heated channel of 2 million, force with
+// the corrector: FP32 189 us on runs, 182 on pieces; FP64 377 and 369).
+constexpr int CAP = GAP_RECORDS;
 
 // Byte offset 4 l of a 4-byte LDS record.  Computed out of the compiler's
 // sight: otherwise it derives this address from the 16-byte records' l << 4
@@ -68,8 +74,8 @@ __device__ __forceinline__ void tile_delta(const KParams& K, const LaneF& p, flo
   dy = ty + uy;
 }
 
-template <typename R, int CAP> struct DensTile;
-template <int CAP> struct DensTile<float, CAP> {
+template <typename R> struct DensTile;
+template <> struct DensTile<float> {
   // the neighbour test reads one 16-byte record per candidate
   float4 a[CAP + TPAD];  // offx, offy, cell column as float, vx
   float vy[CAP + TPAD];
@@ -97,7 +103,7 @@ template <int CAP> struct DensTile<float, CAP> {
     return make_float2(a[l].w, lds_at(vy, off4(l)));
   }
 };
-template <int CAP> struct DensTile<double, CAP> {
+template <> struct DensTile<double> {
   double2 x[CAP + TPAD], v[CAP + TPAD];
   struct Raw {
     double2 x, v;
@@ -132,17 +138,17 @@ template <int CAP> struct DensTile<double, CAP> {
 constexpr int FIX = 4096;
 using s16x2 = __attribute__((ext_vector_type(2))) short;
 
-template <int CAP> struct PreTile {
+struct PreTile {
   uint32_t p[CAP + TPAD];
   __device__ __forceinline__ void put(int l, const KParams& K,
-                                      const typename DensTile<float, CAP>::Raw& r) {
+                                      const DensTile<float>::Raw& r) {
     const uint32_t c = r.c;
     const uint32_t x = (c & 0xffffu) * FIX + (uint32_t)(int)__builtin_fmaf(r.o.x, K.fixf, 0.5f);
     const uint32_t y = (c >> 16) * FIX + (uint32_t)(int)__builtin_fmaf(r.o.y, K.fixf, 0.5f);
     p[l] = (x & 0xffffu) | (y << 16);
   }
   __device__ __forceinline__ void put(int l, const KParams& K,
-                                      const typename DensTile<double, CAP>::Raw& r) {
+                                      const DensTile<double>::Raw& r) {
     auto fix = [&](double d) {
       const double u = d * K.fix;
       return (uint32_t)(int)(u - 65536.0 * floor(u * (1.0 / 65536.0)) + 0.5);
@@ -152,13 +158,13 @@ template <int CAP> struct PreTile {
 };
 
 // Neighbour W = c T of the physical viscosity, staged only when VI.
-template <typename R, int CAP, bool VI> struct TauTile {
+template <typename R, bool VI> struct TauTile {
   struct Raw {};
   static __device__ __forceinline__ Raw load(const St<R>&, int) { return {}; }
   __device__ __forceinline__ void put(int, const Raw&, R) {}
   __device__ __forceinline__ Tau3<R> get(int) const { return Tau3<R>{}; }
 };
-template <int CAP> struct TauTile<float, CAP, true> {
+template <> struct TauTile<float, true> {
   float4 w[CAP];
   using Raw = float4;
   static __device__ __forceinline__ Raw load(const St<float>& S, int t) {
@@ -172,7 +178,7 @@ template <int CAP> struct TauTile<float, CAP, true> {
     return {q.x, q.y, q.z};
   }
 };
-template <int CAP> struct TauTile<double, CAP, true> {
+template <> struct TauTile<double, true> {
   double2 w01[CAP];
   double w2[CAP];
   struct Raw {
@@ -201,21 +207,21 @@ __device__ __forceinline__ void own_tau(const St<R>& S, ForceOwn<R>& o, int i, c
   o.tds = S.tau[4 * (size_t)i + 3];
 }
 
-template <typename R, int CAP, bool VI = false> struct ForceTile;
-template <int CAP, bool VI> struct ForceTile<float, CAP, VI> {
+template <typename R, bool VI = false> struct ForceTile;
+template <bool VI> struct ForceTile<float, VI> {
   float4 a[CAP + TPAD];  // offx, offy, vx, vy
   float4 b[CAP + TPAD];  // Q = 1/rho, A = p/rho, psi, u
   float cx[CAP + TPAD];  // cell column as float
-  TauTile<float, CAP + TPAD, VI> tw;
+  TauTile<float, VI> tw;
   struct Raw {
     float2 o, v;
     float rho, p, psi, u;
     uint32_t c;
-    typename TauTile<float, CAP + TPAD, VI>::Raw w;
+    typename TauTile<float, VI>::Raw w;
   };
   static __device__ __forceinline__ Raw load(const St<float>& S, int t) {
     return {S.off[t], S.v[t],  S.rho[t], S.p[t],
-            S.psi[t], S.uf[t], S.cxy[t], TauTile<float, CAP + TPAD, VI>::load(S, t)};
+            S.psi[t], S.uf[t], S.cxy[t], TauTile<float, VI>::load(S, t)};
   }
   __device__ __forceinline__ void put(int l, const KParams& K, const Raw& r) {
     a[l] = make_float4(r.o.x, r.o.y, r.v.x, r.v.y);
@@ -256,17 +262,17 @@ template <int CAP, bool VI> struct ForceTile<float, CAP, VI> {
                                                  w.w, tw.get(l));
   }
 };
-template <int CAP, bool VI> struct ForceTile<double, CAP, VI> {
+template <bool VI> struct ForceTile<double, VI> {
   double2 x[CAP + TPAD], v[CAP + TPAD], rp[CAP + TPAD], pu[CAP + TPAD];  // rp = (Q, A), pu = (psi, u)
-  TauTile<double, CAP + TPAD, VI> tw;
+  TauTile<double, VI> tw;
   struct Raw {
     double2 x, v;
     double rho, p, psi, u;
-    typename TauTile<double, CAP + TPAD, VI>::Raw w;
+    typename TauTile<double, VI>::Raw w;
   };
   static __device__ __forceinline__ Raw load(const St<double>& S, int t) {
     return {S.xy[t],  S.v[t], S.rho[t], S.p[t],
-            S.psi[t], S.u[t], TauTile<double, CAP + TPAD, VI>::load(S, t)};
+            S.psi[t], S.u[t], TauTile<double, VI>::load(S, t)};
   }
   __device__ __forceinline__ void put(int l, const KParams& K, const Raw& r) {
     x[l] = r.x;
@@ -308,15 +314,15 @@ template <int CAP, bool VI> struct ForceTile<double, CAP, VI> {
 };
 
 // Positions, velocities and Q = 1/rho for the shear tensor pass.
-template <typename R, int CAP> struct TensTile {
-  DensTile<R, CAP> d;
+template <typename R> struct TensTile {
+  DensTile<R> d;
   R q[CAP + TPAD];
   struct Raw {
-    typename DensTile<R, CAP>::Raw d;
+    typename DensTile<R>::Raw d;
     R rho;
   };
   static __device__ __forceinline__ Raw load(const St<R>& S, int t) {
-    return {DensTile<R, CAP>::load(S, t), S.rho[t]};
+    return {DensTile<R>::load(S, t), S.rho[t]};
   }
   __device__ __forceinline__ void put(int l, const KParams& K, const Raw& r) {
     d.put(l, K, r.d);
@@ -331,138 +337,144 @@ template <typename R, int CAP> struct TensTile {
 };
 
 // ---- segment geometry ------------------------------------------------------
-// A segment: the particles [O0, O1) of cell row cy, which lie in cells
-// slo .. shi of that row; the tile holds the rows cy-1 .. cy+1 over those
-// cells (rs[k], rl[k]: sorted start and length of row k's range, lo[k]: its
-// first tile entry).
+// The piece of a workgroup: the particles [O0, O1) of cell row cy; the tile
+// holds the candidate ranges of rows cy-1 .. cy+1 (rs[k], rl[k]: sorted start
+// and length of row k's, lo[k]: its first tile entry).
 struct Segment {
-  int cy, slo, O0, O1;
+  int cy, O0, O1, x0, x1;
   int rs[3], rl[3], lo[3];
   int total;
 };
 
-// How a workgroup finds its segment.
-//  CW > 0: a fixed run of CW cells of a row (segment row * nseg + run).
-//  CW = 0: a piece of at most PIECE consecutive sorted positions of one row
-//          (RowPieces); every wavefront of a piece but the row's last is
-//          full.
 struct SegArg {
-  int nseg;
   const PieceRec* tab;
   int masks;  // the density pass has recorded the neighbour masks
 };
 
-// Width of the LDS copy of the cell starts (none for pieces, whose cells are
-// looked up in global memory: their span is not bounded).
-template <int CW> constexpr int csw() { return CW > 0 ? CW + 3 : 1; }
-
-// cell_start of cell c of tile row k (grid row cy-1+k): from the segment's
-// LDS copy (CW > 0) or from global memory (CW = 0).
-template <int CW> struct CellBounds {
-  const int (*cs)[csw<CW>()];
-  int slo;
-  __device__ __forceinline__ int at(int k, int c) const { return cs[k][c - slo]; }
-};
-template <> struct CellBounds<0> {
-  const int* __restrict__ cstart;
-  int base;  // (cy - 1) nx
-  int nx;
-  __device__ __forceinline__ int at(int k, int c) const { return cstart[base + k * nx + c]; }
-};
-
-template <int CW>
-__device__ __forceinline__ CellBounds<CW> bounds_of(const KParams& K, const Segment& g,
-                                                    const int* __restrict__ cstart,
-                                                    const int (*cs)[csw<CW>()]) {
-  if constexpr (CW > 0)
-    return CellBounds<CW>{cs, g.slo};
-  else
-    return CellBounds<0>{cstart, (g.cy - 1) * K.nx, K.nx};
+// O0 >= O1 when the workgroup has no particles.
+__device__ __forceinline__ Segment segment_of(const SegArg& sa) {
+  const PieceRec r = sa.tab[blockIdx.x];
+  Segment g;
+  g.cy = r.cy;
+  g.O0 = r.O0;
+  g.O1 = r.O1;
+  g.x0 = r.x0;
+  g.x1 = r.x1;
+  g.total = r.total;
+  int l = 0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    g.rs[k] = r.rs[k];
+    g.rl[k] = r.rl[k];
+    g.lo[k] = l;
+    l += r.rl[k];
+  }
+  return g;
 }
 
 // A lane particle's cell column and its candidates [ta_k, tb_k) of row k
-// (sorted positions; empty for a row outside the grid).  On pieces a lane
-// looks them up before the tile is filled, so that the two loads they take
-// one after the other run beside the staging.
+// (sorted positions; empty where the row has none), looked up before the tile
+// is filled, so that the loads run beside the staging.
 struct LaneRows {
   int cx;
   int ta[3], tb[3];
 };
-template <typename BD>
-__device__ __forceinline__ LaneRows lane_rows(const KParams& K, const Segment& g, const BD& B,
-                                              uint32_t key) {
+__device__ __forceinline__ LaneRows lane_rows(const KParams& K, const Segment& g,
+                                              const int* __restrict__ cstart, uint32_t key) {
   LaneRows r;
   r.cx = (int)key - g.cy * K.nx;
   const int ca = r.cx > 0 ? r.cx - 1 : 0;
   const int cb = (r.cx + 1 < K.nx ? r.cx + 1 : K.nx - 1) + 1;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const int kk = g.rl[k] ? k : 1;
-    const int a = B.at(kk, ca), b = B.at(kk, cb);
+    const int row = (g.cy - 1 + (g.rl[k] ? k : 1)) * K.nx;
+    const int a = cstart[row + ca], b = cstart[row + cb];
     r.ta[k] = g.rl[k] ? a : 0;
     r.tb[k] = g.rl[k] ? b : 0;
   }
   return r;
 }
 
-// The segment of this workgroup; O0 >= O1 when it has no particles.  With
-// CW > 0 the workgroup also copies the cell starts of its rows into cs.
-template <int CW>
-__device__ __forceinline__ Segment segment_of(const KParams& K, const int* __restrict__ cstart,
-                                              const SegArg& sa, int (*cs)[csw<CW>()]) {
-  Segment g;
-  if constexpr (CW > 0) {
-    // plain order: most cell runs of a tank are empty, and contiguous
-    // shares per XCD would leave the XCDs of the empty rows idle
-    const int nx = K.nx;
-    g.cy = blockIdx.x / sa.nseg;
-    const int cx0 = (blockIdx.x - g.cy * sa.nseg) * CW;
-    const int cx1 = min(cx0 + CW, nx);
-    g.O0 = cstart[g.cy * nx + cx0];
-    g.O1 = cstart[g.cy * nx + cx1];
-    g.slo = cx0 > 0 ? cx0 - 1 : 0;
-    const int shi = cx1 < nx ? cx1 : nx - 1;
-    g.total = 0;
+// On a grid periodic in x (PER) the particles of the first and last cell
+// columns also see the column at the other end.  A piece that holds some keeps
+// those cells in its tile after the rows: ranges 0 .. 2 are the last column's
+// (for cells of column 0), 3 .. 5 column 0's (for the last column's).
+// Particles of the seam that walked their nine cells in global memory instead
+// set the time of every launch (FP64 channel of 10,000 particles: force 40 us,
+// density and tensor 24 us).
+template <bool PER> struct Wrap {
+  static constexpr int total = 0;
+  __device__ __forceinline__ Wrap(const KParams&, const Segment&, const int*) {}
+};
+template <> struct Wrap<true> {
+  int rs[6], rl[6], lo[6];
+  int total;  // 0 off the seam
+  __device__ __forceinline__ Wrap(const KParams& K, const Segment& g,
+                                  const int* __restrict__ cstart) {
+    total = 0;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int ry = g.cy - 1 + k;
-      if (ry < 0 || ry >= K.ny || g.O0 >= g.O1) {
-        g.rs[k] = 0;
-        g.rl[k] = 0;
-      } else {
-        g.rs[k] = cstart[ry * nx + g.slo];
-        g.rl[k] = cstart[ry * nx + shi + 1] - g.rs[k];
-        const int ncs = shi + 2 - g.slo;
-        for (int j = threadIdx.x; j < ncs; j += blockDim.x) cs[k][j] = cstart[ry * nx + g.slo + j];
+    for (int k = 0; k < 6; ++k) {
+      const int ry = g.cy - 1 + k % 3;
+      rs[k] = rl[k] = 0;
+      if ((k < 3 ? g.x0 == 0 : g.x1 == K.nx - 1) && ry >= 0 && ry < K.ny) {
+        const int* e = cstart + ry * K.nx + (k < 3 ? K.nx - 1 : 0);
+        rs[k] = e[0];
+        rl[k] = e[1] - e[0];
       }
-      g.lo[k] = g.total;
-      g.total += g.rl[k];
-    }
-  } else {
-    const PieceRec r = sa.tab[blockIdx.x];
-    g.cy = r.cy;
-    g.slo = 0;
-    g.O0 = r.O0;
-    g.O1 = r.O1;
-    g.total = r.total;
-    int l = 0;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      g.rs[k] = r.rs[k];
-      g.rl[k] = r.rl[k];
-      g.lo[k] = l;
-      l += r.rl[k];
+      lo[k] = g.total + total;
+      total += rl[k];
     }
   }
-  return g;
+};
+
+// The lane particle as its candidates at the other end see it: sh cells on
+// (the operations of delta() with a shift).
+__device__ __forceinline__ LaneF image(LaneF p, int sh) {
+  p.cxf = p.cxf + (float)sh;
+  return p;
+}
+__device__ __forceinline__ PosD image(PosD p, int) { return p; }
+__device__ __forceinline__ float image_dx(const KParams&, const LaneF&, float dx, int) {
+  return dx;
+}
+__device__ __forceinline__ double image_dx(const KParams& K, const PosD&, double dx, int sh) {
+  return dx + (double)sh * K.cell;
 }
 
-// Tile entries q0 + u BLK + lane, u < UN, of the three rows, read (load(t): the
+// Calls visit(l, dx, dy, r2) for the neighbours of a lane particle at the
+// other end of the grid, after those of its own rows.
+template <typename R, typename Tile, typename LP, typename Visit>
+__device__ __forceinline__ void for_wrapped(const KParams& K, const Wrap<true>& W, const Tile& T,
+                                            int cx, const LP& pi, Visit&& visit) {
+  const bool left = cx == 0;
+  if (!left && cx != K.nx - 1) return;
+  const int sh = left ? K.nx : -K.nx;
+  const LP p = image(pi, sh);
+  const R cut2 = cutoff2<R>(K);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const R uy = (R)row_uy(K, k);
+    const int l0 = left ? W.lo[k] : W.lo[3 + k];
+    const int l1 = l0 + (left ? W.rl[k] : W.rl[3 + k]);
+    for (int l = l0; l < l1; ++l) {
+      R dx, dy;
+      T.delta(K, p, l, uy, dx, dy);
+      dx = image_dx(K, pi, dx, sh);
+      const R r2 = dx * dx + dy * dy;
+      if (r2 < cut2) visit(l, dx, dy, r2);
+    }
+  }
+}
+template <typename R, typename Tile, typename LP, typename Visit>
+__device__ __forceinline__ void for_wrapped(const KParams&, const Wrap<false>&, const Tile&, int,
+                                            const LP&, Visit&&) {}
+
+// Tile entries q0 + u PIECE + lane, u < UN, of the three rows, read (load(t): the
 // record of sorted position t) before any is written (put(l, record)), so that
 // filling a tile waits for memory once or twice.  Past the last entry the last
 // one is read and written again: no branch for the compiler to move the loads
 // into.
-template <int BLK, int UN, typename Raw> struct Stage {
+template <int UN, typename Raw> struct Stage {
   Raw r[UN];
   template <typename Load>
   __device__ __forceinline__ void load(const Segment& g, int q0, Load&& ld) {
@@ -481,69 +493,60 @@ template <int BLK, int UN, typename Raw> struct Stage {
     for (int u = 0; u < UN; ++u) pt(at(g, q0, u), r[u]);
   }
   static __device__ __forceinline__ int at(const Segment& g, int q0, int u) {
-    return min(q0 + u * BLK + (int)threadIdx.x, g.total - 1);
+    return min(q0 + u * PIECE + (int)threadIdx.x, g.total - 1);
   }
 };
 
-// The batches after the first.
-template <int BLK, int UN, typename Raw, typename Load, typename Put>
-__device__ __forceinline__ void stage_rest(const Segment& g, Load&& ld, Put&& pt) {
-  for (int q0 = UN * BLK; q0 < g.total; q0 += UN * BLK) {
-    Stage<BLK, UN, Raw> st;
+// The batches after the first, and the seam's cells.
+template <int UN, typename Raw, bool PER, typename Load, typename Put>
+__device__ __forceinline__ void stage_rest(const Segment& g, const Wrap<PER>& W, Load&& ld,
+                                           Put&& pt) {
+  for (int q0 = UN * PIECE; q0 < g.total; q0 += UN * PIECE) {
+    Stage<UN, Raw> st;
     st.load(g, q0, ld);
     st.put(g, q0, pt);
+  }
+  if constexpr (PER) {
+    for (int q = g.total + (int)threadIdx.x; q < g.total + W.total; q += PIECE) {
+      int t = 0;
+#pragma unroll
+      for (int k = 0; k < 6; ++k)
+        if (q >= W.lo[k]) t = q - W.lo[k] + W.rs[k];  // an empty range gives way to the next
+      pt(q, ld(t));
+    }
   }
 }
 
 // Fills the tile (if tiled), then calls lane(i, key, rows) for the workgroup's
 // particles, one lane each, and done(i, on) in all lanes (on: it has one);
-// early(i) loads what else lane() needs, late(i) what depends on that.  On pieces
-// (CW = 0) every lane has at most one particle, and its key, its rows and
-// early() are read beside the tile's records: after the piece's record that
-// takes two dependent loads, where a chain of staging, key and cell bounds
-// takes six, most of a workgroup's life on the small tiles of 2D.
-template <int CW, int BLK, int UN, typename Raw, typename BD, typename Early, typename Late,
-          typename Load, typename Put, typename Lane, typename Done>
-__device__ __forceinline__ void for_segment(const KParams& K, const Segment& g, const BD& B,
-                                            const uint32_t* __restrict__ skey, bool tiled,
+// early(i) loads what else lane() needs, late(i) what depends on that.  All of
+// it is read beside the tile's records: after the piece's record that takes
+// two dependent loads, where a chain of staging, key and cell bounds takes six,
+// most of a workgroup's life on the small tiles of 2D (720,000 particles, FP32:
+// force 43.5 -> 34.3 us, density 41.8 -> 35.1; 1,972, FP64: 12.7 -> 11.5 and
+// 13.0 -> 10.8).
+template <int UN, typename Raw, bool PER, typename Early, typename Late, typename Load,
+          typename Put, typename Lane, typename Done>
+__device__ __forceinline__ void for_segment(const KParams& K, const Segment& g,
+                                            const Wrap<PER>& W, const uint32_t* __restrict__ skey,
+                                            const int* __restrict__ cstart, bool tiled,
                                             Early&& early, Late&& late, Load&& ld, Put&& pt,
                                             Lane&& lane, Done&& done) {
-  if constexpr (CW == 0) {
-    static_assert(BLK >= PIECE, "a lane for every particle of a piece");
-    const int i = g.O0 + (int)threadIdx.x;
-    const int ic = min(i, g.O1 - 1);
-    const uint32_t key = skey[ic];
-    early(ic);
-    Stage<BLK, UN, Raw> st;
-    st.load(g, 0, ld);
-    const LaneRows r = lane_rows(K, g, B, key);
-    late(ic);
-    if (tiled) {
-      st.put(g, 0, pt);
-      stage_rest<BLK, UN, Raw>(g, ld, pt);
-    }
-    __syncthreads();
-    if (i < g.O1) lane(i, key, r);
-    done(i, i < g.O1);
-  } else {
-    if (tiled) {
-      Stage<BLK, UN, Raw> st;
-      st.load(g, 0, ld);
-      st.put(g, 0, pt);
-      stage_rest<BLK, UN, Raw>(g, ld, pt);
-    }
-    __syncthreads();
-    for (int i0 = g.O0; i0 < g.O1; i0 += BLK) {
-      const int i = i0 + threadIdx.x;
-      if (i < g.O1) {
-        const uint32_t key = skey[i];
-        early(i);
-        late(i);
-        lane(i, key, lane_rows(K, g, B, key));
-      }
-      done(i, i < g.O1);
-    }
+  const int i = g.O0 + (int)threadIdx.x;
+  const int ic = min(i, g.O1 - 1);  // no branch, so that the loads overlap
+  const uint32_t key = skey[ic];
+  early(ic);
+  Stage<UN, Raw> st;
+  st.load(g, 0, ld);
+  const LaneRows r = lane_rows(K, g, cstart, key);
+  late(ic);
+  if (tiled) {
+    st.put(g, 0, pt);
+    stage_rest<UN, Raw>(g, W, ld, pt);
   }
+  __syncthreads();
+  if (i < g.O1) lane(i, key, r);
+  done(i, i < g.O1);
 }
 
 // The row pieces on their own (after a sort that does not build them).
@@ -552,17 +555,6 @@ __global__ __launch_bounds__(BLOCK) void k_row_pieces(const int* __restrict__ cs
                                                       RowPieces rp, Halt hl) {
   if (hl.on()) return;
   row_pieces_block<BLOCK>(cstart, skey, rp, blockIdx.x, gridDim.x);
-}
-
-// A particle of the first or last cell column of a grid periodic in x: its
-// neighbours wrap to the other end, outside the segment's tile, so the
-// direct path (which walks the wrapped cells) takes it.  PER = false: the
-// kernel was launched for a grid without periodic x.
-template <bool PER>
-__device__ __forceinline__ bool seam(const KParams& K, const Segment& g, uint32_t key) {
-  if (!PER) return false;
-  const int cx = (int)key - g.cy * K.nx;
-  return cx == 0 || cx == K.nx - 1;
 }
 
 // Neighbour mask of candidates l0 .. l0+len-1 (len <= 32) of row k: eight
@@ -666,8 +658,7 @@ __device__ __forceinline__ void walk_rows(uint32_t m0, uint32_t m1, uint32_t m2,
 // K.fix2, a bound on (2h)^2 in units of the fixed-point positions (own: the
 // lane's) that covers their rounding; the survivors (about one in two thousand
 // too many) take the exact test in the walk.
-template <int CAP>
-__device__ __forceinline__ uint32_t row_mask_pre(const KParams& K, const PreTile<CAP>& P, s16x2 own,
+__device__ __forceinline__ uint32_t row_mask_pre(const KParams& K, const PreTile& P, s16x2 own,
                                                  int l0, int len, int self) {
   const int bound = -K.fix2;
   uint32_t m = 0;
@@ -692,9 +683,9 @@ __device__ __forceinline__ uint32_t row_mask_pre(const KParams& K, const PreTile
 // adds nothing (dens_pair with ok = false) and leaves the recorded mask.
 // Same visiting order and sums as for_neighbours; the exact masks in rm.
 // Taken by dens_walk for a particle with a row of more than 32 candidates.
-template <typename R, bool SUM, int CAP, typename LP, typename V>
+template <typename R, bool SUM, typename LP, typename V>
 __device__ __forceinline__ void dens_walk_rows(const KParams& K, const Segment& g, const LaneRows& lr,
-                                               const DensTile<R, CAP>& T, const PreTile<CAP>& P,
+                                               const DensTile<R>& T, const PreTile& P,
                                                const LP& pi, const V& vi, int i, DensOwn<R>& o,
                                                uint32_t* rm, bool* ok) {
   const int self = g.lo[1] + (i - g.rs[1]);
@@ -735,9 +726,9 @@ __device__ __forceinline__ void dens_walk_rows(const KParams& K, const Segment& 
 // branch.  Failed survivors are collected per row (fc, flushed at each row
 // change) and taken out of the recorded masks.  Same visiting order and sums
 // as for_neighbours; the exact masks in rm.
-template <typename R, bool SUM, int CAP, typename LP, typename V>
+template <typename R, bool SUM, typename LP, typename V>
 __device__ __forceinline__ void dens_walk(const KParams& K, const Segment& g, const LaneRows& lr,
-                                          const DensTile<R, CAP>& T, const PreTile<CAP>& P,
+                                          const DensTile<R>& T, const PreTile& P,
                                           const LP& pi, const V& vi, int i, DensOwn<R>& o,
                                           uint32_t* rm, bool* ok) {
   const int self = g.lo[1] + (i - g.rs[1]);
@@ -814,23 +805,22 @@ __device__ __forceinline__ void for_masked_rows(const KParams& K, const Segment&
             visit);
 }
 
-template <typename R, bool SUM, bool EOS, bool PER, int BLK, int CW, int CAP>
-__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && !PER ? 8 : 1))) void k_density_tiled(St<R> S, KParams K,
+template <typename R, bool SUM, bool EOS, bool PER>
+__global__ __launch_bounds__(PIECE) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && !PER ? 8 : 1))) void k_density_tiled(St<R> S, KParams K,
                                                        const uint32_t* __restrict__ skey,
                                                        const int* __restrict__ cstart, SegArg sa,
                                                        uint4* __restrict__ nbm) {
-  __shared__ DensTile<R, CAP> T;
-  __shared__ PreTile<CAP> P;
-  __shared__ int cs[3][csw<CW>()];
-  const Segment g = segment_of<CW>(K, cstart, sa, cs);
+  __shared__ DensTile<R> T;
+  __shared__ PreTile P;
+  const Segment g = segment_of(sa);
   if (halted(K) || g.O0 >= g.O1) return;
-  const auto B = bounds_of<CW>(K, g, cstart, cs);
-  const bool tiled = g.total <= CAP;
-  using Raw = typename DensTile<R, CAP>::Raw;
+  const Wrap<PER> W(K, g, cstart);
+  const bool tiled = g.total + W.total <= CAP;
+  using Raw = typename DensTile<R>::Raw;
   int id = 0;
   R rho = (R)0;
-  for_segment<CW, BLK, 4, Raw>(
-      K, g, B, skey, tiled,
+  for_segment<4, Raw>(
+      K, g, W, skey, cstart, tiled,
       [&](int i) {
         id = S.id[i];
         if (EOS) rho = S.rho[i];
@@ -841,8 +831,8 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
         T.put(l, K, r);
         P.put(l, K, r);
       },
-      [&](int i, uint32_t key, const LaneRows& lr) {
-        if (!tiled || seam<PER>(K, g, key)) {
+      [&](int i, uint32_t, const LaneRows& lr) {
+        if (!tiled) {
           density_direct<R, SUM, EOS, PER>(S, K, i, skey, cstart, nbm);
           return;
         }
@@ -854,35 +844,38 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(sizeof(R) =
         uint32_t rm[3] = {0u, 0u, 0u};
         bool ok = true;
         dens_walk<R, SUM>(K, g, lr, T, P, pi, vi, i, o, rm, &ok);
+        for_wrapped<R>(K, W, T, lr.cx, pi, [&](int l, R dx, R dy, R r2) {
+          const auto vj = T.vel(l);
+          dens_pair<R, SUM>(K, dx, dy, r2, vi.x - vj.x, vi.y - vj.y, o.sum, o.rs);
+        });
         nbm[i] = make_uint4(rm[0], rm[1], rm[2], ok ? 1u : 0u);
         dens_end<R, SUM, EOS>(S, K, i, o, id, rho);
       },
       [](int, bool) {});
 }
 
-template <typename R, bool PER, int BLK, int CW, int CAP>
-__global__ __launch_bounds__(BLK) void k_tensor_tiled(St<R> S, KParams K,
+template <typename R, bool PER>
+__global__ __launch_bounds__(PIECE) void k_tensor_tiled(St<R> S, KParams K,
                                                       const uint32_t* __restrict__ skey,
                                                       const int* __restrict__ cstart, SegArg sa,
                                                       const uint4* __restrict__ nbm) {
-  __shared__ TensTile<R, CAP> T;
-  __shared__ int cs[3][csw<CW>()];
-  const Segment g = segment_of<CW>(K, cstart, sa, cs);
+  __shared__ TensTile<R> T;
+  const Segment g = segment_of(sa);
   if (halted(K) || g.O0 >= g.O1) return;
-  const auto B = bounds_of<CW>(K, g, cstart, cs);
-  const bool tiled = g.total <= CAP;
-  using Raw = typename TensTile<R, CAP>::Raw;
+  const Wrap<PER> W(K, g, cstart);
+  const bool tiled = g.total + W.total <= CAP;
+  using Raw = typename TensTile<R>::Raw;
   uint4 nm;
-  for_segment<CW, BLK, 4, Raw>(
-      K, g, B, skey, tiled,
+  for_segment<4, Raw>(
+      K, g, W, skey, cstart, tiled,
       [&](int i) {
         nm = nbm[i];
         if (!sa.masks) nm.w = 0u;
       },
       [](int) {},
       [&](int t) { return T.load(S, t); }, [&](int l, const Raw& r) { T.put(l, K, r); },
-      [&](int i, uint32_t key, const LaneRows& lr) {
-        if (!tiled || seam<PER>(K, g, key)) {
+      [&](int i, uint32_t, const LaneRows& lr) {
+        if (!tiled) {
           tensor_direct<R, PER>(S, K, i, skey, cstart);
           return;
         }
@@ -890,12 +883,14 @@ __global__ __launch_bounds__(BLK) void k_tensor_tiled(St<R> S, KParams K,
         const auto pi = T.lane(self);
         const auto vi = T.d.vel(self);
         TensOwn<R> o;
+        auto pair = [&](int l, R dx, R dy, R r2) {
+          const auto vj = T.d.vel(l);
+          tens_pair(K, o, dx, dy, r2, vj.x - vi.x, vj.y - vi.y, T.q[l]);
+        };
         auto visit = [&](int l, R uy) {
           R dx, dy;
           T.delta(K, pi, l, uy, dx, dy);
-          const R r2 = dx * dx + dy * dy;
-          const auto vj = T.d.vel(l);
-          tens_pair(K, o, dx, dy, r2, vj.x - vi.x, vj.y - vi.y, T.q[l]);
+          pair(l, dx, dy, dx * dx + dy * dy);
         };
         if (nm.w && sizeof(R) == 4)
           for_masked_rows<R>(K, g, lr, nm, visit);
@@ -903,6 +898,7 @@ __global__ __launch_bounds__(BLK) void k_tensor_tiled(St<R> S, KParams K,
           for_masked<R>(K, g, lr, nm, visit);
         else
           for_neighbours<R>(K, g, lr, T, pi, i, visit);
+        for_wrapped<R>(K, W, T, lr.cx, pi, pair);
         tens_end(S, K, i, T.q[self], o);
       },
       [](int, bool) {});
@@ -914,25 +910,23 @@ __global__ __launch_bounds__(BLK) void k_tensor_tiled(St<R> S, KParams K,
 // particles, 4.4 of 41 us with 1,972 in FP64) costs a store.
 // PC: pa_sph and same_e2 fixed at compile time for the FP32 pair body
 // (force_pair_f32), -1 to read them from K (k_force_hot fixes them).
-template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool VI, bool PER, int BLK, int CW,
-          int CAP, int PC = -1>
-__global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
+template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool VI, bool PER, int PC = -1>
+__global__ __launch_bounds__(PIECE) void k_force_tiled(St<R> S, KParams K,
                                                      const uint32_t* __restrict__ skey,
                                                      const int* __restrict__ cstart, SegArg sa,
                                                      const uint4* __restrict__ nbm, Moved<R> M) {
-  __shared__ ForceTile<R, CAP, VI> T;
-  __shared__ int cs[3][csw<CW>()];
-  const Segment g = segment_of<CW>(K, cstart, sa, cs);
+  __shared__ ForceTile<R, VI> T;
+  const Segment g = segment_of(sa);
   if (halted(K) || g.O0 >= g.O1) return;
-  const auto B = bounds_of<CW>(K, g, cstart, cs);
-  const bool tiled = g.total <= CAP;
-  using Raw = typename ForceTile<R, CAP, VI>::Raw;
+  const Wrap<PER> W(K, g, cstart);
+  const bool tiled = g.total + W.total <= CAP;
+  using Raw = typename ForceTile<R, VI>::Raw;
   uint4 nm;
   int id = 0;
   MoveIn<R> m;
   Rates<R> rates;
-  for_segment<CW, BLK, VI ? 3 : 4, Raw>(
-      K, g, B, skey, tiled,
+  for_segment<VI ? 3 : 4, Raw>(
+      K, g, W, skey, cstart, tiled,
       [&](int i) {
         nm = nbm[i];
         if (!sa.masks) nm.w = 0u;
@@ -942,8 +936,8 @@ __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
         if (PRESS && M.its) m = move_load(S, K, M.its, i, id);
       },
       [&](int t) { return T.load(S, t); }, [&](int l, const Raw& r) { T.put(l, K, r); },
-      [&](int i, uint32_t key, const LaneRows& lr) {
-        if (!tiled || seam<PER>(K, g, key)) {
+      [&](int i, uint32_t, const LaneRows& lr) {
+        if (!tiled) {
           rates = force_direct<R, PRESS, AV, AH, XS, VI, PER>(S, K, i, skey, cstart);
           return;
         }
@@ -951,11 +945,13 @@ __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
         const auto pi = T.lane(self);
         ForceOwn<R> o;
         T.own(S, K, o, i, self);
+        auto pair = [&](int l, R dx, R dy, R r2) {
+          T.template pair<PRESS, AV, AH, XS, PC>(K, o, l, dx, dy, r2);
+        };
         auto visit = [&](int l, R uy) {
           R dx, dy;
           T.delta(K, pi, l, uy, dx, dy);
-          const R r2 = dx * dx + dy * dy;
-          T.template pair<PRESS, AV, AH, XS, PC>(K, o, l, dx, dy, r2);
+          pair(l, dx, dy, dx * dx + dy * dy);
         };
         if (nm.w && sizeof(R) == 4)
           for_masked_rows<R>(K, g, lr, nm, visit);  // the row-refill walk
@@ -963,6 +959,7 @@ __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
           for_masked<R>(K, g, lr, nm, visit);  // FP64 (walk_rows measured 0.6 % slower here)
         else
           for_neighbours<R>(K, g, lr, T, pi, i, visit);
+        for_wrapped<R>(K, W, T, lr.cx, pi, pair);
         rates = force_end<R, PRESS, XS, VI>(S, K, i, o, id);
       },
       [&](int i, bool on) {
@@ -980,7 +977,7 @@ __global__ __launch_bounds__(BLK) void k_force_tiled(St<R> S, KParams K,
 // where cells cx and cx+1 start), the exact value the FP32 delta computes.
 // The smaller tile lets eight workgroups share a CU.  Particles without
 // complete masks take the direct path.
-template <int CAP> struct HotForceTile {
+struct HotForceTile {
   float4 a[CAP];  // offx, offy, vx, vy
   float4 b[CAP];  // Q = 1/rho, A = p/rho, psi, u
   struct Raw {
@@ -1045,22 +1042,20 @@ __device__ __forceinline__ void walk_rows2_hot(uint32_t m0, uint32_t m1, uint32_
   }
 }
 
-template <int BLK, int CAP, int PC>
-__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) void k_force_hot(
+template <int PC>
+__global__ __launch_bounds__(PIECE) __attribute__((amdgpu_waves_per_eu(4))) void k_force_hot(
     St<float> S, KParams K, const uint32_t* __restrict__ skey, const int* __restrict__ cstart,
     SegArg sa, const uint4* __restrict__ nbm, Moved<float> M) {
-  __shared__ HotForceTile<CAP> T;
-  __shared__ int cs[3][csw<0>()];
-  const Segment g = segment_of<0>(K, cstart, sa, cs);
+  __shared__ HotForceTile T;
+  const Segment g = segment_of(sa);
   if (halted(K) || g.O0 >= g.O1) return;
-  const auto B = bounds_of<0>(K, g, cstart, cs);
   const bool tiled = g.total <= CAP;
   const int i = g.O0 + (int)threadIdx.x;
   const int ic = min(i, g.O1 - 1);
   const uint32_t key = skey[ic];
   const int id = S.id[ic];
-  using Raw = typename HotForceTile<CAP>::Raw;
-  Stage<BLK, 4, Raw> st;  // as for_segment
+  using Raw = HotForceTile::Raw;
+  Stage<4, Raw> st;  // as for_segment
   auto ld = [&](int t) { return T.load(S, t); };
   auto pt = [&](int l, const Raw& r) { T.put(l, K, r); };
   st.load(g, 0, ld);
@@ -1070,17 +1065,17 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) void k
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const int d = g.lo[k] - g.rs[k];
-    const int kk = g.rl[k] ? k : 1;  // a row outside the grid has an empty mask
-    rw[k].base = d + B.at(kk, cx > 0 ? cx - 1 : 0);
-    rw[k].e1 = d + B.at(kk, cx);
-    rw[k].e2 = d + B.at(kk, cx + 1);
+    const int* e = cstart + (g.cy - 1 + (g.rl[k] ? k : 1)) * K.nx;  // an empty row has no mask
+    rw[k].base = d + e[cx > 0 ? cx - 1 : 0];
+    rw[k].e1 = d + e[cx];
+    rw[k].e2 = d + e[cx + 1];
     rw[k].uy = row_uy(K, k);
   }
   MoveIn<float> m;
   if (M.its) m = move_load(S, K, M.its, ic, id);
   if (tiled) {
     st.put(g, 0, pt);
-    stage_rest<BLK, 4, Raw>(g, ld, pt);
+    stage_rest<4, Raw>(g, Wrap<false>(K, g, cstart), ld, pt);
   }
   __syncthreads();
   Rates<float> rates;
@@ -1130,33 +1125,5 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(4))) void k
   }
   if (M.its) move_particle(K, M, on, i, id, m, rates);
 }
-
-// Launch shapes: cells per segment (0: row pieces of PIECE particles), lanes,
-// LDS record capacity.  Both forms run on row pieces, except the force
-// gathers with the physical viscosity (ForceCfg), which run on cell runs.
-template <typename R> struct TileCfg;
-template <> struct TileCfg<float> {
-  static constexpr int BLK = PIECE, CW = 0, CAP = 592;
-};
-// The hot FP32 force gather (k_force_hot): row pieces; the tile (592 records
-// of 32 bytes, 18.9 KB) lets eight workgroups share a CU (a piece's three
-// rows hold about 3 x 140 records on the dam-break lattice, 584 at most).
-struct HotForceCfg {
-  static constexpr int BLK = PIECE, CW = 0, CAP = 592;
-};
-template <> struct TileCfg<double> {
-  static constexpr int BLK = PIECE, CW = 0, CAP = 600;
-};
-// The force gathers with the physical viscosity stage 16 (FP32) or 24 (FP64)
-// more bytes per record: a piece's 600-record tile would leave four (FP32)
-// or two (FP64) workgroups per CU, so they run on runs of cells with smaller
-// tiles (heated channel: FP32 force 218 -> 164 us, FP64 360 -> 334 us).
-template <typename R, bool VI> struct ForceCfg : TileCfg<R> {};
-template <> struct ForceCfg<float, true> {
-  static constexpr int BLK = 256, CW = 32, CAP = 720;
-};
-template <> struct ForceCfg<double, true> {
-  static constexpr int BLK = 128, CW = 16, CAP = 400;
-};
 
 }  // namespace arm
