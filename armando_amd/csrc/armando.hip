@@ -801,7 +801,6 @@ template <typename R> int fused_step(arm_ctx* c, int its, const StepHooks& hk) {
     std::swap(A, B);
     c->masks_valid = false;
   }
-  if (!xs && (rc = zero_av<R>(c))) return rc;
   c->sorted = true;
   if ((rc = density_t<R>(c, c->prm.density_method, true))) return rc;
   if (hk.jpart)
@@ -812,6 +811,7 @@ template <typename R> int fused_step(arm_ctx* c, int its, const StepHooks& hk) {
   bool moved = false;
   if ((rc = force_and_move_t<R>(c, true, c->prm.flags, xs, hk.tape ? nullptr : &mv, &moved)))
     return rc;
+  if (!xs && !moved && (rc = zero_av<R>(c))) return rc;
   take_new_h<R>(c);
   if (hk.tape) {
     const int nb = std::max(grid_of(n), grid_of(c->K.ncell + 1));

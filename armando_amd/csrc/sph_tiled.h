@@ -963,7 +963,10 @@ __global__ __launch_bounds__(PIECE) void k_force_tiled(St<R> S, KParams K,
         rates = force_end<R, PRESS, XS, VI>(S, K, i, o, id);
       },
       [&](int i, bool on) {
-        if (PRESS && M.its) move_particle(K, M, on, i, id, m, rates);
+        if (PRESS && M.its) {
+          if (!XS && on) S.av[i] = {};  // no XSPH: zero, as the host's fill leaves it
+          move_particle(K, M, on, i, id, m, rates);
+        }
       });
 }
 
