@@ -1512,11 +1512,31 @@ template <typename R> Pack3<R> pack3(arm_ctx* c) {
   return Pack3<R>{static_cast<R4*>(c->pack3_vq)};
 }
 
-// 3D density gather, one wavefront per workgroup (k3_density).  Records the
+// Wavefronts per workgroup of the 3D gathers: as many as the chip still holds
+// at once with all the others, four a SIMD in FP32, three in FP64 (two of the
+// adjoint's).  Density + force with 1, 2, 4, 8 wavefronts, us: 24,874 particles
+// FP32 93, 70, 52, 47, FP64 123, 93, 68, 75; 83,630 FP32 110, 97, 97, 111, FP64
+// 154, 141, 156, 198; 163,000 FP32 132, 146, 149, 185, FP64 201, 235, 261, 339.
+// Adjoint of both passes: 24,874 FP32 94, 79, 59, 54, FP64 118, 102, 71, 85;
+// 83,630 FP32 127, 119, 108, 127, FP64 170, 176, 180, 231.
+int share3(const arm_ctx* c, bool adjoint = false) {
+  const long long nw = (c->n + 63) / 64, room = 1024 * (is32(c) ? 4 : adjoint ? 2 : 3);
+  return 8 * nw <= room ? 8 : 4 * nw <= room ? 4 : 2 * nw <= room ? 2 : 1;
+}
+
+// 3D density gather, 64 particles per workgroup (k3_density).  Records the
 // neighbour masks for the force pass.
+template <typename R, bool SUM, bool EOS, int NS> void launch_density3_s(arm_ctx* c) {
+  hipLaunchKernelGGL((k3_density<R, SUM, EOS, NS>), dim3((c->n + 63) / 64), dim3(64 * NS), 0,
+                     c->stream, st3A<R>(c), c->K, c->skey, c->cstart, c->mask3, pack3<R>(c));
+}
 template <typename R, bool SUM, bool EOS> void launch_density3(arm_ctx* c) {
-  hipLaunchKernelGGL((k3_density<R, SUM, EOS>), dim3((c->n + 63) / 64), dim3(64), 0, c->stream,
-                     st3A<R>(c), c->K, c->skey, c->cstart, c->mask3, pack3<R>(c));
+  switch (share3(c)) {
+    case 8: launch_density3_s<R, SUM, EOS, 8>(c); break;
+    case 4: launch_density3_s<R, SUM, EOS, 4>(c); break;
+    case 2: launch_density3_s<R, SUM, EOS, 2>(c); break;
+    default: launch_density3_s<R, SUM, EOS, 1>(c);
+  }
   c->masks_valid = true;
 }
 
@@ -1537,6 +1557,17 @@ template <typename R> int eos3_t(arm_ctx* c) {
   return ARM_OK;
 }
 
+template <typename R, bool P, bool AV, bool AH, bool XS, int NS>
+void launch_force3_s(arm_ctx* c, const Pack3<R>& pk, const Mask3& m) {
+  const dim3 g((c->n + 63) / 64), b(64 * NS);
+  if (AV && AH && c->K.same_e2)
+    hipLaunchKernelGGL((k3_force<R, P, AV, AH, XS, AV && AH, NS>), g, b, 0, c->stream,
+                       st3A<R>(c), pk, c->K, c->skey, c->cstart, m);
+  else
+    hipLaunchKernelGGL((k3_force<R, P, AV, AH, XS, false, NS>), g, b, 0, c->stream, st3A<R>(c),
+                       pk, c->K, c->skey, c->cstart, m);
+}
+
 // packed: the records are those of the current state (density3_t with eos)
 template <typename R, bool P, bool AV, bool AH, bool XS>
 void launch_force3(arm_ctx* c, bool packed) {
@@ -1545,13 +1576,12 @@ void launch_force3(arm_ctx* c, bool packed) {
   if (!packed)
     hipLaunchKernelGGL(k3_force_pack<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream,
                        st3A<R>(c), c->K, pk);
-  const dim3 g((c->n + 63) / 64), b(64);
-  if (AV && AH && c->K.same_e2)
-    hipLaunchKernelGGL((k3_force<R, P, AV, AH, XS, AV && AH>), g, b, 0, c->stream, st3A<R>(c), pk,
-                       c->K, c->skey, c->cstart, m);
-  else
-    hipLaunchKernelGGL((k3_force<R, P, AV, AH, XS, false>), g, b, 0, c->stream, st3A<R>(c), pk,
-                       c->K, c->skey, c->cstart, m);
+  switch (share3(c)) {
+    case 8: launch_force3_s<R, P, AV, AH, XS, 8>(c, pk, m); break;
+    case 4: launch_force3_s<R, P, AV, AH, XS, 4>(c, pk, m); break;
+    case 2: launch_force3_s<R, P, AV, AH, XS, 2>(c, pk, m); break;
+    default: launch_force3_s<R, P, AV, AH, XS, 1>(c, pk, m);
+  }
 }
 
 template <typename R>
@@ -1855,20 +1885,44 @@ template <typename R> int alloc_tape3(Scratch& sc, Tape3<R>& t, int n, int ncell
   return ARM_OK;
 }
 
-template <typename R>
-void adj_force3(arm_ctx* c, const Tape3<R>& T, const AdjScratch3<R>& W, double* apart) {
+template <typename R, int NS>
+void adj_force3_s(arm_ctx* c, const Tape3<R>& T, const AdjScratch3<R>& W, double* apart) {
   const int f = c->prm.flags;
   const int code = ((f & ARM_ART_VISC) ? 4 : 0) | ((f & ARM_ART_HEAT) ? 2 : 0) | ((f & ARM_AV_VEL) ? 1 : 0);
-  const dim3 g((c->n + 63) / 64), b(64);
+  const dim3 g((c->n + 63) / 64), b(64 * NS);
   switch (code) {
-    case 0: hipLaunchKernelGGL((k3_adj_force<R, false, false, false>), g, b, 0, c->stream, T, c->K, W, apart); break;
-    case 1: hipLaunchKernelGGL((k3_adj_force<R, false, false, true>), g, b, 0, c->stream, T, c->K, W, apart); break;
-    case 2: hipLaunchKernelGGL((k3_adj_force<R, false, true, false>), g, b, 0, c->stream, T, c->K, W, apart); break;
-    case 3: hipLaunchKernelGGL((k3_adj_force<R, false, true, true>), g, b, 0, c->stream, T, c->K, W, apart); break;
-    case 4: hipLaunchKernelGGL((k3_adj_force<R, true, false, false>), g, b, 0, c->stream, T, c->K, W, apart); break;
-    case 5: hipLaunchKernelGGL((k3_adj_force<R, true, false, true>), g, b, 0, c->stream, T, c->K, W, apart); break;
-    case 6: hipLaunchKernelGGL((k3_adj_force<R, true, true, false>), g, b, 0, c->stream, T, c->K, W, apart); break;
-    default: hipLaunchKernelGGL((k3_adj_force<R, true, true, true>), g, b, 0, c->stream, T, c->K, W, apart); break;
+    case 0: hipLaunchKernelGGL((k3_adj_force<R, false, false, false, NS>), g, b, 0, c->stream, T, c->K, W, apart); break;
+    case 1: hipLaunchKernelGGL((k3_adj_force<R, false, false, true, NS>), g, b, 0, c->stream, T, c->K, W, apart); break;
+    case 2: hipLaunchKernelGGL((k3_adj_force<R, false, true, false, NS>), g, b, 0, c->stream, T, c->K, W, apart); break;
+    case 3: hipLaunchKernelGGL((k3_adj_force<R, false, true, true, NS>), g, b, 0, c->stream, T, c->K, W, apart); break;
+    case 4: hipLaunchKernelGGL((k3_adj_force<R, true, false, false, NS>), g, b, 0, c->stream, T, c->K, W, apart); break;
+    case 5: hipLaunchKernelGGL((k3_adj_force<R, true, false, true, NS>), g, b, 0, c->stream, T, c->K, W, apart); break;
+    case 6: hipLaunchKernelGGL((k3_adj_force<R, true, true, false, NS>), g, b, 0, c->stream, T, c->K, W, apart); break;
+    default: hipLaunchKernelGGL((k3_adj_force<R, true, true, true, NS>), g, b, 0, c->stream, T, c->K, W, apart); break;
+  }
+}
+
+template <typename R>
+void adj_force3(arm_ctx* c, const Tape3<R>& T, const AdjScratch3<R>& W, double* apart) {
+  switch (share3(c, true)) {
+    case 8: adj_force3_s<R, 8>(c, T, W, apart); break;
+    case 4: adj_force3_s<R, 4>(c, T, W, apart); break;
+    case 2: adj_force3_s<R, 2>(c, T, W, apart); break;
+    default: adj_force3_s<R, 1>(c, T, W, apart);
+  }
+}
+
+template <typename R, int NS>
+void adj_density3_s(arm_ctx* c, const Tape3<R>& T, const AdjScratch3<R>& W) {
+  hipLaunchKernelGGL((k3_adj_density<R, NS>), dim3((c->n + 63) / 64), dim3(64 * NS), 0, c->stream,
+                     T, c->K, W);
+}
+template <typename R> void adj_density3(arm_ctx* c, const Tape3<R>& T, const AdjScratch3<R>& W) {
+  switch (share3(c, true)) {
+    case 8: adj_density3_s<R, 8>(c, T, W); break;
+    case 4: adj_density3_s<R, 4>(c, T, W); break;
+    case 2: adj_density3_s<R, 2>(c, T, W); break;
+    default: adj_density3_s<R, 1>(c, T, W);
   }
 }
 
@@ -1991,7 +2045,7 @@ int rollout_backward3(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0
                          L, W, R->obj, R->kind, seed);
       adj_force3<Rf>(c, T, W, R->apart);
       hipLaunchKernelGGL(k3_adj_eos<Rf>, dim3(nb), dim3(BLOCK), 0, c->stream, T, c->K, W);
-      hipLaunchKernelGGL(k3_adj_density<Rf>, dim3(nw), dim3(64), 0, c->stream, T, c->K, W);
+      adj_density3<Rf>(c, T, W);
       hipLaunchKernelGGL(k3_adj_predictor<Rf>, dim3(nb), dim3(BLOCK), 0, c->stream, T, c->K, its,
                          L, W);
       HIPCHK(c, hipGetLastError());

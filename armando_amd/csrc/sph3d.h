@@ -435,13 +435,81 @@ __device__ __forceinline__ void window3(const uint32_t* p, int ch, int d, int le
   m[2] = l2 <= 0 ? 0u : (uint32_t)hi & (l2 >= 32 ? ~0u : (1u << l2) - 1u);
 }
 
-// Mask words lw[3k + q][lane] of the nine rows of every lane with on set (rows
-// of at most 96 candidates), the particle's own bit cleared.  Called by the
-// whole wavefront.  cx, row = cy + cz ny: the lane's cell; rec: LDS for the
+// Orders a wavefront's own LDS accesses (it needs no barrier: they execute in
+// order; the compiler must keep them so).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ---- the waves of a workgroup ---------------------------------------------
+// A 3D gather's workgroup has 64 particles, one lane of each of its S
+// wavefronts for each.  S = 1 where the launch fills the chip; below that a
+// wavefront's serial walk of some 75 neighbours is the launch (58 us of FP64
+// force at 25,000 particles, whose 389 wavefronts leave most SIMDs idle), so
+// S wavefronts share it: the density pass deals them the rows of the pre-test,
+// and in every pass wavefront s takes the candidates whose number in their row
+// is s modulo S; the sums are added in the order of s.  share3 on the host
+// picks S.  24,874 particles in FP64, S = 1 and 4: density 70 -> 35 us, force
+// 60 -> 33, their adjoints 44 -> 25 and 77 -> 46.
+template <int S> __device__ __forceinline__ uint32_t share_bits(int s) {
+  return (S == 1 ? 0xffffffffu : S == 2 ? 0x55555555u : S == 4 ? 0x11111111u : 0x01010101u) << s;
+}
+template <int S> __device__ __forceinline__ int wave_of() {
+  return S == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+}
+// Wavefronts 1 .. S-1 leave their W sums (put(v)), wavefront 0 adds them to its
+// own in order (add(v)); called by the whole workgroup.  lds: (S - 1) W x 64.
+template <int S, int W, typename R, typename Put, typename Add>
+__device__ __forceinline__ void share_sum(R (*lds)[64], int s, int lane, Put&& put, Add&& add) {
+  if constexpr (S > 1) {
+    R v[W];
+    if (s > 0) {
+      put(v);
+#pragma unroll
+      for (int q = 0; q < W; ++q) lds[(s - 1) * W + q][lane] = v[q];
+    }
+    __syncthreads();
+    if (s == 0) {
+#pragma unroll
+      for (int p = 0; p < S - 1; ++p) {
+#pragma unroll
+        for (int q = 0; q < W; ++q) v[q] = lds[p * W + q][lane];
+        add(v);
+      }
+    }
+  }
+}
+__device__ __forceinline__ void acc_put(double* v, const Acc<double>& a) { v[0] = a.s; }
+__device__ __forceinline__ void acc_add(Acc<double>& a, const double* v) { a.add(v[0]); }
+__device__ __forceinline__ void acc_put(float* v, const Acc<float>& a) {
+  v[0] = a.s;
+  v[1] = a.c;
+}
+__device__ __forceinline__ void acc_add(Acc<float>& a, const float* v) {
+  a.add(v[0]);
+  a.add(-v[1]);  // the sum is s - c
+}
+// Enters a lane's next word with neighbours in m (of one wavefront every
+// non-empty word has some).
+template <int S, typename Enter>
+__device__ __forceinline__ void next_word(const uint32_t& m, const uint32_t& nz, Enter&& enter) {
+  if (S == 1) {
+    if (m == 0u && nz != 0u) enter();
+  } else {
+    while (m == 0u && nz != 0u) enter();
+  }
+}
+template <typename R> constexpr int acc_words() { return sizeof(R) == 4 ? 2 : 1; }
+
+// Mask words lw[3k + q][lane] of the nine rows (wavefront s of S: rows k = s
+// modulo S) of every lane with on set (rows of at most 96 candidates), the
+// particle's own bit cleared.  Called by the whole wavefront.  cx, row = cy + cz ny: the lane's cell; rec: LDS for the
 // records staged of a row, P3_CAP and P3_TILE + 16 more that may be read.
-template <typename R>
-__device__ __forceinline__ void pretest3(const St3<R>& S, const KParams& K, int i, bool on, int cx,
-                                         int row, const Rows9& rw, float4* __restrict__ rec,
+template <int NS, typename R>
+__device__ __forceinline__ void pretest3(const St3<R>& S, const KParams& K, int s0, int i, bool on,
+                                         int cx, int row, const Rows9& rw, float4* __restrict__ rec,
                                          uint32_t (*__restrict__ lw)[64]) {
   const int* t0 = rw.t0;
   const int* t1 = rw.t1;
@@ -480,6 +548,7 @@ __device__ __forceinline__ void pretest3(const St3<R>& S, const KParams& K, int 
     bool fits = true;
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
+      if (k % NS != s0) continue;
       uint32_t p[4] = {0u, 0u, 0u, 0u};
       int u0 = 0, ch = 0;  // of the lane's tile: first candidate, candidates per word
 #pragma unroll
@@ -506,7 +575,7 @@ __device__ __forceinline__ void pretest3(const St3<R>& S, const KParams& K, int 
           rec[q] = make_float4(-2.f * r.x, -2.f * r.y, -2.f * r.z,
                                __builtin_fmaf(r.x, r.x, __builtin_fmaf(r.y, r.y, r.z * r.z)));
         }
-        __syncthreads();
+        wave_sync();
         const float* ap[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e)
@@ -526,7 +595,7 @@ __device__ __forceinline__ void pretest3(const St3<R>& S, const KParams& K, int 
               p[2 * h + e] =
                   __builtin_amdgcn_alignbit(p[2 * h + e], __float_as_uint(d[e][r]), 31);
         }
-        __syncthreads();
+        wave_sync();
         if ((lane >> 5) == h) {
           u0 = (lane >> 4) & 1 ? at[1] : at[0];
           ch = 4 * steps;
@@ -573,8 +642,8 @@ __device__ __forceinline__ void pretest3(const St3<R>& S, const KParams& K, int 
 // are kept in the lane's own LDS column, which the staged records use
 // before.  A lane with a row of more than 96 candidates tests and sums its
 // candidates one by one instead, in the same order.
-template <typename R, bool SUM, bool EOS>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3))) void k3_density(St3<R> S, KParams K,
+template <typename R, bool SUM, bool EOS, int NS>
+__global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3))) void k3_density(St3<R> S, KParams K,
                                                  const uint32_t* __restrict__ skey,
                                                  const int* __restrict__ cstart, Mask3 nbm,
                                                  Pack3<R> P) {
@@ -585,14 +654,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) ==
   // past the records end in the words
   struct Lds {
     union {
-      float4 rec[P3_CAP];
+      float4 rec[NS][P3_CAP];
       int lt[9][64];
     };
     uint32_t lw[M3_OK][64];
+    R part[NS > 1 ? (NS - 1) * 2 * acc_words<R>() : 1][64];
   };
   __shared__ Lds L;
-  static_assert(sizeof(Lds) >= sizeof(float4) * (P3_CAP + P3_TILE + 16), "reads past the records");
-  const int lane = threadIdx.x;
+  static_assert(sizeof(Lds) >= sizeof(float4) * (NS * P3_CAP + P3_TILE + 16), "reads past the records");
+  const int lane = threadIdx.x & 63, s0 = wave_of<NS>();
   const int i0 = xcd_block() * 64 + lane;
   const bool valid = i0 < K.n;
   const int i = valid ? i0 : K.n - 1;
@@ -602,7 +672,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) ==
   bool ok = true;
 #pragma unroll
   for (int k = 0; k < 9; ++k) ok = ok && rw.t1[k] - rw.t0[k] <= 32 * M3_WORDS;
-  pretest3(S, K, i, valid && ok, cx, row, rw, L.rec, L.lw);
+  pretest3<NS>(S, K, s0, i, valid && ok, cx, row, rw, L.rec[s0], L.lw);
+  __syncthreads();
   uint32_t(*lw)[64] = L.lw;
   int(*lt)[64] = L.lt;
   uint32_t nz = 0u;  // the lane's non-empty words
@@ -610,15 +681,18 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) ==
 #pragma unroll
     for (int q = 0; q < M3_OK; ++q) nz |= (lw[q][lane] != 0u ? 1u : 0u) << q;
   }
+  if (s0 == 0) {
 #pragma unroll
-  for (int k = 0; k < 9; ++k) lt[k][lane] = rw.t0[k];
-  if (!valid) return;
+    for (int k = 0; k < 9; ++k) lt[k][lane] = rw.t0[k];
+  }
+  __syncthreads();
   const auto pi = load_pos3(S, i);
   const auto vi = S.v[i];
   const R cut2 = cutoff2<R>(K);
   DensOwn<R> o;
-  dens_begin<R, SUM>(K, o);
-  if (ok) {
+  if (s0 == 0) dens_begin<R, SUM>(K, o);
+  const uint32_t mine = share_bits<NS>(s0);
+  if (valid && ok) {
     uint32_t m = 0u;
     int tb = 0, wc = 0;
     R uy = (R)0, uz = (R)0;
@@ -626,7 +700,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) ==
     auto enter = [&]() {
       wc = __builtin_ctz(nz);
       nz &= nz - 1u;
-      m = lw[wc][lane];
+      m = lw[wc][lane] & mine;
       const int k = (wc * 11) >> 5;  // wc / 3 for wc < 27
       const int ky = (k * 11) >> 5;  // k / 3 for k < 9
       uy = row_u3<R>(K, 1 - (k - 3 * ky));
@@ -634,14 +708,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) ==
       tb = lt[k][lane] + 32 * (wc - 3 * k);
     };
     while (true) {
-      if (m == 0u) {
-        if (nz == 0u) break;
-        enter();
-      }
+      next_word<NS>(m, nz, enter);
+      if (m == 0u) break;
       const int b0 = __builtin_ctz(m), w0 = wc, t0 = tb + b0;
       const R uy0 = uy, uz0 = uz;
       m &= m - 1u;
-      if (m == 0u && nz != 0u) enter();
+      next_word<NS>(m, nz, enter);
       const bool two = m != 0u;
       const int b1 = two ? __builtin_ctz(m) : b0, t1 = two ? tb + b1 : t0;
       m &= m - 1u;  // 0 stays 0
@@ -656,17 +728,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) ==
       dens3_pair<R, SUM>(K, bx, by, bz, rb, vi.x - v1.x, vi.y - v1.y, vi.z - v1.z, o.sum, o.rs,
                          in1);
       // passed the pre-test only: out of the recorded masks
-      if (!in0) lw[w0][lane] &= ~(1u << b0);
-      if (two && !in1) lw[wc][lane] &= ~(1u << b1);
+      if (!in0) atomicAnd(&lw[w0][lane], ~(1u << b0));
+      if (two && !in1) atomicAnd(&lw[wc][lane], ~(1u << b1));
     }
-    if (nbm.w)
-      for (int q = 0; q < M3_OK; ++q) nbm.put(q, i, lw[q][lane]);
-  } else {
+  } else if (valid) {
     for (int k = 0; k < 9; ++k) {
       const int t0 = rw.t0[k], t1 = rw.t1[k];
       const R uy = row_u3<R>(K, 1 - k % 3), uz = row_u3<R>(K, 1 - k / 3);
       for (int t = t0; t < t1; ++t) {
-        if (t == i) continue;
+        if (t == i || (t - t0) % NS != s0) continue;
         const auto pj = load_pos3(S, t);
         R dx, dy, dz;
         const R r2 = delta3(pi, pj, K, uy, uz, dx, dy, dz);
@@ -676,6 +746,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(R) ==
       }
     }
   }
+  constexpr int AW = acc_words<R>();
+  share_sum<NS, 2 * AW>(
+      L.part, s0, lane,
+      [&](R* v) {
+        acc_put(v, o.sum);
+        acc_put(v + AW, o.rs);
+      },
+      [&](const R* v) {
+        acc_add(o.sum, v);
+        acc_add(o.rs, v + AW);
+      });
+  if (!valid) return;
+  if (nbm.w && ok)
+#pragma unroll
+    for (int q = 0; q < M3_OK; ++q)
+      if (q % NS == s0) nbm.put(q, i, lw[q][lane]);
+  if (s0 != 0) return;
   if (nbm.w) nbm.put(M3_OK, i, ok ? 1u : 0u);
   dens_end<R, SUM, EOS>(S, K, i, o);
   if (EOS) force3_record(S, K, P, i);
@@ -891,16 +978,18 @@ __global__ __launch_bounds__(BLOCK) void k3_force_pack(St3<R> S, KParams K, Pack
 // once leave it at 790 us.  Below that size latency: 83,630 particles FP32
 // 51.6 -> 39.8 us; FP64 at 2.2M 1638 -> 1398 us.  The records written by the
 // density pass take 41 us there instead of a launch of 53 (FP64 106 of 121).
-template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool SE>
-__global__ __launch_bounds__(64) void k3_force(
+template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool SE, int NS>
+__global__ __launch_bounds__(64 * NS) void k3_force(
     St3<R> S, Pack3<R> P, KParams K, const uint32_t* __restrict__ skey,
     const int* __restrict__ cstart, Mask3 nbm) {
   if (halted(K)) return;
   __shared__ uint32_t lw[M3_OK][64];
   __shared__ int lt[9][64];
-  const int lane = threadIdx.x;
-  const int i = xcd_block() * 64 + lane;
-  if (i >= K.n) return;
+  __shared__ R part[NS > 1 ? (NS - 1) * (6 + acc_words<R>()) : 1][64];
+  const int lane = threadIdx.x & 63, s0 = wave_of<NS>();
+  const int i0 = xcd_block() * 64 + lane;
+  const bool valid = i0 < K.n;
+  const int i = valid ? i0 : K.n - 1;
   const auto pi = load_pos3(S, i);
   ForceOwn3<R> o;
   force3_begin(S, K, i, o);
@@ -915,8 +1004,9 @@ __global__ __launch_bounds__(64) void k3_force(
     return force3_terms<R, PRESS, AV, AH, XS, SE>(K, o, dx, dy, dz, r2, vq.x, vq.y, vq.z, vq.w,
                                                   ap.x, ap.y, ap.z);
   };
-  if (nbm.w && nbm.get(M3_OK, i)) {
-    uint32_t nz = 0u;
+  const bool masked = nbm.w && nbm.get(M3_OK, i);
+  uint32_t nz = 0u;
+  if (masked) {  // wavefronts that share the lanes write the same words
 #pragma unroll
     for (int q = 0; q < M3_OK; ++q) {
       const uint32_t m = nbm.get(q, i);
@@ -925,6 +1015,9 @@ __global__ __launch_bounds__(64) void k3_force(
     }
 #pragma unroll
     for (int k = 0; k < 9; ++k) lt[k][lane] = rw.t0[k];
+  }
+  if (valid && masked) {
+    const uint32_t mine = share_bits<NS>(s0);
     uint32_t m = 0u;
     int tb = 0;
     R uy = (R)0, uz = (R)0;
@@ -932,7 +1025,7 @@ __global__ __launch_bounds__(64) void k3_force(
     auto enter = [&]() {
       const int w = __builtin_ctz(nz);
       nz &= nz - 1u;
-      m = lw[w][lane];
+      m = lw[w][lane] & mine;
       const int k = (w * 11) >> 5;   // w / 3 for w < 27
       const int ky = (k * 11) >> 5;  // k / 3 for k < 9
       uy = row_u3<R>(K, 1 - (k - 3 * ky));
@@ -940,15 +1033,13 @@ __global__ __launch_bounds__(64) void k3_force(
       tb = lt[k][lane] + 32 * (w - 3 * k);
     };
     while (true) {
-      if (m == 0u) {
-        if (nz == 0u) break;
-        enter();
-      }
+      next_word<NS>(m, nz, enter);
+      if (m == 0u) break;
       const int ta = tb + (int)__builtin_ctz(m);
       const R ya = uy, za = uz;
       m &= m - 1u;
-      if constexpr (sizeof(R) == 4) {
-        if (m == 0u && nz != 0u) enter();
+      if constexpr (sizeof(R) == 4 || NS > 1) {
+        next_word<NS>(m, nz, enter);
         const bool two = m != 0u;
         const int tc = two ? tb + (int)__builtin_ctz(m) : ta;
         m &= m - 1u;  // 0 stays 0
@@ -960,12 +1051,12 @@ __global__ __launch_bounds__(64) void k3_force(
         force3_acc<R, PRESS, AV, AH, XS>(o, terms(ta, ya, za), true);
       }
     }
-  } else {
+  } else if (valid) {
     const R cut2 = cutoff2<R>(K);
     for (int k = 0; k < 9; ++k) {
       const R uy = row_u3<R>(K, 1 - k % 3), uz = row_u3<R>(K, 1 - k / 3);
       for (int t = rw.t0[k]; t < rw.t1[k]; ++t) {
-        if (t == i) continue;
+        if (t == i || (t - rw.t0[k]) % NS != s0) continue;
         const auto pj = load_pos3(S, t);
         R dx, dy, dz;
         const R r2 = delta3(pi, pj, K, uy, uz, dx, dy, dz);
@@ -974,7 +1065,19 @@ __global__ __launch_bounds__(64) void k3_force(
       }
     }
   }
-  force3_end<R, PRESS, XS>(S, K, i, o);
+  share_sum<NS, 6 + acc_words<R>()>(
+      part, s0, lane,
+      [&](R* v) {
+        v[0] = o.fx, v[1] = o.fy, v[2] = o.fz;
+        v[3] = o.xsx, v[4] = o.xsy, v[5] = o.xsz;
+        acc_put(v + 6, o.du);
+      },
+      [&](const R* v) {
+        o.fx += v[0], o.fy += v[1], o.fz += v[2];
+        o.xsx += v[3], o.xsy += v[4], o.xsz += v[5];
+        acc_add(o.du, v + 6);
+      });
+  if (valid && s0 == 0) force3_end<R, PRESS, XS>(S, K, i, o);
 }
 
 // ------------------------------------------------------------------------

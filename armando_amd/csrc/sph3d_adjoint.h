@@ -125,10 +125,10 @@ struct WalkLds3 {
 // step, in the forward's order: from the recorded masks when they are
 // complete, in one loop over the set bits of all 27 words (a wavefront runs
 // for its longest lane's neighbour count), else by testing the candidates
-// again.
-template <typename R, typename Visit>
-__device__ __forceinline__ void for_tape_neighbours3(const Tape3<R>& T, const KParams& K, int k,
-                                                     WalkLds3& L, Visit&& visit) {
+// again.  Wavefront s0 of NS visits its share of them (share_bits).
+template <int NS, typename R, typename Visit>
+__device__ __forceinline__ void for_tape_neighbours3(const Tape3<R>& T, const KParams& K, int s0,
+                                                     int k, WalkLds3& L, Visit&& visit) {
   const Rows9 rw = rows3_of(K, T.skey[k], T.cstart);
   const size_t st = (size_t)K.n;
   const int lane = threadIdx.x & 63;
@@ -145,18 +145,20 @@ __device__ __forceinline__ void for_tape_neighbours3(const Tape3<R>& T, const KP
     uint32_t m = 0u;
     int tb = 0;
     R uy = (R)0, uz = (R)0;
+    const uint32_t mine = share_bits<NS>(s0);
+    auto enter = [&]() {
+      const int w = __builtin_ctz(nz);
+      nz &= nz - 1u;
+      m = L.w[w][lane] & mine;
+      const int row = (w * 11) >> 5;   // w / 3 for w < 27
+      const int ky = (row * 11) >> 5;  // row / 3 for row < 9
+      uy = row_u3<R>(K, 1 - (row - 3 * ky));
+      uz = row_u3<R>(K, 1 - ky);
+      tb = L.t0[row][lane] + 32 * (w - 3 * row);
+    };
     while (true) {
-      if (m == 0u) {
-        if (nz == 0u) break;
-        const int w = __builtin_ctz(nz);
-        nz &= nz - 1u;
-        m = L.w[w][lane];
-        const int row = (w * 11) >> 5;   // w / 3 for w < 27
-        const int ky = (row * 11) >> 5;  // row / 3 for row < 9
-        uy = row_u3<R>(K, 1 - (row - 3 * ky));
-        uz = row_u3<R>(K, 1 - ky);
-        tb = L.t0[row][lane] + 32 * (w - 3 * row);
-      }
+      next_word<NS>(m, nz, enter);
+      if (m == 0u) break;
       const int l = tb + (int)__builtin_ctz(m);
       m &= m - 1u;
       visit(l, uy, uz);
@@ -168,7 +170,7 @@ __device__ __forceinline__ void for_tape_neighbours3(const Tape3<R>& T, const KP
   for (int row = 0; row < 9; ++row) {
     const R uy = row_u3<R>(K, 1 - row % 3), uz = row_u3<R>(K, 1 - row / 3);
     for (int l = rw.t0[row]; l < rw.t1[row]; ++l) {
-      if (l == k) continue;
+      if (l == k || (l - rw.t0[row]) % NS != s0) continue;
       R d0, d1, d2;
       const R r2 = delta3(pk, tape_pos3(T, l), K, uy, uz, d0, d1, d2);
       if (!(r2 < cut2)) continue;
@@ -270,13 +272,18 @@ __global__ __launch_bounds__(BLOCK) void k3_adj_corrector(Tape3<R> T, KParams K,
 //    Bound by VALU issue and the records' latency.  Measured: FP32, 2.2M
 //    particles 2130 -> 1233 us; FP64, 24,874 particles 206 -> 78 us.  Contiguous
 //    shares per XCD: 1384 -> 1233 us.
-template <typename R, bool AV, bool AH, bool XS>
-__global__ __launch_bounds__(64) void k3_adj_force(Tape3<R> T, KParams K, AdjScratch3<R> W,
+template <typename R, bool AV, bool AH, bool XS, int NS>
+__global__ __launch_bounds__(64 * NS) void k3_adj_force(Tape3<R> T, KParams K, AdjScratch3<R> W,
                                                    double* __restrict__ alpha_part) {
   __shared__ WalkLds3 L;
+  __shared__ R part[NS > 1 ? (NS - 1) * 10 : 1][64];
+  __shared__ double lals[NS];
+  const int lane = threadIdx.x & 63, s0 = wave_of<NS>();
   double lal = 0.0;
   const int kb = xcd_block();
-  const int k = kb * 64 + threadIdx.x;
+  const int k = kb * 64 + lane;
+  R lr_acc[3] = {0, 0, 0}, lv_acc[3] = {0, 0, 0};
+  R lQ = 0, lA = 0, lpsi = 0, lu = 0;
   if (k < K.n) {
     using R4 = typename V4<R>::type;
     const R m = (R)K.mass, h = (R)K.h, invh = (R)K.invh, C1 = (R)K.C1;
@@ -290,9 +297,7 @@ __global__ __launch_bounds__(64) void k3_adj_force(Tape3<R> T, KParams K, AdjScr
     const R em = (R)(K.xsph_eps * K.mass), wn = (R)K.wnorm;
     const R iq2 = (R)(0.5 / (K.h * K.h)), c3 = (R)(3.0 * K.C1);
     const bool pa0 = K.pa_sph == 0, se = K.same_e2 != 0;
-    R lr_acc[3] = {0, 0, 0}, lv_acc[3] = {0, 0, 0};
-    R lQ = 0, lA = 0, lpsi = 0, lu = 0;
-    for_tape_neighbours3<R>(T, K, k, L, [&](int l, R uy, R uz) {
+    for_tape_neighbours3<NS, R>(T, K, s0, k, L, [&](int l, R uy, R uz) {
       const R4* o = W.rec + ((unsigned)l << 1);
       const R4* f = W.frec + (((unsigned)l << 1) + (unsigned)l);
       const auto pl = pos_of_rec(o[0]);
@@ -373,6 +378,18 @@ __global__ __launch_bounds__(64) void k3_adj_force(Tape3<R> T, KParams K, AdjScr
         lv_acc[c] += ldv[c];
       }
     });
+  }
+  share_sum<NS, 10>(
+      part, s0, lane,
+      [&](R* v) {
+        for (int c = 0; c < 3; ++c) v[c] = lr_acc[c], v[3 + c] = lv_acc[c];
+        v[6] = lQ, v[7] = lA, v[8] = lpsi, v[9] = lu;
+      },
+      [&](const R* v) {
+        for (int c = 0; c < 3; ++c) lr_acc[c] += v[c], lv_acc[c] += v[3 + c];
+        lQ += v[6], lA += v[7], lpsi += v[8], lu += v[9];
+      });
+  if (k < K.n && s0 == 0) {
     W.lx[k] = lr_acc[0];
     W.ly[k] = lr_acc[1];
     W.lz[k] = lr_acc[2];
@@ -388,6 +405,12 @@ __global__ __launch_bounds__(64) void k3_adj_force(Tape3<R> T, KParams K, AdjScr
   lal *= 0.5;
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) lal += __shfl_down(lal, d, 64);
+  if constexpr (NS > 1) {
+    if (lane == 0) lals[s0] = lal;
+    __syncthreads();
+    lal = 0.0;
+    for (int q = 0; q < NS; ++q) lal += lals[q];
+  }
   if (threadIdx.x == 0) alpha_part[kb] += lal;
 }
 
@@ -420,18 +443,22 @@ __global__ __launch_bounds__(BLOCK) void k3_adj_eos(Tape3<R> T, KParams K, AdjSc
 
 // 4. density adjoint, gathered; adds to the position / velocity adjoints
 //    (FP32, 2.2M particles 726 -> 538 us; FP64, 24,874 particles 73 -> 45 us)
-template <typename R>
-__global__ __launch_bounds__(64) void k3_adj_density(Tape3<R> T, KParams K, AdjScratch3<R> W) {
+template <typename R, int NS>
+__global__ __launch_bounds__(64 * NS) void k3_adj_density(Tape3<R> T, KParams K,
+                                                          AdjScratch3<R> W) {
   __shared__ WalkLds3 L;
-  const int k = xcd_block() * 64 + threadIdx.x;
-  if (k >= K.n) return;
+  __shared__ R part[NS > 1 ? (NS - 1) * 6 : 1][64];
+  const int lane = threadIdx.x & 63, s0 = wave_of<NS>();
+  const int k0 = xcd_block() * 64 + lane;
+  const bool valid = k0 < K.n;
+  const int k = valid ? k0 : K.n - 1;
   using R4 = typename V4<R>::type;
   const R m = (R)K.mass, invh = (R)K.invh, C1 = (R)K.C1;
   const R c3 = (R)(1.5 * K.C1 / (K.h * K.h)) * m;  // m 3 C1 / (2 h^2)
   const auto pk = pos_of_rec(W.rec[2 * (size_t)k]);
   const R4 vk = W.rec[2 * (size_t)k + 1];
   R lr[3] = {0, 0, 0}, lv[3] = {0, 0, 0};
-  for_tape_neighbours3<R>(T, K, k, L, [&](int l, R uy, R uz) {
+  for_tape_neighbours3<NS, R>(T, K, s0, k, L, [&](int l, R uy, R uz) {
     const R4* o = W.rec + ((unsigned)l << 1);
     const auto pl = pos_of_rec(o[0]);
     const R4 vl = o[1];
@@ -450,6 +477,15 @@ __global__ __launch_bounds__(64) void k3_adj_density(Tape3<R> T, KParams K, AdjS
       lv[c] += lvr * r[c];
     }
   });
+  share_sum<NS, 6>(
+      part, s0, lane,
+      [&](R* v) {
+        for (int c = 0; c < 3; ++c) v[c] = lr[c], v[3 + c] = lv[c];
+      },
+      [&](const R* v) {
+        for (int c = 0; c < 3; ++c) lr[c] += v[c], lv[c] += v[3 + c];
+      });
+  if (!valid || s0 != 0) return;
   W.lx[k] += lr[0];
   W.ly[k] += lr[1];
   W.lz[k] += lr[2];
