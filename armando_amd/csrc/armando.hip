@@ -15,6 +15,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/armando.h"
@@ -922,11 +923,46 @@ template <typename R> int alloc_tape(Scratch& sc, Tape<R>& t, int n, int ncell, 
   return ARM_OK;
 }
 
+// Wavefronts that share a workgroup's 64 particles (share_bits): as many, up to
+// most, as keep the launch within f32 (f64) wavefronts for each of the 1024 SIMDs.
+int share_waves(const arm_ctx* c, int f32, int f64, int most) {
+  const long long nw = (c->n + 63) / 64, room = 1024 * (is32(c) ? f32 : f64);
+  int s = most;
+  while (s > 1 && s * nw > room) s /= 2;
+  return s;
+}
+
+// Of the 2D adjoint's gathers.  Force + density with 1, 2, 4 wavefronts, us: 40,000
+// particles FP32 23, 20, 19, FP64 31, 28, 27; 115,000 FP32 29, 31, 33, FP64 52,
+// 62, 61.
+int share_adj2(const arm_ctx* c) { return share_waves(c, 3, 3, 4); }
+
 template <typename R, bool AV, bool AH, bool XS, bool VI>
 void launch_adj_force(arm_ctx* c, const Tape<R>& T, const AdjScratch<R>& W, double* apart,
                       double* qpart, double* epart) {
-  hipLaunchKernelGGL((k_adj_force<R, AV, AH, XS, VI>), dim3(grid_of(c->n)), dim3(BLOCK), 0,
-                     c->stream, T, c->K, W, apart, qpart, epart);
+  auto run = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    hipLaunchKernelGGL((k_adj_force<R, AV, AH, XS, VI, NS>), dim3((c->n + 63) / 64), dim3(64 * NS),
+                       0, c->stream, T, c->K, W, apart, qpart, epart);
+  };
+  switch (share_adj2(c)) {
+    case 4: run(std::integral_constant<int, 4>()); break;
+    case 2: run(std::integral_constant<int, 2>()); break;
+    default: run(std::integral_constant<int, 1>());
+  }
+}
+
+template <typename R> void adj_density(arm_ctx* c, const Tape<R>& T, const AdjScratch<R>& W) {
+  auto run = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    hipLaunchKernelGGL((k_adj_density<R, NS>), dim3((c->n + 63) / 64), dim3(64 * NS), 0, c->stream,
+                       T, c->K, W);
+  };
+  switch (share_adj2(c)) {
+    case 4: run(std::integral_constant<int, 4>()); break;
+    case 2: run(std::integral_constant<int, 2>()); break;
+    default: run(std::integral_constant<int, 1>());
+  }
 }
 
 template <typename R, bool VI>
@@ -1034,8 +1070,9 @@ int rollout_forward(arm_ctx* c, int nsteps, int ckpt, const int32_t* obj_ids, in
   R->ckpt = ckpt;
   R->nck = (nsteps + ckpt - 1) / ckpt;
   R->kind = c->objkind;
-  if ((rc = sc.get(&R->obj, n)) || (rc = sc.get(&R->jpart, nb)) || (rc = sc.get(&R->apart, nb)) ||
-      (rc = sc.get(&R->qpart, nb)) || (rc = sc.get(&R->epart, nb)))
+  const int nw = (n + 63) / 64;  // k_adj_force's partials
+  if ((rc = sc.get(&R->obj, n)) || (rc = sc.get(&R->jpart, nb)) || (rc = sc.get(&R->apart, nw)) ||
+      (rc = sc.get(&R->qpart, nw)) || (rc = sc.get(&R->epart, nw)))
     return rc;
   {
     std::vector<uint8_t> h(n, 0);
@@ -1061,10 +1098,11 @@ int rollout_forward(arm_ctx* c, int nsteps, int ckpt, const int32_t* obj_ids, in
   for (double** q : lf)
     if ((rc = sc.get(q, n))) return rc;
   AdjScratch<Rf>& W = Ar.W;
-  Rf** wf[] = {&W.lax, &W.lay, &W.ldrho, &W.ldu, &W.lavx, &W.lavy, &W.lp,  &W.lQ,  &W.lA,
-               &W.lpsi, &W.lS, &W.lrhoh, &W.lu,  &W.lvx,  &W.lvy,  &W.lx,  &W.ly,  &W.lus};
+  Rf** wf[] = {&W.ldrho, &W.lp, &W.lQ,  &W.lA, &W.lpsi, &W.lrhoh,
+               &W.lu,    &W.lvx, &W.lvy, &W.lx, &W.ly,   &W.lus};
   for (Rf** q : wf)
     if ((rc = sc.get(q, n))) return rc;
+  if ((rc = sc.get(&W.rec, 2 * (size_t)n)) || (rc = sc.get(&W.frec, 2 * (size_t)n))) return rc;
   W.lTxx = W.lTyy = W.lTxy = nullptr;
   if (visc && ((rc = sc.get(&W.lTxx, n)) || (rc = sc.get(&W.lTyy, n)) || (rc = sc.get(&W.lTxy, n))))
     return rc;
@@ -1105,7 +1143,7 @@ int rollout_forward(arm_ctx* c, int nsteps, int ckpt, const int32_t* obj_ids, in
 template <typename Rf>
 int rollout_backward(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0, double* ms) {
   AdjRun* R = c->adj;
-  const int n = c->n, nb = grid_of(n);
+  const int n = c->n, nb = grid_of(n), nw = (n + 63) / 64;
   const int nsteps = R->nsteps, ckpt = R->ckpt, nck = R->nck;
   AdjState& L = R->L;
   AdjArrays<Rf>& Ar = R->arrays<Rf>();
@@ -1113,9 +1151,9 @@ int rollout_backward(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0,
   int rc;
   double** lf[] = {&L.x, &L.y, &L.vx, &L.vy, &L.rho, &L.u, &L.cax, &L.cay, &L.cdrho, &L.cdu};
   for (double** q : lf) HIPCHK(c, hipMemsetAsync(*q, 0, sizeof(double) * n, c->stream));
-  HIPCHK(c, hipMemsetAsync(R->apart, 0, sizeof(double) * nb, c->stream));
-  HIPCHK(c, hipMemsetAsync(R->qpart, 0, sizeof(double) * nb, c->stream));
-  HIPCHK(c, hipMemsetAsync(R->epart, 0, sizeof(double) * nb, c->stream));
+  HIPCHK(c, hipMemsetAsync(R->apart, 0, sizeof(double) * nw, c->stream));
+  HIPCHK(c, hipMemsetAsync(R->qpart, 0, sizeof(double) * nw, c->stream));
+  HIPCHK(c, hipMemsetAsync(R->epart, 0, sizeof(double) * nw, c->stream));
   hipEvent_t e0, e1;
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
@@ -1135,7 +1173,7 @@ int rollout_backward(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0,
                          L, W, R->obj, R->kind, seed);
       adj_force<Rf>(c, T, W, R->apart, R->qpart, R->epart);
       hipLaunchKernelGGL(k_adj_eos<Rf>, dim3(nb), dim3(BLOCK), 0, c->stream, T, c->K, W);
-      hipLaunchKernelGGL(k_adj_density<Rf>, dim3(nb), dim3(BLOCK), 0, c->stream, T, c->K, W);
+      adj_density<Rf>(c, T, W);
       hipLaunchKernelGGL(k_adj_predictor<Rf>, dim3(nb), dim3(BLOCK), 0, c->stream, T, c->K, its,
                          L, W);
       HIPCHK(c, hipGetLastError());
@@ -1151,10 +1189,10 @@ int rollout_backward(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0,
   HIPCHK(c, hipEventRecord(e1, c->stream));
   // leave the context at the final forward state
   if ((rc = copy_checkpoint(c, stA<Rf>(c), Ar.ck[nck], false))) return rc;
-  std::vector<double> ap(nb), qp(nb), ep(nb), gx(n), gy(n);
-  HIPCHK(c, hipMemcpyAsync(ap.data(), R->apart, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(qp.data(), R->qpart, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(ep.data(), R->epart, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
+  std::vector<double> ap(nw), qp(nw), ep(nw), gx(n), gy(n);
+  HIPCHK(c, hipMemcpyAsync(ap.data(), R->apart, sizeof(double) * nw, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipMemcpyAsync(qp.data(), R->qpart, sizeof(double) * nw, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipMemcpyAsync(ep.data(), R->epart, sizeof(double) * nw, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(gx.data(), L.vx, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipMemcpyAsync(gy.data(), L.vy, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1163,7 +1201,7 @@ int rollout_backward(arm_ctx* c, double seed, double* dJ_dalpha, double* dJ_dv0,
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   double As = 0, Qs = 0, Es = 0;
-  for (int k = 0; k < nb; ++k) {
+  for (int k = 0; k < nw; ++k) {
     As += ap[k];
     Qs += qp[k];
     Es += ep[k];
@@ -1520,8 +1558,7 @@ template <typename R> Pack3<R> pack3(arm_ctx* c) {
 // Adjoint of both passes: 24,874 FP32 94, 79, 59, 54, FP64 118, 102, 71, 85;
 // 83,630 FP32 127, 119, 108, 127, FP64 170, 176, 180, 231.
 int share3(const arm_ctx* c, bool adjoint = false) {
-  const long long nw = (c->n + 63) / 64, room = 1024 * (is32(c) ? 4 : adjoint ? 2 : 3);
-  return 8 * nw <= room ? 8 : 4 * nw <= room ? 4 : 2 * nw <= room ? 2 : 1;
+  return share_waves(c, 4, adjoint ? 2 : 3, 8);
 }
 
 // 3D density gather, 64 particles per workgroup (k3_density).  Records the

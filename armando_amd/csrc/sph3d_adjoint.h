@@ -79,14 +79,6 @@ template <typename R> struct AdjScratch3 {
 __device__ __forceinline__ float4 tape_rec3(const Tape3<float>& T, int t) { return T.pf[t]; }
 __device__ __forceinline__ double4 tape_rec3(const Tape3<double>& T, int t) { return T.xyz[t]; }
 
-// 1/x: the FP32 form's from the hardware's reciprocal (1 ulp) and one Newton
-// step, which rounds it as well as a division in a third of the instructions.
-__device__ __forceinline__ double rcp_n(double x) { return 1.0 / x; }
-__device__ __forceinline__ float rcp_n(float x) {
-  const float y = __builtin_amdgcn_rcpf(x);
-  return __builtin_fmaf(__builtin_fmaf(-x, y, 1.f), y, y);
-}
-
 template <typename R>
 __global__ __launch_bounds__(BLOCK) void k3_tape(St3<R> S, KParams K,
                                                  const uint32_t* __restrict__ skey,

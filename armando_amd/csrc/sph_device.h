@@ -345,6 +345,74 @@ template <> struct Acc<float> {
   __device__ __forceinline__ float get() const { return s; }
 };
 
+// ---- the wavefronts of a workgroup ----------------------------------------
+// A workgroup of the 3D gathers and of the adjoint's has 64 particles, one lane
+// of each of its S wavefronts for each.  S = 1 where the launch fills the chip; below that a
+// wavefront's serial walk of some 75 neighbours is the launch (58 us of FP64
+// force at 25,000 particles, whose 389 wavefronts leave most SIMDs idle), so
+// S wavefronts share it: the density pass deals them the rows of the pre-test,
+// and in every pass wavefront s takes the candidates whose number in their row
+// is s modulo S; the sums are added in the order of s.  The host
+// picks S (share_waves).  24,874 particles in FP64, S = 1 and 4: density 70 -> 35 us, force
+// 60 -> 33, their adjoints 44 -> 25 and 77 -> 46.
+template <int S> __device__ __forceinline__ uint32_t share_bits(int s) {
+  return (S == 1 ? 0xffffffffu : S == 2 ? 0x55555555u : S == 4 ? 0x11111111u : 0x01010101u) << s;
+}
+template <int S> __device__ __forceinline__ int wave_of() {
+  return S == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+}
+// Wavefronts 1 .. S-1 leave their W sums (put(v)), wavefront 0 adds them to its
+// own in order (add(v)); called by the whole workgroup.  lds: (S - 1) W x 64.
+template <int S, int W, typename R, typename Put, typename Add>
+__device__ __forceinline__ void share_sum(R (*lds)[64], int s, int lane, Put&& put, Add&& add) {
+  if constexpr (S > 1) {
+    R v[W];
+    if (s > 0) {
+      put(v);
+#pragma unroll
+      for (int q = 0; q < W; ++q) lds[(s - 1) * W + q][lane] = v[q];
+    }
+    __syncthreads();
+    if (s == 0) {
+#pragma unroll
+      for (int p = 0; p < S - 1; ++p) {
+#pragma unroll
+        for (int q = 0; q < W; ++q) v[q] = lds[p * W + q][lane];
+        add(v);
+      }
+    }
+  }
+}
+__device__ __forceinline__ void acc_put(double* v, const Acc<double>& a) { v[0] = a.s; }
+__device__ __forceinline__ void acc_add(Acc<double>& a, const double* v) { a.add(v[0]); }
+__device__ __forceinline__ void acc_put(float* v, const Acc<float>& a) {
+  v[0] = a.s;
+  v[1] = a.c;
+}
+__device__ __forceinline__ void acc_add(Acc<float>& a, const float* v) {
+  a.add(v[0]);
+  a.add(-v[1]);  // the sum is s - c
+}
+// Enters a lane's next word with neighbours in m (of one wavefront every
+// non-empty word has some).
+template <int S, typename Enter>
+__device__ __forceinline__ void next_word(const uint32_t& m, const uint32_t& nz, Enter&& enter) {
+  if (S == 1) {
+    if (m == 0u && nz != 0u) enter();
+  } else {
+    while (m == 0u && nz != 0u) enter();
+  }
+}
+template <typename R> constexpr int acc_words() { return sizeof(R) == 4 ? 2 : 1; }
+
+// 1/x: the FP32 form's from the hardware's reciprocal (1 ulp) and one Newton
+// step, which rounds it as well as a division in a third of the instructions.
+__device__ __forceinline__ double rcp_n(double x) { return 1.0 / x; }
+__device__ __forceinline__ float rcp_n(float x) {
+  const float y = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, y, 1.f), y, y);
+}
+
 // Linear EOS p = c0^2 rho + p0 from the stored density.
 __device__ __forceinline__ double linear_p(const KParams& K, double rho) {
   return K.lin_c2 * rho + K.lin_p0;
