@@ -608,7 +608,7 @@ def main():
         "pair_interactions_per_s": 2 * r32["niac"] / t_force,
         "passes_ms": {k: pass_ms(r32, k) for k in r32["passes"]},
         "roofline": {
-            "kernel": "k_force_hot<...> (internal_force + art_visc + art_heat + av_vel)",
+            "kernel": "k_force_hot<...> (internal_force + art_visc + art_heat + av_vel, then the corrector)",
             "bound": "hbm",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,

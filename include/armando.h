@@ -321,8 +321,9 @@ int arm_conservation3(arm_ctx* ctx, double out[6]);
                                 time_integration) */
 #define ARM_PASS_EOS 4       /* EOS + art_heat coefficient (arm_eos alone) */
 #define ARM_PASS_FORCE 5     /* [shear tensor +] internal_force + art_visc + art_heat
-                                + av_vel gather */
-#define ARM_PASS_INTEGRATE 6 /* predictor / corrector (+ keys of the next step) */
+                                + av_vel gather; in arm_time_integration in 2D also
+                                the corrector (+ keys of the next step) */
+#define ARM_PASS_INTEGRATE 6 /* predictor / corrector where a pass of its own */
 #define ARM_PASS_COUNT 7
 int arm_pass_times(arm_ctx* ctx, int n, double* ms, int* counts);
 int arm_reset_pass_times(arm_ctx* ctx);
