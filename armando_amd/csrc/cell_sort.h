@@ -328,8 +328,8 @@ struct RowPieces {
   int nx = 0, ny = 0, slots = 0;
 };
 
-// The workgroup of a run of workgroups that xcd_share gives logical block L
-// of count.
+// The workgroup that takes logical block L of count: workgroup b runs on XCD
+// b mod 8, and XCD x takes the x-th contiguous share of the blocks.
 __device__ __forceinline__ int share_slot(int count, int L) {
   constexpr int X = 8;
   const int q = count / X, r = count - q * X;
