@@ -284,22 +284,18 @@ __device__ __forceinline__ Rows9 rows3_of(const KParams& K, uint32_t key,
 // pair arithmetic (the 2D forms with a z component)
 // ------------------------------------------------------------------------
 // ok = false: no neighbour, the sums keep every word.
+// The constants of the pair bodies are not folded in FP32 as in 2D: with the
+// products m C1, -8 C1 m and wnorm eps m / 2 rounded once, the rates of an
+// 83,630-particle tank were further from FP64 (rel. L2: drho 1.56e-7 instead of
+// 1.27e-7, av 1.91e-7 instead of 1.63e-7), and the dam break's velocities after
+// 125 steps 1.8e-7 off instead of 1.3e-7: the rounded factors m, C1, wnorm are
+// together 5e-8 to 8e-8 low, which offsets the hardware square root (1.3e-8 low
+// in the mean, entering (q - 2)^3 threefold and more), while the folded ones
+// are within 1e-8.  It costs nothing at 2.2M particles (force 792 us, 794
+// folded; density 648 and 647), and 43.7 us instead of 40.6 of the force at 83,630.
 template <typename R, bool SUM>
 __device__ __forceinline__ void dens3_pair(const KParams& K, R dx, R dy, R dz, R r2, R dvx,
                                            R dvy, R dvz, Acc<R>& sum, Acc<R>& rs, bool ok = true) {
-  if constexpr (sizeof(R) == 4) {
-    // m dW.dv = m C1 (q - 2)^3 (dx dvx + dy dvy + dz dvz), m C1 one constant
-    const float q = fsqrt(r2) * K.kf.invh;
-    const float tq = q - 2.f;
-    const float vr = __builtin_fmaf(dvz, dz, __builtin_fmaf(dvy, dy, dvx * dx));
-    sum.add_if(K.kf.mC1 * ((tq * tq) * tq * vr), ok);
-    if (SUM) {
-      const float s = __builtin_fmaf(-0.5f, q, 1.f);
-      const float s2 = s * s;
-      rs.add_if(K.kf.mw * ((s2 * s2) * __builtin_fmaf(2.f, q, 1.f)), ok);
-    }
-    return;
-  }
   const R q = fsqrt(r2) * (R)K.invh;
   const R tq = q - (R)2;
   const R F = (R)K.C1 * (tq * tq * tq);
@@ -721,9 +717,6 @@ template <typename R> struct ForceOwn3 {
   using R4 = typename V4<R>::type;
   R4 v;
   R Q, A, psi, u;
-  // FP32 pair body: the particle's factors as in ForceOwn, and the pressure
-  // term f_cm (..) = (a1 Q_j + a0) + A_j (b1 Q_j + b0) for either pa_sph
-  R a0, a1, b0, b1, avb, ava, c4, c4psi, xw, xw2;
   R fx = 0, fy = 0, fz = 0, xsx = 0, xsy = 0, xsz = 0;
   Acc<R> du;
 };
@@ -734,23 +727,7 @@ __device__ __forceinline__ void force3_begin(const St3<R>& S, const KParams& K, 
   o.v = S.v[i];
   q_and_a(K, S.rho[i], S.p[i], o.Q, o.A);
   o.psi = S.psi[i];
-  if constexpr (sizeof(R) == 4) {
-    o.u = S.uf[i];
-    const float cm = K.kf.cm, q4 = 4.f * o.Q, c4 = cm * q4, cA = cm * o.A;
-    const bool pa0 = K.pa_sph == 0;
-    o.a0 = pa0 ? 0.f : cA * o.Q;
-    o.a1 = pa0 ? cA : 0.f;
-    o.b0 = pa0 ? cm * o.Q : 0.f;
-    o.b1 = pa0 ? 0.f : cm;
-    o.avb = c4 * K.kf.avbh2;
-    o.ava = c4 * K.kf.avah;
-    o.c4 = c4;
-    o.c4psi = c4 * o.psi;
-    o.xw = K.kf.xs * q4;
-    o.xw2 = 2.f * o.xw;
-  } else {
-    o.u = (R)S.u[i];
-  }
+  o.u = u3_of(S, i);
 }
 
 // The terms of one pair apart from their accumulation: the particle gains
@@ -759,9 +736,7 @@ template <typename R> struct Terms3 {
   R G, dx, dy, dz, d, wf, dvx, dvy, dvz;
 };
 
-// SE: artificial viscosity and heat share (h eta)^2.  The FP32 form has the
-// operations of force_terms_f32 (sph_kernels.h), the energy rate doubled; the
-// FP64 form the plain products and sums.
+// SE: artificial viscosity and heat share (h eta)^2.
 template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool SE>
 __device__ __forceinline__ Terms3<R> force3_terms(const KParams& K, const ForceOwn3<R>& o, R dx,
                                                   R dy, R dz, R r2, R vjx, R vjy, R vjz, R Qj,
@@ -777,32 +752,6 @@ __device__ __forceinline__ Terms3<R> force3_terms(const KParams& K, const ForceO
   t.d = (R)0;
   t.wf = (R)0;
   const R vr = fmr(t.dvz, dz, fmr(t.dvy, dy, t.dvx * dx));
-  if constexpr (sizeof(R) == 4) {
-    const float rr = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-    const float q = fsqrt(rr) * K.kf.invh;
-    const float s = __builtin_fmaf(-0.5f, q, 1.f);
-    const float s3 = s * s * s;
-    const float M = s3 * (Qj * frcp(o.Q + Qj));
-    float G = 0.f, inv_ea = 0.f;
-    if (PRESS) G = s3 * __builtin_fmaf(Aj, __builtin_fmaf(o.b1, Qj, o.b0), __builtin_fmaf(o.a1, Qj, o.a0));
-    if (AV) {
-      inv_ea = frcp(rr + K.kf.ave2);
-      const float e = __builtin_fminf(vr, 0.f) * inv_ea;
-      G = __builtin_fmaf(e * __builtin_fmaf(o.avb, e, o.ava), M, G);
-    }
-    float d = 0.f;
-    if (PRESS || AV) {
-      t.G = G;
-      d = G * vr;
-    }
-    if (AH) {
-      const float inv_eh = (AV && SE) ? inv_ea : frcp(rr + K.kf.ahe2);
-      d = __builtin_fmaf(__builtin_fmaf(o.c4, psij, o.c4psi) * M * (rr * inv_eh), o.u - uj, d);
-    }
-    t.d = d;
-    if (XS) t.wf = __builtin_fmaf(o.xw2, q, o.xw) * s * M;
-    return t;
-  }
   const R m = (R)K.mass;
   const R q = fsqrt(r2) * (R)K.invh;
   const R tq = q - (R)2;
@@ -878,7 +827,7 @@ __device__ __forceinline__ void force3_end(St3<R>& S, const KParams& K, int i,
     acc.z = o.fz + (grav ? (R)K.gz : (R)0);
     acc.w = (R)0;
     S.a[i] = acc;
-    S.du[i] = sizeof(R) == 4 ? (R)0.5 * o.du.get() : o.du.get();  // FP32: doubled sums
+    S.du[i] = o.du.get();
   }
   if (XS) {
     R4 w;
@@ -914,10 +863,10 @@ __global__ __launch_bounds__(BLOCK) void k3_force_pack(St3<R> S, KParams K, Pack
 // one L2 (3.6x less traffic beyond L2, 915 -> 880 us in FP32 at 2.2M).
 // Bound at 2.2M particles in FP32: the vector cache's tag accesses, one a cycle
 // (a record load of 64 lanes touches 46 lines; three loads a neighbour keep it
-// 92 % busy), so fewer instructions (2.71e8 -> 2.39e8) and two neighbours at
-// once leave it at 790 us.  Below that size latency: 83,630 particles FP32
-// 51.6 -> 39.8 us; FP64 at 2.2M 1638 -> 1398 us.  The records written by the
-// density pass take 41 us there instead of a launch of 53 (FP64 106 of 121).
+// 92 % busy), so two neighbours at once leave it at 792 us.  Below that size
+// latency: 83,630 particles FP32 51.6 -> 43.7 us; FP64 at 2.2M 1638 -> 1398 us.
+// The records written by the density pass take 41 us there instead of a launch
+// of 53 (FP64 106 of 121).
 template <typename R, bool PRESS, bool AV, bool AH, bool XS, bool SE, int NS>
 __global__ __launch_bounds__(64 * NS) void k3_force(
     St3<R> S, Pack3<R> P, KParams K, const uint32_t* __restrict__ skey,
