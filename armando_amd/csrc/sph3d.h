@@ -410,6 +410,20 @@ __device__ __forceinline__ Local3 local3(const KParams& K, double4 q, int cx0, i
           (float)(q.z - (K.oz + (double)cz * K.cell))};
 }
 
+// Whether the particle lies within a few cells of the cell it is sorted into, so
+// that local3 and pre3f hold.  One outside the grid does not (arm_link_list sorts it into
+// cell 0 and returns ARM_ERR_DOMAIN; the gathers still run for a caller that goes
+// on): it takes the exact test of every candidate.
+__device__ __forceinline__ bool local3_holds(const KParams& K, float4 q) {
+  const float c = 2.f * K.cellf;
+  return fabsf(q.x) <= c && fabsf(q.y) <= c && fabsf(q.z) <= c;
+}
+__device__ __forceinline__ bool local3_holds(const KParams& K, double4 q) {
+  const double x = q.x - K.ox, y = q.y - K.oy, z = q.z - K.oz;
+  return x >= -K.cell && x <= (K.nx + 1) * K.cell && y >= -K.cell && y <= (K.ny + 1) * K.cell &&
+         z >= -K.cell && z <= (K.nz + 1) * K.cell;
+}
+
 // The 96-bit window [d, d + len) of the four words p of ch bits each
 // (ch a multiple of 4, at most 32; len <= 96).
 __device__ __forceinline__ void window3(const uint32_t* p, int ch, int d, int len, uint32_t* m) {
@@ -576,8 +590,8 @@ __device__ __forceinline__ void pretest3(const St3<R>& S, const KParams& K, int 
 // loads are in flight together, each through the exact test and the pair
 // sums (a wavefront runs for its longest lane's survivor count).  The words
 // are kept in the lane's own LDS column, which the staged records use
-// before.  A lane with a row of more than 96 candidates tests and sums its
-// candidates one by one instead, in the same order.
+// before.  A lane with a row of more than 96 candidates, or outside the grid, tests
+// and sums its candidates one by one instead, in the same order.
 template <typename R, bool SUM, bool EOS, int NS>
 __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3))) void k3_density(St3<R> S, KParams K,
                                                  const uint32_t* __restrict__ skey,
@@ -605,7 +619,7 @@ __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(sizeof(
   const uint32_t key = skey[i];
   const int row = (int)(key / (uint32_t)K.nx), cx = (int)key - row * K.nx;
   const Rows9 rw = rows3_of(K, key, cstart);
-  bool ok = true;
+  bool ok = local3_holds(K, pos_rec3(S, i));
 #pragma unroll
   for (int k = 0; k < 9; ++k) ok = ok && rw.t1[k] - rw.t0[k] <= 32 * M3_WORDS;
   pretest3<NS>(S, K, s0, i, valid && ok, cx, row, rw, L.rec[s0], L.lw);
