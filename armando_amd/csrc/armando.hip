@@ -85,7 +85,6 @@ struct arm_ctx {
   St3<double> A3_64{}, B3_64{};
   St3<float> A3_32{}, B3_32{};
   uint32_t* nbm3 = nullptr;  // 3D neighbour masks (M3_TOTAL words per particle)
-  Mask3 mask3{};             // where the current step's masks lie: nbm3, or a tape's own
   void* pack3_vq = nullptr;  // 3D force pass: packed neighbour records (Pack3)
   void* d_cd = nullptr;      // ARM_CONTACT: contact displacement per slot (V2<R>)
   // sort workspace
@@ -1561,28 +1560,36 @@ int share3(const arm_ctx* c, bool adjoint = false) {
   return share_waves(c, 4, adjoint ? 2 : 3, 8);
 }
 
+// The context's own neighbour masks of the 3D gathers (nbm3), and what a force
+// pass may read of them.  A recorded step's masks lie in its tape: they are
+// handed down from call to call and leave no trace in the context, which
+// outlives the tape.
+Mask3 own_masks3(const arm_ctx* c) { return Mask3{c->nbm3, c->cap}; }
+Mask3 valid_masks3(const arm_ctx* c) { return Mask3{c->masks_valid ? c->nbm3 : nullptr, c->cap}; }
+
 // 3D density gather, 64 particles per workgroup (k3_density).  Records the
-// neighbour masks for the force pass.
-template <typename R, bool SUM, bool EOS, int NS> void launch_density3_s(arm_ctx* c) {
+// neighbour masks for the force pass in m.
+template <typename R, bool SUM, bool EOS, int NS>
+void launch_density3_s(arm_ctx* c, const Mask3& m) {
   hipLaunchKernelGGL((k3_density<R, SUM, EOS, NS>), dim3((c->n + 63) / 64), dim3(64 * NS), 0,
-                     c->stream, st3A<R>(c), c->K, c->skey, c->cstart, c->mask3, pack3<R>(c));
+                     c->stream, st3A<R>(c), c->K, c->skey, c->cstart, m, pack3<R>(c));
 }
-template <typename R, bool SUM, bool EOS> void launch_density3(arm_ctx* c) {
+template <typename R, bool SUM, bool EOS> void launch_density3(arm_ctx* c, const Mask3& m) {
   switch (share3(c)) {
-    case 8: launch_density3_s<R, SUM, EOS, 8>(c); break;
-    case 4: launch_density3_s<R, SUM, EOS, 4>(c); break;
-    case 2: launch_density3_s<R, SUM, EOS, 2>(c); break;
-    default: launch_density3_s<R, SUM, EOS, 1>(c);
+    case 8: launch_density3_s<R, SUM, EOS, 8>(c, m); break;
+    case 4: launch_density3_s<R, SUM, EOS, 4>(c, m); break;
+    case 2: launch_density3_s<R, SUM, EOS, 2>(c, m); break;
+    default: launch_density3_s<R, SUM, EOS, 1>(c, m);
   }
-  c->masks_valid = true;
+  if (m.w == c->nbm3) c->masks_valid = true;
 }
 
-template <typename R> int density3_t(arm_ctx* c, int method, bool eos) {
+template <typename R> int density3_t(arm_ctx* c, int method, bool eos, const Mask3& m) {
   PassTimer tm(c, ARM_PASS_DENSITY);
   if (method == 1)
-    eos ? launch_density3<R, true, true>(c) : launch_density3<R, true, false>(c);
+    eos ? launch_density3<R, true, true>(c, m) : launch_density3<R, true, false>(c, m);
   else
-    eos ? launch_density3<R, false, true>(c) : launch_density3<R, false, false>(c);
+    eos ? launch_density3<R, false, true>(c, m) : launch_density3<R, false, false>(c, m);
   HIPCHK(c, hipGetLastError());
   return ARM_OK;
 }
@@ -1605,10 +1612,10 @@ void launch_force3_s(arm_ctx* c, const Pack3<R>& pk, const Mask3& m) {
                        pk, c->K, c->skey, c->cstart, m);
 }
 
-// packed: the records are those of the current state (density3_t with eos)
+// packed: the records are those of the current state (density3_t with eos);
+// m: the neighbour masks of the current order, m.w null where there are none
 template <typename R, bool P, bool AV, bool AH, bool XS>
-void launch_force3(arm_ctx* c, bool packed) {
-  const Mask3 m{c->masks_valid ? c->mask3.w : nullptr, c->mask3.stride};
+void launch_force3(arm_ctx* c, bool packed, const Mask3& m) {
   const Pack3<R> pk = pack3<R>(c);
   if (!packed)
     hipLaunchKernelGGL(k3_force_pack<R>, dim3(grid_of(c->n)), dim3(BLOCK), 0, c->stream,
@@ -1622,7 +1629,7 @@ void launch_force3(arm_ctx* c, bool packed) {
 }
 
 template <typename R>
-int force3_t(arm_ctx* c, bool press, int flags, bool xs, bool packed = false) {
+int force3_t(arm_ctx* c, bool press, int flags, bool xs, bool packed, const Mask3& m) {
   const bool av = (flags & ARM_ART_VISC) != 0, ah = (flags & ARM_ART_HEAT) != 0;
   if (press && (flags & ARM_VISC))
     return fail(c, ARM_ERR_UNSUPPORTED, "physical viscosity is implemented in 2D only");
@@ -1630,15 +1637,15 @@ int force3_t(arm_ctx* c, bool press, int flags, bool xs, bool packed = false) {
   PassTimer tm(c, ARM_PASS_FORCE);
   const int code = (press ? 8 : 0) | (av ? 4 : 0) | (ah ? 2 : 0) | (xs ? 1 : 0);
   switch (code) {
-    case 8: launch_force3<R, true, false, false, false>(c, packed); break;
-    case 9: launch_force3<R, true, false, false, true>(c, packed); break;
-    case 10: launch_force3<R, true, false, true, false>(c, packed); break;
-    case 11: launch_force3<R, true, false, true, true>(c, packed); break;
-    case 12: launch_force3<R, true, true, false, false>(c, packed); break;
-    case 13: launch_force3<R, true, true, false, true>(c, packed); break;
-    case 14: launch_force3<R, true, true, true, false>(c, packed); break;
-    case 15: launch_force3<R, true, true, true, true>(c, packed); break;
-    case 1: launch_force3<R, false, false, false, true>(c, packed); break;
+    case 8: launch_force3<R, true, false, false, false>(c, packed, m); break;
+    case 9: launch_force3<R, true, false, false, true>(c, packed, m); break;
+    case 10: launch_force3<R, true, false, true, false>(c, packed, m); break;
+    case 11: launch_force3<R, true, false, true, true>(c, packed, m); break;
+    case 12: launch_force3<R, true, true, false, false>(c, packed, m); break;
+    case 13: launch_force3<R, true, true, false, true>(c, packed, m); break;
+    case 14: launch_force3<R, true, true, true, false>(c, packed, m); break;
+    case 15: launch_force3<R, true, true, true, true>(c, packed, m); break;
+    case 1: launch_force3<R, false, false, false, true>(c, packed, m); break;
     default: return fail(c, ARM_ERR_ARG, "force pass with nothing to compute");
   }
   if (press && (c->K.flags & KF_DEPOSITION))
@@ -1654,9 +1661,10 @@ template <typename R> int zero_av3(arm_ctx* c) {
 
 template <typename R> int single_step3_t(arm_ctx* c) {
   int rc;
-  if ((rc = density3_t<R>(c, c->prm.density_method, true))) return rc;
+  const Mask3 m = own_masks3(c);
+  if ((rc = density3_t<R>(c, c->prm.density_method, true, m))) return rc;
   const bool xs = (c->prm.flags & ARM_AV_VEL) != 0;
-  if ((rc = force3_t<R>(c, true, c->prm.flags, xs, true))) return rc;
+  if ((rc = force3_t<R>(c, true, c->prm.flags, xs, true, m))) return rc;
   if (!xs && (rc = zero_av3<R>(c))) return rc;
   c->have_rates = true;
   return ARM_OK;
@@ -1705,18 +1713,16 @@ template <typename R> int fused_step3(arm_ctx* c, int its, const StepHooks& hk =
   if (!xs && (rc = zero_av3<R>(c))) return rc;
   c->sorted = true;
   const Tape3<R>* tape = static_cast<const Tape3<R>*>(hk.tape);
-  c->mask3 = tape ? Mask3{tape->nbm, n} : Mask3{c->nbm3, c->cap};
-  if ((rc = density3_t<R>(c, c->prm.density_method, true))) return rc;
+  const Mask3 m = tape ? Mask3{tape->nbm, n} : own_masks3(c);
+  if ((rc = density3_t<R>(c, c->prm.density_method, true, m))) return rc;
   if (hk.jpart)
     hipLaunchKernelGGL(k3_objective<R>, dim3(grid_of(n)), dim3(BLOCK), 0, c->stream, st3A<R>(c),
                        c->K, hk.kind, hk.objmask, hk.jpart);
-  if ((rc = force3_t<R>(c, true, c->prm.flags, xs, true))) return rc;
+  if ((rc = force3_t<R>(c, true, c->prm.flags, xs, true, m))) return rc;
   if (tape) {
     const int nb = std::max(grid_of(n), grid_of(c->K.ncell + 1));
     hipLaunchKernelGGL(k3_tape<R>, dim3(nb), dim3(BLOCK), 0, c->stream, st3A<R>(c), c->K, c->skey,
                        c->cstart, *tape);
-    c->mask3 = Mask3{c->nbm3, c->cap};
-    c->masks_valid = false;
   }
   return corrector3_t<R>(c, its, true);
 }
@@ -2380,7 +2386,6 @@ int arm_create(const arm_params* prm, int capacity, arm_ctx** out) {
     rc = dalloc(c, &c->pieces, (size_t)capacity / PIECE + 2 * (size_t)c->K.ny + 2);
   }
   if (!rc && is3d(c)) rc = dalloc(c, &c->nbm3, (size_t)M3_TOTAL * capacity);
-  if (!rc && is3d(c)) c->mask3 = Mask3{c->nbm3, capacity};
   if (!rc && is3d(c)) {
     const size_t r4 = is32(c) ? sizeof(float4) : sizeof(double4);
     double4* q = nullptr;
@@ -2624,7 +2629,7 @@ int arm_density(arm_ctx* c, int method) {
   if (method != 0 && method != 1) return fail(c, ARM_ERR_UNSUPPORTED, "density method %d", method);
   int rc = need_sorted(c);
   if (rc) return rc;
-  rc = is3d(c) ? DISPATCH(c, density3_t)(c, method, false)
+  rc = is3d(c) ? DISPATCH(c, density3_t)(c, method, false, own_masks3(c))
                : DISPATCH(c, density_t)(c, method, false);
   if (!rc) HIPCHK(c, hipStreamSynchronize(c->stream));
   return rc;
@@ -2643,7 +2648,7 @@ int arm_internal_force(arm_ctx* c, int flags) {
   if (!c) return ARM_ERR_ARG;
   int rc = need_sorted(c);
   if (rc) return rc;
-  rc = is3d(c) ? DISPATCH(c, force3_t)(c, true, flags, false, false)
+  rc = is3d(c) ? DISPATCH(c, force3_t)(c, true, flags, false, false, valid_masks3(c))
                : DISPATCH(c, force_t)(c, true, flags, false);
   if (!rc) HIPCHK(c, hipStreamSynchronize(c->stream));
   return rc;
@@ -2653,7 +2658,7 @@ int arm_av_vel(arm_ctx* c) {
   if (!c) return ARM_ERR_ARG;
   int rc = need_sorted(c);
   if (rc) return rc;
-  rc = is3d(c) ? DISPATCH(c, force3_t)(c, false, 0, true, false)
+  rc = is3d(c) ? DISPATCH(c, force3_t)(c, false, 0, true, false, valid_masks3(c))
                : DISPATCH(c, force_t)(c, false, 0, true);
   if (!rc) HIPCHK(c, hipStreamSynchronize(c->stream));
   return rc;
