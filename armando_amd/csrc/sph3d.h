@@ -167,13 +167,12 @@ __global__ __launch_bounds__(BLOCK) void k3_reorder_all(St3<R> A, St3<R> Bs, KPa
   const int t = ord.place(skey, cstart, p, id);
   Bs.id[t] = id;
   Bs.xyz[t] = A.xyz[s];
-  if constexpr (sizeof(R) == 4) {
-    Bs.pf[t] = A.pf[s];
-    Bs.uf[t] = A.uf[s];
-  }
+  if constexpr (sizeof(R) == 4) Bs.pf[t] = A.pf[s];
   Bs.v[t] = A.v[s];
   Bs.rho[t] = A.rho[s];
-  Bs.u[t] = A.u[s];
+  const double u = A.u[s];
+  Bs.u[t] = u;
+  if constexpr (sizeof(R) == 4) Bs.uf[t] = (float)u;  // a rollout leaves A.uf behind
   Bs.p[t] = A.p[s];
   Bs.psi[t] = A.psi[s];
   Bs.drho[t] = A.drho[s];
