@@ -68,6 +68,7 @@ struct arm_ctx {
   uint4* nbm = nullptr;
   // 2D tiled gathers: the row pieces of the current order (RowPieces)
   PieceRec* pieces = nullptr;
+  int* row_sums = nullptr;
   int piece_slots = 0;  // of the table last built
   bool pieces_valid = false;
   // deposition heat source (arm_set_deposition): the map on the device, the
@@ -263,8 +264,8 @@ Ent ent_of(arm_ctx* c) {
 
 RowPieces row_pieces_of(arm_ctx* c) {
   if (!c->pieces) return {};
-  c->piece_slots = (c->n + PIECE - 1) / PIECE + c->K.ny;
-  return {c->pieces, c->K.nx, c->K.ny, c->piece_slots};
+  c->piece_slots = (int)piece_slots(c->n, c->K.ny);
+  return {c->pieces, c->row_sums, c->K.nx, c->K.ny, c->piece_slots};
 }
 
 // Sorts the first n_sort slots (c->n when n_sort < 0) by (cell, id): skey holds
@@ -287,8 +288,10 @@ int run_sort(arm_ctx* c, const int32_t* id_of, Order* order, bool* ranges_done,
     ++c->scan_epoch;
     hipLaunchKernelGGL(k_cs_scan1, dim3(c->cs_tiles), dim3(CS_THREADS), 0, c->stream, c->cnt,
                        ncell, n, c->cstart, c->tstat, c->scan_epoch, hl);
-    hipLaunchKernelGGL(k_cs_scatter, dim3(nb), dim3(CS_THREADS), 0, c->stream, c->key_by_id,
-                       id_of, n, c->cstart, c->cnt, ent_of(c), c->sk[1], hl);
+    const RowPieces rp = row_pieces_of(c);
+    hipLaunchKernelGGL(k_cs_scatter, dim3(nb + (rp.tab ? row_chunks(rp.ny) : 0)), dim3(CS_THREADS),
+                       0, c->stream, c->key_by_id, id_of, n, c->cstart, c->cnt, ent_of(c),
+                       c->sk[1], hl, rp);
     HIPCHK(c, hipGetLastError());
     c->skey = c->sk[1];
     *order = Order{ent_of(c).id, ent_of(c).slot};
@@ -448,17 +451,19 @@ template <typename R> int link_list_t(arm_ctx* c) {
 }
 
 // The row pieces of the tiled gathers (rebuilt after each sort) and how many
-// workgroups they take: ny for the cut parts and piece_slots.
+// workgroups they take.
 SegArg seg_arg(arm_ctx* c) {
   if (!c->pieces_valid) {
     const RowPieces rp = row_pieces_of(c);
+    hipLaunchKernelGGL(k_row_sums, dim3(row_chunks(rp.ny)), dim3(ROW_CHUNK), 0, c->stream,
+                       c->cstart, rp, Halt{c->K.halt, c->K.its});
     hipLaunchKernelGGL(k_row_pieces, dim3(row_blocks(rp)), dim3(BLOCK), 0, c->stream,
                        c->cstart, c->skey, rp, Halt{c->K.halt, c->K.its});
     c->pieces_valid = true;
   }
   return SegArg{c->pieces, c->masks_valid};
 }
-int seg_grid(const arm_ctx* c) { return c->K.ny + c->piece_slots; }
+int seg_grid(const arm_ctx* c) { return c->piece_slots; }
 
 template <typename R, bool SUM, bool EOS> void launch_density(arm_ctx* c) {
   St<R>& A = stA<R>(c);
@@ -2383,7 +2388,8 @@ int arm_create(const arm_params* prm, int capacity, arm_ctx** out) {
   if (!rc) rc = dalloc(c, &c->d_cnt, capacity);
   if (!rc) rc = dalloc(c, &c->nbm, capacity);
   if (!rc && !is3d(c)) {
-    rc = dalloc(c, &c->pieces, (size_t)capacity / PIECE + 2 * (size_t)c->K.ny + 2);
+    rc = dalloc(c, &c->pieces, (size_t)piece_slots(capacity, c->K.ny));
+    if (!rc) rc = dalloc(c, &c->row_sums, (size_t)row_chunks(c->K.ny));
   }
   if (!rc && is3d(c)) rc = dalloc(c, &c->nbm3, (size_t)M3_TOTAL * capacity);
   if (!rc && is3d(c)) {
@@ -3073,7 +3079,7 @@ extern "C" int arm_link_list_static(const arm_params* prm, int n, const double* 
   if (n > 0) {
     hipLaunchKernelGGL(k_cs_scatter, dim3(nb), dim3(CS_THREADS), 0, s, key,
                        static_cast<const int32_t*>(nullptr), n,
-                       reinterpret_cast<const int*>(cell_start), count, ent, entc, Halt{});
+                       reinterpret_cast<const int*>(cell_start), count, ent, entc, Halt{}, RowPieces{});
     hipLaunchKernelGGL(k_cs_rank, dim3(nb), dim3(CS_THREADS), 0, s, ent, entc, n,
                        reinterpret_cast<const int*>(cell_start),
                        reinterpret_cast<uint32_t*>(key_sorted),

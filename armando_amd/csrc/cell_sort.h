@@ -264,6 +264,94 @@ __global__ __launch_bounds__(CS_THREADS) void k_cs_scan1(const int* __restrict__
   if (b == 0 && threadIdx.x == 0) cstart[ncell] = n;
 }
 
+// Pieces of the cell rows, for the gathers that give each workgroup a run of
+// consecutive sorted positions of one row: the sorted range of row y,
+// [cstart[y nx], cstart[(y+1) nx]), cut into runs of PIECE positions from its
+// start (the last one shorter).  tab[b] is all that workgroup b of a gather
+// needs to begin: its particles [O0, O1) of row cy and the three ranges of
+// sorted positions that hold their candidates, so that one load stands
+// between the launch and the filling of the tile (a chain of five before, a
+// microsecond each for every workgroup).
+//
+// Above a tank's free surface a row holds wall particles on either side only,
+// and the row below everything between them, so that a piece over the gap needs
+// more records than a gather's tile holds and its workgroup runs on the direct
+// path, as long as a whole launch of the others (FP32 force of the
+// 111,119-particle dam break: 28.6 us, 12.8 without; density 20.5 and 14.5).  A
+// piece of more than GAP_SPAN cells whose three rows hold more than GAP_RECORDS
+// particles is therefore cut at the middle of its cells, at most one of each row.
+//
+// A row has its pieces in order, then, where it and its neighbours hold more than
+// GAP_RECORDS particles, one place for the part cut off (empty if none is).  The
+// places of all rows, count in all, are dealt so that the workgroups of one XCD
+// take one contiguous share (neighbouring pieces, which stage the same rows, then
+// share an L2); the rest of the table is empty.  The host bounds count by
+// n / PIECE + min(ny, n) + min(ny, 3 n / GAP_RECORDS) (piece_slots).
+constexpr int PIECE = 128;
+constexpr int GAP_SPAN = 40;      // a full piece of 2h cells spans about 20
+constexpr int GAP_RECORDS = 592;  // the records of a gather's tile
+struct alignas(16) PieceRec {
+  int O0, O1, cy, total;  // total = rl[0] + rl[1] + rl[2]
+  int rs[3], rl[3];       // sorted start and length of rows cy-1, cy, cy+1
+  int x0, x1;             // cells of its first and last particle
+};
+// sums[c]: the places of rows ROW_CHUNK c .. (row_sums_block)
+struct RowPieces {
+  PieceRec* tab = nullptr;
+  int* sums = nullptr;
+  int nx = 0, ny = 0, slots = 0;
+};
+constexpr int ROW_CHUNK = 256;
+__host__ __device__ inline int row_chunks(int ny) { return (ny + ROW_CHUNK - 1) / ROW_CHUNK; }
+// Bound on count for n particles.
+__host__ inline long long piece_slots(long long n, long long ny) {
+  const long long cuts = 3 * n / GAP_RECORDS;
+  return (n + PIECE - 1) / PIECE + (ny < n ? ny : n) + (ny < cuts ? ny : cuts);
+}
+
+// A row's pieces and its places in the table.
+struct RowCount {
+  int a, b;  // its sorted range
+  int pieces, places;
+};
+__device__ __forceinline__ RowCount row_count(const int* __restrict__ cstart, const RowPieces& rp,
+                                              int y) {
+  RowCount r;
+  r.a = cstart[y * rp.nx];
+  r.b = cstart[(y + 1) * rp.nx];
+  r.pieces = (r.b - r.a + PIECE - 1) / PIECE;
+  const int lo = cstart[max(y - 1, 0) * rp.nx], hi = cstart[min(y + 2, rp.ny) * rp.nx];
+  r.places = r.pieces + (r.pieces && hi - lo > GAP_RECORDS ? 1 : 0);
+  return r;
+}
+
+// The workgroup that takes logical block L of count: workgroup b runs on XCD
+// b mod 8, and XCD x takes the x-th contiguous share of the blocks.
+__device__ __forceinline__ int share_slot(int count, int L) {
+  constexpr int X = 8;
+  const int q = count / X, r = count - q * X;
+  if (L < r * (q + 1)) return (L % (q + 1)) * X + L / (q + 1);
+  const int m = L - r * (q + 1);
+  return (m % q) * X + r + m / q;
+}
+
+// The places of the ROW_CHUNK rows of chunk c, one lane per row.  They are added
+// up before the table is made (beside the scatter), so that a workgroup of
+// row_pieces_block reads its chunk's rows and a word for each other chunk: with
+// every workgroup counting every row, ny^2 / 2 loads, the reorder of 2,400 particles
+// in 60,000 rows took 2,283 us (26 now; 8 in 48 rows of as many cells in all), that
+// of 1.2 million in 12,510 rows 154 us (40).
+template <int THREADS>
+__device__ __forceinline__ void row_sums_block(const int* __restrict__ cstart, const RowPieces& rp,
+                                               int c) {
+  static_assert(THREADS == ROW_CHUNK, "one lane per row");
+  __shared__ int wsum[THREADS / 64];
+  const int y = c * ROW_CHUNK + (int)threadIdx.x;
+  int total;
+  block_exclusive_scan<THREADS>(y < rp.ny ? row_count(cstart, rp, y).places : 0, wsum, &total);
+  if (threadIdx.x == 0) rp.sums[c] = total;
+}
+
 // The scattered entries: id and slot of the particle at each position of
 // its cell range (two arrays, so that the rank's loop reads 4 bytes per
 // entry); entc = its cell.
@@ -273,13 +361,21 @@ struct Ent {
 };
 
 // Particles in slot order; with id_of null the particle in slot t has id t.
+// With row pieces (rp.tab set) the first row_chunks(ny) workgroups add up the
+// rows' places instead.
 __global__ __launch_bounds__(CS_THREADS) void k_cs_scatter(const uint32_t* __restrict__ key_by_slot,
                                                            const int32_t* __restrict__ id_of,
                                                            int n, const int* __restrict__ cstart,
                                                            int* __restrict__ count, Ent ent,
-                                                           uint32_t* __restrict__ entc, Halt hl) {
+                                                           uint32_t* __restrict__ entc, Halt hl,
+                                                           RowPieces rp) {
   if (hl.on()) return;
-  const int t = blockIdx.x * CS_THREADS + threadIdx.x;
+  const int rc = rp.tab ? row_chunks(rp.ny) : 0;
+  if ((int)blockIdx.x < rc) {
+    row_sums_block<CS_THREADS>(cstart, rp, blockIdx.x);
+    return;
+  }
+  const int t = ((int)blockIdx.x - rc) * CS_THREADS + threadIdx.x;
   const bool valid = t < n;
   const uint32_t c = valid ? key_by_slot[t] : 0xffffffffu;
   const WaveRun r = wave_run(c, valid);
@@ -293,134 +389,101 @@ __global__ __launch_bounds__(CS_THREADS) void k_cs_scatter(const uint32_t* __res
   entc[pos] = c;
 }
 
-// Pieces of the cell rows, for the gathers that give each workgroup a run of
-// consecutive sorted positions of one row: the sorted range of row y,
-// [cstart[y nx], cstart[(y+1) nx]), cut into runs of PIECE positions from its
-// start (the last one shorter).  tab[b] is all that workgroup b of a gather
-// needs to begin: its particles [O0, O1) of row cy and the three ranges of
-// sorted positions that hold their candidates, so that one load stands
-// between the launch and the filling of the tile (a chain of five before, a
-// microsecond each for every workgroup).
-//
-// tab[0 .. ny) hold the parts cut off the rows' pieces: above a tank's free
-// surface a row holds wall particles on either side only, and the row below
-// everything between them, so that a piece over the gap needs more records
-// than a gather's tile holds and its workgroup runs on the direct path, as
-// long as a whole launch of the others (FP32 force of the 111,119-particle
-// dam break: 28.6 us, 12.8 without; density 20.5 and 14.5).  A piece of more
-// than GAP_SPAN cells whose three rows hold more than GAP_RECORDS particles is
-// therefore cut at the middle of its cells, at most one of each row.
-//
-// tab[ny .. ny + slots) hold the pieces: the first count of them, dealt so
-// that the workgroups of one XCD take one contiguous share (neighbouring
-// pieces, which stage the same rows, then share an L2); the others are empty.
-// slots = n / PIECE + ny bounds the count.
-constexpr int PIECE = 128;
-constexpr int GAP_SPAN = 40;      // a full piece of 2h cells spans about 20
-constexpr int GAP_RECORDS = 592;  // the records of a gather's tile
-struct alignas(16) PieceRec {
-  int O0, O1, cy, total;  // total = rl[0] + rl[1] + rl[2]
-  int rs[3], rl[3];       // sorted start and length of rows cy-1, cy, cy+1
-  int x0, x1;             // cells of its first and last particle
-};
-struct RowPieces {
-  PieceRec* tab = nullptr;
-  int nx = 0, ny = 0, slots = 0;
-};
-
-// The workgroup that takes logical block L of count: workgroup b runs on XCD
-// b mod 8, and XCD x takes the x-th contiguous share of the blocks.
-__device__ __forceinline__ int share_slot(int count, int L) {
-  constexpr int X = 8;
-  const int q = count / X, r = count - q * X;
-  if (L < r * (q + 1)) return (L % (q + 1)) * X + L / (q + 1);
-  const int m = L - r * (q + 1);
-  return (m % q) * X + r + m / q;
-}
-
-// Workgroup wg of a grid of row_blocks() lists the pieces of rows
-// wg ROWS_PER_WG .., one wavefront per row and one lane per piece (a lane that
-// walked a row's pieces itself waited for the keys of each in turn: 32 us for
-// a 17 us reorder).  It counts the pieces of all rows itself, so the table
-// needs neither atomics nor a cleared counter.  keys: the cell of every sorted
-// position.
+// Workgroup wg of a grid of nwg = row_blocks() lists the pieces of its share of
+// the rows, one wavefront per row and one lane per piece (a lane that walked a
+// row's pieces itself waited for the keys of each in turn: 32 us for a 17 us
+// reorder).  rp.sums are those of all chunks, so the table needs neither atomics
+// nor a cleared counter.  keys: the cell of every sorted position.
 constexpr int ROWS_PER_WG = 4;
+constexpr int ROW_WGS = 1024;  // at most; above 4096 rows a wavefront takes several
 template <int THREADS>
 __device__ __forceinline__ void row_pieces_block(const int* __restrict__ cstart,
                                                  const uint32_t* __restrict__ keys,
                                                  const RowPieces& rp, int wg, int nwg) {
   static_assert(THREADS == 64 * ROWS_PER_WG, "one wavefront per row");
+  static_assert(THREADS == ROW_CHUNK, "one lane per row of a chunk");
   __shared__ int wsum[THREADS / 64];
   const int nx = rp.nx, ny = rp.ny;
-  const int y0 = wg * ROWS_PER_WG;
-  auto count = [&](int y) { return (cstart[(y + 1) * nx] - cstart[y * nx] + PIECE - 1) / PIECE; };
+  const int per = (ny + nwg * ROWS_PER_WG - 1) / (nwg * ROWS_PER_WG);  // rows of a wavefront
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int y0 = (wg * ROWS_PER_WG + w) * per, y1 = min(y0 + per, ny);
+  // the places before the workgroup's first row, and all
+  const int first = min(wg * ROWS_PER_WG * per, ny), c0 = first / ROW_CHUNK;
   int before = 0, all = 0;
-  for (int y = threadIdx.x; y < ny; y += THREADS) {
-    const int c = count(y);
-    all += c;
-    before += y < y0 ? c : 0;
+  for (int c = threadIdx.x; c < row_chunks(ny); c += THREADS) {
+    const int p = rp.sums[c];
+    all += p;
+    before += c < c0 ? p : 0;
   }
+  const int yc = c0 * ROW_CHUNK + (int)threadIdx.x;
+  if (yc < first) before += row_count(cstart, rp, yc).places;
   int base, total;
   block_exclusive_scan<THREADS>(before, wsum, &base);
   __syncthreads();  // wsum is reused
   block_exclusive_scan<THREADS>(all, wsum, &total);
-  PieceRec* slots = rp.tab + ny;
+  PieceRec* slots = rp.tab;
   for (int s = total + wg * THREADS + (int)threadIdx.x; s < rp.slots; s += nwg * THREADS)
     slots[s] = PieceRec{};
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int y = y0 + w;
-  if (y >= ny) return;
-  for (int r = y0; r < y; ++r) base += count(r);
-  const int a = cstart[y * nx], b = cstart[(y + 1) * nx];
-  const int np = (b - a + PIECE - 1) / PIECE;
-  // the rows' ranges of the particles [p, e) in cells x0 .. x1
-  auto make = [&](int p, int e, int x0, int x1) {
-    PieceRec r{};
-    const int lo = x0 > 0 ? x0 - 1 : 0, hi = (x1 + 1 < nx ? x1 + 1 : nx - 1) + 1;
-    r.O0 = p;
-    r.O1 = e;
-    r.cy = y;
-    r.x0 = x0;
-    r.x1 = x1;
+  // ... and before the wavefront's
+  int mine = 0;
+  for (int y = first + lane; y < min(y0, ny); y += 64) mine += row_count(cstart, rp, y).places;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int ry = y - 1 + k;
-      if (ry >= 0 && ry < ny) {
-        r.rs[k] = cstart[ry * nx + lo];
-        r.rl[k] = cstart[ry * nx + hi] - r.rs[k];
+  for (int d = 32; d > 0; d >>= 1) mine += __shfl_xor(mine, d, 64);
+  base += mine;
+  for (int y = y0; y < y1; ++y) {
+    const RowCount row = row_count(cstart, rp, y);
+    const int a = row.a, b = row.b;
+    // the rows' ranges of the particles [p, e) in cells x0 .. x1
+    auto make = [&](int p, int e, int x0, int x1) {
+      PieceRec r{};
+      const int lo = x0 > 0 ? x0 - 1 : 0, hi = (x1 + 1 < nx ? x1 + 1 : nx - 1) + 1;
+      r.O0 = p;
+      r.O1 = e;
+      r.cy = y;
+      r.x0 = x0;
+      r.x1 = x1;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int ry = y - 1 + k;
+        if (ry >= 0 && ry < ny) {
+          r.rs[k] = cstart[ry * nx + lo];
+          r.rl[k] = cstart[ry * nx + hi] - r.rs[k];
+        }
+        r.total += r.rl[k];
       }
-      r.total += r.rl[k];
-    }
-    return r;
-  };
-  bool found = false;
-  for (int j0 = 0; j0 < np; j0 += 64) {
-    const int p = a + (j0 + lane) * PIECE;
-    int m = 0;
-    PieceRec rec{}, cut{};
-    if (p < b) {
-      const int e = min(p + PIECE, b);
-      const int x0 = (int)keys[p] - y * nx, x1 = (int)keys[e - 1] - y * nx;
-      rec = make(p, e, x0, x1);
-      if (!found && x1 - x0 > GAP_SPAN && rec.total > GAP_RECORDS) {
-        m = cstart[y * nx + (x0 + x1 + 1) / 2];
-        if (m > p && m < e)
-          cut = make(m, e, (int)keys[m] - y * nx, x1);
-        else
-          m = 0;
+      return r;
+    };
+    bool found = false;
+    for (int j0 = 0; j0 < row.pieces; j0 += 64) {
+      const int p = a + (j0 + lane) * PIECE;
+      int m = 0;
+      PieceRec rec{}, cut{};
+      if (p < b) {
+        const int e = min(p + PIECE, b);
+        const int x0 = (int)keys[p] - y * nx, x1 = (int)keys[e - 1] - y * nx;
+        rec = make(p, e, x0, x1);
+        if (!found && x1 - x0 > GAP_SPAN && rec.total > GAP_RECORDS) {
+          m = cstart[y * nx + (x0 + x1 + 1) / 2];
+          if (m > p && m < e)
+            cut = make(m, e, (int)keys[m] - y * nx, x1);
+          else
+            m = 0;
+        }
       }
-    }
-    const uint64_t cutters = __ballot(m != 0);
-    if (cutters && !found) {
-      found = true;
-      if (lane == __builtin_ctzll(cutters)) {
-        rp.tab[y] = cut;
-        rec = make(p, m, (int)keys[p] - y * nx, (int)keys[m - 1] - y * nx);
+      const uint64_t cutters = __ballot(m != 0);
+      if (cutters && !found) {
+        found = true;
+        if (lane == __builtin_ctzll(cutters)) {  // rec.total > GAP_RECORDS: the row has the place
+          slots[share_slot(total, base + row.pieces)] = cut;
+          rec = make(p, m, (int)keys[p] - y * nx, (int)keys[m - 1] - y * nx);
+        }
       }
+      if (p < b) slots[share_slot(total, base + j0 + lane)] = rec;
     }
-    if (p < b) slots[share_slot(total, base + j0 + lane)] = rec;
+    if (!found && row.places > row.pieces && lane == 0)
+      slots[share_slot(total, base + row.pieces)] = PieceRec{};
+    base += row.places;
   }
-  if (!found && lane == 0) rp.tab[y] = PieceRec{};
 }
 
 // Where the particle of position p of a scattered cell range goes: its rank

@@ -185,13 +185,15 @@ __device__ __forceinline__ void ghost_slot(const St<R>& A, St<R>& Bs, const KPar
   G.gpid[t] = A.id[ps];
 }
 
-// A reorder kernel launched with row pieces (rp.tab set; cell_start
-// written by the sort) has row_blocks(rp) extra workgroups in front, one
-// wavefront per cell row, which list the rows' pieces (they run beside the
+// A reorder kernel launched with row pieces (rp.tab set; cell_start and the
+// rows' sums written by the sort) has row_blocks(rp) extra workgroups in front,
+// one wavefront per cell row, which list the rows' pieces (they run beside the
 // first particles' workgroups).  Returns true in those; *t is the position
 // of the lane in the others.
 __host__ __device__ inline int row_blocks(const RowPieces& rp) {
-  return rp.tab ? (rp.ny + ROWS_PER_WG - 1) / ROWS_PER_WG : 0;
+  if (!rp.tab) return 0;
+  const int b = (rp.ny + ROWS_PER_WG - 1) / ROWS_PER_WG;
+  return b < ROW_WGS ? b : ROW_WGS;
 }
 __device__ __forceinline__ bool reorder_row_pieces(const int* __restrict__ cstart,
                                                    const uint32_t* __restrict__ keys,

@@ -549,7 +549,13 @@ __device__ __forceinline__ void for_segment(const KParams& K, const Segment& g,
   done(i, i < g.O1);
 }
 
-// The row pieces on their own (after a sort that does not build them).
+// The row pieces on their own (after a sort that does not build them): first the
+// chunks' sums, then the table.
+__global__ __launch_bounds__(ROW_CHUNK) void k_row_sums(const int* __restrict__ cstart, RowPieces rp,
+                                                        Halt hl) {
+  if (hl.on()) return;
+  row_sums_block<ROW_CHUNK>(cstart, rp, blockIdx.x);
+}
 __global__ __launch_bounds__(BLOCK) void k_row_pieces(const int* __restrict__ cstart,
                                                       const uint32_t* __restrict__ skey,
                                                       RowPieces rp, Halt hl) {
