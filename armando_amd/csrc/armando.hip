@@ -331,7 +331,9 @@ template <typename R> St<R>& stB(arm_ctx* c);
 template <> St<double>& stB<double>(arm_ctx* c) { return c->B64; }
 template <> St<float>& stB<float>(arm_ctx* c) { return c->B32; }
 
-// Swaps the active state buffer with the other one.
+// Swaps the four fields that the corrector of a run's 2D step moves: they were
+// written to the inactive state (moved_of), all others of the particle, rates and
+// order included, are in the active one and stay.
 template <typename R> void swap_moved(St<R>& A, St<R>& B) {
   std::swap(A.xy, B.xy);
   std::swap(A.v, B.v);
@@ -339,8 +341,9 @@ template <typename R> void swap_moved(St<R>& A, St<R>& B) {
   std::swap(A.u, B.u);
 }
 
-// Undoes the swaps of one step of a run: the reorder's of the two states and,
-// in 2D, the corrector's of the moved fields.
+// Undoes the swaps of one step of a run: the reorder's of the two states and, in
+// 2D, the corrector's of the moved fields, which between them leave the moved
+// fields where they were and the others swapped.
 void unstep_state(arm_ctx* c) {
   if (c->prm.dim != 3) {
     if (c->prm.precision == ARM_FP32)
