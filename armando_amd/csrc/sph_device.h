@@ -405,8 +405,15 @@ __device__ __forceinline__ void next_word(const uint32_t& m, const uint32_t& nz,
 }
 template <typename R> constexpr int acc_words() { return sizeof(R) == 4 ? 2 : 1; }
 
-// 1/x: the FP32 form's from the hardware's reciprocal (1 ulp) and one Newton
-// step, which rounds it as well as a division in a third of the instructions.
+// 1/x: the FP32 form's from the hardware's reciprocal and one Newton step, a third
+// of a division's instructions.  For x and 1/x normal it is the division's value:
+// the hardware's is within 0.882 ulp, the step's rounding error is then the last
+// rounding's (0.500001 ulp for any start within an ulp), and on every one of the
+// 2^23 mantissas, at seven exponents from 2^-120 to 2^120, it gave the correctly
+// rounded 1/x.  For x zero, infinite or subnormal it is NaN, where a division
+// gives infinity or zero; of what the adjoint's pairs divide by, Q_i + Q_j and
+// r^2 + (h eta)^2 are normal, and q = r / h is zero only for coincident particles,
+// whose term infinity 0 is NaN either way.
 __device__ __forceinline__ double rcp_n(double x) { return 1.0 / x; }
 __device__ __forceinline__ float rcp_n(float x) {
   const float y = __builtin_amdgcn_rcpf(x);
