@@ -409,18 +409,17 @@ __device__ __forceinline__ Local3 local3(const KParams& K, double4 q, int cx0, i
           (float)(q.z - (K.oz + (double)cz * K.cell))};
 }
 
-// Whether the particle lies within a few cells of the cell it is sorted into, so
-// that local3 and pre3f hold.  One outside the grid does not (arm_link_list sorts it into
-// cell 0 and returns ARM_ERR_DOMAIN; the gathers still run for a caller that goes
-// on): it takes the exact test of every candidate.
+// Whether a particle sorted into cell 0 lies in it or near it, so that local3 and
+// pre3f hold.  One outside the grid does not (arm_link_list sorts it into cell 0
+// and returns ARM_ERR_DOMAIN; the gathers still run for a caller that goes on):
+// it takes the exact test of every candidate.
 __device__ __forceinline__ bool local3_holds(const KParams& K, float4 q) {
   const float c = 2.f * K.cellf;
   return fabsf(q.x) <= c && fabsf(q.y) <= c && fabsf(q.z) <= c;
 }
 __device__ __forceinline__ bool local3_holds(const KParams& K, double4 q) {
-  const double x = q.x - K.ox, y = q.y - K.oy, z = q.z - K.oz;
-  return x >= -K.cell && x <= (K.nx + 1) * K.cell && y >= -K.cell && y <= (K.ny + 1) * K.cell &&
-         z >= -K.cell && z <= (K.nz + 1) * K.cell;
+  const double c = 2.0 * K.cell;
+  return fabs(q.x - K.ox) <= c && fabs(q.y - K.oy) <= c && fabs(q.z - K.oz) <= c;
 }
 
 // The 96-bit window [d, d + len) of the four words p of ch bits each
@@ -450,6 +449,72 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Sweeps that pretest3 makes of the lanes on.
+__device__ __forceinline__ int sweeps3(bool on, int cx, int row) {
+  int n = 0;
+  for (uint64_t todo = __ballot(on); todo; ++n) {
+    const int a = __builtin_ctzll(todo);
+    const int row0 = __builtin_amdgcn_readlane(row, a), cx0 = __builtin_amdgcn_readlane(cx, a);
+    todo &= ~__ballot(row == row0 && cx - cx0 <= P3_SPAN);
+  }
+  return n;
+}
+
+// pretest3 lane by lane: the exact test of a lane's own candidates, NB at a time (in
+// FP64 two: eight double4 loads of which one is a candidate took 52 us instead of 42
+// on the thinnest spray below).  For wavefronts whose particles lie in many cell rows
+// and have few candidates: spray, thin sheets, narrow channels.  pretest3 makes a
+// sweep of nine rows for every row and 13 cells of it that the wavefront touches, one
+// after the other; here they run side by side.  Measured, density pass of 300,000
+// particles, FP32 (FP64), us: a sweep adds 10 (12), a hundred candidates 20 (35),
+// so that lanes take less below 10 + 50 (10 + 45) candidates a sweep, FEW3:
+//   spray, 0.3 / 1 / 3 per cell   sweeps 212 / 108 / 81 (239 / 124 / 97)
+//                                 lanes 31 / 39 / 63 (42 / 57 / 89)
+//   sheets of 2 / 3 particles     sweeps 125 / 125 (154 / 159), lanes 71 / 101 (116 / 148)
+// Dense fluid has 490 candidates and one to three sweeps.
+constexpr int FEW3_MAX = 288;  // beyond it no count of sweeps is looked for
+template <typename R> struct Few3;
+template <> struct Few3<float> { static constexpr int base = 10, sweep = 50, batch = 4; };
+template <> struct Few3<double> { static constexpr int base = 10, sweep = 45, batch = 2; };
+template <int NS, typename R>
+__device__ __forceinline__ void pretest3_lanes(const St3<R>& S, const KParams& K, int s0, int i,
+                                               bool on, const Rows9& rw,
+                                               int (*__restrict__ lt)[64],
+                                               uint32_t (*__restrict__ lw)[64]) {
+  constexpr int NB = Few3<R>::batch;
+  const int lane = threadIdx.x & 63;
+  const auto pi = load_pos3(S, i);
+  const R cut2 = cutoff2<R>(K);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {  // the rows' bounds, for a loop that is not unrolled
+    if (k % NS != s0) continue;
+    lt[k][lane] = rw.t0[k];
+    lw[3 * k][lane] = (uint32_t)rw.t1[k];
+  }
+  for (int k = s0; k < 9; k += NS) {
+    const int ky = (k * 11) >> 5;  // k / 3 for k < 9
+    const R uy = row_u3<R>(K, 1 - (k - 3 * ky)), uz = row_u3<R>(K, 1 - ky);
+    const int t0 = lt[k][lane], t1 = on ? (int)lw[3 * k][lane] : t0;
+#pragma unroll
+    for (int q = 0; q < M3_WORDS; ++q) {
+      const int c0 = t0 + 32 * q, end = min(c0 + 32, t1);
+      uint32_t m = 0u;
+      for (int c = c0; c < end; c += NB) {
+        uint32_t bb = 0u;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const int t = min(c + b, end - 1);
+          R dx, dy, dz;
+          const R r2 = delta3(pi, load_pos3(S, t), K, uy, uz, dx, dy, dz);
+          bb |= (r2 < cut2 && c + b < end && t != i ? 1u : 0u) << b;
+        }
+        m |= bb << (c - c0);
+      }
+      if (on) lw[3 * k + q][lane] = m;
+    }
+  }
 }
 
 // Mask words lw[3k + q][lane] of the nine rows (wavefront s of S: rows k = s
@@ -618,10 +683,22 @@ __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(sizeof(
   const uint32_t key = skey[i];
   const int row = (int)(key / (uint32_t)K.nx), cx = (int)key - row * K.nx;
   const Rows9 rw = rows3_of(K, key, cstart);
-  bool ok = local3_holds(K, pos_rec3(S, i));
+  bool ok = key != 0u || local3_holds(K, pos_rec3(S, i));
+  int candidates = 0;
 #pragma unroll
-  for (int k = 0; k < 9; ++k) ok = ok && rw.t1[k] - rw.t0[k] <= 32 * M3_WORDS;
-  pretest3<NS>(S, K, s0, i, valid && ok, cx, row, rw, L.rec[s0], L.lw);
+  for (int k = 0; k < 9; ++k) {
+    const int len = rw.t1[k] - rw.t0[k];
+    ok = ok && len <= 32 * M3_WORDS;
+    candidates += len;
+  }
+  const bool on = valid && ok;
+  // (unlikely: so that the registers of what follows stay with the sweeps)
+  auto none_has = [&](int c) { return __ballot(on && candidates >= c) == 0ull; };
+  if (__builtin_expect(none_has(FEW3_MAX) && none_has(Few3<R>::base + Few3<R>::sweep *
+                                                      sweeps3(on, cx, row)), 0))
+    pretest3_lanes<NS>(S, K, s0, i, on, rw, L.lt, L.lw);
+  else
+    pretest3<NS>(S, K, s0, i, on, cx, row, rw, L.rec[s0], L.lw);
   __syncthreads();
   uint32_t(*lw)[64] = L.lw;
   int(*lt)[64] = L.lt;
@@ -680,7 +757,7 @@ __global__ __launch_bounds__(64 * NS) __attribute__((amdgpu_waves_per_eu(sizeof(
       if (!in0) atomicAnd(&lw[w0][lane], ~(1u << b0));
       if (two && !in1) atomicAnd(&lw[wc][lane], ~(1u << b1));
     }
-  } else if (valid) {
+  } else if (__builtin_expect(valid, 0)) {
     for (int k = 0; k < 9; ++k) {
       const int t0 = rw.t0[k], t1 = rw.t1[k];
       const R uy = row_u3<R>(K, 1 - k % 3), uz = row_u3<R>(K, 1 - k / 3);
