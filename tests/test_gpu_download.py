@@ -5,6 +5,7 @@ for bit, nothing written past a field's end.  The downloads unsort into the
 inactive state's arrays: steps after them equal those of a run that was never
 looked at."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -67,3 +68,32 @@ def test_interleaved_downloads(name, prec):
         assert np.array_equal(v, sim.state()[k]), k
     sim.close()
     plain.close()
+
+
+@pytest.mark.parametrize("prec", [cases.FP64, cases.FP32])
+@pytest.mark.parametrize("name", ["2d", "3d"])
+def test_arrays_of_a_small_download(name, prec):
+    """state() and rates() fetch a small state in fewer copies than fields: they
+    take at most 1.1 of arm_download's five.  The arrays are the caller's own."""
+    c = make(name, prec)
+    sim = armando_amd.Simulation(c)
+    sim.time_integration(1, 2)
+    buf = {k: np.empty((sim.dim if k in VECTORS else 1) * sim.n) for k in STATE}
+    ptr = [buf[k].ctypes.data_as(C.POINTER(C.c_double)) for k in STATE]
+
+    def best(call):
+        t = []
+        for _ in range(200):
+            t0 = time.perf_counter()
+            call()
+            t.append(time.perf_counter() - t0)
+        return 1e6 * min(t)
+
+    us = {"state": best(sim.state), "rates": best(sim.rates),
+          "arm_download": best(lambda: sim.L.arm_download(sim.ctx, *ptr))}
+    print(f"[gpu] small download {name} n={sim.n} prec={prec}: {us}", flush=True)
+    for v in {**sim.state(), **sim.rates()}.values():
+        assert v.flags.owndata and v.flags.writeable and v.flags.c_contiguous
+    sim.close()
+    assert us["state"] <= 1.1 * us["arm_download"]
+    assert us["rates"] <= 1.1 * us["arm_download"]
