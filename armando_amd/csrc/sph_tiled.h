@@ -25,22 +25,30 @@
 namespace arm {
 
 // ---- LDS tiles ------------------------------------------------------------
-// Every tile has TPAD spare records after CAP so that the eight-wide
-// neighbour test may read up to seven records past a row's end (their bits
-// are masked off).  In the FP32 form a record keeps the cell column as a
+// The eight-wide neighbour test may read up to seven records past a row's end
+// (their bits are masked off).  After the last row of a full tile these lie in
+// the array that follows in the tile, so what the test reads is never its last
+// member.  In the FP32 form a record keeps the cell column as a
 // float, and the cell-row difference of a candidate row is the constant
 // 1 - k of row k of the segment, so
 //   dx = (off_i.x - off_j.x) + (cx_i - cx_j) cell
 //   dy = (off_i.y - off_j.y) + (1 - k) cell
 // are the same operations, with the same roundings, as delta() on PosF.
-constexpr int TPAD = 8;
-// Records of a tile: a piece's three rows hold about 3 x 140 on the dam-break
-// lattice, 584 at most.  The FP32 force gather's 18.9 KB let eight workgroups
-// share a CU; with the physical viscosity's 52 bytes (FP32) or 88 (FP64) a
-// record, runs of 32 or 16 cells with smaller tiles were the faster form until
-// the loads of the prologue overlapped (heated channel of 2 million, force with
-// the corrector: FP32 189 us on runs, 182 on pieces; FP64 377 and 369).
-constexpr int CAP = GAP_RECORDS;
+// Records of a tile.  A piece's three rows hold about 3 x 140 on the dam-break
+// lattice, 584 at most, but up to 640 where a row has fewer particles than its
+// neighbours (h = 1.7 or 1.8 dx on a lattice); a piece of more runs on the direct
+// path.  FP32: 640 (ten workgroups a CU in the density pass, seven in the force),
+// and 592 with the physical viscosity (five) and in the hot force gather, whose
+// 18.9 KB let eight share a CU.  FP64: 600 (seven and four).  With 592 in all of
+// them the passes at h = 1.8 dx, 350,000 particles, took in FP64 92 us (density) and
+// 197 (force with the corrector), now 83 and 165; in FP32 64 (density), now 55.
+// With the physical viscosity runs of 32 or 16 cells with smaller tiles were the
+// faster form until the loads of the prologue overlapped (heated channel of 2
+// million, force with the corrector: FP32 189 us on runs, 182 on pieces; FP64 377
+// and 369).
+template <typename R, bool VI = false> constexpr int tile_cap() {
+  return sizeof(R) == 8 ? 600 : (VI ? GAP_RECORDS : 640);
+}
 
 // Byte offset 4 l of a 4-byte LDS record.  Computed out of the compiler's
 // sight: otherwise it derives this address from the 16-byte records' l << 4
@@ -77,8 +85,8 @@ __device__ __forceinline__ void tile_delta(const KParams& K, const LaneF& p, flo
 template <typename R> struct DensTile;
 template <> struct DensTile<float> {
   // the neighbour test reads one 16-byte record per candidate
-  float4 a[CAP + TPAD];  // offx, offy, cell column as float, vx
-  float vy[CAP + TPAD];
+  float4 a[tile_cap<float>()];  // offx, offy, cell column as float, vx
+  float vy[tile_cap<float>()];
   struct Raw {
     float2 o, v;
     uint32_t c;
@@ -104,7 +112,7 @@ template <> struct DensTile<float> {
   }
 };
 template <> struct DensTile<double> {
-  double2 x[CAP + TPAD], v[CAP + TPAD];
+  double2 x[tile_cap<double>()], v[tile_cap<double>()];
   struct Raw {
     double2 x, v;
   };
@@ -138,8 +146,8 @@ template <> struct DensTile<double> {
 constexpr int FIX = 4096;
 using s16x2 = __attribute__((ext_vector_type(2))) short;
 
-struct PreTile {
-  uint32_t p[CAP + TPAD];
+template <typename R> struct PreTile {
+  uint32_t p[tile_cap<R>()];
   __device__ __forceinline__ void put(int l, const KParams& K,
                                       const DensTile<float>::Raw& r) {
     const uint32_t c = r.c;
@@ -165,7 +173,7 @@ template <typename R, bool VI> struct TauTile {
   __device__ __forceinline__ Tau3<R> get(int) const { return Tau3<R>{}; }
 };
 template <> struct TauTile<float, true> {
-  float4 w[CAP];
+  float4 w[tile_cap<float, true>()];
   using Raw = float4;
   static __device__ __forceinline__ Raw load(const St<float>& S, int t) {
     return reinterpret_cast<const float4*>(S.tau)[t];
@@ -179,8 +187,8 @@ template <> struct TauTile<float, true> {
   }
 };
 template <> struct TauTile<double, true> {
-  double2 w01[CAP];
-  double w2[CAP];
+  double2 w01[tile_cap<double, true>()];
+  double w2[tile_cap<double, true>()];
   struct Raw {
     double xx, yy, xy;
   };
@@ -209,9 +217,10 @@ __device__ __forceinline__ void own_tau(const St<R>& S, ForceOwn<R>& o, int i, c
 
 template <typename R, bool VI = false> struct ForceTile;
 template <bool VI> struct ForceTile<float, VI> {
-  float4 a[CAP + TPAD];  // offx, offy, vx, vy
-  float4 b[CAP + TPAD];  // Q = 1/rho, A = p/rho, psi, u
-  float cx[CAP + TPAD];  // cell column as float
+  static constexpr int CAP = tile_cap<float, VI>();
+  float cx[CAP];  // cell column as float
+  float4 a[CAP];  // offx, offy, vx, vy
+  float4 b[CAP];  // Q = 1/rho, A = p/rho, psi, u
   TauTile<float, VI> tw;
   struct Raw {
     float2 o, v;
@@ -263,7 +272,8 @@ template <bool VI> struct ForceTile<float, VI> {
   }
 };
 template <bool VI> struct ForceTile<double, VI> {
-  double2 x[CAP + TPAD], v[CAP + TPAD], rp[CAP + TPAD], pu[CAP + TPAD];  // rp = (Q, A), pu = (psi, u)
+  static constexpr int CAP = tile_cap<double, VI>();
+  double2 x[CAP], v[CAP], rp[CAP], pu[CAP];  // rp = (Q, A), pu = (psi, u)
   TauTile<double, VI> tw;
   struct Raw {
     double2 x, v;
@@ -316,7 +326,7 @@ template <bool VI> struct ForceTile<double, VI> {
 // Positions, velocities and Q = 1/rho for the shear tensor pass.
 template <typename R> struct TensTile {
   DensTile<R> d;
-  R q[CAP + TPAD];
+  R q[tile_cap<R>()];
   struct Raw {
     typename DensTile<R>::Raw d;
     R rho;
@@ -664,7 +674,8 @@ __device__ __forceinline__ void walk_rows(uint32_t m0, uint32_t m1, uint32_t m2,
 // K.fix2, a bound on (2h)^2 in units of the fixed-point positions (own: the
 // lane's) that covers their rounding; the survivors (about one in two thousand
 // too many) take the exact test in the walk.
-__device__ __forceinline__ uint32_t row_mask_pre(const KParams& K, const PreTile& P, s16x2 own,
+template <typename R>
+__device__ __forceinline__ uint32_t row_mask_pre(const KParams& K, const PreTile<R>& P, s16x2 own,
                                                  int l0, int len, int self) {
   const int bound = -K.fix2;
   uint32_t m = 0;
@@ -691,7 +702,7 @@ __device__ __forceinline__ uint32_t row_mask_pre(const KParams& K, const PreTile
 // Taken by dens_walk for a particle with a row of more than 32 candidates.
 template <typename R, bool SUM, typename LP, typename V>
 __device__ __forceinline__ void dens_walk_rows(const KParams& K, const Segment& g, const LaneRows& lr,
-                                               const DensTile<R>& T, const PreTile& P,
+                                               const DensTile<R>& T, const PreTile<R>& P,
                                                const LP& pi, const V& vi, int i, DensOwn<R>& o,
                                                uint32_t* rm, bool* ok) {
   const int self = g.lo[1] + (i - g.rs[1]);
@@ -734,7 +745,7 @@ __device__ __forceinline__ void dens_walk_rows(const KParams& K, const Segment& 
 // as for_neighbours; the exact masks in rm.
 template <typename R, bool SUM, typename LP, typename V>
 __device__ __forceinline__ void dens_walk(const KParams& K, const Segment& g, const LaneRows& lr,
-                                          const DensTile<R>& T, const PreTile& P,
+                                          const DensTile<R>& T, const PreTile<R>& P,
                                           const LP& pi, const V& vi, int i, DensOwn<R>& o,
                                           uint32_t* rm, bool* ok) {
   const int self = g.lo[1] + (i - g.rs[1]);
@@ -816,12 +827,16 @@ __global__ __launch_bounds__(PIECE) __attribute__((amdgpu_waves_per_eu(sizeof(R)
                                                        const uint32_t* __restrict__ skey,
                                                        const int* __restrict__ cstart, SegArg sa,
                                                        uint4* __restrict__ nbm) {
-  __shared__ DensTile<R> T;
-  __shared__ PreTile P;
+  __shared__ struct {
+    PreTile<R> P;
+    DensTile<R> T;
+  } L;
+  PreTile<R>& P = L.P;
+  DensTile<R>& T = L.T;
   const Segment g = segment_of(sa);
   if (halted(K) || g.O0 >= g.O1) return;
   const Wrap<PER> W(K, g, cstart);
-  const bool tiled = g.total + W.total <= CAP;
+  const bool tiled = g.total + W.total <= tile_cap<R>();
   using Raw = typename DensTile<R>::Raw;
   int id = 0;
   R rho = (R)0;
@@ -869,7 +884,7 @@ __global__ __launch_bounds__(PIECE) void k_tensor_tiled(St<R> S, KParams K,
   const Segment g = segment_of(sa);
   if (halted(K) || g.O0 >= g.O1) return;
   const Wrap<PER> W(K, g, cstart);
-  const bool tiled = g.total + W.total <= CAP;
+  const bool tiled = g.total + W.total <= tile_cap<R>();
   using Raw = typename TensTile<R>::Raw;
   uint4 nm;
   for_segment<4, Raw>(
@@ -925,7 +940,7 @@ __global__ __launch_bounds__(PIECE) void k_force_tiled(St<R> S, KParams K,
   const Segment g = segment_of(sa);
   if (halted(K) || g.O0 >= g.O1) return;
   const Wrap<PER> W(K, g, cstart);
-  const bool tiled = g.total + W.total <= CAP;
+  const bool tiled = g.total + W.total <= tile_cap<R, VI>();
   using Raw = typename ForceTile<R, VI>::Raw;
   uint4 nm;
   int id = 0;
@@ -987,6 +1002,7 @@ __global__ __launch_bounds__(PIECE) void k_force_tiled(St<R> S, KParams K,
 // The smaller tile lets eight workgroups share a CU.  Particles without
 // complete masks take the direct path.
 struct HotForceTile {
+  static constexpr int CAP = GAP_RECORDS;
   float4 a[CAP];  // offx, offy, vx, vy
   float4 b[CAP];  // Q = 1/rho, A = p/rho, psi, u
   struct Raw {
@@ -1058,7 +1074,7 @@ __global__ __launch_bounds__(PIECE) __attribute__((amdgpu_waves_per_eu(4))) void
   __shared__ HotForceTile T;
   const Segment g = segment_of(sa);
   if (halted(K) || g.O0 >= g.O1) return;
-  const bool tiled = g.total <= CAP;
+  const bool tiled = g.total <= HotForceTile::CAP;
   const int i = g.O0 + (int)threadIdx.x;
   const int ic = min(i, g.O1 - 1);
   const uint32_t key = skey[ic];
