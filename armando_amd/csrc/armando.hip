@@ -68,7 +68,7 @@ struct arm_ctx {
   uint4* nbm = nullptr;
   // 2D tiled gathers: the row pieces of the current order (RowPieces)
   PieceRec* pieces = nullptr;
-  int* row_sums = nullptr;
+  uint64_t* row_sums = nullptr;
   int piece_slots = 0;  // of the table last built
   bool pieces_valid = false;
   // deposition heat source (arm_set_deposition): the map on the device, the
