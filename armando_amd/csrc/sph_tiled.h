@@ -215,12 +215,25 @@ __device__ __forceinline__ void own_tau(const St<R>& S, ForceOwn<R>& o, int i, c
   o.tds = S.tau[4 * (size_t)i + 3];
 }
 
+// The FP32 records: offx, offy, vx, vy; Q = 1/rho, A = p/rho, psi, u; cell column
+// as float.  With the shear tensor behind them the columns come last, with the spare records
+// of their own (first, as without it: force of 100,000 particles 56 -> 58 us).
+template <bool VI> struct ForceRecs {
+  float cx[tile_cap<float>()];
+  float4 a[tile_cap<float>()];
+  float4 b[tile_cap<float>()];
+};
+template <> struct ForceRecs<true> {
+  float4 a[tile_cap<float, true>() + 8];
+  float4 b[tile_cap<float, true>() + 8];
+  float cx[tile_cap<float, true>() + 8];
+};
+
 template <typename R, bool VI = false> struct ForceTile;
-template <bool VI> struct ForceTile<float, VI> {
-  static constexpr int CAP = tile_cap<float, VI>();
-  float cx[CAP];  // cell column as float
-  float4 a[CAP];  // offx, offy, vx, vy
-  float4 b[CAP];  // Q = 1/rho, A = p/rho, psi, u
+template <bool VI> struct ForceTile<float, VI> : ForceRecs<VI> {
+  using ForceRecs<VI>::a;
+  using ForceRecs<VI>::b;
+  using ForceRecs<VI>::cx;
   TauTile<float, VI> tw;
   struct Raw {
     float2 o, v;
