@@ -174,8 +174,9 @@ template <typename R> int alloc_state(arm_ctx* c, St<R>& S, int cap) {
   AL(psi, cap);
   AL(drho, cap);
   AL(du, cap);
-  AL(a, 2 * (size_t)cap);  // one block with av (out_scratch)
-  S.av = S.a + cap;
+  const size_t lines = ((size_t)cap + 31) / 32 * 32;  // av at the start of a cache line
+  AL(a, lines + cap);  // one block with av (out_scratch)
+  S.av = S.a + lines;
   AL(divv, cap);
   AL(rho_min, cap);
   AL(u_min, cap);

@@ -425,6 +425,52 @@ __device__ __forceinline__ void row_pieces_block(const int* __restrict__ cstart,
   const int per = (ny + nwg * ROWS_PER_WG - 1) / (nwg * ROWS_PER_WG);  // rows of a wavefront
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int y0 = (wg * ROWS_PER_WG + w) * per, y1 = min(y0 + per, ny);
+  // the ranges of rows y-1 .. y+1 of the particles [p, e) of row y in cells x0 .. x1
+  auto make = [&](int y, int p, int e, int x0, int x1) {
+    PieceRec r{};
+    const int lo = x0 > 0 ? x0 - 1 : 0, hi = (x1 + 1 < nx ? x1 + 1 : nx - 1) + 1;
+    r.O0 = p;
+    r.O1 = e;
+    r.cy = y;
+    r.x0 = x0;
+    r.x1 = x1;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int ry = y - 1 + k;
+      if (ry >= 0 && ry < ny) {
+        r.rs[k] = cstart[ry * nx + lo];
+        r.rl[k] = cstart[ry * nx + hi] - r.rs[k];
+      }
+      r.total += r.rl[k];
+    }
+    return r;
+  };
+  // the lane's piece of the 64 from j0 on of row y, and where it would be cut (0: not)
+  struct Piece {
+    PieceRec rec;
+    int m;
+  };
+  auto piece = [&](int y, const RowCount& row, int j0) {
+    Piece q{};
+    const int p = row.a + (j0 + lane) * PIECE;
+    if (p < row.b) {
+      const int e = min(p + PIECE, row.b);
+      const int x0 = (int)keys[p] - y * nx, x1 = (int)keys[e - 1] - y * nx;
+      q.rec = make(y, p, e, x0, x1);
+      if (x1 - x0 > GAP_SPAN && q.rec.total > GAP_RECORDS) {
+        const int m = cstart[y * nx + (x0 + x1 + 1) / 2];
+        q.m = m > p && m < e ? m : 0;
+      }
+    }
+    return q;
+  };
+  // the first row's pieces, whose loads run beside the counting
+  RowCount row{};
+  Piece q{};
+  if (y0 < y1) {
+    row = row_count(cstart, rp, y0);
+    q = piece(y0, row, 0);
+  }
   // what comes before the workgroup's first row, and all
   const int first = min(wg * ROWS_PER_WG * per, ny), c0 = first / ROW_CHUNK;
   uint64_t before = 0, all = 0;
@@ -448,9 +494,9 @@ __device__ __forceinline__ void row_pieces_block(const int* __restrict__ cstart,
   __syncthreads();
   all = 0;
 #pragma unroll
-  for (int q = 0; q < ROWS_PER_WG; ++q) {
-    mine += part[0][q];
-    all += part[1][q];
+  for (int k = 0; k < ROWS_PER_WG; ++k) {
+    mine += part[0][k];
+    all += part[1][k];
   }
   const int total = (int)(uint32_t)all;
   int base = (int)(uint32_t)mine, parts = total + (int)(mine >> 32);  // the next places
@@ -458,59 +504,28 @@ __device__ __forceinline__ void row_pieces_block(const int* __restrict__ cstart,
   for (int s = total + (int)(all >> 32) + wg * THREADS + (int)threadIdx.x; s < rp.slots;
        s += nwg * THREADS)
     slots[s] = PieceRec{};
-  for (int y = y0; y < y1; ++y) {
-    const RowCount row = row_count(cstart, rp, y);
-    const int a = row.a, b = row.b;
-    // the rows' ranges of the particles [p, e) in cells x0 .. x1
-    auto make = [&](int p, int e, int x0, int x1) {
-      PieceRec r{};
-      const int lo = x0 > 0 ? x0 - 1 : 0, hi = (x1 + 1 < nx ? x1 + 1 : nx - 1) + 1;
-      r.O0 = p;
-      r.O1 = e;
-      r.cy = y;
-      r.x0 = x0;
-      r.x1 = x1;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const int ry = y - 1 + k;
-        if (ry >= 0 && ry < ny) {
-          r.rs[k] = cstart[ry * nx + lo];
-          r.rl[k] = cstart[ry * nx + hi] - r.rs[k];
-        }
-        r.total += r.rl[k];
-      }
-      return r;
-    };
+  for (int y = y0; y < y1;) {
     bool found = false;
     for (int j0 = 0; j0 < row.pieces; j0 += 64) {
-      const int p = a + (j0 + lane) * PIECE;
-      int m = 0;
-      PieceRec rec{}, cut{};
-      if (p < b) {
-        const int e = min(p + PIECE, b);
-        const int x0 = (int)keys[p] - y * nx, x1 = (int)keys[e - 1] - y * nx;
-        rec = make(p, e, x0, x1);
-        if (!found && x1 - x0 > GAP_SPAN && rec.total > GAP_RECORDS) {
-          m = cstart[y * nx + (x0 + x1 + 1) / 2];
-          if (m > p && m < e)
-            cut = make(m, e, (int)keys[m] - y * nx, x1);
-          else
-            m = 0;
-        }
-      }
-      const uint64_t cutters = __ballot(m != 0);
+      if (j0) q = piece(y, row, j0);
+      const uint64_t cutters = __ballot(q.m != 0);
       if (cutters && !found) {
         found = true;
         if (lane == __builtin_ctzll(cutters)) {  // rec.total > GAP_RECORDS: the row has the place
-          slots[parts] = cut;
-          rec = make(p, m, (int)keys[p] - y * nx, (int)keys[m - 1] - y * nx);
+          const PieceRec r = q.rec;
+          slots[parts] = make(y, q.m, r.O1, (int)keys[q.m] - y * nx, r.x1);
+          q.rec = make(y, r.O0, q.m, r.x0, (int)keys[q.m - 1] - y * nx);
         }
       }
-      if (p < b) slots[share_slot(total, base + j0 + lane)] = rec;
+      if (row.a + (j0 + lane) * PIECE < row.b) slots[share_slot(total, base + j0 + lane)] = q.rec;
     }
     if (!found && row.parts && lane == 0) slots[parts] = PieceRec{};
     base += row.pieces;
     parts += row.parts;
+    if (++y < y1) {
+      row = row_count(cstart, rp, y);
+      q = piece(y, row, 0);
+    }
   }
 }
 
