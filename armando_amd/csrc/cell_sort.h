@@ -352,8 +352,8 @@ __device__ __forceinline__ int share_slot(int count, int L) {
 // up before the table is made (beside the scatter), so that a workgroup of
 // row_pieces_block reads its chunk's rows and a word for each other chunk: with
 // every workgroup counting every row, ny^2 / 2 loads, the reorder of 2,400 particles
-// in 60,000 rows took 2,283 us (26 now; 8 in 48 rows of as many cells in all), that
-// of 1.2 million in 12,510 rows 154 us (40).
+// in 60,000 rows took 2,283 us (24 now; 8 in 48 rows of as many cells in all), that
+// of 1.2 million in 12,510 rows 154 us (39).
 template <int THREADS>
 __device__ __forceinline__ void row_sums_block(const int* __restrict__ cstart, const RowPieces& rp,
                                                int c) {
